@@ -24,13 +24,13 @@ OUT_DIR = os.path.join(HERE, "nanovllm", "_lib")
 LIB = os.path.join(OUT_DIR, "libqlinear.so")
 SEQMIX_LIB = os.path.join(OUT_DIR, "libseqmix.so")
 HYMIX_LIB = os.path.join(OUT_DIR, "libhymix.so")
-FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-fno-gpu-rdc"]
-# the packed-f32 VALU forms stay off in the newer library (plain f32 code only)
-NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# the packed-f32 VALU forms stay off (plain f32 code only): some of them have given wrong results on this hardware
+FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-fno-gpu-rdc", "-Xclang", "-target-feature", "-Xclang",
+         "-packed-fp32-ops"]
 TARGETS = {
     "qlinear": dict(src=CSRC, lib=LIB, header="qlinear.h", flags=FLAGS, obj=""),
-    "seqmix": dict(src=os.path.join(CSRC, "seqmix"), lib=SEQMIX_LIB, header="seqmix.h", flags=FLAGS + NO_PACKED_F32, obj="seqmix_"),
-    "hymix": dict(src=os.path.join(CSRC, "hymix"), lib=HYMIX_LIB, header="hymix.h", flags=FLAGS + NO_PACKED_F32, obj="hymix_"),
+    "seqmix": dict(src=os.path.join(CSRC, "seqmix"), lib=SEQMIX_LIB, header="seqmix.h", flags=FLAGS, obj="seqmix_"),
+    "hymix": dict(src=os.path.join(CSRC, "hymix"), lib=HYMIX_LIB, header="hymix.h", flags=FLAGS, obj="hymix_"),
 }
 
 
