@@ -51,11 +51,15 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 // the gated forms: g' = min(g, limit), u' = clamp(u, +-limit), g' sigmoid(alpha g') (u' + 1) (SM_ACT_CLAMPED_GLU), or with
 // SM_ACT_SILU_GLU the same without the one: silu(g) u for limit = +inf and alpha = 1; SM_ACT_GELU_TANH_GLU: gelu_tanh(g) u
+// RCP: the quotient by the hardware's reciprocal (1 ulp) instead of the full division, for results that leave in bf16: in the
+// matrix-core expert kernels a quarter of the epilogue was the division
+template <bool RCP = false>
 __device__ __forceinline__ float gated_act(float g, float u, float limit, float alpha, int act) {
     if (act == SM_ACT_GELU_TANH_GLU) return gelu_tanh(g) * u;
     g = fminf(g, limit);
     u = fminf(fmaxf(u, -limit), limit);
-    return g / (1.f + __expf(-alpha * g)) * (u + (act == SM_ACT_SILU_GLU ? 0.f : 1.f));
+    const float den = 1.f + __expf(-alpha * g);
+    return (RCP ? g * __builtin_amdgcn_rcpf(den) : g / den) * (u + (act == SM_ACT_SILU_GLU ? 0.f : 1.f));
 }
 __host__ __device__ __forceinline__ bool act_is_gated(int act) {
     return act == SM_ACT_CLAMPED_GLU || act == SM_ACT_SILU_GLU || act == SM_ACT_GELU_TANH_GLU;
@@ -64,6 +68,10 @@ __device__ __forceinline__ float plain_act(float z, int act) {
     if (act == SM_ACT_RELU_SQ) { z = fmaxf(z, 0.f); return z * z; }
     return act == SM_ACT_GELU_TANH ? gelu_tanh(z) : gelu_erf(z);
 }
+
+// the grouping of (token, choice) pairs by expert into tiles of `unit` rows (sm_moe_align.hip); SM_OK or an error code
+int launch_moe_align(const int32_t* idx, int64_t P, int E, int unit, int max_tiles, int32_t* row_pair, int32_t* tile_expert,
+                     int32_t* pair_row, hipStream_t s);
 
 static inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 

@@ -7,19 +7,25 @@ namespace sm {
 
 constexpr int kMaxExperts = 1024, kMaxTop = 32;
 
-// largest value over the wave, smallest index among equals; every lane gets both
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
+// The wave's sums of d[0 .. N - 1]: halving the values with every step, lane l ends with value l / (64 / N) in d[0].
+template <int N, int O, int M>
+__device__ __forceinline__ void fold_wave(float (&d)[M], int lane) {
+    if constexpr (O == 0) {
+        return;
+    } else if constexpr (N > 1) {
+        const bool up = (lane & O) != 0;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(v, o);
-        const int oi = __shfl_xor(i, o);
-        if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
+        for (int i = 0; i < N / 2; ++i) d[i] = (up ? d[i + N / 2] : d[i]) + __shfl_xor(up ? d[i] : d[i + N / 2], O);
+        fold_wave<N / 2, O / 2>(d, lane);
+    } else {
+        d[0] += __shfl_xor(d[0], O);
+        fold_wave<1, O / 2>(d, lane);
     }
 }
 
 // kRouteTokens = tokens per workgroup: every router row read serves all of them
 template <typename T, int kRouteTokens>
-__global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ h, const float* __restrict__ router_w,
+__global__ __launch_bounds__(256, kRouteTokens == 8 ? 3 : 4) void moe_route_kernel(const T* __restrict__ h, const float* __restrict__ router_w,
                                                         int32_t* __restrict__ idx, float* __restrict__ wts, int64_t T_all, int W,
                                                         int E, int top, int groups, int keep, int score,
                                                         const float* __restrict__ correction, int group_top, int renorm,
@@ -37,26 +43,51 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ h,
         T* h_lds = (T*)(z_all + (kRouteTokens * RS + 3) / 4 * 4);
         const T* src = h + (size_t)t0 * W;
         struct alignas(sizeof(T) * 4) Pack4 { T v[4]; };
-        for (int i = threadIdx.x * 4; i < nt * W; i += 1024) *(Pack4*)(h_lds + i) = *(const Pack4*)(src + i);     // W % 4 == 0
-        __syncthreads();
-        for (int e = wave; e < rows; e += 4) {
-            const float* wr = e < E ? router_w + (size_t)e * W : gate_w;
-            float d[kRouteTokens];
-            for (int i = 0; i < kRouteTokens; ++i) d[i] = 0.f;
-#pragma unroll 4
-            for (int c = lane * 4; c < W; c += 256) {
-                const float4 wv = *(const float4*)(wr + c);
+        for (int i0 = threadIdx.x * 4; i0 < nt * W; i0 += 8 * 1024) {     // W % 4 == 0; eight pieces of a thread in flight
+            Pack4 piece[8];
 #pragma unroll
-                for (int i = 0; i < kRouteTokens; ++i)
-                    if (i < nt) {
-                        const Pack4 hv = *(const Pack4*)(h_lds + (size_t)i * W + c);
-                        d[i] += to_f(hv.v[0]) * wv.x + to_f(hv.v[1]) * wv.y + to_f(hv.v[2]) * wv.z + to_f(hv.v[3]) * wv.w;
-                    }
+            for (int j = 0; j < 8; ++j) piece[j] = *(const Pack4*)(src + min(i0 + 1024 * j, nt * W - 4));
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (i0 + 1024 * j < nt * W) *(Pack4*)(h_lds + i0 + 1024 * j) = piece[j];
+        }
+        __syncthreads();
+        // four experts at a time: a token's piece read from LDS and widened meets four router rows (one row at a time, the
+        // LDS reads and the 6 lane moves of every single sum were most of the kernel: 8192 tokens of 2048 channels, 16
+        // experts: 53 -> 29 us; 64 tokens 16 -> 9)
+        for (int e0 = 4 * wave; e0 < rows; e0 += 16) {
+            const float* wr[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int e = min(e0 + j, rows - 1);
+                wr[j] = e < E ? router_w + (size_t)e * W : gate_w;
             }
-            for (int i = 0; i < kRouteTokens; ++i) {
-                const float sum = wave_sum(d[i]);
-                if (lane == 0) z_all[i * RS + (e < E ? e : RS - 1)] = sum;
+            constexpr int N = 4 * kRouteTokens;
+            float d[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) d[i] = 0.f;
+            float4 nxt[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) nxt[j] = *(const float4*)(wr[j] + min(lane * 4, W - 4));
+#pragma unroll 1
+            for (int c = lane * 4; c < W; c += 256) {
+                float4 wv[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    wv[j] = nxt[j];
+                    nxt[j] = *(const float4*)(wr[j] + min(c + 256, W - 4));
+                }
+#pragma unroll
+                for (int i = 0; i < kRouteTokens; ++i) {           // (rows past nt: whatever LDS holds, nobody reads their sums)
+                    const Pack4 hv = *(const Pack4*)(h_lds + (size_t)i * W + c);
+                    const float x0 = to_f(hv.v[0]), x1 = to_f(hv.v[1]), x2 = to_f(hv.v[2]), x3 = to_f(hv.v[3]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) d[4 * i + j] += x0 * wv[j].x + x1 * wv[j].y + x2 * wv[j].z + x3 * wv[j].w;
+                }
             }
+            fold_wave<N, 32>(d, lane);
+            const int v = lane / (64 / N), e = e0 + v % 4;
+            if (lane % (64 / N) == 0 && e < rows) z_all[v / 4 * RS + (e < E ? e : RS - 1)] = d[0];
         }
     } else {
         for (int e = wave; e < rows; e += 4) {
@@ -106,14 +137,19 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ h,
             }
             float tot = 0.f, my_w = 0.f;
             int my_e = 0;
+            const int span = E <= 16 ? 16 : E <= 32 ? 32 : 64;
             for (int k = 0; k < top; ++k) {
                 float bv = -INFINITY;
                 int be = E;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     if (c[j] > bv) { bv = c[j]; be = lane + 64 * j; }
-                wave_argmax(bv, be);
-                be = min(be, E - 1);
+                for (int o = span >> 1; o > 0; o >>= 1) {        // (the lanes past the experts hold -inf)
+                    const float ov = __shfl_xor(bv, o);
+                    const int oe = __shfl_xor(be, o);
+                    if (ov > bv || (ov == bv && oe < be)) { bv = ov; be = oe; }
+                }
+                be = min(__builtin_amdgcn_readfirstlane(be), E - 1);
                 float w = 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
@@ -147,6 +183,19 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ h,
         for (int e = 0; e < E; ++e) z[e] *= inv;
     }
     float* gs = z + E;
+    // a chosen expert's score becomes -inf (no score is); the weights wait in wts for their sum.  (No array per thread: those
+    // cost every token of this kernel its registers.)
+    auto take = [&](int k, int best, float& tot) {
+        const float w = best < 0 ? 0.f : z[best];
+        idx[(size_t)t * top + k] = best < 0 ? 0 : best;
+        wts[(size_t)t * top + k] = w;
+        tot += w;
+        if (best >= 0) z[best] = -INFINITY;
+    };
+    auto leave = [&](float tot) {
+        const float rn = renorm ? 1.f / (tot + 1e-20f) : 1.f;
+        for (int k = 0; k < top; ++k) wts[(size_t)t * top + k] *= rn;
+    };
     if (correction != nullptr || group_top > 1) {
         // The general form: choice scores c = s + correction (they may be negative) decide, the weights are s.  A group
         // scores the sum of its `group_top` largest c; experts outside the best `keep` groups count as -inf.
@@ -179,27 +228,18 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ h,
                 if (best >= 0) gs[best] = INFINITY;
             }
         }
-        int chosen[kMaxTop];
-        float cw[kMaxTop], tot = 0.f;
+        float tot = 0.f;
         for (int k = 0; k < top; ++k) {
             int best = -1;
             float bv = -INFINITY;
             for (int e = 0; e < E; ++e) {
                 if (!ok_all && gs[e / per] != INFINITY) continue;
-                bool taken = false;
-                for (int j = 0; j < k; ++j) taken |= chosen[j] == e;
                 const float c = z[e] + (correction ? correction[e] : 0.f);
-                if (!taken && (best < 0 || c > bv)) { bv = c; best = e; }
+                if (z[e] != -INFINITY && (best < 0 || c > bv)) { bv = c; best = e; }
             }
-            chosen[k] = best < 0 ? 0 : best;
-            cw[k] = best < 0 ? 0.f : z[best];
-            tot += cw[k];
+            take(k, best, tot);
         }
-        const float rn = renorm ? 1.f / (tot + 1e-20f) : 1.f;
-        for (int k = 0; k < top; ++k) {
-            idx[(size_t)t * top + k] = chosen[k];
-            wts[(size_t)t * top + k] = cw[k] * rn;
-        }
+        leave(tot);
         return;
     }
     if (groups > 1) {
@@ -218,27 +258,17 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ h,
             if (best >= 0) gs[best] = -2.f;                     // -2 = kept
         }
     }
-    int chosen[kMaxTop];
-    float cw[kMaxTop];
     float tot = 0.f;
     for (int k = 0; k < top; ++k) {
         int best = -1;
         float bv = -1.f;
         for (int e = 0; e < E; ++e) {
             if (groups > 1 && gs[e / (E / groups)] != -2.f) continue;
-            bool taken = false;
-            for (int j = 0; j < k; ++j) taken |= chosen[j] == e;
-            if (!taken && z[e] > bv) { bv = z[e]; best = e; }
+            if (z[e] != -INFINITY && z[e] > bv) { bv = z[e]; best = e; }
         }
-        chosen[k] = best < 0 ? 0 : best;
-        cw[k] = best < 0 ? 0.f : bv;
-        tot += cw[k];
+        take(k, best, tot);
     }
-    const float rn = renorm ? 1.f / (tot + 1e-20f) : 1.f;
-    for (int k = 0; k < top; ++k) {
-        idx[(size_t)t * top + k] = chosen[k];
-        wts[(size_t)t * top + k] = cw[k] * rn;
-    }
+    leave(tot);
 }
 
 // workgroup = one (token, expert) pair; every wave produces outputs f = wave, wave + 4, ...

@@ -1,0 +1,99 @@
+// The grouping in front of the expert products: (token, choice) pairs sorted by expert into tiles of `unit` rows.
+//
+// One workgroup, because every row number depends on every count.  What it spends its time in are the LDS counters: with one
+// counter per expert all waves meet on a few addresses, so every wave (or a few of them, for very many experts) counts on a
+// copy of its own, and the position that its counter returned is kept, so that pairs are counted once and not twice; and the
+// loads, which a thread therefore requests sixteen at a time (32768 pairs over 16 experts: 35 -> 25 us).
+#include "sm_common.h"
+
+namespace sm {
+
+constexpr int kAlignThreads = 1024, kAlignWaves = kAlignThreads / 64, kBatch = 16;
+
+__global__ __launch_bounds__(kAlignThreads) void moe_align_kernel(const int32_t* __restrict__ idx, int P, int E, int copies, int unit,
+                                                                  int max_tiles, int32_t* __restrict__ row_pair,
+                                                                  int32_t* __restrict__ tile_expert, int32_t* __restrict__ pair_row) {
+    extern __shared__ int cnt[];                // [copies][E]: counts, then the first row of the copy's pairs
+    const int lane = threadIdx.x & 63;
+    int* mine = cnt + (threadIdx.x >> 6) % copies * E;
+    const int max_rows = max_tiles * unit;
+    for (int i = threadIdx.x; i < copies * E; i += kAlignThreads) cnt[i] = 0;
+    for (int i = threadIdx.x; i < max_tiles; i += kAlignThreads) tile_expert[i] = -1;
+    for (int i = threadIdx.x; i < max_rows; i += kAlignThreads) row_pair[i] = -1;
+    __syncthreads();
+    for (int p0 = threadIdx.x; p0 < P; p0 += kBatch * kAlignThreads) {
+        int e[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int p = p0 + j * kAlignThreads;
+            e[j] = p < P ? idx[p] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) e[j] = e[j] >= 0 && e[j] < E ? atomicAdd(&mine[e[j]], 1) : 0;
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int p = p0 + j * kAlignThreads;
+            if (p < P) pair_row[p] = e[j];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {                     // a wave takes 64 experts at a time
+        int tiles = 0;
+        for (int e0 = 0; e0 < E; e0 += 64) {
+            const int e = e0 + lane;
+            int total = 0;
+            if (e < E)
+                for (int c = 0; c < copies; ++c) total += cnt[c * E + e];
+            const int n = (total + unit - 1) / unit;
+            int upto = n;                       // tiles of the experts up to this one
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int v = __shfl_up(upto, o);
+                if (lane >= o) upto += v;
+            }
+            const int first = tiles + upto - n;
+            if (e < E) {
+                for (int i = 0; i < n && first + i < max_tiles; ++i) tile_expert[first + i] = e;
+                int row = first * unit;
+                for (int c = 0; c < copies; ++c) {
+                    const int k = cnt[c * E + e];
+                    cnt[c * E + e] = row;
+                    row += k;
+                }
+            }
+            tiles += __shfl(upto, 63);
+        }
+    }
+    __syncthreads();
+    for (int p0 = threadIdx.x; p0 < P; p0 += kBatch * kAlignThreads) {
+        int e[kBatch], r[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int p = p0 + j * kAlignThreads;
+            e[j] = p < P ? idx[p] : -1;
+            r[j] = p < P ? pair_row[p] : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            const int p = p0 + j * kAlignThreads;
+            if (e[j] < 0 || e[j] >= E) continue;
+            const int row = mine[e[j]] + r[j];
+            if (row < max_rows) row_pair[row] = p;
+            pair_row[p] = min(row, max_rows - 1);
+        }
+    }
+}
+
+// tiles of `unit` rows: every pair of idx gets a row, a tile's rows belong to one expert; rows without a pair hold -1, tiles
+// without rows expert -1
+int launch_moe_align(const int32_t* idx, int64_t P, int E, int unit, int max_tiles, int32_t* row_pair, int32_t* tile_expert,
+                     int32_t* pair_row, hipStream_t s) {
+    int copies = kAlignWaves;
+    while ((int64_t)copies * E * sizeof(int) > 64 * 1024) copies >>= 1;      // (E <= 4096: four copies at least)
+    hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(kAlignThreads), (size_t)copies * E * sizeof(int), s, idx, (int)P, E, copies, unit,
+                       max_tiles, row_pair, tile_expert, pair_row);
+    SM_CHECK_LAUNCH("sm_moe_align");
+    return SM_OK;
+}
+
+}  // namespace sm

@@ -1,5 +1,5 @@
 // Expert products for many tokens on the matrix cores (bf16): the (token, expert) pairs are grouped by expert into
-// tiles of 32 rows (sm_moe_align), so that one workgroup multiplies 32 rows of one expert by 128 of its output
+// tiles of 32 rows (sm_moe_align.hip), so that one wave multiplies 32 rows of one expert by 32 of its output
 // columns; gate and up are produced together and leave as the clamped GLU, the down product leaves per pair and a
 // last launch sums a token's pairs with their weights (and the shared expert) in a fixed order.
 //
@@ -15,40 +15,9 @@ namespace sm {
 
 constexpr int kRowsPerTile = 32;
 
-__global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restrict__ idx, int P, int E, int max_tiles,
-                                                         int32_t* __restrict__ row_pair, int32_t* __restrict__ tile_expert,
-                                                         int32_t* __restrict__ pair_row) {
-    extern __shared__ int sh[];                 // counts[E], offs[E], cursor[E]
-    int* counts = sh;
-    int* offs = sh + E;
-    int* cursor = sh + 2 * E;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) { counts[e] = 0; cursor[e] = 0; }
-    __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) atomicAdd(&counts[idx[p]], 1);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tiles = 0;
-        for (int e = 0; e < E; ++e) {
-            offs[e] = tiles * kRowsPerTile;
-            const int n = (counts[e] + kRowsPerTile - 1) / kRowsPerTile;
-            for (int i = 0; i < n; ++i) tile_expert[tiles + i] = e;
-            tiles += n;
-        }
-        for (int i = tiles; i < max_tiles; ++i) tile_expert[i] = -1;
-    }
-    for (int r = threadIdx.x; r < max_tiles * kRowsPerTile; r += blockDim.x) row_pair[r] = -1;
-    __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
-        const int e = idx[p];
-        const int r = offs[e] + atomicAdd(&cursor[e], 1);
-        row_pair[r] = p;
-        pair_row[p] = r;
-    }
-}
-
 __device__ __forceinline__ float glu_bf16(float g, float u, float limit, float alpha, int act) {
     // the products leave the matrix unit in bf16, as a GEMM's output would
-    return gated_act((float)(bf16_t)g, (float)(bf16_t)u, limit, alpha, act);
+    return gated_act<true>((float)(bf16_t)g, (float)(bf16_t)u, limit, alpha, act);
 }
 
 __device__ __forceinline__ bf16x8 load8(const unsigned short* p, int k, int K) {
@@ -61,8 +30,12 @@ __device__ __forceinline__ bf16x8 load8(const unsigned short* p, int k, int K) {
 // else:    A = act rows,                 B = the expert's down rows,       out = per-row products [rows, N] (N = W, K = F)
 // MODE 0: the down product; 1: gate and up with a gated activation (act_kind); 2: the up product alone with a plain one.
 // in_wts != NULL (modes 1, 2): pair p's products are scaled by in_wts[p] before the activation (a weight on the expert's input)
+//
+// A wave is a workgroup: sixteen tiles by 48 column blocks are three waves for every CU, where workgroups of four waves left a
+// quarter of the CUs without work (64 tokens, top 4 of 16 experts of 2048 x 1536: gate and up 76 -> 43 us, 4.6 TB/s of weights;
+// down 43 -> 37).
 template <int MODE>
-__global__ __launch_bounds__(256) void moe_grouped_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
+__global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                           const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                           unsigned short* __restrict__ out, int top, int N, int K, float limit,
                                                           float alpha, int act_kind, const float* __restrict__ in_wts) {
@@ -70,10 +43,8 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const unsigned short* 
     const int tile = blockIdx.x;
     const int e = tile_expert[tile];
     if (e < 0) return;
-    const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n0 = blockIdx.y * 128 + wave * 32;
-    if (n0 >= N) return;
+    const int lane = threadIdx.x, l31 = lane & 31, hi = lane >> 5;
+    const int n0 = blockIdx.y * 32;
     const int row = tile * kRowsPerTile + l31;
     const int pair = row_pair[row];
     const unsigned short* ap = FROM_TOKENS ? a + (size_t)(pair < 0 ? 0 : pair / top) * K : a + (size_t)row * K;
@@ -83,19 +54,18 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const unsigned short* 
     const unsigned short* bp = w + (((size_t)e * (GATE_UP ? 2 : 1) * nb32 + n0 / 32) * ksteps) * 2048 + 8 * lane;
     const unsigned short* bp2 = bp + (size_t)nb32 * ksteps * 2048;      // the up blocks follow the gate blocks
     f32x16 acc = {0}, acc2 = {0};
-    // A ring of three 64-k steps in flight: with a handful of rows per expert (decode) a wave's eight MFMAs per step
-    // hide nothing, so the weight stream has to be kept busy by outstanding loads (3 x 12 KB per wave).  Steps past K
-    // load zeros (both operands), which leave the sums as they are.
+    // A ring of 64-k steps in flight: with a handful of rows per expert (decode) a wave's few MFMAs per step hide nothing, so
+    // the weight stream has to be kept busy by outstanding loads: three steps of gate and up (36 KB per wave), six of a single
+    // product (24 KB of weights).  No condition stands around a load of the ring (one would make every load wait for the one
+    // before it): past the last whole step it loads that step again, and a shorter last step comes by itself.
+    constexpr int RING = GATE_UP ? 3 : 6;
     struct Stage { bf16x8 a[4], b[4], b2[4]; };
-    auto request = [&](Stage& st, int k0) {
-        const int kb = k0 + 32 * hi;
+    auto request = [&](Stage& st, int step) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            st.a[s] = load8(ap, kb + 8 * s, K);
-            // (steps past K: the ring runs up to two steps over; clamp to the last block and let A's zeros cancel it)
-            const size_t boff = (size_t)min(k0 / 64, ksteps - 1) * 2048 + 512 * s;
-            st.b[s] = *(const bf16x8*)(bp + boff);
-            if (GATE_UP) st.b2[s] = *(const bf16x8*)(bp2 + boff);
+            st.a[s] = *(const bf16x8*)(ap + (size_t)step * 64 + 32 * hi + 8 * s);
+            st.b[s] = *(const bf16x8*)(bp + (size_t)step * 2048 + 512 * s);
+            if (GATE_UP) st.b2[s] = *(const bf16x8*)(bp2 + (size_t)step * 2048 + 512 * s);
         }
     };
     auto consume = [&](const Stage& st) {
@@ -105,17 +75,31 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const unsigned short* 
             if (GATE_UP) acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(st.a[s], st.b2[s], acc2, 0, 0, 0);
         }
     };
-    Stage s0, s1, s2;
-    request(s0, 0);
-    request(s1, 64);
-    request(s2, 128);
-    for (int k0 = 0; k0 < K; k0 += 192) {
-        consume(s0);
-        request(s0, k0 + 192);
-        consume(s1);
-        request(s1, k0 + 256);
-        consume(s2);
-        request(s2, k0 + 320);
+    const int full = K / 64;
+    if (full > 0) {
+        Stage st[RING];
+#pragma unroll
+        for (int i = 0; i < RING; ++i) request(st[i], min(i, full - 1));
+        int step = 0;
+        for (; step + RING <= full; step += RING)
+#pragma unroll
+            for (int i = 0; i < RING; ++i) {
+                consume(st[i]);
+                request(st[i], min(step + RING + i, full - 1));
+            }
+#pragma unroll
+        for (int i = 0; i < RING; ++i)
+            if (step + i < full) consume(st[i]);
+    }
+    if (K % 64 != 0) {                                        // zeros past the end of a row (the weights end in zeros)
+        Stage st;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            st.a[s] = load8(ap, full * 64 + 32 * hi + 8 * s, K);
+            st.b[s] = *(const bf16x8*)(bp + (size_t)full * 2048 + 512 * s);
+            if (GATE_UP) st.b2[s] = *(const bf16x8*)(bp2 + (size_t)full * 2048 + 512 * s);
+        }
+        consume(st);
     }
     if (n0 + l31 >= N) return;
 #pragma unroll
@@ -130,19 +114,41 @@ __global__ __launch_bounds__(256) void moe_grouped_kernel(const unsigned short* 
     }
 }
 
-__global__ void moe_combine_kernel(const unsigned short* __restrict__ prod, const int32_t* __restrict__ pair_row,
-                                   const float* __restrict__ wts, const unsigned short* __restrict__ shared,
-                                   unsigned short* __restrict__ y, int top, int W, const float* __restrict__ shared_scale) {
-    const size_t t = blockIdx.x;
-    for (int c = threadIdx.x; c < W; c += blockDim.x) {
-        float tot = 0.f;
-        for (int k = 0; k < top; ++k) {
-            const size_t r = pair_row[t * top + k];
-            tot += (wts ? wts[t * top + k] : 1.f) * (float)__builtin_bit_cast(bf16_t, prod[r * W + c]);
-        }
-        if (shared) tot += (shared_scale ? shared_scale[t] : 1.f) * (float)__builtin_bit_cast(bf16_t, shared[t * W + c]);
-        y[t * W + c] = __builtin_bit_cast(unsigned short, (bf16_t)tot);
+// A token's pairs summed with their weights, in a fixed order, V channels per thread: 8 where rows and pointers allow 16-byte
+// accesses (64 tokens of 2048 channels: 4 us, 8192 tokens: 29 us, 5.8 TB/s; two bytes per access and a workgroup per token took 12
+// and 80).
+template <int V>
+__global__ __launch_bounds__(256) void moe_combine_kernel(const unsigned short* __restrict__ prod, const int32_t* __restrict__ pair_row,
+                                                          const float* __restrict__ wts, const unsigned short* __restrict__ shared,
+                                                          unsigned short* __restrict__ y, int64_t items, int top, int W,
+                                                          const float* __restrict__ shared_scale) {
+    struct alignas(2 * V) Pack { bf16_t v[V]; };
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= items) return;
+    const int per = W / V;
+    const int64_t t = i / per;
+    const int c = (int)(i - t * per) * V;
+    float tot[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) tot[v] = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < top; ++k) {
+        const size_t r = pair_row[t * top + k];
+        const float w = wts ? wts[t * top + k] : 1.f;
+        const Pack x = *(const Pack*)(prod + r * W + c);
+#pragma unroll
+        for (int v = 0; v < V; ++v) tot[v] += w * (float)x.v[v];
     }
+    if (shared) {
+        const float w = shared_scale ? shared_scale[t] : 1.f;
+        const Pack x = *(const Pack*)(shared + t * W + c);
+#pragma unroll
+        for (int v = 0; v < V; ++v) tot[v] += w * (float)x.v[v];
+    }
+    Pack o;
+#pragma unroll
+    for (int v = 0; v < V; ++v) o.v[v] = (bf16_t)tot[v];
+    *(Pack*)(y + t * W + c) = o;
 }
 
 }  // namespace sm
@@ -169,19 +175,17 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     if (T == 0) return SM_OK;
     const int tiles = sm_moe_grouped_tiles(T, top, E);
     hipStream_t s = as_stream(stream);
-    hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), (size_t)3 * E * sizeof(int), s, idx, (int)(T * top), E, tiles, row_pair,
-                       tile_expert, pair_row);
-    SM_CHECK_LAUNCH("sm_moe_grouped (align)");
+    if (int rc = launch_moe_align(idx, T * top, E, kRowsPerTile, tiles, row_pair, tile_expert, pair_row, s)) return rc;
     if (act_is_gated(act_kind))
-        hipLaunchKernelGGL(moe_grouped_kernel<1>, dim3((unsigned)tiles, (unsigned)((F + 127) / 128)), dim3(256), 0, s,
+        hipLaunchKernelGGL(moe_grouped_kernel<1>, dim3((unsigned)tiles, (unsigned)((F + 31) / 32)), dim3(64), 0, s,
                            (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, top, F,
                            W, limit, alpha, act_kind, weight_in ? wts : nullptr);
     else
-        hipLaunchKernelGGL(moe_grouped_kernel<2>, dim3((unsigned)tiles, (unsigned)((F + 127) / 128)), dim3(256), 0, s,
+        hipLaunchKernelGGL(moe_grouped_kernel<2>, dim3((unsigned)tiles, (unsigned)((F + 31) / 32)), dim3(64), 0, s,
                            (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, top, F,
                            W, limit, alpha, act_kind, weight_in ? wts : nullptr);
     SM_CHECK_LAUNCH("sm_moe_grouped (gate/up)");
-    hipLaunchKernelGGL(moe_grouped_kernel<0>, dim3((unsigned)tiles, (unsigned)((W + 127) / 128)), dim3(256), 0, s,
+    hipLaunchKernelGGL(moe_grouped_kernel<0>, dim3((unsigned)tiles, (unsigned)((W + 31) / 32)), dim3(64), 0, s,
                        (const unsigned short*)act, (const unsigned short*)w_down, row_pair, tile_expert, (unsigned short*)prod, top, W,
                        F, 0.f, 0.f, 0, (const float*)nullptr);
     SM_CHECK_LAUNCH("sm_moe_grouped (down)");
@@ -198,10 +202,8 @@ extern "C" int sm_moe_align(const int32_t* idx, int64_t T, int top, int E, int32
         return SM_EINVAL;
     }
     if (T == 0) return SM_OK;
-    hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), (size_t)3 * E * sizeof(int), as_stream(stream), idx, (int)(T * top), E,
-                       sm_moe_grouped_tiles(T, top, E), row_pair, tile_expert, pair_row);
-    SM_CHECK_LAUNCH("sm_moe_align");
-    return SM_OK;
+    return launch_moe_align(idx, T * top, E, kRowsPerTile, sm_moe_grouped_tiles(T, top, E), row_pair, tile_expert, pair_row,
+                            as_stream(stream));
 }
 
 extern "C" int sm_moe_combine(const void* prod, const int32_t* pair_row, const float* wts, const void* shared,
@@ -211,8 +213,14 @@ extern "C" int sm_moe_combine(const void* prod, const int32_t* pair_row, const f
         return SM_EINVAL;
     }
     if (T == 0) return SM_OK;
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)T), dim3(256), 0, as_stream(stream), (const unsigned short*)prod, pair_row,
-                       wts, (const unsigned short*)shared, (unsigned short*)y, top, W, shared_scale);
+    const bool wide = W % 8 == 0 && ((uintptr_t)prod | (uintptr_t)shared | (uintptr_t)y) % 16 == 0;
+    const int64_t items = T * (wide ? W / 8 : W), blocks = (items + 255) / 256;
+    if (blocks > 0x7fffffff) { set_error("sm_moe_combine: too many rows"); return SM_ESHAPE; }
+#define SM_COMBINE(V_)                                                                                                         \
+    hipLaunchKernelGGL(moe_combine_kernel<V_>, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), (const unsigned short*)prod, \
+                       pair_row, wts, (const unsigned short*)shared, (unsigned short*)y, items, top, W, shared_scale)
+    if (wide) SM_COMBINE(8); else SM_COMBINE(1);
+#undef SM_COMBINE
     SM_CHECK_LAUNCH("sm_moe_combine");
     return SM_OK;
 }

@@ -1,152 +1,253 @@
-// Expert products for large groups (prefill) on the matrix cores, bf16: tiles of 128 rows of one expert by 128 output
-// columns.  The 128 x 64 activation block of a k-step is staged once in LDS and shared by the four waves (each wave
-// owns 32 columns and all 128 rows: four row fragments reuse every weight fragment), the weights go from global
-// memory straight to the MFMA registers (a lane owns one weight row and 32 consecutive k of the 64-k step).
-// Against the 32-row form of sm_moe_grouped.hip this reads an expert's weights 4x less often and the activations
-// once per workgroup instead of once per wave.
+// Expert products for large groups (prefill) on the matrix cores, bf16: tiles of 64 MB rows of one expert (MB = 4 or 2 by the
+// size of the groups) by 256 rows of its weights (128 gate and the 128 up rows of the same outputs, or 256 plain ones).
 //
-// Row r of a group is the same sum whatever else shares its tile, so both forms agree bit for bit on a row's
-// products (same k order inside a 64-k step, same accumulation).
+// Row r of a group is the same sum whatever else shares its tile, so every form agrees bit for bit on a row's products
+// (same k order inside a 64-k step, same accumulation).
 #include "sm_common.h"
 
 namespace sm {
 
-constexpr int kBigRows = 128;                 // rows per tile
-constexpr int kAStride = 64 * 2 + 16;         // bytes between rows of the staged block (odd number of 16-byte chunks)
+constexpr int kBigRows = 128;                 // tiles are one or two times as many rows
 
-__global__ __launch_bounds__(1024) void moe_align128_kernel(const int32_t* __restrict__ idx, int P, int E, int max_tiles,
-                                                            int32_t* __restrict__ row_pair, int32_t* __restrict__ tile_expert,
-                                                            int32_t* __restrict__ pair_row) {
-    extern __shared__ int sh[];                 // counts[E], offs[E], cursor[E]
-    int* counts = sh;
-    int* offs = sh + E;
-    int* cursor = sh + 2 * E;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) { counts[e] = 0; cursor[e] = 0; }
-    __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
-        const int e = idx[p];
-        if (e >= 0 && e < E) atomicAdd(&counts[e], 1);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tiles = 0;
-        for (int e = 0; e < E; ++e) {
-            offs[e] = tiles * kBigRows;
-            const int n = (counts[e] + kBigRows - 1) / kBigRows;
-            for (int i = 0; i < n && tiles + i < max_tiles; ++i) tile_expert[tiles + i] = e;
-            tiles += n;
-        }
-        for (int i = tiles; i < max_tiles; ++i) tile_expert[i] = -1;
-    }
-    for (int r = threadIdx.x; r < max_tiles * kBigRows; r += blockDim.x) row_pair[r] = -1;
-    __syncthreads();
-    for (int p = threadIdx.x; p < P; p += blockDim.x) {
-        const int e = idx[p];
-        if (e < 0 || e >= E) { pair_row[p] = 0; continue; }
-        const int r = offs[e] + atomicAdd(&cursor[e], 1);
-        if (r < max_tiles * kBigRows) row_pair[r] = p;
-        pair_row[p] = min(r, max_tiles * kBigRows - 1);
-    }
-}
-
-__device__ __forceinline__ float glu_bf16_big(float g, float u, float limit, float alpha, int act) {
-    // the products leave the matrix unit in bf16, as a GEMM's output would
-    return gated_act((float)(bf16_t)g, (float)(bf16_t)u, limit, alpha, act);
-}
-
-__device__ __forceinline__ i32x4 load16(const unsigned short* p, int k, int K) {
-    i32x4 v = {0, 0, 0, 0};
-    if (k + 8 <= K) v = *(const i32x4*)(p + k);
-    return v;
-}
-
-// GATE_UP: A = h rows gathered by token, B = the expert's gate and up rows, out = act [rows, N] (N = F, K = W)
-// else:    A = act rows,                 B = the expert's down rows,       out = per-row products [rows, N] (N = W, K = F)
-// MODE 0: the down product; 1: gate and up with a gated activation (act_kind); 2: the up product alone with a plain one.
-// in_wts != NULL (modes 1, 2): pair p's products are scaled by in_wts[p] before the activation (a weight on the expert's input)
-template <int MODE>
-__global__ __launch_bounds__(256) void moe_tiles128_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
+// MODE 0: the down product, A = act rows;  1: gate and up with a gated activation (act_kind), 2: the up product alone with a
+// plain one, both with A = h rows gathered by token.  B = the expert's weight rows in the tiled layout (4 KB blocks of 32 rows
+// x 64 k in lane order, see seq_ops.tile_expert_weights).  in_wts != NULL (modes 1, 2): pair p's products are scaled by
+// in_wts[p] before the activation (a weight on the expert's input).
+//
+// Four waves, two by two: a wave owns 32 MB rows by 128 weight rows.  Both operands of a 64-k step go from global memory
+// straight to LDS (16 bytes per lane, no registers in between): the weights as they lie, a token row as eight 16-byte chunks,
+// chunk c of row r at place c ^ (r / 2 & 7), which spreads the 16-byte reads of 16 lanes over the 64 banks.  Two LDS buffers: the
+// loads of step k + 2 are issued as soon as every wave has read step k, one whole step ahead of their use, and a wave's
+// fragments are read from LDS one 16-k product ahead, across the barrier too.  (The buffers are two arrays and the loop is
+// unrolled by two, so that the compiler sees that a read of one does not wait for the loads into the other.)
+//
+// Bound by the matrix cores: 128 x 128 per wave needs half of what LDS delivers (smaller wave tiles need all of it).  32768
+// rows over 16 experts: gate and up of 2 x 1536 x 2048 in 449 us (0.92 PFLOP/s), down in 252 us (0.82), against 950 and 434 us
+// of tiles of 128 rows with one LDS buffer, two barriers per step and the weights loaded to registers by every wave.  What is
+// left: a first load and a last store per tile that no other workgroup of the CU covers, and a last round of tiles that does
+// not fill the chip.
+template <int MODE, int MB>
+__global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                            const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
-                                                           unsigned short* __restrict__ out, int top, int N, int K, float limit,
-                                                           float alpha, int act_kind, const float* __restrict__ in_wts) {
-    __shared__ __attribute__((aligned(16))) unsigned char a_lds[kBigRows * kAStride];
+                                                           unsigned short* __restrict__ out, int top, int N, int K, int tiles, int nct,
+                                                           float limit, float alpha, int act_kind, const float* __restrict__ in_wts) {
     constexpr bool GATE_UP = MODE == 1, FROM_TOKENS = MODE != 0;
-    const int tile = blockIdx.x;
+    constexpr int ROWS = 64 * MB, A_BYTES = ROWS * 128, BUF = A_BYTES + 8 * 4096;
+    constexpr int NA = 2 * MB;                                // 1 KB pieces of A a wave loads per step (and 8 of B)
+    __shared__ __attribute__((aligned(1024))) unsigned char buf0[BUF];
+    __shared__ __attribute__((aligned(1024))) unsigned char buf1[BUF];
+    // Workgroups go to the eight dies in turn; a die takes two neighbouring row tiles and all their column tiles before its next
+    // two, so that its L2 sees a row tile's activations nct times and a column tile's weights twice.
+    const int id = blockIdx.x >> 3, unit = id / (2 * nct), in_unit = id - unit * 2 * nct;
+    const int tile = (unit * 8 + (blockIdx.x & 7)) * 2 + (in_unit & 1), ct = in_unit >> 1;
+    if (tile >= tiles) return;
     const int e = tile_expert[tile];
     if (e < 0) return;                                        // (uniform over the workgroup)
-    const int tid = threadIdx.x, lane = tid & 63, l31 = lane & 31, hi = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.y * 128 + wave * 32;              // (n0 >= N: the wave still stages and keeps the barriers)
-    // staging: thread -> row tid / 2, k half tid % 2 (32 consecutive k = 64 bytes)
-    const int srow = tid >> 1, shalf = tid & 1;
-    const int spair = row_pair[tile * kBigRows + srow];
-    const unsigned short* ap = FROM_TOKENS ? a + (size_t)(spair < 0 ? 0 : spair / top) * K : a + ((size_t)tile * kBigRows + srow) * K;
-    // weights in the tiled layout of sm_moe_tile_weights (see sm_moe_grouped.hip): a wave's load is one contiguous KB
+    const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = wave >> 1, wc = wave & 1;
     const int nb32 = (N + 31) / 32, ksteps = (K + 63) / 64;
-    const unsigned short* bp = w + (((size_t)e * (GATE_UP ? 2 : 1) * nb32 + min(n0, N - 1) / 32) * ksteps) * 2048 + 8 * lane;
-    const unsigned short* bp2 = bp + (size_t)nb32 * ksteps * 2048;      // the up blocks follow the gate blocks
-    f32x16 acc[4], acc2[4];
+
+    // what this lane loads: rows 8 (wave NA + i) + lane / 8 of the tile, the chunk that belongs at place lane % 8
+    const int chunk = (lane & 7) ^ (lane >> 4);               // (i even; i odd: chunk ^ 4)
+    const unsigned short* arow[NA];
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) { acc[m][r] = 0.f; acc2[m][r] = 0.f; }
-    // software pipeline: the operands of step k+1 are requested before the MFMAs of step k
-    i32x4 ar[4], bn[4], bn2[4];
-    auto request = [&](int k0) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            ar[s] = load16(ap, k0 + 32 * shalf + 8 * s, K);
-            const size_t boff = (size_t)(k0 / 64) * 2048 + 512 * s;
-            bn[s] = *(const i32x4*)(bp + boff);
-            if (GATE_UP) bn2[s] = *(const i32x4*)(bp2 + boff);
-        }
-    };
-    request(0);
-    for (int k0 = 0; k0 < K; k0 += 64) {
-        i32x4 bf[4], bf2[4];
-        __syncthreads();                                      // the previous step's reads of a_lds are done
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            *(i32x4*)(a_lds + srow * kAStride + 64 * shalf + 16 * s) = ar[s];
-            bf[s] = bn[s];
-            if (GATE_UP) bf2[s] = bn2[s];
-        }
-        __syncthreads();
-        if (k0 + 64 < K) request(k0 + 64);
-        if (n0 < N) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const bf16x8 af = *(const bf16x8*)(a_lds + (32 * m + l31) * kAStride + 64 * hi + 16 * s);
-                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, __builtin_bit_cast(bf16x8, bf[s]), acc[m], 0, 0, 0);
-                    if (GATE_UP)
-                        acc2[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, __builtin_bit_cast(bf16x8, bf2[s]), acc2[m], 0, 0, 0);
-                }
+    for (int i = 0; i < NA; ++i) {
+        const int row = tile * ROWS + 8 * (wave * NA + i) + (lane >> 3), ch = chunk ^ (4 * (i & 1));
+        if (FROM_TOKENS) {
+            const int p = row_pair[row];
+            arow[i] = a + (size_t)(p < 0 ? 0 : p / top) * K + 8 * ch;
+        } else {
+            arow[i] = a + (size_t)row * K + 8 * ch;
         }
     }
-    if (n0 + l31 >= N) return;
+    // weight blocks 2 wave and 2 wave + 1 of the tile's eight: gate blocks first, then up blocks (blocks past N: the last one)
+    const unsigned short* bblk[2];
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int j = 0; j < 2; ++j) {
+        const int blk = 2 * wave + j;
+        const int nb = GATE_UP ? min(4 * ct + (blk & 3), nb32 - 1) + (blk >= 4 ? nb32 : 0) : min(8 * ct + blk, nb32 - 1);
+        bblk[j] = w + (((size_t)e * (GATE_UP ? 2 : 1) * nb32 + nb) * ksteps) * 2048 + 8 * lane;
+    }
+    typedef __attribute__((address_space(1))) const void gvoid;
+    typedef __attribute__((address_space(3))) void lvoid;
+    auto load_a = [&](unsigned char* buf, int ks, int i) {
+        __builtin_amdgcn_global_load_lds((gvoid*)(arow[i] + (size_t)ks * 64), (lvoid*)(buf + 1024 * (wave * NA + i)), 16, 0, 0);
+    };
+    auto load_b = [&](unsigned char* buf, int ks, int i) {
+        __builtin_amdgcn_global_load_lds((gvoid*)(bblk[i >> 2] + (size_t)ks * 2048 + 512 * (i & 3)),
+                                         (lvoid*)(buf + A_BYTES + 4096 * (2 * wave + (i >> 2)) + 1024 * (i & 3)), 16, 0, 0);
+    };
+    auto load_step = [&](unsigned char* buf, int ks) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int orow = tile * kBigRows + 32 * m + (r & 3) + 8 * (r >> 2) + 4 * hi;
-            const int p = row_pair[orow];
-            if (p < 0) continue;
-            const float iw = FROM_TOKENS && in_wts ? in_wts[p] : 1.f;
-            const float v = GATE_UP ? glu_bf16_big(acc[m][r] * iw, acc2[m][r] * iw, limit, alpha, act_kind)
-                                    : (MODE == 2 ? plain_act((float)(bf16_t)(acc[m][r] * iw), act_kind) : acc[m][r]);
-            out[(size_t)orow * N + n0 + l31] = __builtin_bit_cast(unsigned short, (bf16_t)v);
+        for (int i = 0; i < NA; ++i) load_a(buf, ks, i);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) load_b(buf, ks, i);
+    };
+    auto landed = [&]() {                                     // this wave's loads are in LDS, then everybody's
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+
+    f32x16 acc[MB][4];
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+
+    struct Frags { bf16x8 a[MB], b[4]; };
+    const int a_base = (32 * MB * wr + l31) * 128, a_x = (l31 >> 1) & 7;
+    auto read = [&](Frags& f, const unsigned char* buf, int s) {       // k = 32 hi + 8 s .. + 8 of the step
+        const int place = 16 * ((4 * hi + s) ^ a_x);
+#pragma unroll
+        for (int m = 0; m < MB; ++m) f.a[m] = *(const bf16x8*)(buf + a_base + 4096 * m + place);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int blk = GATE_UP ? 2 * wc + (n & 1) + 4 * (n >> 1) : 4 * wc + n;
+            f.b[n] = *(const bf16x8*)(buf + A_BYTES + 4096 * blk + 1024 * s + 16 * lane);
         }
+    };
+    auto multiply = [&](const Frags& f) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[n], f.a[m], acc[m][n], 0, 0, 0);
+    };
+
+    // The order of a product's instructions: the next product's LDS reads one by one between the first MFMAs, then the loads of
+    // the step after next.  Left alone the compiler puts the reads in front of their use, and every product waits for LDS.
+    auto interleave = [&](int loads) {
+#pragma unroll
+        for (int i = 0; i < MB + 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);          // an MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);          // an LDS read
+        }
+#pragma unroll
+        for (int i = 0; i < 3 * MB - 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (loads) __builtin_amdgcn_sched_group_barrier(0x020, (NA + 8 + 3 * MB - 5) / (3 * MB - 4), 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Frags f0, f1;
+    const int full = K / 64, last = full - 1;                 // whole steps; a shorter one follows them
+    auto step = [&](unsigned char* cur, unsigned char* nxt, int ks) {
+        read(f1, cur, 1);
+        multiply(f0);
+        interleave(0);
+        read(f0, cur, 2);
+        multiply(f1);
+        interleave(0);
+        read(f1, cur, 3);
+        multiply(f0);
+        interleave(0);
+        landed();                                             // the next step is there, and nobody reads this one any more
+        read(f0, nxt, 0);
+        load_step(cur, min(ks + 2, last));                    // (past the end: the last step again, which nobody reads)
+        multiply(f1);
+        interleave(NA + 8);
+    };
+    if (full > 0) {
+        load_step(buf0, 0);
+        landed();
+        load_step(buf1, min(1, last));
+        read(f0, buf0, 0);
+        int ks = 0;
+        for (; ks + 1 < full; ks += 2) {
+            step(buf0, buf1, ks);
+            step(buf1, buf0, ks + 1);
+        }
+        if (ks < full) step(buf0, buf1, ks);
+        landed();
+    }
+    if (K % 64 != 0) {                                        // zeros past the end of a token's row (the weights end in zeros)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            i32x4 v = {0, 0, 0, 0};
+            if (full * 64 + 8 * (chunk ^ (4 * (i & 1))) + 8 <= K) v = *(const i32x4*)(arow[i] + (size_t)full * 64);
+            *(i32x4*)(buf0 + 1024 * (wave * NA + i) + 16 * lane) = v;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) load_b(buf0, full, i);
+        landed();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            read(f0, buf0, s);
+            multiply(f0);
+        }
+        __syncthreads();
+    }
+
+    // The products leave the matrix unit in bf16, as a GEMM's output would, and go through LDS (rows 0 .. 32 MB - 1 in buf0, the
+    // others in buf1; 16-byte chunk c of row r at place c ^ (r & 31)), so that a thread finishes eight neighbouring outputs.
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+        float iw = 1.f;
+        if (FROM_TOKENS && in_wts) {
+            const int p = row_pair[tile * ROWS + 32 * (MB * wr + m) + l31];
+            if (p >= 0) iw = in_wts[p];
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int blk = GATE_UP ? 2 * wc + (n & 1) + 4 * (n >> 1) : 4 * wc + n;
+                u16x4 o4;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o4[r] = __builtin_bit_cast(unsigned short, (bf16_t)(acc[m][n][4 * q + r] * iw));
+                *(u16x4*)((wr ? buf1 : buf0) + (32 * m + l31) * 512 + 16 * ((4 * blk + q) ^ l31) + 8 * hi) = o4;
+            }
+    }
+    __syncthreads();
+    constexpr int CH = GATE_UP ? 16 : 32;                     // finished chunks per row
+#pragma unroll 4
+    for (int i = threadIdx.x; i < ROWS * CH; i += 256) {          // (rows without a pair too: nobody reads what they leave)
+        const int row = i / CH, c = i % CH, lrow = row & (32 * MB - 1);
+        const int col = (GATE_UP ? 128 : 256) * ct + 8 * c;
+        if (col >= N) continue;                               // (N % 8 == 0)
+        const unsigned char* src = (row >= 32 * MB ? buf1 : buf0) + lrow * 512;
+        bf16x8 x = *(const bf16x8*)(src + 16 * (c ^ (row & 31)));
+        if (GATE_UP) {
+            const bf16x8 u = *(const bf16x8*)(src + 16 * ((c + 16) ^ (row & 31)));
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x[r] = (bf16_t)gated_act<true>((float)x[r], (float)u[r], limit, alpha, act_kind);
+        } else if (MODE == 2) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x[r] = (bf16_t)plain_act((float)x[r], act_kind);
+        }
+        *(bf16x8*)(out + ((size_t)tile * ROWS + row) * N + col) = x;
+    }
+}
+
+// Rows of a tile: 256 from 128 rows per expert on average, else 128 (us with 128 / 256 rows, two sizes: 16 experts of 2048 x
+// 1536, 32 of 1024 x 768: 96 rows per expert 99 / 120, 53 / 75; 128 rows 142 / 120, 78 / 76; 384 rows 229 / 189, 126 / 124;
+// 2048 rows 942 / 734, 634 / 514).
+static int tile_rows(int64_t T, int top, int E) { return T * top >= (int64_t)128 * E ? 256 : 128; }
+
+template <int MODE>
+static void launch_tiles(int rows, const void* a, const void* w, const int32_t* row_pair, const int32_t* tile_expert, void* out, int top,
+                         int tiles, int N, int K, float limit, float alpha, int act_kind, const float* in_wts, hipStream_t s) {
+    const int nct = MODE == 1 ? (N + 127) / 128 : (N + 255) / 256, units = (tiles + 1) / 2;
+    dim3 grid((unsigned)((units + 7) / 8 * 8 * 2 * nct));
+    if (rows == 256)
+        hipLaunchKernelGGL((moe_tiles_kernel<MODE, 4>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, row_pair,
+                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, limit, alpha, act_kind, in_wts);
+    else
+        hipLaunchKernelGGL((moe_tiles_kernel<MODE, 2>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, row_pair,
+                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, limit, alpha, act_kind, in_wts);
 }
 
 }  // namespace sm
 
 using namespace sm;
 
+// room for a call's rows, in units of 128 rows
 extern "C" int sm_moe_tiles128_count(int64_t T, int top, int E) {
     if (T <= 0 || top <= 0 || E <= 0) return 0;
-    return (int)((T * top + kBigRows - 1) / kBigRows + E);
+    const int rows = tile_rows(T, top, E);
+    return (int)((T * top + rows - 1) / rows + E) * (rows / kBigRows);
 }
 
 extern "C" int sm_moe_tiles128(const void* h, const int32_t* idx, const float* wts, const void* w_gu, const void* w_down,
@@ -162,23 +263,16 @@ extern "C" int sm_moe_tiles128(const void* h, const int32_t* idx, const float* w
         return SM_ESHAPE;
     }
     if (T == 0) return SM_OK;
-    const int tiles = sm_moe_tiles128_count(T, top, E);
+    const int rows = tile_rows(T, top, E), tiles = sm_moe_tiles128_count(T, top, E) / (rows / kBigRows);
     hipStream_t s = as_stream(stream);
-    hipLaunchKernelGGL(moe_align128_kernel, dim3(1), dim3(1024), (size_t)3 * E * sizeof(int), s, idx, (int)(T * top), E, tiles, row_pair,
-                       tile_expert, pair_row);
-    SM_CHECK_LAUNCH("sm_moe_tiles128 (align)");
+    if (int rc = launch_moe_align(idx, T * top, E, rows, tiles, row_pair, tile_expert, pair_row, s)) return rc;
+    const float* in_wts = weight_in ? wts : nullptr;
     if (act_is_gated(act_kind))
-        hipLaunchKernelGGL(moe_tiles128_kernel<1>, dim3((unsigned)tiles, (unsigned)((F + 127) / 128)), dim3(256), 0, s,
-                           (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, top, F,
-                           W, limit, alpha, act_kind, weight_in ? wts : nullptr);
+        launch_tiles<1>(rows, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
     else
-        hipLaunchKernelGGL(moe_tiles128_kernel<2>, dim3((unsigned)tiles, (unsigned)((F + 127) / 128)), dim3(256), 0, s,
-                           (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, top, F,
-                           W, limit, alpha, act_kind, weight_in ? wts : nullptr);
+        launch_tiles<2>(rows, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
     SM_CHECK_LAUNCH("sm_moe_tiles128 (gate/up)");
-    hipLaunchKernelGGL(moe_tiles128_kernel<0>, dim3((unsigned)tiles, (unsigned)((W + 127) / 128)), dim3(256), 0, s,
-                       (const unsigned short*)act, (const unsigned short*)w_down, row_pair, tile_expert, (unsigned short*)prod, top, W,
-                       F, 0.f, 0.f, 0, (const float*)nullptr);
+    launch_tiles<0>(rows, act, w_down, row_pair, tile_expert, prod, top, tiles, W, F, 0.f, 0.f, 0, nullptr, s);
     SM_CHECK_LAUNCH("sm_moe_tiles128 (down)");
     if (y == nullptr) return SM_OK;               // the caller sums a token's pairs itself
     return sm_moe_combine(prod, pair_row, weight_in ? nullptr : wts, shared, shared_scale, y, T, top, W, stream);

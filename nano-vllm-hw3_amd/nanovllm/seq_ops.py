@@ -248,7 +248,9 @@ def moe_route(h, router_w, top, groups=1, keep=1, score=ROUTE_SOFTMAX, correctio
     return (idx, wts) if gate is None else (idx, wts, gate)
 
 
-TILES128_MIN_ROWS_PER_EXPERT = 64
+# rows per expert on average from which tiles of 128 and 256 rows beat tiles of 32 (us of the 32-row form / the other, 16 experts
+# of 2048 x 1536 and 32 of 1024 x 768: 16 rows 82 / 100 and 45 / 50, 32 rows 106 / 96 and 62 / 51)
+TILES128_MIN_ROWS_PER_EXPERT = 24
 
 
 def tile_expert_weights(w, parts=1):
@@ -291,7 +293,6 @@ def moe_experts(h, idx, wts, w_gu, w_down, limit, alpha=1.702, shared=None, form
     lib, code = SM.load(), SM.dtype_code(h.dtype)
     can_group = h.dtype == torch.bfloat16 and W % 8 == 0 and F % 8 == 0
     if form is None:
-        # groups of 64 rows and more on average fill 128-row tiles well enough to pay for their padding
         form = "pairs" if not can_group else ("tiles128" if T * top >= TILES128_MIN_ROWS_PER_EXPERT * E else "grouped")
     if form in ("grouped", "tiles128"):
         assert can_group

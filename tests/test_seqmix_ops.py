@@ -298,6 +298,43 @@ def test_moe_grouped_equals_pairs(T, W, F, E, top):
     assert torch.equal(b, c)          # a row's sums do not depend on the tile it sits in: both grouped forms agree exactly
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,W,F,E,top,act", [(900, 64, 128, 3, 2, "silu"), (1024, 136, 264, 1, 1, "silu"), (2100, 200, 72, 2, 1, "relu"),
+                                             (1500, 8, 8, 2, 1, "gelu"), (700, 320, 640, 5, 2, "clamped"), (260, 64, 256, 2, 1, "silu")])
+def test_moe_large_tiles_equal_small_ones(T, W, F, E, top, act):
+    """Tiles of 256 and of 128 rows (512 pairs per expert and more, and fewer) against tiles of 32: one and several k steps,
+    k that is no multiple of 64 or below it, columns off the 256-column tile, ragged groups, an expert without tokens.  A
+    row's sums are the same in every form, so the outputs agree bit for bit; and all are near float32 (bf16 products of
+    unit size: 2^-8 of the largest term of a sum of F, and the activation's own rounding)."""
+    g = gen(T + W + F)
+    h = rnd(g, T, W).cuda().bfloat16()
+    idx = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int()
+    if E > 4:
+        idx[idx == 2] = 3
+    wts = torch.rand(T, top, generator=g).cuda()
+    kind = dict(silu=seq_ops.ACT_SILU_GLU, relu=seq_ops.ACT_RELU_SQ, gelu=seq_ops.ACT_GELU, clamped=seq_ops.ACT_CLAMPED_GLU)[act]
+    parts = 2 if kind in seq_ops.GATED_ACTS else 1
+    w_gu, w_down = rnd(g, E, parts * F, W, s=W ** -0.5).cuda().bfloat16(), rnd(g, E, W, F, s=F ** -0.5).cuda().bfloat16()
+    limit, alpha = (1.2, 1.702) if act == "clamped" else (float("inf"), 1.0)
+    for weight_in in (False, True):
+        y = [seq_ops.moe_experts(h, idx.cuda(), wts, w_gu, w_down, limit, alpha, form=f, act_kind=kind, weight_in=weight_in)
+             for f in ("grouped", "tiles128")]
+        assert torch.equal(*y)
+    ref = torch.zeros(T, W, device="cuda")
+    for e in range(E):
+        tok, k = (idx.cuda() == e).nonzero(as_tuple=True)
+        z = (h[tok].float() @ w_gu[e].float().t()) * wts[tok, k][:, None]
+        if act == "silu":
+            a = torch.nn.functional.silu(z[:, :F]) * z[:, F:]
+        elif act == "clamped":
+            gt = z[:, :F].clamp(max=1.2)
+            a = gt * torch.sigmoid(1.702 * gt) * (z[:, F:].clamp(-1.2, 1.2) + 1)
+        else:
+            a = torch.relu(z) ** 2 if act == "relu" else torch.nn.functional.gelu(z)
+        ref.index_add_(0, tok, a @ w_down[e].float().t())
+    assert (y[1].float() - ref).norm() < 2 ** -7 * ref.norm()
+
+
 def test_oracle_absorbed_form_is_the_explicit_one():
     """The oracle's two statements of the attention agree: explicit keys / values, and queries that carry W_uk."""
     g = gen(11)
