@@ -24,8 +24,9 @@ __device__ __forceinline__ float mode_pre(float scale, float softcap, const floa
     return MODE == kSigmoid && head_bias ? head_bias[head] * 1.4426950408889634f : 0.f;
 }
 
-template <int NBK, int NBV, int MODE>
-__global__ __launch_bounds__(256) void attn_tiles_kernel(const unsigned short* __restrict__ q, const unsigned short* __restrict__ kc,
+// SLIM: head sizes of exactly 32 NBK and 32 NBV channels, in the loop whose tiles go straight to LDS (kv_slim_loop)
+template <int NBK, int NBV, int MODE, bool SLIM>
+__global__ __launch_bounds__(256, 2) void attn_tiles_kernel(const unsigned short* __restrict__ q, const unsigned short* __restrict__ kc,
                                                          const unsigned short* __restrict__ vc,
                                                          const int32_t* __restrict__ block_tables,
                                                          const int32_t* __restrict__ qstart, const int32_t* __restrict__ seq_pos0,
@@ -33,12 +34,24 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(const unsigned short* _
                                                          unsigned short* __restrict__ o, int H, int G, int D, int V, int block_size,
                                                          int max_blocks, const unsigned short* __restrict__ kp,
                                                          const unsigned short* __restrict__ vp, int pool, int pool_rows,
-                                                         int chunk, const float* __restrict__ head_bias, float softcap, OutArgs out) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds_k[TileGeom<NBK>::LDS_BYTES];
-    __shared__ __attribute__((aligned(16))) unsigned char lds_v[TileGeom<NBV>::LDS_BYTES];
-    const int b = blockIdx.y, g = blockIdx.z, rep = H / G;
+                                                         int chunk, const float* __restrict__ head_bias, float softcap, OutArgs out, int B, int tiles,
+                                                         int by_die) {
+    // (the two LDS arrays are the slim loop's buffers, or the key and the value tile)
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_k[SLIM ? SlimGeom<NBK>::BYTES + SlimGeom<NBV>::BYTES : TileGeom<NBK>::LDS_BYTES];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_v[SLIM ? SlimGeom<NBK>::BYTES + SlimGeom<NBV>::BYTES : TileGeom<NBV>::LDS_BYTES];
+    // Workgroups go to the eight dies in turn: all row tiles of a (sequence, key/value head) on one die, whose L2 then reads its
+    // keys and values once (by_die; with few pairs the row tiles are dealt to the dies instead)
+    int pair = blockIdx.x / tiles, xt = blockIdx.x - pair * tiles;
+    if (by_die) {
+        const int j = blockIdx.x >> 3;
+        pair = j / tiles;
+        xt = j - pair * tiles;
+        pair = 8 * pair + (blockIdx.x & 7);
+    }
+    const int b = pair / G, g = pair - b * G, rep = H / G;
+    if (b >= B) return;
     const int q0 = qstart[b], rows = (qstart[b + 1] - q0) * rep;
-    const int tile0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 128;            // heaviest tiles first
+    const int tile0 = (tiles - 1 - xt) * 128;                                  // heaviest tiles first
     if (tile0 >= rows) return;
     const int pos0 = seq_pos0[b];
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
@@ -50,14 +63,22 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(const unsigned short* _
     const int wave_min_pos = pos0 + min(tile0 + 32 * wave, rows - 1) / rep;
     const int n_keys = pos0 + min(tile0 + 127, rows - 1) / rep + 1;
     const int wave_max_pos = pos0 + min(tile0 + 32 * wave + 31, rows - 1) / rep;
-    const TileWalk walk = make_walk(pos0 + tile0 / rep, n_keys - 1, window, keep_first, pool, chunk);
     const float unit = MODE == kSoftcap ? softcap : scale, c_log2 = unit * 1.4426950408889634f;      // what a raw score is worth
     const float pre = mode_pre<MODE>(scale, softcap, head_bias, head);
     f32x16 oacc[NBV];
     float m_run, l_tot;
-    kv_tile_loop<NBK, NBV, 4, MODE>(q + ((size_t)(q0 + tok) * H + head) * D, kc, vc, block_tables + (size_t)b * max_blocks, D, V, G, g,
-                                   block_size, walk, 0, walk.count(n_keys), n_keys, row_pos, wave_min_pos, wave_max_pos, window, keep_first, c_log2,
-                                   kp, vp, pool, pool_rows, lds_k, lds_v, oacc, m_run, l_tot, chunk, pre);
+    const unsigned short* qrow = q + ((size_t)(q0 + tok) * H + head) * D;
+    if constexpr (SLIM) {
+        const auto walk = make_walk<kSlimKeys>(pos0 + tile0 / rep, n_keys - 1, window, keep_first, pool, chunk);
+        kv_slim_loop<NBK, NBV, MODE>(qrow, kc, vc, block_tables + (size_t)b * max_blocks, G, g, block_size, walk, walk.count(n_keys), n_keys,
+                                     row_pos, wave_min_pos, wave_max_pos, window, keep_first, c_log2, kp, vp, pool, pool_rows, lds_k, lds_v,
+                                     oacc, m_run, l_tot, chunk, pre);
+    } else {
+        const auto walk = make_walk(pos0 + tile0 / rep, n_keys - 1, window, keep_first, pool, chunk);
+        kv_tile_loop<NBK, NBV, 4, MODE>(qrow, kc, vc, block_tables + (size_t)b * max_blocks, D, V, G, g, block_size, walk, 0,
+                                        walk.count(n_keys), n_keys, row_pos, wave_min_pos, wave_max_pos, window, keep_first, c_log2, kp, vp,
+                                        pool, pool_rows, lds_k, lds_v, oacc, m_run, l_tot, chunk, pre);
+    }
     if (r >= rows) return;
     // the sink joins the denominator with its own score, which is not scaled (m_run is finite: a row sees itself);
     // sigmoid weights are not normalised
@@ -97,7 +118,7 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(const unsigned short* _
     __shared__ __attribute__((aligned(16))) unsigned char lds_v[TileGeom<NBV>::LDS_BYTES];
     const int sp = blockIdx.x, b = blockIdx.y, g = blockIdx.z, rep = H / G;
     const int n = ctx[b];
-    const TileWalk walk = make_walk(n - 1, n - 1, window, keep_first, pool, chunk);
+    const auto walk = make_walk(n - 1, n - 1, window, keep_first, pool, chunk);
     const int nt = walk.count(n), per = (nt + splits - 1) / splits;
     const int vt_lo = sp * per, vt_hi = min(nt, vt_lo + per);
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
@@ -237,17 +258,24 @@ extern "C" int hm_attn_tiles(const void* q, const void* k_cache, const void* v_c
     }
     if (B == 0 || max_q == 0) return HM_OK;
     const int64_t tiles = ((int64_t)max_q * (H / G) + 127) / 128;
-    dim3 grid((unsigned)tiles, (unsigned)B, (unsigned)G), block(256);
+    const int64_t pairs = (int64_t)B * G;
+    const int by_die = pairs >= 32 || pairs % 8 == 0;          // (fewer pairs would leave dies idle)
+    const int64_t groups = (by_die ? (pairs + 7) / 8 * 8 : pairs) * tiles;
+    if (groups > 0x7fffffff) { set_error("hm_attn_tiles: too many rows"); return HM_ESHAPE; }
+    dim3 grid((unsigned)groups), block(256);
     hipStream_t s = as_stream(stream);
     const int nbk = padded_nb(D), nbv = padded_nb(V);
+    const bool slim = D == 32 * nbk && V == 32 * nbv;
     const OutArgs out = {o_stride, (const unsigned short*)gate, gate_stride, out_scale};
-#define HM_TILES(K_, V_, S_)                                                                                                 \
-    hipLaunchKernelGGL((attn_tiles_kernel<K_, V_, S_>), grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k_cache, \
+#define HM_TILES(K_, V_, S_) do { if (slim) HM_TILES_(K_, V_, S_, true); else HM_TILES_(K_, V_, S_, false); } while (0)
+#define HM_TILES_(K_, V_, S_, SLIM_)                                                                                         \
+    hipLaunchKernelGGL((attn_tiles_kernel<K_, V_, S_, SLIM_>), grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k_cache, \
                        (const unsigned short*)v_cache, block_tables, qstart, seq_pos0, sink, window, keep_first, scale,       \
                        (unsigned short*)o, H, G, D, V, block_size, max_blocks, (const unsigned short*)kp_cache,               \
-                       (const unsigned short*)vp_cache, pool, pool_rows, chunk, head_bias, softcap, out)
+                       (const unsigned short*)vp_cache, pool, pool_rows, chunk, head_bias, softcap, out, B, (int)tiles, by_die)
     HM_BY_HEAD_SIZE(nbk, nbv, sigmoid_w, softcap, HM_TILES);
 #undef HM_TILES
+#undef HM_TILES_
     HM_CHECK_LAUNCH("hm_attn_tiles");
     return HM_OK;
 }

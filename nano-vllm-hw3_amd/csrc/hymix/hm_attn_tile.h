@@ -32,30 +32,32 @@ struct TileGeom {
     static constexpr int P = 32 * NB, CH = P / 8, RS = P * 2 + 16, LDS_BYTES = kTileKeys * RS;
 };
 
-// The list of tiles a group of rows walks.  keep_tiles tiles from key 0, then tiles from key win_lo (a multiple of 64,
-// >= 64 keep_tiles) up to the causal end.
+// The list of tiles of TK keys a group of rows walks.  keep_tiles tiles from key 0, then tiles from key win_lo (a multiple of
+// TK, >= TK keep_tiles) up to the causal end.
+template <int TK = kTileKeys>
 struct TileWalk {
     int pool_tiles, n_pool, keep_tiles, win_lo;
-    // first key of token tile vt (vt >= pool_tiles); a pooled tile vt < pool_tiles starts at entry 64 vt
+    // first key of token tile vt (vt >= pool_tiles); a pooled tile vt < pool_tiles starts at entry TK vt
     __device__ __forceinline__ int key0(int vt) const {
         const int u = vt - pool_tiles;
-        return u < keep_tiles ? u * kTileKeys : win_lo + (u - keep_tiles) * kTileKeys;
+        return u < keep_tiles ? u * TK : win_lo + (u - keep_tiles) * TK;
     }
     __device__ __forceinline__ int count(int n_keys) const {
-        return pool_tiles + keep_tiles + (n_keys - win_lo + kTileKeys - 1) / kTileKeys;
+        return pool_tiles + keep_tiles + (n_keys - win_lo + TK - 1) / TK;
     }
 };
 
 // min_pos / max_pos = the smallest / largest position among the rows that walk together
 // chunk > 0: a row also sees nothing before the start of its own chunk of `chunk` positions
-__device__ __forceinline__ TileWalk make_walk(int min_pos, int max_pos, int window, int keep_first, int pool, int chunk = 0) {
-    TileWalk w;
+template <int TK = kTileKeys>
+__device__ __forceinline__ TileWalk<TK> make_walk(int min_pos, int max_pos, int window, int keep_first, int pool, int chunk = 0) {
+    TileWalk<TK> w;
     w.n_pool = pooled_seen(max_pos, window, pool);
-    w.pool_tiles = (w.n_pool + kTileKeys - 1) / kTileKeys;
+    w.pool_tiles = (w.n_pool + TK - 1) / TK;
     int lo = window > 0 ? max(0, min_pos - window + 1) : 0;
     if (chunk > 0) lo = max(lo, min_pos / chunk * chunk);
-    w.win_lo = lo / kTileKeys * kTileKeys;
-    w.keep_tiles = window > 0 ? min((keep_first + kTileKeys - 1) / kTileKeys, w.win_lo / kTileKeys) : 0;
+    w.win_lo = lo / TK * TK;
+    w.keep_tiles = window > 0 ? min((keep_first + TK - 1) / TK, w.win_lo / TK) : 0;
     return w;
 }
 
@@ -71,7 +73,7 @@ constexpr int kSoftmax = 0, kSigmoid = 1, kSoftcap = 2;
 template <int NBK, int NBV, int WAVES, int MODE = kSoftmax>
 __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ qrow, const unsigned short* __restrict__ kc,
                                              const unsigned short* __restrict__ vc, const int32_t* __restrict__ table, int D, int V,
-                                             int G, int g, int block_size, TileWalk walk, int vt_lo, int vt_hi, int n_keys,
+                                             int G, int g, int block_size, TileWalk<> walk, int vt_lo, int vt_hi, int n_keys,
                                              int row_pos, int wave_min_pos, int wave_max_pos, int window, int keep_first, float c_log2,
                                              const unsigned short* __restrict__ kp, const unsigned short* __restrict__ vp,
                                              int pool, int pool_rows, unsigned char* lds_k, unsigned char* lds_v, f32x16 (&oacc)[NBV], float& m_run,
@@ -278,6 +280,203 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
             store_tile();
             __syncthreads();
         }
+    }
+    l_tot = l_run + __shfl_xor(l_run, 32);
+    if (SIG) { m_run = 0.f; l_tot = 1.f; }
+}
+
+// The same walk for head sizes of exactly 32 NBK and 32 NBV channels, whose tiles go from global memory straight to LDS: two
+// buffers, one barrier per tile.  The loop above holds a tile in registers on its way (a wave then has 350 of them and its SIMD
+// to itself, with nothing to fill its waits; held to 256 it takes 110 us where this one takes 83 and the first took 174: eight
+// prompts of about 1000 tokens, 16 / 8 heads of 128, a window of 512, capped scores).  What is left is the vector unit's:
+// three exponentials or reciprocals per capped score.  Tiles of 32 keys, which fit three waves, measured the same.
+// A row of 2 P bytes is kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows
+// that differ mod 16, one chunk) and the 32 of a transposed read (four rows, four chunks) then touch every bank once.  A
+// wave none of whose rows sees a tile leaves it out: a masked score would add an exact zero.
+constexpr int kSlimKeys = 64, kSlimParts = kSlimKeys / 32;
+
+template <int NB>
+struct SlimGeom {
+    static constexpr int P = 32 * NB, CH = P / 8, RB = 2 * P, BYTES = kSlimKeys * RB, PIECES = BYTES / 1024;
+    __device__ static __forceinline__ int swz(int r) {
+        return CH % 16 == 0 ? ((r & 3) << 2 | (r >> 2 & 3)) : CH % 8 == 0 ? ((r >> 1 & 1) << 2 | (r >> 2 & 3)) : (r >> 2 & 3);
+    }
+    __device__ static __forceinline__ int at(int r, int ch) { return RB * r + 16 * (ch ^ swz(r)); }
+};
+
+template <int NBK, int NBV, int MODE>
+__device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ qrow, const unsigned short* __restrict__ kc,
+                                             const unsigned short* __restrict__ vc, const int32_t* __restrict__ table, int G, int g,
+                                             int block_size, TileWalk<kSlimKeys> walk, int nt, int n_keys, int row_pos, int wave_min_pos,
+                                             int wave_max_pos, int window, int keep_first, float c_log2,
+                                             const unsigned short* __restrict__ kp, const unsigned short* __restrict__ vp, int pool,
+                                             int pool_rows, unsigned char* buf0, unsigned char* buf1, f32x16 (&oacc)[NBV], float& m_run,
+                                             float& l_tot, int chunk, float pre) {
+    constexpr bool SIG = MODE == kSigmoid;
+    typedef SlimGeom<NBK> GK;
+    typedef SlimGeom<NBV> GV;
+    typedef __attribute__((address_space(1))) const void gvoid;
+    typedef __attribute__((address_space(3))) void lvoid;
+    const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    bf16x8 qf[2 * NBK];                                    // Q^T as the B operand: k-step ks = columns 16 ks + 8 hi .. +8
+#pragma unroll
+    for (int ks = 0; ks < 2 * NBK; ++ks) qf[ks] = *(const bf16x8*)(qrow + 16 * ks + 8 * hi);
+
+    // one tile: pieces of 1 KB, dealt to the four waves; lane l of a piece brings the chunk that belongs at 16 l
+    auto load_part = [&](auto geom, unsigned char* to, const unsigned short* src, const unsigned short* psrc, int vt, int kt0, size_t row0) {
+        typedef decltype(geom) GG;
+        constexpr int LPR = GG::CH;                        // lanes per row
+#pragma unroll
+        for (int i0 = 0; i0 < GG::PIECES; i0 += 4) {
+            const int i = i0 + wave;
+            if (GG::PIECES < 4 && i >= GG::PIECES) break;
+            const int row = i * (64 / LPR) + lane / LPR, ch = (lane % LPR) ^ GG::swz(row);
+            const unsigned short* from;
+            if (vt < walk.pool_tiles) {                    // pooled entries, each found through the block table
+                const int e = min(vt * kSlimKeys + row, walk.n_pool - 1);
+                from = psrc + (((size_t)table[e / pool_rows] * pool_rows + e % pool_rows) * G + g) * GG::P;
+            } else {
+                from = src + ((row0 + min(row, n_keys - 1 - kt0)) * G + g) * GG::P;
+            }
+            __builtin_amdgcn_global_load_lds((gvoid*)(from + 8 * ch), (lvoid*)(to + 1024 * i), 16, 0, 0);
+        }
+    };
+    auto load_tile = [&](unsigned char* buf, int vt) {
+        int kt0 = 0;
+        size_t row0 = 0;
+        if (vt >= walk.pool_tiles) {                       // (a tile lies in one cache block)
+            kt0 = __builtin_amdgcn_readfirstlane(walk.key0(vt));
+            const int page = kt0 / block_size;
+            row0 = (size_t)table[page] * block_size + (kt0 - page * block_size);
+        }
+        load_part(GK(), buf, kc, kp, vt, kt0, row0);
+        load_part(GV(), buf + GK::BYTES, vc, vp, vt, kt0, row0);
+    };
+    auto landed = [&]() {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+
+#pragma unroll
+    for (int d = 0; d < NBV; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
+    m_run = -INFINITY;
+    float l_run = 0.f;
+    const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;      // transposed-read address pieces
+    // a chunk's number enters its place by exclusive or: the reads' addresses are one base each, changed in the chunk's bits
+    const int k_at = GK::at(l31, hi), v_at = GV::at(4 * hi + tq, 2 * gq + (tp >> 1)) + 8 * (tp & 1),
+              v_at8 = GV::at(4 * hi + tq + 8, 2 * gq + (tp >> 1)) + 8 * (tp & 1);
+    const int my_pool = pooled_seen(row_pos, window, pool);
+    const int chunk_lo = chunk > 0 ? row_pos / chunk * chunk : 0;
+    const int wave_chunk_lo = chunk > 0 ? wave_max_pos / chunk * chunk : 0, wave_chunk_first = chunk > 0 ? wave_min_pos / chunk * chunk : 0;
+
+    auto work = [&](const unsigned char* buf, int vt) {
+        const bool pooled = vt < walk.pool_tiles;
+        const int kt0 = pooled ? vt * kSlimKeys : walk.key0(vt), kt1 = kt0 + kSlimKeys - 1;
+        if (!pooled && (kt0 > wave_max_pos || kt1 < wave_chunk_first || (window > 0 && wave_min_pos - kt1 >= window && kt0 >= keep_first)))
+            return;
+        f32x16 s[kSlimParts];
+#pragma unroll
+        for (int j = 0; j < kSlimParts; ++j) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[j][r] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < 2 * NBK; ++ks) {
+                const bf16x8 kf = *(const bf16x8*)(buf + (k_at ^ (32 * ks)) + 32 * GK::RB * j);        // row 32 j + l31, chunk 2 ks + hi
+                s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[j], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kSlimParts; ++j) {
+            if (SIG) {                                       // the logit in log2 units, before the mask
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[j][r] = __builtin_fmaf(s[j][r], c_log2, pre);
+            }
+            if (MODE == kSoftcap) {                          // tanh(z) = 1 - 2 / (1 + e^2z); both infinities come out right
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    s[j][r] = 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[j][r] * pre));
+            }
+        }
+        if (pooled) {
+#pragma unroll
+            for (int j = 0; j < kSlimParts; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi >= my_pool) s[j][r] = -INFINITY;
+        } else if (kt1 > wave_min_pos || (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo) {
+            // (a tile that every row of the wave sees whole needs no mask)
+#pragma unroll
+            for (int j = 0; j < kSlimParts; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi;
+                    const bool seen = key <= row_pos && key >= chunk_lo && (window <= 0 || row_pos - key < window || key < keep_first);
+                    if (!seen) s[j][r] = -INFINITY;
+                }
+        }
+        bf16x8 pf[2 * kSlimParts];
+        if (SIG) {
+#pragma unroll
+            for (int t = 0; t < 2 * kSlimParts; ++t)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)              // a masked logit is -inf: exp2(+inf) = inf and the weight is 0
+                    pf[t][e] = (bf16_t)__builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-s[t >> 1][8 * (t & 1) + e]));
+        } else {
+            float mx = s[0][0];
+#pragma unroll
+            for (int j = 0; j < kSlimParts; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[j][r]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float m_new = fmaxf(m_run, mx);
+            const bool none = m_new == -INFINITY;            // the row has seen nothing yet: no rescale, and every weight is zero
+            const float alpha = none ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_log2);
+            const float mc = none ? 0.f : m_new * c_log2;
+            float psum = 0.f;
+#pragma unroll
+            for (int t = 0; t < 2 * kSlimParts; ++t)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t >> 1][8 * (t & 1) + e], c_log2, -mc));
+                    psum += p;
+                    pf[t][e] = (bf16_t)p;
+                }
+            l_run = l_run * alpha + psum;
+            m_run = m_new;
+            if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+                for (int d = 0; d < NBV; ++d)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) oacc[d][r] *= alpha;
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < NBV; ++d)
+#pragma unroll
+            for (int t = 0; t < 2 * kSlimParts; ++t) {
+                // rows 16 t + 4 hi + tq and 8 further on, chunk 4 d + 2 gq + tp / 2
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (s16x4 __attribute__((address_space(3)))*)(buf + GK::BYTES + (v_at ^ (64 * d)) + 16 * GV::RB * t));
+                const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (s16x4 __attribute__((address_space(3)))*)(buf + GK::BYTES + (v_at8 ^ (64 * d)) + 16 * GV::RB * t));
+                const s16x8 vv = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pf[t], oacc[d], 0, 0, 0);
+            }
+    };
+    load_tile(buf0, 0);
+    landed();
+    for (int vt = 0; vt < nt; vt += 2) {
+        if (vt + 1 < nt) load_tile(buf1, vt + 1);
+        work(buf0, vt);
+        landed();
+        if (vt + 1 >= nt) break;
+        if (vt + 2 < nt) load_tile(buf0, vt + 2);
+        work(buf1, vt + 1);
+        landed();
     }
     l_tot = l_run + __shfl_xor(l_run, 32);
     if (SIG) { m_run = 0.f; l_tot = 1.f; }

@@ -13,40 +13,56 @@
 // The k index of the second product is the KEY; its order inside a 16-key MFMA step is free as long
 // as both operands agree, and it is chosen to be exactly the order in which the S^T accumulator
 // registers already hold the keys - P never moves between lanes.
-// K/V tiles (64 keys) are staged through one LDS image per tensor, 256-byte rows with an XOR swizzle of
-// the 16-byte chunk index that keeps both the row reads (K) and the transposed reads (V) conflict-free;
-// the next tile's global loads are issued before the current tile's math and land in LDS after it.
+// K/V tiles (64 keys) go from global memory straight to LDS, 256-byte rows with an XOR swizzle of the 16-byte chunk
+// index that keeps both the row reads (K) and the transposed reads (V) conflict-free: two buffers, one barrier per
+// tile, the next tile's loads issued before the current tile's math.  Held in registers on its way a tile made it 294
+// per wave, one wave per SIMD, and nothing filled its waits; at 191 two waves run one's exponentials beside the
+// other's products: 8 prompts of 1024 tokens, 16 / 8 heads, 133 -> 74 us, one of 4096 tokens 222 -> 110, two of 1024 34 -> 30.
+// (Tiles of 32 keys fit three waves and are no faster with full CUs, 76 and 128 us, and slower where a CU has one
+// workgroup and a tile's chain of dependent steps is what counts: 128 us and 38.)
 #include "ql_common.h"
 
 namespace ql {
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTileKeys = 64;
+
+constexpr int kTileKeys = 64, NH = kTileKeys / 32;
 
 __device__ __forceinline__ int kv_off(int row, int ch) {
     return 256 * row + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
 template <int G>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(const unsigned short* __restrict__ q,
-                                                           const unsigned short* __restrict__ k,
-                                                           const unsigned short* __restrict__ v,
-                                                           const int* __restrict__ cu_seqlens,
-                                                           unsigned short* __restrict__ out, float c_log2, int Hq,
-                                                           int Hkv, int kv_group) {
+__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const unsigned short* __restrict__ q,
+                                                              const unsigned short* __restrict__ k,
+                                                              const unsigned short* __restrict__ v,
+                                                              const int* __restrict__ cu_seqlens,
+                                                              unsigned short* __restrict__ out, float c_log2, int Hq,
+                                                              int Hkv, int kv_group, int blocks, int pairs, int by_die) {
     constexpr int SUBS = 4 / G;            // 32-row query blocks per head in this workgroup
     constexpr int QROWS = 32 * SUBS;
-    __shared__ __attribute__((aligned(256))) unsigned char k_lds[kTileKeys * 256];
-    __shared__ __attribute__((aligned(256))) unsigned char v_lds[kTileKeys * 256];
+    constexpr int V_AT = kTileKeys * 256;  // the value tile behind the key tile
+    __shared__ __attribute__((aligned(1024))) unsigned char buf0[2 * kTileKeys * 256];
+    __shared__ __attribute__((aligned(1024))) unsigned char buf1[2 * kTileKeys * 256];
 
-    // blockIdx.y counts groups of G query heads; a group reads the K/V of kv head (group * G) / kv_group, which is
-    // the group itself when a kv head's query heads form one group (kv_group == G: ratios 1, 2, 4); other ratios
-    // are dealt to several groups per kv head
-    const int seq = blockIdx.z, hgrp = blockIdx.y, hk = (hgrp * G) / kv_group;
+    // Workgroups go to the eight dies in turn: all query blocks of a (sequence, group of heads) on one die, whose L2 then
+    // reads its keys and values once (by_die; with few such pairs the query blocks are dealt to the dies instead)
+    int pair = blockIdx.x / blocks, xb = blockIdx.x - pair * blocks;
+    if (by_die) {
+        const int j = blockIdx.x >> 3;
+        pair = j / blocks;
+        xb = j - pair * blocks;
+        pair = 8 * pair + (blockIdx.x & 7);
+    }
+    if (pair >= pairs) return;
+    // a group of G query heads reads the K/V of kv head (group * G) / kv_group, which is the group itself when a kv
+    // head's query heads form one group (kv_group == G: ratios 1, 2, 4); other ratios are dealt to several groups per
+    // kv head
+    const int ngroups = Hq / G, seq = pair / ngroups, hgrp = pair - seq * ngroups, hk = (hgrp * G) / kv_group;
     const int s0 = cu_seqlens[seq];
     const int L = cu_seqlens[seq + 1] - s0;
-    const int q0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * QROWS;      // heaviest query blocks first
+    const int q0 = (blocks - 1 - xb) * QROWS;                           // heaviest query blocks first
     if (q0 >= L) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -66,25 +82,23 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const unsigned short*
         for (int ks = 0; ks < 8; ++ks) qf[ks] = *(const bf16x8*)(qp + 16 * ks);
     }
 
-    // cooperative tile staging: thread moves chunks c = tid + 256*j: row c >> 4, 16-byte chunk c & 15
-    const int st_row = tid >> 4, st_ch = tid & 15;
-    i32x4 kreg[4], vreg[4];
-    auto load_tile = [&](int kt0) {
+    // a tile: eight pieces of 1 KB (four rows) per tensor, two per wave; lane l brings the chunk that belongs at 16 l
+    typedef __attribute__((address_space(1))) const void gvoid;
+    typedef __attribute__((address_space(3))) void lvoid;
+    const unsigned short *ks0 = k + ((size_t)s0 * Hkv + hk) * 128, *vs0 = v + ((size_t)s0 * Hkv + hk) * 128;
+    auto load_tile = [&](unsigned char* buf, int kt0) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int key = min(kt0 + st_row + 16 * j, L - 1);
-            const size_t off = ((size_t)(s0 + key) * Hkv + hk) * 128 + st_ch * 8;
-            kreg[j] = *(const i32x4*)(k + off);
-            vreg[j] = *(const i32x4*)(v + off);
+        for (int j = 0; j < 2 * NH; ++j) {
+            const int i = wave + 4 * j, row = 4 * i + (lane >> 4);
+            const int ch = (lane & 15) ^ (((row & 3) << 2) | ((row >> 2) & 3));
+            const size_t off = (size_t)min(kt0 + row, L - 1) * Hkv * 128 + 8 * ch;
+            __builtin_amdgcn_global_load_lds((gvoid*)(ks0 + off), (lvoid*)(buf + 1024 * i), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gvoid*)(vs0 + off), (lvoid*)(buf + V_AT + 1024 * i), 16, 0, 0);
         }
     };
-    auto store_tile = [&]() {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int o = kv_off(st_row + 16 * j, st_ch);
-            *(i32x4*)(k_lds + o) = kreg[j];
-            *(i32x4*)(v_lds + o) = vreg[j];
-        }
+    auto landed = [&]() {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
     };
 
     f32x16 oacc[4];
@@ -94,37 +108,30 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const unsigned short*
         for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
     float m_run = -INFINITY, l_run = 0.f;
 
-    // transposed-read address pieces of this lane: 16-lane group gq picks dims 16*gq .. +16 of a 32-dim block
+    // Transposed-read address pieces of this lane: 16-lane group gq picks dims 16*gq .. +16 of a 32-dim block.  A chunk's
+    // number enters its place by exclusive or, so the reads' addresses are one base each, changed in the chunk's bits.
     const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;
+    const int k_at = kv_off(l31, hi), v_at = kv_off(4 * hi + tq, 2 * gq + (tp >> 1)) + 8 * (tp & 1),
+              v_at8 = kv_off(4 * hi + tq + 8, 2 * gq + (tp >> 1)) + 8 * (tp & 1);
 
-    load_tile(0);
-    store_tile();
-    __syncthreads();
-    // Pin the Q fragments as loaded HERE.  Otherwise their loads are sunk to the loop entry, and because the
-    // wait counter is positional every MFMA of the loop that reads them also waits for the next tile's K/V
-    // loads issued just before it: the prefetch would have to land within the first product of each tile.
+    auto work = [&](const unsigned char* buf, int kt0) {
+        if (kt0 > qw0 + 31) return;                                  // no row of this wave sees the tile
+        // ---- S^T = K . Q^T
+        f32x16 s[NH];
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) asm volatile("" ::"v"(__builtin_bit_cast(i32x4, qf[ks])));
-    for (int it = 0; it < ntiles; ++it) {
-        const int kt0 = it * kTileKeys;
-        if (it + 1 < ntiles) load_tile(kt0 + kTileKeys);
-
-        // ---- S^T = K . Q^T for the two 32-key halves of the tile
-        f32x16 s[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NH; ++j) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[j][r] = 0.f;
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks) {
-                const bf16x8 kf = *(const bf16x8*)(k_lds + kv_off(32 * j + l31, 2 * ks + hi));
+                const bf16x8 kf = *(const bf16x8*)(buf + (k_at ^ (32 * ks)) + 8192 * j);
                 s[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[j], 0, 0, 0);
             }
         }
         // ---- causal mask (only tiles that reach past this wave's first query) and online softmax
         if (kt0 + kTileKeys - 1 > qw0) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < NH; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int key = kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi;
@@ -133,25 +140,23 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const unsigned short*
         }
         float mx = s[0][0];
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NH; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[j][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));                          // the other 32 keys of this query
+        mx = fmaxf(mx, __shfl_xor(mx, 32));                          // the other half of this query's keys
         const float m_new = fmaxf(m_run, mx);                        // finite: key 0 is visible to every query
         const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c_log2);
         const float mc = m_new * c_log2;
         float psum = 0.f;
-        bf16x8 pf[2][2];                                             // P^T fragments: [32-key half][16-key step]
+        bf16x8 pf[2 * NH];                                           // P^T fragments, 16 keys each
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int t = 0; t < 2 * NH; ++t)
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][8 * t + e], c_log2, -mc));
-                    psum += p;
-                    pf[j][t][e] = (bf16_t)p;
-                }
+            for (int e = 0; e < 8; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t >> 1][8 * (t & 1) + e], c_log2, -mc));
+                psum += p;
+                pf[t][e] = (bf16_t)p;
+            }
         l_run = l_run * alpha + psum;
         m_run = m_new;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {        // skip the rescale while no maximum moved
@@ -160,28 +165,30 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const unsigned short*
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[d][r] *= alpha;
         }
-        // ---- O^T += V^T . P^T
+        // ---- O^T += V^T . P^T: rows 16 t + 4 hi + tq and 8 further on, chunk 4 d + 2 gq + tp / 2
 #pragma unroll
         for (int d = 0; d < 4; ++d)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const int r0 = 32 * j + 16 * t + 4 * hi;
-                    const int c0 = 4 * d + 2 * gq;
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (s16x4 __attribute__((address_space(3)))*)(v_lds + kv_off(r0 + tq, c0 + (tp >> 1)) + 8 * (tp & 1)));
-                    const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (s16x4 __attribute__((address_space(3)))*)(v_lds + kv_off(r0 + 8 + tq, c0 + (tp >> 1)) + 8 * (tp & 1)));
-                    typedef short s16x8 __attribute__((ext_vector_type(8)));
-                    const s16x8 vv = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
-                    oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pf[j][t], oacc[d], 0, 0, 0);
-                }
-        __syncthreads();                                             // every wave is done with this tile
-        if (it + 1 < ntiles) {
-            store_tile();
-            __syncthreads();
-        }
+            for (int t = 0; t < 2 * NH; ++t) {
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (s16x4 __attribute__((address_space(3)))*)(buf + V_AT + (v_at ^ (64 * d)) + 4096 * t));
+                const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (s16x4 __attribute__((address_space(3)))*)(buf + V_AT + (v_at8 ^ (64 * d)) + 4096 * t));
+                typedef short s16x8 __attribute__((ext_vector_type(8)));
+                const s16x8 vv = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pf[t], oacc[d], 0, 0, 0);
+            }
+    };
+    load_tile(buf0, 0);
+    landed();
+    for (int it = 0; it < ntiles; it += 2) {
+        if (it + 1 < ntiles) load_tile(buf1, (it + 1) * kTileKeys);
+        work(buf0, it * kTileKeys);
+        landed();
+        if (it + 1 >= ntiles) break;
+        if (it + 2 < ntiles) load_tile(buf0, (it + 2) * kTileKeys);
+        work(buf1, (it + 1) * kTileKeys);
+        landed();
     }
 
     // ---- normalise and store: lane holds dims 32*d + 8*(r>>2) + 4*hi + (r&3) of its query
@@ -216,13 +223,17 @@ extern "C" int ql_attn_prefill(const void* q, const void* k, const void* v, cons
     const int G = (kv_group % 4 == 0) ? 4 : (kv_group % 2 == 0) ? 2 : 1;     // query heads per workgroup
     if (num_seqs == 0 || max_seqlen == 0) return QL_OK;
     if (num_seqs > 65535 || Hq / G > 65535) { set_error("ql_attn_prefill: too many sequences or heads"); return QL_ESHAPE; }
-    const int qrows = 128 / G;
-    dim3 grid((unsigned)((max_seqlen + qrows - 1) / qrows), (unsigned)(Hq / G), (unsigned)num_seqs), block(256);
+    const int qrows = 128 / G, blocks = (max_seqlen + qrows - 1) / qrows;
+    const int64_t pairs = (int64_t)num_seqs * (Hq / G);
+    const int by_die = pairs >= 32 || pairs % 8 == 0;
+    const int64_t groups = (by_die ? (pairs + 7) / 8 * 8 : pairs) * blocks;
+    if (groups > 0x7fffffff) { set_error("ql_attn_prefill: too many rows"); return QL_ESHAPE; }
+    dim3 grid((unsigned)groups), block(256);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
 #define QL_PF(G_)                                                                                              \
     hipLaunchKernelGGL(attn_prefill_kernel<G_>, grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k, \
-                       (const unsigned short*)v, cu_seqlens, (unsigned short*)out, c, Hq, Hkv, kv_group)
+                       (const unsigned short*)v, cu_seqlens, (unsigned short*)out, c, Hq, Hkv, kv_group, blocks, (int)pairs, by_die)
     if (G == 1) QL_PF(1); else if (G == 2) QL_PF(2); else QL_PF(4);
 #undef QL_PF
     QL_CHECK_LAUNCH("ql_attn_prefill");

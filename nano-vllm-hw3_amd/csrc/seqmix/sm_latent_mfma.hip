@@ -5,20 +5,31 @@
 
 namespace sm {
 
-template <int NB, int NBV>
-__global__ __launch_bounds__(256) void latent_attn_tiles_kernel(const unsigned short* __restrict__ q,
+// SLIM: rows of exactly 32 NB columns, in the loop of 32-key tiles (latent_slim_loop)
+template <int NB, int NBV, bool SLIM>
+__global__ __launch_bounds__(256, SLIM ? 2 : 1) void latent_attn_tiles_kernel(const unsigned short* __restrict__ q,
                                                                 const unsigned short* __restrict__ cache,
                                                                 const int32_t* __restrict__ block_tables,
                                                                 const int32_t* __restrict__ qstart,
                                                                 const int32_t* __restrict__ seq_pos0,
                                                                 unsigned short* __restrict__ o, float c_log2, int H, int R,
                                                                 int block_size, int max_blocks, int RV, int window,
-                                                                const float* __restrict__ sink) {
-    typedef TileGeom<NB> G;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[G::LDS_BYTES];
-    const int b = blockIdx.y;
+                                                                const float* __restrict__ sink, int B, int tiles, int by_die) {
+    // (the slim loop has two buffers of half a tile)
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[SLIM ? SlimGeom<NB>::BYTES : TileGeom<NB>::LDS_BYTES];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds2[SLIM ? SlimGeom<NB>::BYTES : 16];
+    // Workgroups go to the eight dies in turn: all row tiles of a sequence on one die, whose L2 then reads its rows once (by_die;
+    // with few sequences the row tiles are dealt to the dies instead)
+    int b = blockIdx.x / tiles, xt = blockIdx.x - b * tiles;
+    if (by_die) {
+        const int j = blockIdx.x >> 3;
+        b = j / tiles;
+        xt = j - b * tiles;
+        b = 8 * b + (blockIdx.x & 7);
+    }
+    if (b >= B) return;
     const int q0 = qstart[b], rows = (qstart[b + 1] - q0) * H;
-    const int tile0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 128;            // heaviest tiles first
+    const int tile0 = (tiles - 1 - xt) * 128;                                  // heaviest tiles first
     if (tile0 >= rows) return;
     const int pos0 = seq_pos0[b];
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
@@ -29,11 +40,20 @@ __global__ __launch_bounds__(256) void latent_attn_tiles_kernel(const unsigned s
     const int wave_min_pos = pos0 + min(tile0 + 32 * wave, rows - 1) / H;
     const int k_hi = pos0 + min(tile0 + 127, rows - 1) / H + 1;
     // with a window the walk starts at the tile that holds the first key the workgroup's first row sees
-    const int k_lo = window > 0 ? max(0, pos0 + tile0 / H - window + 1) / kTileKeys * kTileKeys : 0;
+    constexpr int TK = SLIM ? kSlimKeys : kTileKeys;
+    const int k_lo = window > 0 ? max(0, pos0 + tile0 / H - window + 1) / TK * TK : 0;
     f32x16 oacc[NBV];
     float m_run, l_tot;
-    latent_tile_loop<NB, NBV, 4>(q + ((size_t)q0 * H + rc) * R, cache, block_tables + (size_t)b * max_blocks, R, block_size, k_lo,
-                                 k_hi, row_pos, wave_min_pos, c_log2, window, lds, oacc, m_run, l_tot);
+    const unsigned short* qrow = q + ((size_t)q0 * H + rc) * R;
+    const int32_t* table = block_tables + (size_t)b * max_blocks;
+    if constexpr (SLIM) {
+        const int wave_max_pos = pos0 + min(tile0 + 32 * wave + 31, rows - 1) / H;
+        latent_slim_loop<NB, NBV>(qrow, cache, table, block_size, k_lo, k_hi, row_pos, wave_min_pos, wave_max_pos, c_log2, window, lds, lds2,
+                                  oacc, m_run, l_tot);
+    } else {
+        latent_tile_loop<NB, NBV, 4>(qrow, cache, table, R, block_size, k_lo, k_hi, row_pos, wave_min_pos, c_log2, window, lds, oacc, m_run,
+                                     l_tot);
+    }
     if (r >= rows) return;
     const float inv = sink ? sink_inv(m_run * c_log2, l_tot, sink[r % H]) : 1.f / l_tot;
     unsigned short* op = o + ((size_t)q0 * H + r) * RV + 4 * hi;
@@ -68,16 +88,21 @@ extern "C" int sm_latent_attn_tiles(const void* q, const void* cache, const int3
     }
     if (B == 0 || max_q == 0) return SM_OK;
     const int64_t tiles = ((int64_t)max_q * H + 127) / 128;
-    dim3 grid((unsigned)tiles, (unsigned)B), block(256);
+    const int by_die = B >= 32 || B % 8 == 0;
+    const int64_t groups = (by_die ? ((int64_t)B + 7) / 8 * 8 : B) * tiles;
+    if (groups > 0x7fffffff) { set_error("sm_latent_attn_tiles: too many rows"); return SM_ESHAPE; }
+    dim3 grid((unsigned)groups), block(256);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
     const int nb = (R + 31) / 32, nbv = (RV + 31) / 32;
-#define SM_TILES(NB_, NBV_)                                                                                               \
-    hipLaunchKernelGGL((latent_attn_tiles_kernel<NB_, NBV_>), grid, block, 0, s, (const unsigned short*)q,                 \
+#define SM_TILES(NB_, NBV_) do { if (R == 32 * NB_) SM_TILES_(NB_, NBV_, true); else SM_TILES_(NB_, NBV_, false); } while (0)
+#define SM_TILES_(NB_, NBV_, SLIM_)                                                                                       \
+    hipLaunchKernelGGL((latent_attn_tiles_kernel<NB_, NBV_, SLIM_>), grid, block, 0, s, (const unsigned short*)q,                 \
                        (const unsigned short*)cache, block_tables, qstart, seq_pos0, (unsigned short*)o, c, H, R, block_size, \
-                       max_blocks, RV, window, sink)
+                       max_blocks, RV, window, sink, B, (int)tiles, by_die)
     SM_BY_LATENT_SIZE(nb, nbv, SM_TILES);
 #undef SM_TILES
+#undef SM_TILES_
     SM_CHECK_LAUNCH("sm_latent_attn_tiles");
     return SM_OK;
 }

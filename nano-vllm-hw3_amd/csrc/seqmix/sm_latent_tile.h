@@ -172,6 +172,140 @@ __device__ __forceinline__ void latent_tile_loop(const unsigned short* __restric
     l_tot = l_run + __shfl_xor(l_run, 32);
 }
 
+// The same walk for cache rows of exactly 32 NB columns, in tiles of 32 keys that go from global memory straight to LDS (the loop
+// above holds a tile in registers on its way: a wave of 256 columns then needs nearly 400, one wave per SIMD, with nothing to
+// fill its waits).  Two buffers, one barrier per tile; with the scores and weights of 32 keys at a time two waves share a SIMD:
+// eight prompts of about 1000 tokens, 16 heads, rows of 192 + 64: 160 -> 81 us (0.65 PFLOP/s).  A row is kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows that differ
+// mod 16, one chunk) and the 32 of a transposed read (four rows, four chunks) touch every bank once.  A wave none of whose rows
+// sees a tile leaves it out: a masked score would add an exact zero.
+constexpr int kSlimKeys = 32;
+
+template <int NB>
+struct SlimGeom {
+    static constexpr int P = 32 * NB, CH = P / 8, RB = 2 * P, BYTES = kSlimKeys * RB, PIECES = BYTES / 1024;
+    __device__ static __forceinline__ int swz(int r) {
+        return CH % 16 == 0 ? ((r & 3) << 2 | (r >> 2 & 3)) : CH % 8 == 0 ? ((r >> 1 & 1) << 2 | (r >> 2 & 3)) : (r >> 2 & 3);
+    }
+    __device__ static __forceinline__ int at(int r, int ch) { return RB * r + 16 * (ch ^ swz(r)); }
+};
+
+template <int NB, int NBV>
+__device__ __forceinline__ void latent_slim_loop(const unsigned short* __restrict__ qrow, const unsigned short* __restrict__ cache,
+                                                 const int32_t* __restrict__ table, int block_size, int k_lo, int k_hi, int row_pos,
+                                                 int wave_min_pos, int wave_max_pos, float c_log2, int window, unsigned char* buf0,
+                                                 unsigned char* buf1, f32x16 (&oacc)[NBV], float& m_run, float& l_tot) {
+    typedef SlimGeom<NB> G;
+    typedef __attribute__((address_space(1))) const void gvoid;
+    typedef __attribute__((address_space(3))) void lvoid;
+    const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    bf16x8 qf[2 * NB];                                     // Q^T as the B operand: k-step ks = columns 16 ks + 8 hi .. +8
+#pragma unroll
+    for (int ks = 0; ks < 2 * NB; ++ks) qf[ks] = *(const bf16x8*)(qrow + 16 * ks + 8 * hi);
+
+    // one tile: pieces of 1 KB, dealt to the four waves; lane l of a piece brings the chunk that belongs at 16 l
+    auto load_tile = [&](unsigned char* buf, int kt0) {
+        const int page = __builtin_amdgcn_readfirstlane(kt0 / block_size);             // (a tile lies in one cache block)
+        const size_t row0 = (size_t)table[page] * block_size + (kt0 - page * block_size);
+#pragma unroll
+        for (int i0 = 0; i0 < G::PIECES; i0 += 4) {
+            const int i = i0 + wave;
+            if (G::PIECES % 4 != 0 && i >= G::PIECES) break;
+            const int c = 64 * i + lane, row = c / G::CH, ch = (c % G::CH) ^ G::swz(row);
+            __builtin_amdgcn_global_load_lds((gvoid*)(cache + (row0 + min(row, k_hi - 1 - kt0)) * G::P + 8 * ch), (lvoid*)(buf + 1024 * i),
+                                             16, 0, 0);
+        }
+    };
+    auto landed = [&]() {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+
+#pragma unroll
+    for (int d = 0; d < NBV; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
+    m_run = -INFINITY;
+    float l_run = 0.f;
+    const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;      // transposed-read address pieces
+    // Where the chunk's bits that an address steps through are none that the row changes by addition, the reads' addresses are one
+    // base each, changed by exclusive or.
+    constexpr bool XOR = G::CH % 16 == 0;
+    const int k_at = G::at(l31, hi), v_at = G::at(4 * hi + tq, 2 * gq + (tp >> 1)) + 8 * (tp & 1),
+              v_at8 = G::at(4 * hi + tq + 8, 2 * gq + (tp >> 1)) + 8 * (tp & 1);
+
+    auto work = [&](const unsigned char* buf, int kt0) {
+        const int kt1 = kt0 + kSlimKeys - 1;
+        if (kt0 > wave_max_pos || (window > 0 && wave_min_pos - kt1 >= window)) return;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < 2 * NB; ++ks) {
+            const bf16x8 cf = *(const bf16x8*)(buf + (XOR ? k_at ^ (32 * ks) : G::at(l31, 2 * ks + hi)));
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cf, qf[ks], s, 0, 0, 0);
+        }
+        if (kt1 > wave_min_pos || (window > 0 && wave_max_pos - kt0 >= window)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = kt0 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+                if (key > row_pos || (window > 0 && row_pos - key >= window)) s[r] = -INFINITY;
+            }
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        const float m_new = fmaxf(m_run, mx);
+        const bool none = m_new == -INFINITY;                // the row has seen nothing yet: no rescale, and every weight is zero
+        const float alpha = none ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_log2);
+        const float mc = none ? 0.f : m_new * c_log2;
+        float psum = 0.f;
+        bf16x8 pf[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * t + e], c_log2, -mc));
+                psum += p;
+                pf[t][e] = (bf16_t)p;
+            }
+        l_run = l_run * alpha + psum;
+        m_run = m_new;
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+            for (int d = 0; d < NBV; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) oacc[d][r] *= alpha;
+        }
+#pragma unroll
+        for (int d = 0; d < NBV; ++d)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                // rows 16 t + 4 hi + tq and 8 further on, chunk 4 d + 2 gq + tp / 2
+                const int a0 = XOR ? v_at ^ (64 * d) : G::at(4 * hi + tq, 4 * d + 2 * gq + (tp >> 1)) + 8 * (tp & 1);
+                const int a8 = XOR ? v_at8 ^ (64 * d) : G::at(4 * hi + tq + 8, 4 * d + 2 * gq + (tp >> 1)) + 8 * (tp & 1);
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(buf + a0 + 16 * G::RB * t));
+                const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(buf + a8 + 16 * G::RB * t));
+                const s16x8 vv = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
+                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vv), pf[t], oacc[d], 0, 0, 0);
+            }
+    };
+    load_tile(buf0, k_lo);
+    landed();
+    for (int kt0 = k_lo; kt0 < k_hi; kt0 += 2 * kSlimKeys) {
+        if (kt0 + kSlimKeys < k_hi) load_tile(buf1, kt0 + kSlimKeys);
+        work(buf0, kt0);
+        landed();
+        if (kt0 + kSlimKeys >= k_hi) break;
+        if (kt0 + 2 * kSlimKeys < k_hi) load_tile(buf0, kt0 + 2 * kSlimKeys);
+        work(buf1, kt0 + kSlimKeys);
+        landed();
+    }
+    l_tot = l_run + __shfl_xor(l_run, 32);
+}
+
 }  // namespace sm
 
 // run M(NB, NBV) with the padded key and value widths of a latent row: rows whose values are the whole row, and the

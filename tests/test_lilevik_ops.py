@@ -211,6 +211,49 @@ def test_matrix_core_attention_equals_portable(H, G, D, V, chunk):
         near(a, b.double().cpu(), dt, bf16=2e-2)
 
 
+# (B 8: the row tiles of a pair stay on one die; 3 x 2 pairs: dealt to all; 40 pairs: padded to a multiple of eight)
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(32, 32), (64, 64), (128, 128), (64, 128), (128, 32), (96, 64)])
+@pytest.mark.parametrize("B,H,G", [(8, 4, 4), (3, 4, 2), (13, 9, 3)])
+def test_matrix_core_prompts_equal_portable(B, H, G, D, V):
+    """bf16: the prompt kernel at the head sizes whose tiles go straight to LDS (and one, 96, that is padded instead) against
+    the portable kernel: ragged portions around the edges of a tile and of a 128-row block, with and without a cached
+    prefix, for every kind of mask and weights.  Tolerance: two bf16 roundings (weights, result) of values near one."""
+    g = gen(B * D + V)
+    dev, dt = "cuda", torch.bfloat16
+    sizes = [(0, 200), (130, 70), (63, 2), (300, 33), (0, 64), (64, 65), (0, 1), (127, 129)]
+    portions = [sizes[(3 * i) % 8] for i in range(B)]
+    ctx, blocks = batch(portions, device=dev, seed=B)
+    kc = (torch.randn(blocks, 64, G, D, generator=g) * 0.7).to(dt).to(dev)
+    vc = (torch.randn(blocks, 64, G, V, generator=g) * 0.7).to(dt).to(dev)
+    kp, vp = (torch.randn(blocks, 4, G, n, generator=g).to(dt).to(dev) for n in (D, V))
+    q = (torch.randn(ctx.num_tokens, H, D, generator=g) * 0.7).to(dt).to(dev)
+    hb, sink = (torch.randn(H, generator=g).to(dev) for _ in range(2))
+    for kw in (dict(), dict(sink=sink), dict(window=50), dict(window=64, keep_first=70, sink=sink), dict(softcap=3.0, window=100),
+               dict(chunk=50, sigmoid=True, head_bias=hb), dict(chunk=64, softcap=2.0), dict(window=40, pooled=(kp, vp, 16))):
+        a = hy_ops.paged_attention(q, kc, vc, ctx, 0.2, **kw)
+        b = hy_ops.paged_attention(q, kc, vc, ctx, 0.2, force_rows=True, **kw)
+        near(a, b.double().cpu(), dt, bf16=2e-2)
+
+
+# Rows of a multiple of 32 columns go straight to LDS (8, 7, 6, 5, 4, 3, 1 times 32: every swizzle), others (40, 200) do not.
+@pytest.mark.gpu
+@pytest.mark.parametrize("R,RV", [(256, 192), (256, 256), (224, 192), (192, 192), (160, 128), (128, 64), (96, 96), (32, 32), (40, 40), (200, 136)])
+@pytest.mark.parametrize("B,H", [(8, 16), (3, 5)])
+def test_matrix_core_latent_prompts_equal_portable(B, H, R, RV):
+    g = gen(B * R + RV)
+    dev, dt = "cuda", torch.bfloat16
+    sizes = [(0, 100), (130, 70), (63, 2), (200, 33), (0, 32), (64, 65), (0, 1), (31, 33)]
+    ctx, blocks = batch([sizes[(3 * i) % 8] for i in range(B)], device=dev, seed=B)
+    cache = (torch.randn(blocks, 64, R, generator=g) * 0.7).to(dt).to(dev)
+    q = (torch.randn(ctx.num_tokens, H, R, generator=g) * 0.7).to(dt).to(dev)
+    sink = torch.randn(H, generator=g).to(dev)
+    for kw in (dict(), dict(sink=sink), dict(window=30), dict(window=64, sink=sink)):
+        a = seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=RV, **kw)
+        b = seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=RV, force_rows=True, **kw)
+        near(a, b.double().cpu(), dt, bf16=2e-2)
+
+
 # ------------------------------------------------------------------------------------------ latent attention with a query latent
 @pytest.mark.parametrize("device,dtype", CASES)
 @pytest.mark.parametrize("H,D,Rd,V,R,Q", [(3, 8, 8, 16, 24, 20), (1, 4, 2, 4, 8, 4), (2, 40, 24, 72, 136, 56), (4, 24, 8, 40, 112, 64),
