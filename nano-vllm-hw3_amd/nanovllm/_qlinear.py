@@ -96,6 +96,9 @@ SIGNATURES = {
 _lib = None
 
 
+QL_EWORKSPACE = -3
+
+
 class QLinearError(RuntimeError):
     pass
 
@@ -170,17 +173,20 @@ def dtype_code(dtype):
 
 
 def stream_ptr(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of ``device`` as the handle the libraries take (asked for without building a Stream object, which
+    costs half as much as a launch)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_cuda(t, dtype, name):
+    if t.is_cuda and (dtype is None or t.dtype == dtype) and t.is_contiguous():
+        return t
     if not t.is_cuda:
         raise QLinearError(f"{name} must live on the GPU (got {t.device}); the HIP path has no CPU fallback")
     if dtype is not None and t.dtype != dtype:
         raise QLinearError(f"{name} must be {dtype}, got {t.dtype}")
-    if not t.is_contiguous():
-        raise QLinearError(f"{name} must be contiguous")
-    return t
+    raise QLinearError(f"{name} must be contiguous")
 
 
 class _Workspace:
@@ -219,10 +225,18 @@ class _Workspace:
             self.buf[key] = torch.zeros(max(int(nbytes), 1 << 20), dtype=torch.uint8, device=device)
         return self.buf[key]
 
+    def held(self, device):
+        """(address, bytes) of the device's buffer as it is, (None, 0) without one: for calls that say by their status when it
+        is too small, in front of any launch."""
+        b = self.buf.get(device.index)
+        return (None, 0) if b is None else (b.data_ptr(), b.numel())
+
     def get(self, device, nbytes):
         if nbytes == 0:
             return None, 0
-        b = self.reserve(device, nbytes)
+        b = self.buf.get(device.index) if isinstance(device, torch.device) else None        # (an index of None is no key)
+        if b is None or b.numel() < nbytes:
+            b = self.reserve(device, nbytes)
         return b.data_ptr(), b.numel()
 
 

@@ -50,7 +50,6 @@ _WIDE = {torch.float16: 1, torch.float32: 2}
 
 
 # --------------------------------------------------------------------------- quantizers
-@torch.no_grad()
 def per_row_quant(x: torch.Tensor, dtype: torch.dtype):
     """x [T, H] bf16 (or fp16 / fp32: the reference's kernel widens whatever it loads to f32, quantization.py:27)
     -> (q [T, H] dtype, scale [T] f32).  Reference: quantization.py:147-163."""
@@ -161,6 +160,7 @@ def _bf16_terms(x2):
     return terms
 
 
+@torch.no_grad()
 def _w8a16_wide(x, qw, sw32, bias, granularity, group_size, dtype, silu):
     """The weight-only matmuls on fp16 / fp32 activations (reference: ``x.float() @ w.T`` in fp32, result cast to x's
     dtype, quantization.py:258-261, 299-305).  The activations are split exactly into bf16 terms; every term runs the
@@ -195,6 +195,15 @@ def _w8a16_wide(x, qw, sw32, bias, granularity, group_size, dtype, silu):
     return y.view(*x.shape[:-1], y.shape[-1])
 
 
+def _gemm(fn, args, device, M, N, K, granularity):
+    """One GEMM call with the workspace at hand; a call that needs a larger one says so before it launches anything, and is
+    repeated with it.  (Asking first means planning every form of the call, as much host work as the call itself.)"""
+    rc = fn(*args, *Q.workspace.held(device), Q.stream_ptr(device))
+    if rc == Q.QL_EWORKSPACE:
+        rc = fn(*args, *Q.workspace.get(device, Q.load().ql_gemm_workspace_bytes(M, N, K, granularity)), Q.stream_ptr(device))
+    Q.check(rc)
+
+
 def _w8a16(x, qw, sw, bias, granularity, group_size, dtype, silu=False, out=None):
     assert dtype in _DTYPES and qw.dtype == dtype
     if x.dtype in _WIDE:
@@ -203,51 +212,45 @@ def _w8a16(x, qw, sw, bias, granularity, group_size, dtype, silu=False, out=None
         sw_ = sw if sw.dtype == torch.float32 else sw.to(torch.float32)
         sw_ = Q.require_cuda(sw_.reshape(-1) if sw_.dim() == 0 else sw_, torch.float32, "sw")
         return _w8a16_wide(x, qw, sw_, bias, granularity, group_size, dtype, silu)
-    x2, y_shape = _flatten(x, qw.shape[0] // 2 if silu else qw.shape[0])
+    N, K_w = qw.shape
+    n_out = N // 2 if silu else N
+    flat = x.dim() == 2
+    x2 = x if flat else x.reshape(-1, x.shape[-1])
     Q.require_cuda(x2, torch.bfloat16, "x")
     Q.require_cuda(qw, dtype, "qw")
     sw32 = sw if sw.dtype == torch.float32 else sw.to(torch.float32)
-    sw32 = Q.require_cuda(sw32.reshape(-1) if sw32.dim() == 0 else sw32, torch.float32, "sw")
+    sw32 = Q.require_cuda(sw32 if sw32.dim() else sw32.reshape(-1), torch.float32, "sw")
     if bias is not None:
         Q.require_cuda(bias, torch.bfloat16, "bias")
     M, K = x2.shape
-    N = qw.shape[0]
-    assert qw.shape[1] == K, f"x has K={K} but qw has K={qw.shape[1]}"
+    assert K_w == K, f"x has K={K} but qw has K={K_w}"
+    device = x2.device
     lib = Q.load()
-    if silu:
-        y = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
-        ws_ptr, ws_len = Q.workspace.get(x.device, lib.ql_gemm_workspace_bytes(M, N, K, granularity))
-        Q.check(lib.ql_gemm_w8a16_silu(_wcode(qw, dtype), granularity, x2.data_ptr(), qw.data_ptr(), sw32.data_ptr(),
-                                       bias.data_ptr() if bias is not None else None, y.data_ptr(), M, N, K,
-                                       group_size or 0, ws_ptr, ws_len, Q.stream_ptr(x.device)))
-        return y.view(y_shape)
-    if out is not None:
+    if out is not None and not silu:
         assert out.shape == (M, N)
         y = Q.require_cuda(out, torch.bfloat16, "out")
     else:
-        y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    ws_ptr, ws_len = Q.workspace.get(x.device, lib.ql_gemm_workspace_bytes(M, N, K, granularity))
-    Q.check(lib.ql_gemm_w8a16(_wcode(qw, dtype), granularity, x2.data_ptr(), qw.data_ptr(), sw32.data_ptr(),
-                              bias.data_ptr() if bias is not None else None, y.data_ptr(), M, N, K,
-                              group_size or 0, ws_ptr, ws_len, Q.stream_ptr(x.device)))
-    return y if out is not None else y.view(y_shape)
+        y = torch.empty((M, n_out), dtype=torch.bfloat16, device=device)
+    _gemm(lib.ql_gemm_w8a16_silu if silu else lib.ql_gemm_w8a16,
+          (_wcode(qw, dtype), granularity, x2.data_ptr(), qw.data_ptr(), sw32.data_ptr(), bias.data_ptr() if bias is not None else None,
+           y.data_ptr(), M, N, K, group_size or 0), device, M, N, K, granularity)
+    return y if flat or (out is not None and not silu) else y.view(list(x.shape)[:-1] + [n_out])
 
 
-@torch.no_grad()
+# (The matmuls below enter no no_grad block of their own: their results are new tensors written by the library, which autograd
+# does not see; the forms that compute with torch operators, _w8a16_wide and _per_row_matmul_wide, do.)
 def per_tensor_matmul(x, qw, sw, bias, dtype, silu=False, out=None):
     """``(x.float() @ (qw.float() * sw).T).to(bf16) + bias`` fused (quantization.py:237-262).  ``out`` (every
     matmul here): a contiguous [M, N] bf16 tensor to write instead of a new one (x is then [M, K])."""
     return _w8a16(x, qw, sw, bias, Q.QL_PER_TENSOR, 0, dtype, silu, out)
 
 
-@torch.no_grad()
 def per_group_matmul(x, qw, sw, bias, group_size, dtype, silu=False, out=None):
     """Per-group dequant fused into the GEMM (quantization.py:265-307)."""
     assert qw.shape[1] % group_size == 0
     return _w8a16(x, qw, sw, bias, Q.QL_PER_GROUP, group_size, dtype, silu, out)
 
 
-@torch.no_grad()
 def per_row_weight_only_matmul(x, qw, sw, bias, dtype, silu=False, out=None):
     """W8A16 with per-output-channel scales: ``bf16((x @ q.T) * sw + bias)``; the numerics the
     reference reaches through ``F.linear(x, fake_per_row_quant(W))`` (quantization.py:438-439).
@@ -258,7 +261,6 @@ def per_row_weight_only_matmul(x, qw, sw, bias, dtype, silu=False, out=None):
     return _w8a16(x, qw, sw, bias, Q.QL_PER_ROW, 0, dtype, silu, out)
 
 
-@torch.no_grad()
 def w8a8_matmul(qx, sx, qw, sw, bias, dtype, y_shape=None, silu=False, out=None, return_rowmax=False):
     """The dual-scale GEMM on already-quantized activations (quantization.py:54-144, 331-345).  ``return_rowmax``
     (SiLU form only): also f32 [M, N/64], the |max| of every output row over each 32-column strip."""
@@ -274,29 +276,22 @@ def w8a8_matmul(qx, sx, qw, sw, bias, dtype, y_shape=None, silu=False, out=None,
     assert qw.shape[1] == K
     lib = Q.load()
     assert silu or not return_rowmax
+    device = qx.device
+    head = (_wcode(qw, dtype), qx.data_ptr(), sx.data_ptr(), qw.data_ptr(), sw.data_ptr(), bias.data_ptr() if bias is not None else None)
     if silu:
-        y = torch.empty((M, N // 2), dtype=torch.bfloat16, device=qx.device)
-        ws_ptr, ws_len = Q.workspace.get(qx.device, lib.ql_gemm_workspace_bytes(M, N, K, Q.QL_PER_ROW))
+        y = torch.empty((M, N // 2), dtype=torch.bfloat16, device=device)
         if return_rowmax:
-            rowmax = torch.empty((M, N // 64), dtype=torch.float32, device=qx.device)
-            Q.check(lib.ql_gemm_w8a8_silu_rowmax(_wcode(qw, dtype), qx.data_ptr(), sx.data_ptr(), qw.data_ptr(),
-                                                 sw.data_ptr(), bias.data_ptr() if bias is not None else None,
-                                                 y.data_ptr(), rowmax.data_ptr(), M, N, K, ws_ptr, ws_len,
-                                                 Q.stream_ptr(qx.device)))
+            rowmax = torch.empty((M, N // 64), dtype=torch.float32, device=device)
+            _gemm(lib.ql_gemm_w8a8_silu_rowmax, head + (y.data_ptr(), rowmax.data_ptr(), M, N, K), device, M, N, K, Q.QL_PER_ROW)
             return (y if y_shape is None else y.view(y_shape)), rowmax
-        Q.check(lib.ql_gemm_w8a8_silu(_wcode(qw, dtype), qx.data_ptr(), sx.data_ptr(), qw.data_ptr(), sw.data_ptr(),
-                                      bias.data_ptr() if bias is not None else None, y.data_ptr(), M, N, K,
-                                      ws_ptr, ws_len, Q.stream_ptr(qx.device)))
+        _gemm(lib.ql_gemm_w8a8_silu, head + (y.data_ptr(), M, N, K), device, M, N, K, Q.QL_PER_ROW)
         return y if y_shape is None else y.view(y_shape)
     if out is not None:
         assert out.shape == (M, N)
         y = Q.require_cuda(out, torch.bfloat16, "out")
     else:
-        y = torch.empty((M, N), dtype=torch.bfloat16, device=qx.device)
-    ws_ptr, ws_len = Q.workspace.get(qx.device, lib.ql_gemm_workspace_bytes(M, N, K, Q.QL_PER_ROW))
-    Q.check(lib.ql_gemm_w8a8(_wcode(qw, dtype), qx.data_ptr(), sx.data_ptr(), qw.data_ptr(), sw.data_ptr(),
-                             bias.data_ptr() if bias is not None else None, y.data_ptr(), M, N, K, ws_ptr, ws_len,
-                             Q.stream_ptr(qx.device)))
+        y = torch.empty((M, N), dtype=torch.bfloat16, device=device)
+    _gemm(lib.ql_gemm_w8a8, head + (y.data_ptr(), M, N, K), device, M, N, K, Q.QL_PER_ROW)
     return y if y_shape is None else y.view(y_shape)
 
 
@@ -338,6 +333,7 @@ def w8a8_dynq_matmul(x, rowmax_part, qw, sw, bias, dtype, out=None):
     return y if out is not None else y.view(y_shape)
 
 
+@torch.no_grad()
 def _per_row_matmul_wide(x, qw, sw, bias, dtype, silu):
     """per_row_matmul on fp16 / fp32 activations: the quantizer widens them to f32 (as the reference's does), the
     contraction runs in the deferred form (raw int32 / f32 slices) and the reference's epilogue
@@ -366,12 +362,14 @@ def _per_row_matmul_wide(x, qw, sw, bias, dtype, silu):
     return y.view(*x.shape[:-1], y.shape[-1])
 
 
-@torch.no_grad()
 def per_row_matmul(x, qw, sw, bias, dtype, silu=False, out=None):
     """Dynamic per-token activation quant + W8A8 GEMM (quantization.py:310-346)."""
     if x.dtype in _WIDE:
         return _per_row_matmul_wide(x, qw, sw, bias, dtype, silu)
-    x2, y_shape = _flatten(x, qw.size(0) // 2 if silu else qw.size(0))
+    if x.dim() == 2:
+        x2, y_shape = x, None
+    else:
+        x2, y_shape = _flatten(x, qw.size(0) // 2 if silu else qw.size(0))
     assert x2.size(1) % 32 == 0, f"K({x2.size(1)}) must be multiple of 32"
     qx, sx = per_row_quant(x2.contiguous(), dtype)
     return w8a8_matmul(qx, sx, qw, sw, bias, dtype, None if out is not None else y_shape, silu, out)
@@ -657,6 +655,8 @@ class QLinear(_QBase):
 
     def forward(self, x: torch.Tensor):
         fn = per_row_weight_only_matmul if self.weight_only else per_row_matmul
+        if self.tp_size == 1:
+            return fn(x, self.qw, self.sw, self.bias, self.dtype, self.silu_fused)
         x2 = x.reshape(-1, x.shape[-1])
         return self._run(x, lambda rows, out: fn(x if rows is None else x2[rows], self.qw, self.sw,
                                                  self._bias_for_rank(), self.dtype, self.silu_fused, out))
@@ -733,6 +733,8 @@ class QTensorLinear(_QBase):
         return m
 
     def forward(self, x: torch.Tensor):
+        if self.tp_size == 1:
+            return per_tensor_matmul(x, self.qw, self._sw32, self.bias, self.dtype, self.silu_fused)
         x2 = x.reshape(-1, x.shape[-1])
         return self._run(x, lambda rows, out: per_tensor_matmul(x if rows is None else x2[rows], self.qw, self._sw32,
                                                                 self._bias_for_rank(), self.dtype, self.silu_fused, out))
@@ -767,6 +769,8 @@ class QGroupLinear(_QBase):
         return m
 
     def forward(self, x: torch.Tensor):
+        if self.tp_size == 1:
+            return per_group_matmul(x, self.qw, self.sw, self.bias, self.group_size, self.dtype, self.silu_fused)
         x2 = x.reshape(-1, x.shape[-1])
         return self._run(x, lambda rows, out: per_group_matmul(x if rows is None else x2[rows], self.qw, self.sw,
                                                                self._bias_for_rank(), self.group_size, self.dtype,
