@@ -176,6 +176,19 @@ int hm_state_space(int dtype, const void* rows, int64_t stride, int x_off, int b
                    const int32_t* qstart, const int32_t* seq_pos0, const int32_t* seq_slot, float* y, int B, int64_t T, int H, int G,
                    int N, int V, int max_q, void* stream);
 
+/* The two recurrences above over portions of bf16 rows, 32 tokens at a time on the matrix cores; the same arguments, and scratch
+ * `work` of hm_outer_chunk_work_bytes(T, B, H) bytes (16-byte aligned).  64 or 128 key channels (states), value channels a multiple
+ * of 32; rows, stride and every part's offset on 16 bytes.  gates is needed for every max_q. */
+size_t hm_outer_chunk_work_bytes(int64_t T, int B, int H);
+int hm_gated_delta_chunks(const void* rows, int64_t stride, int q_off, int k_off, int v_off, const void* pre, int64_t pre_stride,
+                          int b_off, int a_off, const float* A, const float* dt_bias, float unit_eps, float q_scale, float* gates,
+                          void* work, float* state, const int32_t* qstart, const int32_t* seq_pos0, const int32_t* seq_slot, float* o,
+                          int B, int64_t T, int H, int G, int D, int V, int max_q, void* stream);
+int hm_state_space_chunks(const void* rows, int64_t stride, int x_off, int b_off, int c_off, const void* pre, int64_t pre_stride,
+                          int dt_off, const float* A, const float* dt_bias, const float* D, float* gates, void* work, float* state,
+                          const int32_t* qstart, const int32_t* seq_pos0, const int32_t* seq_slot, float* y, int B, int64_t T, int H,
+                          int G, int N, int V, int max_q, void* stream);
+
 /* Linear attention with a constant decay per head.  q, k [T, H*D] and v [T, H*V] are the columns q_off, k_off, v_off of
  * proj (rows row_stride apart) passed through silu.  For every sequence b and head, over the tokens of its portion:
  *   S <- decay[h] S + k v^T;  o[t] = S^T q

@@ -52,6 +52,11 @@ SIGNATURES = {
                               _int, _i64, _int, _int, _int, _int, _int, _vp]),
     "hm_state_space": (_int, [_int, _vp, _i64, _int, _int, _int, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                               _int, _i64, _int, _int, _int, _int, _int, _vp]),
+    "hm_outer_chunk_work_bytes": (_sz, [_i64, _int, _int]),
+    "hm_gated_delta_chunks": (_int, [_vp, _i64, _int, _int, _int, _vp, _i64, _int, _int, _vp, _vp, _f, _f, _vp, _vp, _vp, _vp, _vp, _vp,
+                                     _vp, _int, _i64, _int, _int, _int, _int, _int, _vp]),
+    "hm_state_space_chunks": (_int, [_vp, _i64, _int, _int, _int, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                     _int, _i64, _int, _int, _int, _int, _int, _vp]),
     "hm_relu_squared": (_int, [_int, _vp, _i64, _vp, _vp, _i64, _i64, _int, _vp]),
 }
 

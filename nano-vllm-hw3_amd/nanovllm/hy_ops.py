@@ -336,6 +336,26 @@ def delta_gate_norm(o, g, norm_w, eps, dtype, act=GATE_SIGMOID, gate_first=False
     return out
 
 
+# Tokens of the longest portion from which a step takes 32 tokens at a time, by key channels, where the portions have half of that on
+# average: below, the chunks cost more than they save (microseconds, chunks / walk, 16 heads of 128 x 128: 1 portion of 32 21 / 17,
+# of 64 22 / 27, of 256 44 / 88; 64 portions of 16 67 / 59, of 32 72 / 94, of 64 107 / 166; 4 heads of 64 x 64: 1 portion of 64
+# 21 / 20, of 128 25 / 33; 64 of 64 25 / 22, of 128 35 / 36).
+CHUNKS_MIN_TOKENS = {64: 128, 128: 64}
+
+
+def _outer_chunked(rows, offsets, D, V, ctx):
+    """Whether a step's portions take the form of 32 tokens at a time (bf16 rows whose parts start on 16 bytes, 64 or 128 key
+    channels, 32 or a multiple of it value channels; long enough)."""
+    least = CHUNKS_MIN_TOKENS.get(D, 0)
+    return (rows.dtype == torch.bfloat16 and 0 < least <= ctx.max_q and 2 * rows.shape[0] >= least * ctx.num_seqs and V % 32 == 0 and
+            rows.data_ptr() % 16 == 0 and all(c % 8 == 0 for c in (rows.stride(0), *offsets)) and ctx.num_seqs <= 65535)
+
+
+def _outer_work(rows, H, ctx):
+    n = HM.load().hm_outer_chunk_work_bytes(rows.shape[0], ctx.num_seqs, H)
+    return torch.empty((n,), dtype=torch.uint8, device=rows.device)
+
+
 def _outer_args(rows, pre, state, o_shape, H, D, V, ctx):
     """Checks of the outer-product recurrences; (output, gates scratch or None)."""
     _rows(rows, "rows")
@@ -360,6 +380,14 @@ def gated_delta(rows, q_off, k_off, v_off, pre, b_off, a_off, A, dt_bias, H, G, 
         return cpu_ops.gated_delta(rows, q_off, k_off, v_off, pre, b_off, a_off, A, dt_bias, H, G, D, V, unit_eps, q_scale, state, ctx)
     assert A.dtype == dt_bias.dtype == torch.float32 and A.numel() == dt_bias.numel() == H
     o, gates = _outer_args(rows, pre, state, (rows.shape[0], H, V), H, D, V, ctx)
+    if _outer_chunked(rows, (q_off, k_off, v_off), D, V, ctx):
+        work = _outer_work(rows, H, ctx)
+        HM.check(HM.load().hm_gated_delta_chunks(rows.data_ptr(), rows.stride(0), q_off, k_off, v_off, pre.data_ptr(), pre.stride(0), b_off,
+                                                 a_off, A.data_ptr(), dt_bias.data_ptr(), float(unit_eps), float(q_scale),
+                                                 gates.data_ptr(), work.data_ptr(), state.data_ptr(), ctx.qstart.data_ptr(),
+                                                 ctx.seq_pos0.data_ptr(), ctx.seq_slot.data_ptr(), o.data_ptr(), ctx.num_seqs,
+                                                 rows.shape[0], H, G, D, V, int(ctx.max_q), _dev(rows)))
+        return o
     HM.check(HM.load().hm_gated_delta(HM.dtype_code(rows.dtype), rows.data_ptr(), rows.stride(0), q_off, k_off, v_off, pre.data_ptr(),
                                       pre.stride(0), b_off, a_off, A.data_ptr(), dt_bias.data_ptr(), float(unit_eps), float(q_scale),
                                       HM.ptr(gates), state.data_ptr(), ctx.qstart.data_ptr(), ctx.seq_pos0.data_ptr(),
@@ -378,6 +406,14 @@ def state_space(rows, x_off, b_off, c_off, pre, dt_off, A, dt_bias, D, H, G, N, 
         return cpu_ops.state_space(rows, x_off, b_off, c_off, pre, dt_off, A, dt_bias, D, H, G, N, V, state, ctx)
     assert A.dtype == dt_bias.dtype == D.dtype == torch.float32 and A.numel() == dt_bias.numel() == D.numel() == H
     y, gates = _outer_args(rows, pre, state, (rows.shape[0], H, V), H, N, V, ctx)
+    if _outer_chunked(rows, (x_off, b_off, c_off), N, V, ctx):
+        work = _outer_work(rows, H, ctx)
+        HM.check(HM.load().hm_state_space_chunks(rows.data_ptr(), rows.stride(0), x_off, b_off, c_off, pre.data_ptr(), pre.stride(0), dt_off,
+                                                 A.data_ptr(), dt_bias.data_ptr(), D.data_ptr(), gates.data_ptr(), work.data_ptr(),
+                                                 state.data_ptr(), ctx.qstart.data_ptr(), ctx.seq_pos0.data_ptr(),
+                                                 ctx.seq_slot.data_ptr(), y.data_ptr(), ctx.num_seqs, rows.shape[0], H, G, N, V,
+                                                 int(ctx.max_q), _dev(rows)))
+        return y
     HM.check(HM.load().hm_state_space(HM.dtype_code(rows.dtype), rows.data_ptr(), rows.stride(0), x_off, b_off, c_off, pre.data_ptr(),
                                       pre.stride(0), dt_off, A.data_ptr(), dt_bias.data_ptr(), D.data_ptr(), HM.ptr(gates),
                                       state.data_ptr(), ctx.qstart.data_ptr(), ctx.seq_pos0.data_ptr(), ctx.seq_slot.data_ptr(),

@@ -203,5 +203,10 @@ def test_hymix_argument_validation_needs_no_gpu():
     assert lib.hm_gated_delta(1, one, 96, 0, 32, 64, one, 64, 0, 2, one, one, 1e-6, 1.0, one, *delta, one, 2, 8, 3, 2, 16, 16, 4, None) == -1   # heads % kv_heads
     assert lib.hm_gated_delta(1, one, 90, 0, 32, 64, one, 64, 0, 2, one, one, 1e-6, 1.0, one, *delta, one, 2, 8, 2, 2, 16, 16, 4, None) == -1   # rows too narrow
     assert lib.hm_gated_delta(1, one, 96, 0, 32, 64, one, 64, 0, 2, one, one, 1e-6, 1.0, None, *delta, one, 2, 8, 2, 2, 16, 16, 4, None) == -1  # no scratch
+    chunks = (2, 8, 2, 1, 64, 32, 64, None)                                                                                                   # B T H G D V max_q stream
+    assert lib.hm_gated_delta_chunks(one, 192, 0, 64, 128, one, 64, 0, 2, one, one, 1e-6, 1.0, one, None, *delta, one, *chunks) == -1          # no work
+    assert lib.hm_gated_delta_chunks(one, 192, 0, 64, 128, one, 64, 0, 2, one, one, 1e-6, 1.0, one, one, *delta, one, 2, 8, 2, 1, 32, 32, 64, None) == -2   # 32 key channels
+    assert lib.hm_gated_delta_chunks(one, 196, 0, 64, 128, one, 64, 0, 2, one, one, 1e-6, 1.0, one, one, *delta, one, *chunks) == -1           # rows off 16 bytes
+    assert lib.hm_state_space_chunks(one, 192, 0, 64, 128, one, 64, 0, one, one, None, one, one, *delta, one, *chunks) == -1                   # no skip weights
     assert lib.hm_state_space(1, one, 4096, 0, 32, 600, one, 64, 0, one, one, one, one, *delta, one, 2, 8, 2, 1, 300, 16, 4, None) == -2         # more than 256 states
     assert lib.hm_state_space(1, one, 96, 0, 32, 48, one, 64, 0, one, one, None, one, *delta, one, 2, 8, 2, 1, 16, 16, 4, None) == -1            # no skip weights

@@ -184,6 +184,68 @@ def test_states_that_hardly_forget_through_portions(device, dtype, sizes):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["delta", "space"])
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 64, 32), (3, 3, 128, 32), (4, 2, 128, 128), (6, 2, 64, 160)])
+def test_portions_by_chunks_equal_the_walk(monkeypatch, kind, H, G, D, V):
+    """32 tokens at a time and token after token: portions around one and two chunks, new ones and ones that continue a state, rows that
+    are a column slice (and one too little aligned for chunks).  Both are float32 sums of exact operands: from the float64 recurrence
+    they are within 16 roundings of 2^-24 in norm (D / 64 terms per lane and fold, up to four chunks' states).  A token that is
+    not finite leaves the tokens in front of it and the other portions as they are."""
+    g = gen(D + V + H)
+    lens, of = [1, 31, 32, 33, 64, 2, 65, 97], torch.arange(H) // (H // G)
+    starts = [0, 40, 0, 7, 0, 3, 9, 0]
+    n, n_qk = sum(lens), 2 * G * D
+    wide = rnd(g, n, n_qk + H * V + 16, dtype=torch.bfloat16)
+    pre = rnd(g, n, 2 * H, s=2.0, dtype=torch.bfloat16).cuda()
+    A, bias = forget(g, H)
+    skip = rnd(g, H)
+    ctx, _ = batch(list(zip(starts, lens)), device="cuda", seed=3)
+    state0 = rnd(g, max(int(s) for s in ctx.seq_slot) + 2, H, D, V)
+    cuda = [t.cuda() for t in (A, bias, skip)]
+
+    def run(rows, least):
+        monkeypatch.setattr(hy_ops, "CHUNKS_MIN_TOKENS", {D: least} if least else {})
+        st = state0.cuda()
+        if kind == "delta":
+            o = hy_ops.gated_delta(rows, 0, G * D, n_qk, pre, 0, H, *cuda[:2], H, G, D, V, st, ctx, q_scale=0.37)
+        else:
+            o = hy_ops.state_space(rows, n_qk, 0, G * D, pre, 0, *cuda, H, G, D, V, st, ctx)
+        return o, st
+    rows = wide.cuda()[:, 8:8 + n_qk + H * V]
+    walk, chunks = run(rows, 0), run(rows, 1)
+    off = torch.zeros(n, wide.shape[1] + 3, dtype=torch.bfloat16, device="cuda")
+    off[:, 3:] = wide
+    off = off[:, 11:11 + n_qk + H * V]
+    odd = run(off, 1)
+    assert [hy_ops._outer_chunked(r, (0, G * D, n_qk), D, V, ctx) for r in (rows, off)] == [True, False]
+    x, p, at = wide[:, 8:].to(F64), pre.cpu().to(F64), 0
+    for b, (start, length) in enumerate(zip(starts, lens)):
+        h, pb, slot = x[at:at + length], p[at:at + length], int(ctx.seq_slot[b])
+        a, c = (h[:, i * G * D:(i + 1) * G * D].reshape(length, G, D) for i in (0, 1))
+        v = h[:, n_qk:n_qk + H * V].reshape(length, H, V)
+        s0 = state0[slot].to(F64) if start else torch.zeros(H, D, V, dtype=F64)
+        if kind == "delta":
+            ref, s_ref = O.gated_delta((O.unit(a) * 0.37)[:, of], O.unit(c)[:, of], v, torch.sigmoid(pb[:, :H]),
+                                       torch.exp(A.to(F64) * O.softplus(pb[:, H:] + bias.to(F64))), s0)
+        else:
+            ref, s_ref = O.state_space(v, a[:, of], c[:, of], O.softplus(pb[:, :H] + bias.to(F64)), A.to(F64), skip.to(F64), s0)
+        for o, st in (walk, chunks, odd):
+            assert (o[at:at + length].cpu().to(F64) - ref).norm() <= 16 * 2 ** -24 * ref.norm()
+            assert (st[slot].cpu().to(F64) - s_ref).norm() <= 16 * 2 ** -24 * s_ref.norm()
+        at += length
+    at = n - 97 + 50                                                    # one token of the last portion's second chunk
+    for column, value in ((n_qk + 5, float("inf")), (3, float("nan")), (G * D + 1, float("inf"))):
+        bad = rows.clone()
+        bad[at, column] = value
+        o = run(bad, 1)[0]
+        assert torch.equal(o[:at], chunks[0][:at]) and not torch.isfinite(o[at, 0]).all()
+        if column > n_qk:                                               # a value channel: the others don't notice
+            keep = torch.ones(H * V, dtype=torch.bool)
+            keep[5] = False
+            assert torch.equal(o.view(n, -1)[:, keep], chunks[0].view(n, -1)[:, keep]) and not torch.isfinite(o[at:, 0, 5]).any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("D,V", [(32, 64), (64, 128), (128, 64), (256, 72)])
 def test_recurrence_forms_agree(dtype, D, V):
