@@ -9,15 +9,22 @@ namespace sm {
 // floats per (sequence, split, head) in the workspace: scaled maximum, sum, RP outputs
 __host__ __device__ constexpr int part_stride(int nb) { return 32 * nb + 2; }
 
-template <int NB, int NBV, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void latent_attn_decode_kernel(const unsigned short* __restrict__ q,
+// SLIM: rows of exactly 32 NB columns, in the loop of 32-key tiles (latent_slim_loop), which goes straight to LDS.  A split is a few
+// tiles behind the latency of its first loads, so what counts is how many workgroups run beside each other; the other loop, with a
+// tile in registers on its way, spills in one wave of 256 columns.  Microseconds with the merge, other loop / this one, rows of
+// 192 + 64: 64 sequences of about 1000 keys 28 / 22 (16 heads), 42 / 35 (64 heads), 8 sequences 21 / 18, 256 of about 450 41 / 31, 16 of
+// 3500 with 128 heads 49 / 40.  256 registers, so that two waves share a SIMD, where a workgroup has two or four waves:
+// 35 against 42 at 64 heads; one wave alone holds more than that and would spill (30 against 22).
+template <int NB, int NBV, int WAVES, bool SLIM>
+__global__ __launch_bounds__(64 * WAVES, SLIM && WAVES > 1 ? 2 : 1) void latent_attn_decode_kernel(const unsigned short* __restrict__ q,
                                                                         const unsigned short* __restrict__ cache,
                                                                         const int32_t* __restrict__ block_tables,
                                                                         const int32_t* __restrict__ ctx, float* __restrict__ ws,
                                                                         float c_log2, int H, int R, int block_size,
                                                                         int max_blocks, int splits, int window) {
-    typedef TileGeom<NB> G;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[G::LDS_BYTES];
+    // (the slim loop has two buffers of half a tile)
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[SLIM ? SlimGeom<NB>::BYTES : TileGeom<NB>::LDS_BYTES];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds2[SLIM ? SlimGeom<NB>::BYTES : 16];
     const int sp = blockIdx.x, b = blockIdx.y;
     const int n = ctx[b];
     // the visible keys start at the tile that holds key n - window; whole tiles per split
@@ -35,8 +42,14 @@ __global__ __launch_bounds__(64 * WAVES) void latent_attn_decode_kernel(const un
     const int rc = min(r, H - 1);
     f32x16 oacc[NBV];
     float m_run, l_tot;
-    latent_tile_loop<NB, NBV, WAVES>(q + ((size_t)b * H + rc) * R, cache, block_tables + (size_t)b * max_blocks, R, block_size,
-                                     k_lo, k_hi, n - 1, n - 1, c_log2, window, lds, oacc, m_run, l_tot);
+    const unsigned short* qrow = q + ((size_t)b * H + rc) * R;
+    const int32_t* table = block_tables + (size_t)b * max_blocks;
+    if constexpr (SLIM)
+        latent_slim_loop<NB, NBV, WAVES>(qrow, cache, table, block_size, k_lo, k_hi, n - 1, n - 1, n - 1, c_log2, window, lds, lds2, oacc,
+                                         m_run, l_tot);
+    else
+        latent_tile_loop<NB, NBV, WAVES>(qrow, cache, table, R, block_size, k_lo, k_hi, n - 1, n - 1, c_log2, window, lds, oacc, m_run,
+                                         l_tot);
     if (r >= H) return;
     if (hi == 0) { part[0] = l_tot > 0.f ? m_run * c_log2 : -INFINITY; part[1] = l_tot; }
 #pragma unroll
@@ -137,13 +150,15 @@ extern "C" int sm_latent_attn_decode(const void* q, const void* cache, const int
     dim3 grid((unsigned)splits, (unsigned)B);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
-#define SM_DEC(NB_, NBV_, W_)                                                                                              \
-    hipLaunchKernelGGL((latent_attn_decode_kernel<NB_, NBV_, W_>), grid, dim3(64 * W_), 0, s, (const unsigned short*)q,    \
+#define SM_DEC(NB_, NBV_, W_) do { if (R == 32 * NB_) SM_DEC_(NB_, NBV_, W_, true); else SM_DEC_(NB_, NBV_, W_, false); } while (0)
+#define SM_DEC_(NB_, NBV_, W_, SLIM_)                                                                                      \
+    hipLaunchKernelGGL((latent_attn_decode_kernel<NB_, NBV_, W_, SLIM_>), grid, dim3(64 * W_), 0, s, (const unsigned short*)q, \
                        (const unsigned short*)cache, block_tables, ctx, (float*)workspace, c, H, R, block_size, max_blocks, \
                        splits, window)
 #define SM_DEC_W(NB_, NBV_) do { if (waves == 1) SM_DEC(NB_, NBV_, 1); else if (waves == 2) SM_DEC(NB_, NBV_, 2); else SM_DEC(NB_, NBV_, 4); } while (0)
     SM_BY_LATENT_SIZE(nb, nbv, SM_DEC_W);
 #undef SM_DEC_W
+#undef SM_DEC_
 #undef SM_DEC
     SM_CHECK_LAUNCH("sm_latent_attn_decode");
     hipLaunchKernelGGL(latent_decode_merge_kernel, dim3((unsigned)(B * H)), dim3(256), 0, s, (const float*)workspace,

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256, SLIM ? 2 : 1) void latent_attn_tiles_kernel(co
     const int32_t* table = block_tables + (size_t)b * max_blocks;
     if constexpr (SLIM) {
         const int wave_max_pos = pos0 + min(tile0 + 32 * wave + 31, rows - 1) / H;
-        latent_slim_loop<NB, NBV>(qrow, cache, table, block_size, k_lo, k_hi, row_pos, wave_min_pos, wave_max_pos, c_log2, window, lds, lds2,
+        latent_slim_loop<NB, NBV, 4>(qrow, cache, table, block_size, k_lo, k_hi, row_pos, wave_min_pos, wave_max_pos, c_log2, window, lds, lds2,
                                   oacc, m_run, l_tot);
     } else {
         latent_tile_loop<NB, NBV, 4>(qrow, cache, table, R, block_size, k_lo, k_hi, row_pos, wave_min_pos, c_log2, window, lds, oacc, m_run,

@@ -175,9 +175,10 @@ __device__ __forceinline__ void latent_tile_loop(const unsigned short* __restric
 // The same walk for cache rows of exactly 32 NB columns, in tiles of 32 keys that go from global memory straight to LDS (the loop
 // above holds a tile in registers on its way: a wave of 256 columns then needs nearly 400, one wave per SIMD, with nothing to
 // fill its waits).  Two buffers, one barrier per tile; with the scores and weights of 32 keys at a time two waves share a SIMD:
-// eight prompts of about 1000 tokens, 16 heads, rows of 192 + 64: 160 -> 81 us (0.65 PFLOP/s).  A row is kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows that differ
-// mod 16, one chunk) and the 32 of a transposed read (four rows, four chunks) touch every bank once.  A wave none of whose rows
-// sees a tile leaves it out: a masked score would add an exact zero.
+// eight prompts of about 1000 tokens, 16 heads, rows of 192 + 64: 160 -> 81 us (0.65 PFLOP/s).  A row is
+// kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows that differ mod 16, one chunk) and
+// the 32 of a transposed read (four rows, four chunks) touch every bank once.  A wave none of whose rows sees a tile leaves it out: a
+// masked score would add an exact zero.
 constexpr int kSlimKeys = 32;
 
 template <int NB>
@@ -189,7 +190,7 @@ struct SlimGeom {
     __device__ static __forceinline__ int at(int r, int ch) { return RB * r + 16 * (ch ^ swz(r)); }
 };
 
-template <int NB, int NBV>
+template <int NB, int NBV, int WAVES>
 __device__ __forceinline__ void latent_slim_loop(const unsigned short* __restrict__ qrow, const unsigned short* __restrict__ cache,
                                                  const int32_t* __restrict__ table, int block_size, int k_lo, int k_hi, int row_pos,
                                                  int wave_min_pos, int wave_max_pos, float c_log2, int window, unsigned char* buf0,
@@ -204,14 +205,14 @@ __device__ __forceinline__ void latent_slim_loop(const unsigned short* __restric
 #pragma unroll
     for (int ks = 0; ks < 2 * NB; ++ks) qf[ks] = *(const bf16x8*)(qrow + 16 * ks + 8 * hi);
 
-    // one tile: pieces of 1 KB, dealt to the four waves; lane l of a piece brings the chunk that belongs at 16 l
+    // one tile: pieces of 1 KB, dealt to the waves; lane l of a piece brings the chunk that belongs at 16 l
     auto load_tile = [&](unsigned char* buf, int kt0) {
         const int page = __builtin_amdgcn_readfirstlane(kt0 / block_size);             // (a tile lies in one cache block)
         const size_t row0 = (size_t)table[page] * block_size + (kt0 - page * block_size);
 #pragma unroll
-        for (int i0 = 0; i0 < G::PIECES; i0 += 4) {
+        for (int i0 = 0; i0 < G::PIECES; i0 += WAVES) {
             const int i = i0 + wave;
-            if (G::PIECES % 4 != 0 && i >= G::PIECES) break;
+            if (G::PIECES % WAVES != 0 && i >= G::PIECES) break;
             const int c = 64 * i + lane, row = c / G::CH, ch = (c % G::CH) ^ G::swz(row);
             __builtin_amdgcn_global_load_lds((gvoid*)(cache + (row0 + min(row, k_hi - 1 - kt0)) * G::P + 8 * ch), (lvoid*)(buf + 1024 * i),
                                              16, 0, 0);

@@ -254,6 +254,23 @@ def test_matrix_core_latent_prompts_equal_portable(B, H, R, RV):
         near(a, b.double().cpu(), dt, bf16=2e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,R,RV", [(9, 1, 32, 32), (9, 16, 256, 256), (9, 33, 96, 64), (3, 65, 256, 192), (2, 128, 160, 160), (40, 16, 256, 200)])
+def test_matrix_core_latent_decode_equals_portable(B, H, R, RV):
+    """Single tokens over contexts around tiles of 32 keys, in one, two and four waves of heads (the bound as for the prompts)."""
+    g = gen(B * R + H)
+    dev, dt = "cuda", torch.bfloat16
+    lens = [1, 31, 32, 33, 64, 65, 129, 300, 700]
+    ctx, blocks = batch([(lens[(4 * i) % 9] - 1, 1) for i in range(B)], device=dev, seed=B)
+    cache = (torch.randn(blocks, 64, R, generator=g) * 0.7).to(dt).to(dev)
+    q = (torch.randn(B, H, R, generator=g) * 0.7).to(dt).to(dev)
+    sink = torch.randn(H, generator=g).to(dev)
+    for kw in (dict(), dict(sink=sink), dict(window=30), dict(window=64, sink=sink)):
+        a = seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=RV, **kw)
+        b = seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=RV, force_rows=True, **kw)
+        near(a, b.double().cpu(), dt, bf16=2e-2)
+
+
 # ------------------------------------------------------------------------------------------ latent attention with a query latent
 @pytest.mark.parametrize("device,dtype", CASES)
 @pytest.mark.parametrize("H,D,Rd,V,R,Q", [(3, 8, 8, 16, 24, 20), (1, 4, 2, 4, 8, 4), (2, 40, 24, 72, 136, 56), (4, 24, 8, 40, 112, 64),
