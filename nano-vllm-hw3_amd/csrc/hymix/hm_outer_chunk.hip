@@ -214,7 +214,11 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
     constexpr int KQ = ROWS / 2048, NP = (DELTA ? kPrepared : kTAt) / 1024, VAT = PREP + 1024 * NP;
     __shared__ __attribute__((aligned(1024))) unsigned char buf0[VAT + kChunk * 64];
     __shared__ __attribute__((aligned(1024))) unsigned char buf1[VAT + kChunk * 64];
-    __shared__ __attribute__((aligned(16))) f32x4 swap_k[2][4][64], swap_o[2][2][64];      // either wave's part of K S; of the other's rows
+    // Either wave's part of K S, and of the other's rows of results.  swap_k: written between a chunk's first and second meeting, read
+    // behind the second one.  swap_o: wave w reads swap_o[.][w] of chunk c behind the first meeting of chunk c + 1, and the other wave
+    // writes the place again at the end of a chunk.  The delta form's second meeting lies between the two; the state-space form
+    // has one meeting per chunk, so its chunks take two places in turn, and the first meeting of chunk c + 2 lies between.
+    __shared__ __attribute__((aligned(16))) f32x4 swap_k[2][4][64], swap_o[DELTA ? 1 : 2][2][2][64];
     const int b = blockIdx.x, h = blockIdx.y, gr = h / (H / G), lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = blockIdx.z * 32 + l31;
@@ -275,12 +279,12 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
     };
     double part[8];                                          // the last chunk's results of tokens 16 wave..: this wave's part
     // (in double: in float32 the state-space form's error was 1 to 5 % above the token-by-token walk's; 1 us of 142)
-    // their sum with the other wave's part, written before the last meeting
-    auto store_rows = [&](int t0, bool whole) {
+    // their sum with the other wave's part, written before the last meeting (turn: 0 for an even chunk of the portion, 1 for an odd one)
+    auto store_rows = [&](int t0, bool whole, int turn) {
         float* orow = o + ((size_t)(q0 + t0 + 16 * wave + 4 * hi) * H + h) * V + col;
 #pragma unroll
         for (int r4 = 0; r4 < 2; ++r4) {
-            const f32x4 y = swap_o[wave][r4][lane];
+            const f32x4 y = swap_o[DELTA ? 0 : turn][wave][r4][lane];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int t = e + 8 * r4;
@@ -288,11 +292,11 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
             }
         }
     };
-    auto chunk = [&](unsigned char* buf, unsigned char* nxt, int t0) {
+    auto chunk = [&](unsigned char* buf, unsigned char* nxt, int t0, int turn) {
         const int left = n - t0;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the chunk has landed (and rows of results a whole chunk old)
         meet();
-        if (t0 > 0) store_rows(t0 - kChunk, true);
+        if (t0 > 0) store_rows(t0 - kChunk, true, turn ^ 1);
         if (left < kChunk) {                                  // an absent token's row: zeros, whatever the one in its place holds
             for (int i = left * GM::RB + 16 * (int)threadIdx.x; i < ROWS; i += 2048) {
                 *(i32x4*)(buf + i) = i32x4{0, 0, 0, 0};
@@ -425,7 +429,7 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
                     part[r] = c * (qb + qs) + (pb + ps);
                     if (!DELTA) part[r] += (double)skip * (double)(wave ? v[g] : v[r]);
                 }
-                swap_o[wave ^ 1][r4][lane] = y;
+                swap_o[DELTA ? 0 : turn][wave ^ 1][r4][lane] = y;
             }
         }
 #pragma unroll
@@ -435,11 +439,11 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
     };
     load_chunk(buf0, 0);
     for (int t0 = 0; t0 < n; t0 += 2 * kChunk) {
-        chunk(buf0, buf1, t0);
-        if (t0 + kChunk < n) chunk(buf1, buf0, t0 + kChunk);
+        chunk(buf0, buf1, t0, 0);
+        if (t0 + kChunk < n) chunk(buf1, buf0, t0 + kChunk, 1);
     }
     meet();
-    store_rows((n - 1) / kChunk * kChunk, false);
+    store_rows((n - 1) / kChunk * kChunk, false, (n - 1) / kChunk & 1);
 #pragma unroll
     for (int blk = 0; blk < NB; ++blk)
 #pragma unroll

@@ -246,6 +246,41 @@ def test_portions_by_chunks_equal_the_walk(monkeypatch, kind, H, G, D, V):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["delta", "space"])
+@pytest.mark.parametrize("H,D,V", [(24, 64, 64), (12, 128, 96)])
+def test_long_portions_by_chunks_keep_every_chunks_results(monkeypatch, kind, H, D, V):
+    """Portions of 8 to 47 chunks on more workgroups than the chip runs at once, several times: the two waves of a workgroup exchange
+    parts of a chunk's results, and a part of another chunk in their place is an error of the size of the results in half a chunk's
+    rows.  Every chunk's rows are within 32 roundings of 2^-24 of the walk's in norm (either is within 16 of the exact sums), and
+    every run gives the same bits."""
+    g = gen(H + D)
+    lens = [1500, 256, 1023, 777, 1337, 288, 640, 1024] * 3
+    n = sum(lens)
+    rows = rnd(g, n, 2 * D + H * V, dtype=torch.bfloat16).cuda()
+    pre = rnd(g, n, 2 * H, s=2.0, dtype=torch.bfloat16).cuda()
+    A, bias = (t.cuda() for t in forget(g, H))
+    skip = rnd(g, H).cuda()
+    ctx, _ = batch([(0, m) for m in lens], device="cuda", seed=1)
+    slots = max(int(s) for s in ctx.seq_slot) + 1
+
+    def run(least):
+        monkeypatch.setattr(hy_ops, "CHUNKS_MIN_TOKENS", {D: least} if least else {})
+        st = torch.zeros(slots, H, D, V, device="cuda")
+        if kind == "delta":
+            return hy_ops.gated_delta(rows, 0, D, 2 * D, pre, 0, H, A, bias, H, 1, D, V, st, ctx, q_scale=0.37)
+        return hy_ops.state_space(rows, 2 * D, 0, D, pre, 0, A, bias, skip, H, 1, D, V, st, ctx)
+    walk, first = run(0).double(), run(1)
+    at = 0
+    for m in lens:
+        for t in range(at, at + m, 32):
+            e = min(t + 32, at + m)
+            assert (first[t:e].double() - walk[t:e]).norm() <= 32 * 2 ** -24 * walk[t:e].norm()
+        at += m
+    for _ in range(10):
+        assert torch.equal(run(1), first)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("D,V", [(32, 64), (64, 128), (128, 64), (256, 72)])
 def test_recurrence_forms_agree(dtype, D, V):
