@@ -60,7 +60,8 @@ def build(force=False, verbose=True, target="qlinear"):
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     hipcc = _hipcc()
-    headers = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".h")]
+    shared = os.path.join(HERE, "csrc")                                   # headers of more than one library lie there
+    headers = [os.path.join(d, f) for d in {CSRC, shared} for f in os.listdir(d) if f.endswith(".h")]
     headers.append(os.path.join(HERE, "..", "include", spec["header"]))
     srcs = sorted(f for f in os.listdir(CSRC) if f.endswith(".hip"))      # every translation unit of the folder
 

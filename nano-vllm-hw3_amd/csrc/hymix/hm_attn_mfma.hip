@@ -4,6 +4,7 @@
 //   single-token queries (decode): the group's query heads of a sequence's one token are the rows of one wave; the tile
 //     list is split over workgroups, every (sequence, split, head) leaves an unnormalised partial state {m c, l, O} in the
 //     workspace, and a second launch merges the splits in order and adds the sink to the denominator.
+#include "../row_deal.h"
 #include "hm_attn_tile.h"
 
 namespace hm {
@@ -35,23 +36,15 @@ __global__ __launch_bounds__(256, 2) void attn_tiles_kernel(const unsigned short
                                                          int max_blocks, const unsigned short* __restrict__ kp,
                                                          const unsigned short* __restrict__ vp, int pool, int pool_rows,
                                                          int chunk, const float* __restrict__ head_bias, float softcap, OutArgs out, int B, int tiles,
-                                                         int by_die) {
+                                                         int run) {
     // (the two LDS arrays are the slim loop's buffers, or the key and the value tile)
     __shared__ __attribute__((aligned(1024))) unsigned char lds_k[SLIM ? SlimGeom<NBK>::BYTES + SlimGeom<NBV>::BYTES : TileGeom<NBK>::LDS_BYTES];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_v[SLIM ? SlimGeom<NBK>::BYTES + SlimGeom<NBV>::BYTES : TileGeom<NBV>::LDS_BYTES];
-    // Workgroups go to the eight dies in turn: all row tiles of a (sequence, key/value head) on one die, whose L2 then reads its
-    // keys and values once (by_die; with few pairs the row tiles are dealt to the dies instead)
-    int pair = blockIdx.x / tiles, xt = blockIdx.x - pair * tiles;
-    if (by_die) {
-        const int j = blockIdx.x >> 3;
-        pair = j / tiles;
-        xt = j - pair * tiles;
-        pair = 8 * pair + (blockIdx.x & 7);
-    }
-    const int b = pair / G, g = pair - b * G, rep = H / G;
-    if (b >= B) return;
+    const RowTile rt = row_tile(blockIdx.x, blockIdx.y, blockIdx.z, run, tiles, B, G);
+    if (rt.b < 0) return;
+    const int b = rt.b, g = rt.g, rep = H / G;
     const int q0 = qstart[b], rows = (qstart[b + 1] - q0) * rep;
-    const int tile0 = (tiles - 1 - xt) * 128;                                  // heaviest tiles first
+    const int tile0 = (tiles - 1 - rt.tile) * 128;                             // heaviest tiles first
     if (tile0 >= rows) return;
     const int pos0 = seq_pos0[b];
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
@@ -258,11 +251,8 @@ extern "C" int hm_attn_tiles(const void* q, const void* k_cache, const void* v_c
     }
     if (B == 0 || max_q == 0) return HM_OK;
     const int64_t tiles = ((int64_t)max_q * (H / G) + 127) / 128;
-    const int64_t pairs = (int64_t)B * G;
-    const int by_die = pairs >= 32 || pairs % 8 == 0;          // (fewer pairs would leave dies idle)
-    const int64_t groups = (by_die ? (pairs + 7) / 8 * 8 : pairs) * tiles;
-    if (groups > 0x7fffffff) { set_error("hm_attn_tiles: too many rows"); return HM_ESHAPE; }
-    dim3 grid((unsigned)groups), block(256);
+    const RowGrid rg = row_grid(tiles, B, G);
+    dim3 grid(rg.x, rg.y, rg.z), block(256);
     hipStream_t s = as_stream(stream);
     const int nbk = padded_nb(D), nbv = padded_nb(V);
     const bool slim = D == 32 * nbk && V == 32 * nbv;
@@ -272,7 +262,7 @@ extern "C" int hm_attn_tiles(const void* q, const void* k_cache, const void* v_c
     hipLaunchKernelGGL((attn_tiles_kernel<K_, V_, S_, SLIM_>), grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k_cache, \
                        (const unsigned short*)v_cache, block_tables, qstart, seq_pos0, sink, window, keep_first, scale,       \
                        (unsigned short*)o, H, G, D, V, block_size, max_blocks, (const unsigned short*)kp_cache,               \
-                       (const unsigned short*)vp_cache, pool, pool_rows, chunk, head_bias, softcap, out, B, (int)tiles, by_die)
+                       (const unsigned short*)vp_cache, pool, pool_rows, chunk, head_bias, softcap, out, B, (int)tiles, rg.run)
     HM_BY_HEAD_SIZE(nbk, nbv, sigmoid_w, softcap, HM_TILES);
 #undef HM_TILES
 #undef HM_TILES_

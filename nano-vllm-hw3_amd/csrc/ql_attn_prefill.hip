@@ -21,6 +21,7 @@
 // (Tiles of 32 keys fit three waves and are no faster with full CUs, 76 and 128 us, and slower where a CU has one
 // workgroup and a tile's chain of dependent steps is what counts: 128 us and 38.)
 #include "ql_common.h"
+#include "row_deal.h"
 
 namespace ql {
 
@@ -39,30 +40,22 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const unsigned sho
                                                               const unsigned short* __restrict__ v,
                                                               const int* __restrict__ cu_seqlens,
                                                               unsigned short* __restrict__ out, float c_log2, int Hq,
-                                                              int Hkv, int kv_group, int blocks, int pairs, int by_die) {
+                                                              int Hkv, int kv_group, int blocks, int num_seqs, int run) {
     constexpr int SUBS = 4 / G;            // 32-row query blocks per head in this workgroup
     constexpr int QROWS = 32 * SUBS;
     constexpr int V_AT = kTileKeys * 256;  // the value tile behind the key tile
     __shared__ __attribute__((aligned(1024))) unsigned char buf0[2 * kTileKeys * 256];
     __shared__ __attribute__((aligned(1024))) unsigned char buf1[2 * kTileKeys * 256];
 
-    // Workgroups go to the eight dies in turn: all query blocks of a (sequence, group of heads) on one die, whose L2 then
-    // reads its keys and values once (by_die; with few such pairs the query blocks are dealt to the dies instead)
-    int pair = blockIdx.x / blocks, xb = blockIdx.x - pair * blocks;
-    if (by_die) {
-        const int j = blockIdx.x >> 3;
-        pair = j / blocks;
-        xb = j - pair * blocks;
-        pair = 8 * pair + (blockIdx.x & 7);
-    }
-    if (pair >= pairs) return;
+    const RowTile rt = row_tile(blockIdx.x, blockIdx.y, blockIdx.z, run, blocks, num_seqs, Hq / G);
+    if (rt.b < 0) return;
     // a group of G query heads reads the K/V of kv head (group * G) / kv_group, which is the group itself when a kv
     // head's query heads form one group (kv_group == G: ratios 1, 2, 4); other ratios are dealt to several groups per
     // kv head
-    const int ngroups = Hq / G, seq = pair / ngroups, hgrp = pair - seq * ngroups, hk = (hgrp * G) / kv_group;
+    const int seq = rt.b, hgrp = rt.g, hk = (hgrp * G) / kv_group;
     const int s0 = cu_seqlens[seq];
     const int L = cu_seqlens[seq + 1] - s0;
-    const int q0 = (blocks - 1 - xb) * QROWS;                           // heaviest query blocks first
+    const int q0 = (blocks - 1 - rt.tile) * QROWS;                      // heaviest query blocks first
     if (q0 >= L) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -224,16 +217,13 @@ extern "C" int ql_attn_prefill(const void* q, const void* k, const void* v, cons
     if (num_seqs == 0 || max_seqlen == 0) return QL_OK;
     if (num_seqs > 65535 || Hq / G > 65535) { set_error("ql_attn_prefill: too many sequences or heads"); return QL_ESHAPE; }
     const int qrows = 128 / G, blocks = (max_seqlen + qrows - 1) / qrows;
-    const int64_t pairs = (int64_t)num_seqs * (Hq / G);
-    const int by_die = pairs >= 32 || pairs % 8 == 0;
-    const int64_t groups = (by_die ? (pairs + 7) / 8 * 8 : pairs) * blocks;
-    if (groups > 0x7fffffff) { set_error("ql_attn_prefill: too many rows"); return QL_ESHAPE; }
-    dim3 grid((unsigned)groups), block(256);
+    const RowGrid rg = row_grid(blocks, num_seqs, Hq / G);
+    dim3 grid(rg.x, rg.y, rg.z), block(256);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
 #define QL_PF(G_)                                                                                              \
     hipLaunchKernelGGL(attn_prefill_kernel<G_>, grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k, \
-                       (const unsigned short*)v, cu_seqlens, (unsigned short*)out, c, Hq, Hkv, kv_group, blocks, (int)pairs, by_die)
+                       (const unsigned short*)v, cu_seqlens, (unsigned short*)out, c, Hq, Hkv, kv_group, blocks, num_seqs, rg.run)
     if (G == 1) QL_PF(1); else if (G == 2) QL_PF(2); else QL_PF(4);
 #undef QL_PF
     QL_CHECK_LAUNCH("ql_attn_prefill");

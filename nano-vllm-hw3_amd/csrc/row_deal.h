@@ -1,0 +1,44 @@
+// How the prompt attention kernels' workgroups are dealt to the eight dies, each with an L2 of its own.  A kernel's work is
+// `tiles` row tiles (tile 0 the heaviest: the last rows, which see most keys) of each of B sequences by G groups of heads; a
+// (sequence, group) pair's tiles read the same keys and values.  A short sequence among longer ones has its last tiles only.
+#pragma once
+#include <stdint.h>
+
+#ifdef __HIPCC__
+#include <hip/hip_runtime.h>
+#define ROW_DEAL_FN __host__ __device__ __forceinline__
+#else
+#define ROW_DEAL_FN inline
+#endif
+
+// Two grids; consecutive workgroups go to the dies in turn.
+// Few pairs, which would leave dies idle: (tiles, B, G), every tile to the next die (run 0).
+// Else eight pairs after eight pairs, (8 tiles, ceil(B G / 8)): a run of kRowRun neighbouring tiles of a pair on one die, whose L2
+// then reads their keys once, and the next run of the pair as many dies further on as a sequence's heads take, so that one long
+// prompt among short ones has the whole chip.  (All tiles of a pair on one die: 2000 tokens and 31 single ones in latent attention, 16
+// heads: 269 us on one die, 94 by runs, 104 dealt one by one in an older kernel; 8192 and 7 single ones 3292 / 495 / 850; 8 x 1000
+// 90 / 82 / 164.  With 2 key/value heads of 16 / 2, 8192 and 7 single ones 1266 / 362 / 792.  Runs of 4 and of 16 are within 3 %.)
+// The number of a pair's places is odd: a die deals its workgroups to its shader engines in turn, too, and with an even one the
+// single tiles of the short sequences all met on one of them (500 tokens and 127 single ones, 16 / 8 heads: 331 -> 126 us).  Below
+// eight tiles the empty place would cost more (8 x 100 tokens, 32 / 8 heads: 8.9 -> 10.7 us).
+constexpr int kRowRun = 8;
+
+struct RowGrid { uint32_t x, y, z; int run; };
+
+static inline RowGrid row_grid(int64_t tiles, int B, int G) {
+    const int64_t pairs = (int64_t)B * G;
+    if (pairs >= 32 || pairs % 8 == 0)
+        return {(uint32_t)(8 * (tiles < 8 ? tiles : tiles | 1)), (uint32_t)((pairs + 7) / 8), 1u, kRowRun};
+    return {(uint32_t)tiles, (uint32_t)B, (uint32_t)G, 0};
+}
+
+struct RowTile { int b, g, tile; };                  // b < 0: nothing to do
+
+// the tile of workgroup (x, y, z)
+ROW_DEAL_FN RowTile row_tile(uint32_t x, uint32_t y, uint32_t z, int run, int tiles, int B, int G) {
+    if (run == 0) return {(int)y, (int)z, (int)x};
+    const int tile = x >> 3, step = G & -G;          // step: a divisor of eight (or a multiple, which stays), 8 / step dies per pair
+    const int pair = 8 * (int)y + (((int)(x & 7) - step * (tile / run)) & 7);
+    if (pair >= B * G || tile >= tiles) return {-1, 0, 0};
+    return {pair / G, pair % G, tile};
+}

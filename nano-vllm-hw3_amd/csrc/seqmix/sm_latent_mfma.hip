@@ -1,6 +1,7 @@
 // Latent attention on the matrix cores, portions of any length: a workgroup of four waves owns 128 consecutive
 // query rows of ONE sequence's portion (rows run token by token, head by head, so a row's last visible key is the
 // position of its token) and walks the cache tiles up to the last row's position.
+#include "../row_deal.h"
 #include "sm_latent_tile.h"
 
 namespace sm {
@@ -14,22 +15,15 @@ __global__ __launch_bounds__(256, SLIM ? 2 : 1) void latent_attn_tiles_kernel(co
                                                                 const int32_t* __restrict__ seq_pos0,
                                                                 unsigned short* __restrict__ o, float c_log2, int H, int R,
                                                                 int block_size, int max_blocks, int RV, int window,
-                                                                const float* __restrict__ sink, int B, int tiles, int by_die) {
+                                                                const float* __restrict__ sink, int B, int tiles, int run) {
     // (the slim loop has two buffers of half a tile)
     __shared__ __attribute__((aligned(1024))) unsigned char lds[SLIM ? SlimGeom<NB>::BYTES : TileGeom<NB>::LDS_BYTES];
     __shared__ __attribute__((aligned(1024))) unsigned char lds2[SLIM ? SlimGeom<NB>::BYTES : 16];
-    // Workgroups go to the eight dies in turn: all row tiles of a sequence on one die, whose L2 then reads its rows once (by_die;
-    // with few sequences the row tiles are dealt to the dies instead)
-    int b = blockIdx.x / tiles, xt = blockIdx.x - b * tiles;
-    if (by_die) {
-        const int j = blockIdx.x >> 3;
-        b = j / tiles;
-        xt = j - b * tiles;
-        b = 8 * b + (blockIdx.x & 7);
-    }
-    if (b >= B) return;
+    const RowTile rt = row_tile(blockIdx.x, blockIdx.y, blockIdx.z, run, tiles, B, 1);
+    if (rt.b < 0) return;
+    const int b = rt.b;
     const int q0 = qstart[b], rows = (qstart[b + 1] - q0) * H;
-    const int tile0 = (tiles - 1 - xt) * 128;                                  // heaviest tiles first
+    const int tile0 = (tiles - 1 - rt.tile) * 128;                             // heaviest tiles first
     if (tile0 >= rows) return;
     const int pos0 = seq_pos0[b];
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
@@ -88,10 +82,8 @@ extern "C" int sm_latent_attn_tiles(const void* q, const void* cache, const int3
     }
     if (B == 0 || max_q == 0) return SM_OK;
     const int64_t tiles = ((int64_t)max_q * H + 127) / 128;
-    const int by_die = B >= 32 || B % 8 == 0;
-    const int64_t groups = (by_die ? ((int64_t)B + 7) / 8 * 8 : B) * tiles;
-    if (groups > 0x7fffffff) { set_error("sm_latent_attn_tiles: too many rows"); return SM_ESHAPE; }
-    dim3 grid((unsigned)groups), block(256);
+    const RowGrid rg = row_grid(tiles, B, 1);
+    dim3 grid(rg.x, rg.y, rg.z), block(256);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
     const int nb = (R + 31) / 32, nbv = (RV + 31) / 32;
@@ -99,7 +91,7 @@ extern "C" int sm_latent_attn_tiles(const void* q, const void* cache, const int3
 #define SM_TILES_(NB_, NBV_, SLIM_)                                                                                       \
     hipLaunchKernelGGL((latent_attn_tiles_kernel<NB_, NBV_, SLIM_>), grid, block, 0, s, (const unsigned short*)q,                 \
                        (const unsigned short*)cache, block_tables, qstart, seq_pos0, (unsigned short*)o, c, H, R, block_size, \
-                       max_blocks, RV, window, sink, B, (int)tiles, by_die)
+                       max_blocks, RV, window, sink, B, (int)tiles, rg.run)
     SM_BY_LATENT_SIZE(nb, nbv, SM_TILES);
 #undef SM_TILES
 #undef SM_TILES_
