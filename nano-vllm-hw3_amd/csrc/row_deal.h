@@ -12,7 +12,7 @@
 #endif
 
 // Two grids; consecutive workgroups go to the dies in turn.
-// Few pairs, which would leave dies idle: (tiles, B, G), every tile to the next die (run 0).
+// Few pairs, which would leave dies idle, or more than the other grid holds: (tiles, B, G), every tile to the next die (run 0).
 // Else eight pairs after eight pairs, (8 tiles, ceil(B G / 8)): a run of kRowRun neighbouring tiles of a pair on one die, whose L2
 // then reads their keys once, and the next run of the pair as many dies further on as a sequence's heads take, so that one long
 // prompt among short ones has the whole chip.  (All tiles of a pair on one die: 2000 tokens and 31 single ones in latent attention, 16
@@ -27,7 +27,7 @@ struct RowGrid { uint32_t x, y, z; int run; };
 
 static inline RowGrid row_grid(int64_t tiles, int B, int G) {
     const int64_t pairs = (int64_t)B * G;
-    if (pairs >= 32 || pairs % 8 == 0)
+    if ((pairs >= 32 || pairs % 8 == 0) && pairs <= 8 * 65535 && tiles < 1 << 20)        // (2^32 threads in x, 65535 groups in y)
         return {(uint32_t)(8 * (tiles < 8 ? tiles : tiles | 1)), (uint32_t)((pairs + 7) / 8), 1u, kRowRun};
     return {(uint32_t)tiles, (uint32_t)B, (uint32_t)G, 0};
 }

@@ -8,11 +8,15 @@ import subprocess
 import pytest
 import torch
 
-from nanovllm import seq_ops
+from nanovllm import ops, seq_ops
 from test_lilevik_ops import batch
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nano-vllm-hw3_amd", "csrc")
 SOURCE = """#include "row_deal.h"
+extern "C" void grid_of(int64_t tiles, int B, int G, uint32_t* out) {
+    const RowGrid g = row_grid(tiles, B, G);
+    out[0] = g.x; out[1] = g.y; out[2] = g.z; out[3] = (uint32_t)g.run;
+}
 extern "C" void walk(int tiles, int B, int G, int* seen, int* die) {     // [B][G][tiles]: how often, and on which die
     const RowGrid g = row_grid(tiles, B, G);
     uint64_t id = 0;
@@ -58,6 +62,15 @@ def test_every_tile_once_and_a_sequence_on_every_die(deal, B, G, tiles):
         assert load.max() - load.min() <= 1
 
 
+@pytest.mark.parametrize("tiles,B,G", [(128, 20000, 8), (8192, 1024, 8), (2 ** 20, 64, 1), (2 ** 20 + 5, 8, 1), (1, 65535, 65535), (4096, 65535, 128)])
+def test_grids_within_the_launch_limits(deal, tiles, B, G):
+    """Fewer than 2^32 threads of 256 in x and at most 65535 groups in y and z, whatever number of sequences and heads is taken."""
+    out = (ctypes.c_uint32 * 4)()
+    deal.grid_of(ctypes.c_int64(tiles), B, G, out)
+    assert out[0] * 256 < 2 ** 32 and out[1] <= 65535 and out[2] <= 65535
+    assert out[0] * out[1] * out[2] >= tiles * B * G
+
+
 def _us(f, n=20):
     for _ in range(5):
         f()
@@ -87,3 +100,19 @@ def test_one_prompt_among_single_tokens_has_the_whole_chip():
     prompt, single = [(0, 2000)], [(899, 1)] * 31
     together, apart = us(prompt + single), us(prompt) + us(single)
     assert together <= 1.6 * apart, (together, apart)
+
+
+@pytest.mark.gpu
+def test_prompt_attention_of_more_pairs_than_one_grid_dimension_holds():
+    """20000 sequences by 8 heads, the longest of 129 row tiles: more workgroups than 2^32 threads.  Every row is what it is in a call
+    of its own sequence."""
+    g = torch.Generator().manual_seed(3)
+    lens = [16500] + [1] * 19999
+    T = sum(lens)
+    q, k, v = (torch.randn(T, 8, 128, generator=g).bfloat16().cuda() for _ in range(3))
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    out = ops.attn_prefill(q, k, v, cu, max(lens), 128 ** -0.5)
+    n = lens[0]
+    alone = ops.attn_prefill(q[:n], k[:n], v[:n], cu[:2], n, 128 ** -0.5)
+    assert torch.equal(out[:n], alone)
+    assert torch.equal(out[n:], v[n:])                     # a sequence of one token returns its value
