@@ -9,6 +9,8 @@
 // Operands go from global memory straight to the MFMA registers: both matrices are K-contiguous, a lane owns one row
 // and 32 consecutive k of a 64-k step (four 16-byte loads, four MFMA steps; the k order inside a step is free as
 // long as both operands agree).
+#include <algorithm>
+
 #include "sm_common.h"
 
 namespace sm {
@@ -214,13 +216,19 @@ extern "C" int sm_moe_combine(const void* prod, const int32_t* pair_row, const f
     }
     if (T == 0) return SM_OK;
     const bool wide = W % 8 == 0 && ((uintptr_t)prod | (uintptr_t)shared | (uintptr_t)y) % 16 == 0;
-    const int64_t items = T * (wide ? W / 8 : W), blocks = (items + 255) / 256;
-    if (blocks > 0x7fffffff) { set_error("sm_moe_combine: too many rows"); return SM_ESHAPE; }
+    const int per = wide ? W / 8 : W;
+    const int64_t most = (((int64_t)1 << 32) - 256) / per;     // tokens of one launch: a grid holds fewer than 2^32 threads
+    for (int64_t t = 0; t < T; t += most) {
+        const int64_t items = std::min(most, T - t) * per;
+        const dim3 grid((unsigned)((items + 255) / 256));
+        const unsigned short* sh = shared ? (const unsigned short*)shared + t * W : nullptr;
 #define SM_COMBINE(V_)                                                                                                         \
-    hipLaunchKernelGGL(moe_combine_kernel<V_>, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), (const unsigned short*)prod, \
-                       pair_row, wts, (const unsigned short*)shared, (unsigned short*)y, items, top, W, shared_scale)
-    if (wide) SM_COMBINE(8); else SM_COMBINE(1);
+    hipLaunchKernelGGL(moe_combine_kernel<V_>, grid, dim3(256), 0, as_stream(stream), (const unsigned short*)prod, pair_row + t * top,    \
+                       wts ? wts + t * top : nullptr, sh, (unsigned short*)y + t * W, items, top, W,                              \
+                       shared_scale ? shared_scale + t : nullptr)
+        if (wide) SM_COMBINE(8); else SM_COMBINE(1);
 #undef SM_COMBINE
-    SM_CHECK_LAUNCH("sm_moe_combine");
+        SM_CHECK_LAUNCH("sm_moe_combine");
+    }
     return SM_OK;
 }

@@ -335,6 +335,20 @@ def test_moe_large_tiles_equal_small_ones(T, W, F, E, top, act):
     assert (y[1].float() - ref).norm() < 2 ** -7 * ref.norm()
 
 
+@pytest.mark.gpu
+def test_moe_combine_of_more_elements_than_a_grid_has_threads():
+    """2.2 million tokens of 2044 channels (a width without 16-byte rows): 4.5e9 elements, more than 2^32 threads."""
+    from nanovllm import _seqmix as SM
+    T, W, rows = 2_200_000, 2044, 8
+    prod = torch.randn(rows, W, generator=gen(1)).cuda().bfloat16()
+    pair_row = torch.randint(0, rows, (T,), generator=gen(2), dtype=torch.int32).cuda()
+    y = torch.zeros(T, W, dtype=torch.bfloat16, device="cuda")
+    SM.check(SM.load().sm_moe_combine(prod.data_ptr(), pair_row.data_ptr(), None, None, None, y.data_ptr(), T, 1, W,
+                                      torch.cuda.current_stream().cuda_stream))
+    for t in range(0, T, 200_000):
+        assert torch.equal(y[t:t + 200_000], prod[pair_row[t:t + 200_000].long()])
+
+
 def test_oracle_absorbed_form_is_the_explicit_one():
     """The oracle's two statements of the attention agree: explicit keys / values, and queries that carry W_uk."""
     g = gen(11)
