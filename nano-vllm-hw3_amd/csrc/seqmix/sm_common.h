@@ -51,15 +51,11 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 // the gated forms: g' = min(g, limit), u' = clamp(u, +-limit), g' sigmoid(alpha g') (u' + 1) (SM_ACT_CLAMPED_GLU), or with
 // SM_ACT_SILU_GLU the same without the one: silu(g) u for limit = +inf and alpha = 1; SM_ACT_GELU_TANH_GLU: gelu_tanh(g) u
-// RCP: the quotient by the hardware's reciprocal (1 ulp) instead of the full division, for results that leave in bf16: in the
-// matrix-core expert kernels a quarter of the epilogue was the division
-template <bool RCP = false>
 __device__ __forceinline__ float gated_act(float g, float u, float limit, float alpha, int act) {
     if (act == SM_ACT_GELU_TANH_GLU) return gelu_tanh(g) * u;
     g = fminf(g, limit);
     u = fminf(fmaxf(u, -limit), limit);
-    const float den = 1.f + __expf(-alpha * g);
-    return (RCP ? g * __builtin_amdgcn_rcpf(den) : g / den) * (u + (act == SM_ACT_SILU_GLU ? 0.f : 1.f));
+    return g / (1.f + __expf(-alpha * g)) * (u + (act == SM_ACT_SILU_GLU ? 0.f : 1.f));
 }
 __host__ __device__ __forceinline__ bool act_is_gated(int act) {
     return act == SM_ACT_CLAMPED_GLU || act == SM_ACT_SILU_GLU || act == SM_ACT_GELU_TANH_GLU;

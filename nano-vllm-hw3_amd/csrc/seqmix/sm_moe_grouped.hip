@@ -19,7 +19,7 @@ constexpr int kRowsPerTile = 32;
 
 __device__ __forceinline__ float glu_bf16(float g, float u, float limit, float alpha, int act) {
     // the products leave the matrix unit in bf16, as a GEMM's output would
-    return gated_act<true>((float)(bf16_t)g, (float)(bf16_t)u, limit, alpha, act);
+    return gated_act((float)(bf16_t)g, (float)(bf16_t)u, limit, alpha, act);
 }
 
 __device__ __forceinline__ bf16x8 load8(const unsigned short* p, int k, int K) {

@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
         if (GATE_UP) {
             const bf16x8 u = *(const bf16x8*)(src + 16 * ((c + 16) ^ (row & 31)));
 #pragma unroll
-            for (int r = 0; r < 8; ++r) x[r] = (bf16_t)gated_act<true>((float)x[r], (float)u[r], limit, alpha, act_kind);
+            for (int r = 0; r < 8; ++r) x[r] = (bf16_t)gated_act((float)x[r], (float)u[r], limit, alpha, act_kind);
         } else if (MODE == 2) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) x[r] = (bf16_t)plain_act((float)x[r], act_kind);

@@ -349,6 +349,28 @@ def test_moe_combine_of_more_elements_than_a_grid_has_threads():
         assert torch.equal(y[t:t + 200_000], prod[pair_row[t:t + 200_000].long()])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["pairs", "grouped", "tiles128"])
+def test_moe_gate_divides_where_the_denominator_is_large(form):
+    """silu(g) u with exp(-g) past 2^126, where the reciprocal of the denominator is below the smallest normal float and the quotient
+    is not: with u = 2^100 the products are of the order of 1e-6.  Exact but for __expf (the rounding of -g log2(e), 2^-24 of 128,
+    times log 2: 6e-6) and the two bf16 roundings, 2^-8 each at most."""
+    W, F, T = 64, 32, 40
+    gate = torch.linspace(-88.5, -87.5, 3).repeat(11)[:F]
+    h = torch.zeros(T, W)
+    h[:, 0] = 1
+    w_gu = torch.zeros(1, 2 * F, W)
+    w_gu[0, :F, 0], w_gu[0, F:, 0] = gate, 2.0 ** 100
+    w_down = torch.zeros(1, W, F)
+    w_down[0, torch.arange(F), torch.arange(F)] = 1
+    args = [t.cuda().bfloat16() for t in (h, w_gu, w_down)]
+    y = seq_ops.moe_experts(args[0], torch.zeros(T, 1, dtype=torch.int32).cuda(), torch.ones(T, 1).cuda(), args[1], args[2], float("inf"), 1.0,
+                            form=form, act_kind=seq_ops.ACT_SILU_GLU).double().cpu()
+    g = gate.double()
+    ref = g / (1 + torch.exp(-g)) * 2.0 ** 100
+    assert ((y[:, :F] - ref).abs() <= (2 * 2.0 ** -8 + 6e-6) * ref.abs()).all()
+
+
 def test_oracle_absorbed_form_is_the_explicit_one():
     """The oracle's two statements of the attention agree: explicit keys / values, and queries that carry W_uk."""
     g = gen(11)
