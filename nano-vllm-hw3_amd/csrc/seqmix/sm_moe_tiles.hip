@@ -29,18 +29,19 @@ constexpr int kBigRows = 128;                 // tiles are one or two times as m
 template <int MODE, int MB>
 __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                            const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
-                                                           unsigned short* __restrict__ out, int top, int N, int K, int tiles, int nct,
+                                                           unsigned short* __restrict__ out, int top, int N, int K, int tiles, int nct, int cols, int segs,
                                                            float limit, float alpha, int act_kind, const float* __restrict__ in_wts) {
     constexpr bool GATE_UP = MODE == 1, FROM_TOKENS = MODE != 0;
     constexpr int ROWS = 64 * MB, A_BYTES = ROWS * 128, BUF = A_BYTES + 8 * 4096;
     constexpr int NA = 2 * MB;                                // 1 KB pieces of A a wave loads per step (and 8 of B)
     __shared__ __attribute__((aligned(1024))) unsigned char buf0[BUF];
     __shared__ __attribute__((aligned(1024))) unsigned char buf1[BUF];
-    // Workgroups go to the eight dies in turn; a die takes two neighbouring row tiles and all their column tiles before its next
-    // two, so that its L2 sees a row tile's activations nct times and a column tile's weights twice.
-    const int id = blockIdx.x >> 3, unit = id / (2 * nct), in_unit = id - unit * 2 * nct;
-    const int tile = (unit * 8 + (blockIdx.x & 7)) * 2 + (in_unit & 1), ct = in_unit >> 1;
-    if (tile >= tiles) return;
+    // Workgroups go to the eight dies in turn; a die takes two neighbouring row tiles and one of `segs` parts of their column tiles
+    // before its next such unit, so that its L2 sees a row tile's activations several times and a column tile's weights twice.
+    const int id = blockIdx.x >> 3, turn = id / (2 * cols), in_unit = id - turn * 2 * cols;
+    const int unit = turn * 8 + (blockIdx.x & 7), rows2 = unit / segs;
+    const int tile = rows2 * 2 + (in_unit & 1), ct = (unit - rows2 * segs) * cols + (in_unit >> 1);
+    if (tile >= tiles || ct >= nct) return;
     const int e = tile_expert[tile];
     if (e < 0) return;                                        // (uniform over the workgroup)
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
@@ -226,17 +227,25 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
 // 2048 rows 942 / 734, 634 / 514).
 static int tile_rows(int64_t T, int top, int E) { return T * top >= (int64_t)128 * E ? 256 : 128; }
 
+// Units of work that a launch makes at least, by cutting the column tiles of its pairs of row tiles into parts: a pair of row tiles is
+// one die's, so few of them left dies without any (us, 128-row tiles, weights not in a cache, whole pairs / parts: one expert of 4096 x
+// 11008 687 / 295, two of 4096 x 4096 257 / 172, four of 2048 x 4096 184 / 138, eight of 4096 x 14336 970 / 807; 16 experts of
+// 1024 x 768 58 / 59).  Two units per die: with one the largest of these is 30 % slower at 512 rows, with four the small ones lose up
+// to 3 % to activations read by more dies.
+constexpr int kUnits = 16;
+
 template <int MODE>
 static void launch_tiles(int rows, const void* a, const void* w, const int32_t* row_pair, const int32_t* tile_expert, void* out, int top,
                          int tiles, int N, int K, float limit, float alpha, int act_kind, const float* in_wts, hipStream_t s) {
-    const int nct = MODE == 1 ? (N + 127) / 128 : (N + 255) / 256, units = (tiles + 1) / 2;
-    dim3 grid((unsigned)((units + 7) / 8 * 8 * 2 * nct));
+    const int nct = MODE == 1 ? (N + 127) / 128 : (N + 255) / 256, pairs = (tiles + 1) / 2;
+    const int want = (kUnits + pairs - 1) / pairs, cols = (nct + want - 1) / want, segs = (nct + cols - 1) / cols;
+    dim3 grid((unsigned)((pairs * segs + 7) / 8 * 8 * 2 * cols));
     if (rows == 256)
         hipLaunchKernelGGL((moe_tiles_kernel<MODE, 4>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, row_pair,
-                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, limit, alpha, act_kind, in_wts);
+                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts);
     else
         hipLaunchKernelGGL((moe_tiles_kernel<MODE, 2>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, row_pair,
-                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, limit, alpha, act_kind, in_wts);
+                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts);
 }
 
 }  // namespace sm

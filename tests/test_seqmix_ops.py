@@ -335,6 +335,45 @@ def test_moe_large_tiles_equal_small_ones(T, W, F, E, top, act):
     assert (y[1].float() - ref).norm() < 2 ** -7 * ref.norm()
 
 
+def _us(f, n=10):
+    for _ in range(3):
+        f()
+    best = float("inf")
+    for _ in range(5):
+        s, e = torch.cuda.Event(True), torch.cuda.Event(True)
+        s.record()
+        for _ in range(n):
+            f()
+        e.record()
+        torch.cuda.synchronize()
+        best = min(best, s.elapsed_time(e) / n * 1e3)
+    return best
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,W,F,E,top", [(100, 1104, 1512, 1, 1), (700, 72, 1160, 2, 2), (900, 520, 392, 5, 2)])
+def test_moe_tiles_cut_into_parts_equal_small_ones(T, W, F, E, top):
+    """Few row tiles: their column tiles go to the dies in parts (12 and 5 in parts of one, 10 in parts of 3, 3, 3
+    and 1, 4 in two).  Every output is written, bit for bit as in the 32-row form."""
+    g = gen(T + W)
+    h, idx = rnd(g, T, W).cuda().bfloat16(), torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int().cuda()
+    w_gu, w_down = rnd(g, E, 2 * F, W, s=W ** -0.5).cuda().bfloat16(), rnd(g, E, W, F, s=F ** -0.5).cuda().bfloat16()
+    y = [seq_ops.moe_experts(h, idx, torch.rand(T, top, generator=gen(5)).cuda(), w_gu, w_down, 1.2, form=f) for f in ("grouped", "tiles128")]
+    assert torch.equal(*y)
+
+
+@pytest.mark.gpu
+def test_moe_tiles_of_one_expert_use_the_whole_chip():
+    """One expert of 4096 x 11008 on 64 rows: about twice the time of the 32-row form (a first load per tile, 16-column-tile
+    products of 172 steps); with all its column tiles on one die it was five times."""
+    T, W, F = 64, 4096, 11008
+    h, idx, wts = torch.randn(T, W, device="cuda").bfloat16(), torch.zeros(T, 1, dtype=torch.int32, device="cuda"), torch.ones(T, 1, device="cuda")
+    w_gu, w_down = (torch.randn(1, *s, device="cuda").bfloat16() * 0.02 for s in ((2 * F, W), (W, F)))
+    tiled = seq_ops.tile_expert_weights(w_gu, 2), seq_ops.tile_expert_weights(w_down)
+    small, large = (_us(lambda: seq_ops.moe_experts(h, idx, wts, w_gu, w_down, 1.2, form=f, tiled=tiled)) for f in ("grouped", "tiles128"))
+    assert large <= 3.2 * small, (small, large)
+
+
 @pytest.mark.gpu
 def test_moe_combine_of_more_elements_than_a_grid_has_threads():
     """2.2 million tokens of 2044 channels (a width without 16-byte rows): 4.5e9 elements, more than 2^32 threads."""
