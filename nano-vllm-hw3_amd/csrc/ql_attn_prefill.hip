@@ -55,8 +55,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const unsigned sho
     const int seq = rt.b, hgrp = rt.g, hk = (hgrp * G) / kv_group;
     const int s0 = cu_seqlens[seq];
     const int L = cu_seqlens[seq + 1] - s0;
-    const int q0 = (blocks - 1 - rt.tile) * QROWS;                      // heaviest query blocks first
-    if (q0 >= L) return;
+    const int q0 = row_first(run, rt.tile, blocks, L, QROWS);           // heaviest query blocks first
+    if (q0 < 0 || q0 >= L) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = wave % G, sub = wave / G;

@@ -23,8 +23,8 @@ __global__ __launch_bounds__(256, SLIM ? 2 : 1) void latent_attn_tiles_kernel(co
     if (rt.b < 0) return;
     const int b = rt.b;
     const int q0 = qstart[b], rows = (qstart[b + 1] - q0) * H;
-    const int tile0 = (tiles - 1 - rt.tile) * 128;                             // heaviest tiles first
-    if (tile0 >= rows) return;
+    const int tile0 = row_first(run, rt.tile, tiles, rows, 128);               // heaviest tiles first
+    if (tile0 < 0 || tile0 >= rows) return;
     const int pos0 = seq_pos0[b];
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
