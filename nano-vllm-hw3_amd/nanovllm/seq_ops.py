@@ -248,9 +248,19 @@ def moe_route(h, router_w, top, groups=1, keep=1, score=ROUTE_SOFTMAX, correctio
     return (idx, wts) if gate is None else (idx, wts, gate)
 
 
-# rows per expert on average from which tiles of 128 and 256 rows beat tiles of 32 (us of the 32-row form / the other, 16 experts
-# of 2048 x 1536 and 32 of 1024 x 768: 16 rows 82 / 100 and 45 / 50, 32 rows 106 / 96 and 62 / 51)
-TILES128_MIN_ROWS_PER_EXPERT = 24
+def experts_form(pairs, E, W, F):
+    """The grouped form that ``pairs`` (token, choice) pairs over ``E`` experts of ``W`` x ``F`` take: "tiles128" or "grouped".
+
+    Tiles of 128 and 256 rows take the time of a tile whatever its rows; those of 32 rows are a wave each, and their time grows with
+    the waves per CU.  So the large ones win from 24 rows per expert on average and, as long as they leave CUs without a
+    tile, only from about 3.5 waves per CU of the small ones (the two products' mean by what they take: their k, and 256 for the
+    rest).  Microseconds, 32-row form / large tiles, weights not in a cache: 16 experts of 2048 x 1536 (4.3 waves at 24 rows) 16
+    rows 84 / 103, 28 rows 108 / 102, 48 rows 130 / 103; 128 of 2048 x 768 (22 at 24) 16 rows 298 / 303, 24 rows 349 / 306; 8 of 1024
+    x 768 (2.1 at 63, 3.8 at 127) 48 rows 37 / 55, 127 rows 54 / 57; 8 of 1024 x 1536 (2.4 at 48, 4.2 at 96) 48 rows 53 / 71, 96
+    rows 67 / 71; 4 of 2048 x 4096 (2.3 at 40, 4.0 at 80) 40 rows 104 / 137, 80 rows 121 / 137, 127 rows 177 / 138."""
+    mean = ((W + 256) * F + (F + 256) * W) / (W + F + 512)
+    waves_per_cu = (pairs / 32 + E / 2) * mean / 32 / 256
+    return "tiles128" if pairs >= 24 * E and waves_per_cu >= 3.5 else "grouped"
 
 
 def tile_expert_weights(w, parts=1):
@@ -293,7 +303,7 @@ def moe_experts(h, idx, wts, w_gu, w_down, limit, alpha=1.702, shared=None, form
     lib, code = SM.load(), SM.dtype_code(h.dtype)
     can_group = h.dtype == torch.bfloat16 and W % 8 == 0 and F % 8 == 0
     if form is None:
-        form = "pairs" if not can_group else ("tiles128" if T * top >= TILES128_MIN_ROWS_PER_EXPERT * E else "grouped")
+        form = experts_form(T * top, E, W, F) if can_group else "pairs"
     if form in ("grouped", "tiles128"):
         assert can_group
         rows = 32 if form == "grouped" else 128

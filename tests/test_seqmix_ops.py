@@ -374,6 +374,28 @@ def test_moe_tiles_of_one_expert_use_the_whole_chip():
     assert large <= 3.2 * small, (small, large)
 
 
+@pytest.mark.parametrize("W,F,E,rows,form", [(2048, 1536, 16, 16, "grouped"), (2048, 1536, 16, 24, "tiles128"), (2048, 1536, 16, 2048, "tiles128"),
+                                             (1024, 768, 8, 48, "grouped"), (1024, 768, 8, 192, "tiles128"), (2048, 768, 128, 24, "tiles128"),
+                                             (2048, 4096, 4, 40, "grouped"), (4096, 11008, 1, 24, "grouped"), (1024, 64, 64, 96, "tiles128")])
+def test_moe_form_by_rows_and_waves(W, F, E, rows, form):
+    assert seq_ops.experts_form(rows * E, E, W, F) == form
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W,F,E,top,rows", [(1024, 768, 8, 2, 48), (1024, 1536, 8, 2, 32), (2048, 4096, 4, 1, 40), (2048, 1536, 16, 4, 48)])
+def test_moe_takes_the_faster_grouped_form(W, F, E, top, rows):
+    """Few experts and few rows, where tiles of 128 rows leave most of the chip idle (they took 1.35 to 1.7 times as long), and more of
+    both: no more than a tenth and 2 us above the faster form."""
+    T = rows * E // top
+    g = gen(W + F)
+    h = torch.randn(T, W, device="cuda").bfloat16()
+    idx, wts = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int().cuda(), torch.rand(T, top, device="cuda")
+    w_gu, w_down = (torch.randn(E, *s, device="cuda").bfloat16() * 0.02 for s in ((2 * F, W), (W, F)))
+    tiled = seq_ops.tile_expert_weights(w_gu, 2), seq_ops.tile_expert_weights(w_down)
+    us = {f: _us(lambda: seq_ops.moe_experts(h, idx, wts, w_gu, w_down, 1.2, form=f, tiled=tiled)) for f in (None, "grouped", "tiles128")}
+    assert us[None] <= 1.1 * min(us["grouped"], us["tiles128"]) + 2, us
+
+
 @pytest.mark.gpu
 def test_moe_combine_of_more_elements_than_a_grid_has_threads():
     """2.2 million tokens of 2044 channels (a width without 16-byte rows): 4.5e9 elements, more than 2^32 threads."""
