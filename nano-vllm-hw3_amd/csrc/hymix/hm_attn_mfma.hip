@@ -25,7 +25,8 @@ __device__ __forceinline__ float mode_pre(float scale, float softcap, const floa
     return MODE == kSigmoid && head_bias ? head_bias[head] * 1.4426950408889634f : 0.f;
 }
 
-// SLIM: head sizes of exactly 32 NBK and 32 NBV channels, in the loop whose tiles go straight to LDS (kv_slim_loop)
+// SLIM: head sizes of exactly 32 NBK and 32 NBV channels and caches on 16 bytes, in the loop whose tiles go straight to LDS
+// (kv_slim_loop)
 template <int NBK, int NBV, int MODE, bool SLIM>
 __global__ __launch_bounds__(256, 2) void attn_tiles_kernel(const unsigned short* __restrict__ q, const unsigned short* __restrict__ kc,
                                                          const unsigned short* __restrict__ vc,
@@ -255,7 +256,8 @@ extern "C" int hm_attn_tiles(const void* q, const void* k_cache, const void* v_c
     dim3 grid(rg.x, rg.y, rg.z), block(256);
     hipStream_t s = as_stream(stream);
     const int nbk = padded_nb(D), nbv = padded_nb(V);
-    const bool slim = D == 32 * nbk && V == 32 * nbv;
+    const bool slim = D == 32 * nbk && V == 32 * nbv &&
+                      ((uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)kp_cache | (uintptr_t)vp_cache) % 16 == 0;
     const OutArgs out = {o_stride, (const unsigned short*)gate, gate_stride, out_scale};
 #define HM_TILES(K_, V_, S_) do { if (slim) HM_TILES_(K_, V_, S_, true); else HM_TILES_(K_, V_, S_, false); } while (0)
 #define HM_TILES_(K_, V_, S_, SLIM_)                                                                                         \

@@ -34,7 +34,8 @@ __device__ __forceinline__ int kv_off(int row, int ch) {
     return 256 * row + 16 * (ch ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
-template <int G>
+// DMA: keys and values on 16 bytes, loaded straight to LDS; rows off 16 bytes go through registers
+template <int G, bool DMA>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const unsigned short* __restrict__ q,
                                                               const unsigned short* __restrict__ k,
                                                               const unsigned short* __restrict__ v,
@@ -76,6 +77,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const unsigned sho
     }
 
     // a tile: eight pieces of 1 KB (four rows) per tensor, two per wave; lane l brings the chunk that belongs at 16 l
+    typedef i32x4 anywhere __attribute__((aligned(2)));
     typedef __attribute__((address_space(1))) const void gvoid;
     typedef __attribute__((address_space(3))) void lvoid;
     const unsigned short *ks0 = k + ((size_t)s0 * Hkv + hk) * 128, *vs0 = v + ((size_t)s0 * Hkv + hk) * 128;
@@ -85,8 +87,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const unsigned sho
             const int i = wave + 4 * j, row = 4 * i + (lane >> 4);
             const int ch = (lane & 15) ^ (((row & 3) << 2) | ((row >> 2) & 3));
             const size_t off = (size_t)min(kt0 + row, L - 1) * Hkv * 128 + 8 * ch;
-            __builtin_amdgcn_global_load_lds((gvoid*)(ks0 + off), (lvoid*)(buf + 1024 * i), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((gvoid*)(vs0 + off), (lvoid*)(buf + V_AT + 1024 * i), 16, 0, 0);
+            if constexpr (DMA) {
+                __builtin_amdgcn_global_load_lds((gvoid*)(ks0 + off), (lvoid*)(buf + 1024 * i), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds((gvoid*)(vs0 + off), (lvoid*)(buf + V_AT + 1024 * i), 16, 0, 0);
+            } else {
+                *(i32x4*)(buf + 1024 * i + 16 * lane) = *(const anywhere*)(ks0 + off);
+                *(i32x4*)(buf + V_AT + 1024 * i + 16 * lane) = *(const anywhere*)(vs0 + off);
+            }
         }
     };
     auto landed = [&]() {
@@ -221,11 +228,14 @@ extern "C" int ql_attn_prefill(const void* q, const void* k, const void* v, cons
     dim3 grid(rg.x, rg.y, rg.z), block(256);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
-#define QL_PF(G_)                                                                                              \
-    hipLaunchKernelGGL(attn_prefill_kernel<G_>, grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k, \
+    const bool dma = ((uintptr_t)k | (uintptr_t)v) % 16 == 0;
+#define QL_PF(G_) do { if (dma) QL_PF_(G_, true); else QL_PF_(G_, false); } while (0)
+#define QL_PF_(G_, DMA_)                                                                                       \
+    hipLaunchKernelGGL((attn_prefill_kernel<G_, DMA_>), grid, block, 0, s, (const unsigned short*)q, (const unsigned short*)k, \
                        (const unsigned short*)v, cu_seqlens, (unsigned short*)out, c, Hq, Hkv, kv_group, blocks, num_seqs, rg.run)
     if (G == 1) QL_PF(1); else if (G == 2) QL_PF(2); else QL_PF(4);
 #undef QL_PF
+#undef QL_PF_
     QL_CHECK_LAUNCH("ql_attn_prefill");
     return QL_OK;
 }

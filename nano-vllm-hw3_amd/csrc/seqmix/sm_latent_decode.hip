@@ -9,7 +9,7 @@ namespace sm {
 // floats per (sequence, split, head) in the workspace: scaled maximum, sum, RP outputs
 __host__ __device__ constexpr int part_stride(int nb) { return 32 * nb + 2; }
 
-// SLIM: rows of exactly 32 NB columns, in the loop of 32-key tiles (latent_slim_loop), which goes straight to LDS.  A split is a few
+// SLIM: rows of exactly 32 NB columns on 16 bytes, in the loop of 32-key tiles (latent_slim_loop), which goes straight to LDS.  A split is a few
 // tiles behind the latency of its first loads, so what counts is how many workgroups run beside each other; the other loop, with a
 // tile in registers on its way, spills in one wave of 256 columns.  Microseconds with the merge, other loop / this one, rows of
 // 192 + 64: 64 sequences of about 1000 keys 28 / 22 (16 heads), 42 / 35 (64 heads), 8 sequences 21 / 18, 256 of about 450 41 / 31, 16 of
@@ -67,7 +67,8 @@ __global__ __launch_bounds__(64 * WAVES, SLIM && WAVES > 1 ? 2 : 1) void latent_
 __global__ __launch_bounds__(256) void latent_decode_merge_kernel(const float* __restrict__ ws, unsigned short* __restrict__ o, int H,
                                                                   int R, int splits, int stride, const float* __restrict__ sink) {
     __shared__ float2 part[4][64];
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2), aligned(2)));      // (workspace and output as the caller has them)
+    typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
     const size_t row = blockIdx.x;                          // b * H + h
     const size_t b = row / H, h = row % H;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -76,12 +77,12 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(const float* _
     // (an empty split has sum 0 and outputs that nobody wrote: it counts for nothing)
     float M = -INFINITY, L = 0.f;
     for (int s = lane; s < splits; s += 64) {
-        const float2 ml = *(const float2*)(first + s * step);
+        const f32x2 ml = *(const f32x2*)(first + s * step);
         if (ml.y > 0.f) M = fmaxf(M, ml.x);
     }
     M = wave_max(M);
     for (int s = lane; s < splits; s += 64) {
-        const float2 ml = *(const float2*)(first + s * step);
+        const f32x2 ml = *(const f32x2*)(first + s * step);
         if (ml.y > 0.f) L += __builtin_amdgcn_exp2f(ml.x - M) * ml.y;
     }
     L = wave_sum(L);
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(const float* _
 #pragma unroll 4
         for (int s = wave; s < splits; s += 4) {
             const float* p = first + s * step;
-            const float2 ml = *(const float2*)p, x = *(const float2*)(p + 2 + min(c, R - 2));
+            const f32x2 ml = *(const f32x2*)p, x = *(const f32x2*)(p + 2 + min(c, R - 2));
             const float f = __builtin_amdgcn_exp2f(ml.x - M);
             if (ml.y > 0.f) { acc.x += f * x.x; acc.y += f * x.y; }
         }
@@ -150,7 +151,7 @@ extern "C" int sm_latent_attn_decode(const void* q, const void* cache, const int
     dim3 grid((unsigned)splits, (unsigned)B);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
-#define SM_DEC(NB_, NBV_, W_) do { if (R == 32 * NB_) SM_DEC_(NB_, NBV_, W_, true); else SM_DEC_(NB_, NBV_, W_, false); } while (0)
+#define SM_DEC(NB_, NBV_, W_) do { if (R == 32 * NB_ && (uintptr_t)cache % 16 == 0) SM_DEC_(NB_, NBV_, W_, true); else SM_DEC_(NB_, NBV_, W_, false); } while (0)
 #define SM_DEC_(NB_, NBV_, W_, SLIM_)                                                                                      \
     hipLaunchKernelGGL((latent_attn_decode_kernel<NB_, NBV_, W_, SLIM_>), grid, dim3(64 * W_), 0, s, (const unsigned short*)q, \
                        (const unsigned short*)cache, block_tables, ctx, (float*)workspace, c, H, R, block_size, max_blocks, \

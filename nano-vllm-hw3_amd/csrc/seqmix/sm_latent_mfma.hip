@@ -6,7 +6,7 @@
 
 namespace sm {
 
-// SLIM: rows of exactly 32 NB columns, in the loop of 32-key tiles (latent_slim_loop)
+// SLIM: rows of exactly 32 NB columns on 16 bytes, in the loop of 32-key tiles (latent_slim_loop)
 template <int NB, int NBV, bool SLIM>
 __global__ __launch_bounds__(256, SLIM ? 2 : 1) void latent_attn_tiles_kernel(const unsigned short* __restrict__ q,
                                                                 const unsigned short* __restrict__ cache,
@@ -87,7 +87,7 @@ extern "C" int sm_latent_attn_tiles(const void* q, const void* cache, const int3
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
     const int nb = (R + 31) / 32, nbv = (RV + 31) / 32;
-#define SM_TILES(NB_, NBV_) do { if (R == 32 * NB_) SM_TILES_(NB_, NBV_, true); else SM_TILES_(NB_, NBV_, false); } while (0)
+#define SM_TILES(NB_, NBV_) do { if (R == 32 * NB_ && (uintptr_t)cache % 16 == 0) SM_TILES_(NB_, NBV_, true); else SM_TILES_(NB_, NBV_, false); } while (0)
 #define SM_TILES_(NB_, NBV_, SLIM_)                                                                                       \
     hipLaunchKernelGGL((latent_attn_tiles_kernel<NB_, NBV_, SLIM_>), grid, block, 0, s, (const unsigned short*)q,                 \
                        (const unsigned short*)cache, block_tables, qstart, seq_pos0, (unsigned short*)o, c, H, R, block_size, \

@@ -26,7 +26,7 @@ constexpr int kBigRows = 128;                 // tiles are one or two times as m
 // of tiles of 128 rows with one LDS buffer, two barriers per step and the weights loaded to registers by every wave.  What is
 // left: a first load and a last store per tile that no other workgroup of the CU covers, and a last round of tiles that does
 // not fill the chip.
-template <int MODE, int MB>
+template <int MODE, int MB, bool DMA>
 __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                            const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                            unsigned short* __restrict__ out, int top, int N, int K, int tiles, int nct, int cols, int segs,
@@ -70,14 +70,16 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
         const int nb = GATE_UP ? min(4 * ct + (blk & 3), nb32 - 1) + (blk >= 4 ? nb32 : 0) : min(8 * ct + blk, nb32 - 1);
         bblk[j] = w + (((size_t)e * (GATE_UP ? 2 : 1) * nb32 + nb) * ksteps) * 2048 + 8 * lane;
     }
+    typedef i32x4 anywhere __attribute__((aligned(2)));
     typedef __attribute__((address_space(1))) const void gvoid;
     typedef __attribute__((address_space(3))) void lvoid;
-    auto load_a = [&](unsigned char* buf, int ks, int i) {
-        __builtin_amdgcn_global_load_lds((gvoid*)(arow[i] + (size_t)ks * 64), (lvoid*)(buf + 1024 * (wave * NA + i)), 16, 0, 0);
+    auto bring = [&](const unsigned short* from, unsigned char* to) {
+        if constexpr (DMA) __builtin_amdgcn_global_load_lds((gvoid*)from, (lvoid*)to, 16, 0, 0);
+        else *(i32x4*)(to + 16 * lane) = *(const anywhere*)from;
     };
+    auto load_a = [&](unsigned char* buf, int ks, int i) { bring(arow[i] + (size_t)ks * 64, buf + 1024 * (wave * NA + i)); };
     auto load_b = [&](unsigned char* buf, int ks, int i) {
-        __builtin_amdgcn_global_load_lds((gvoid*)(bblk[i >> 2] + (size_t)ks * 2048 + 512 * (i & 3)),
-                                         (lvoid*)(buf + A_BYTES + 4096 * (2 * wave + (i >> 2)) + 1024 * (i & 3)), 16, 0, 0);
+        bring(bblk[i >> 2] + (size_t)ks * 2048 + 512 * (i & 3), buf + A_BYTES + 4096 * (2 * wave + (i >> 2)) + 1024 * (i & 3));
     };
     auto load_step = [&](unsigned char* buf, int ks) {
 #pragma unroll
@@ -167,7 +169,7 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             i32x4 v = {0, 0, 0, 0};
-            if (full * 64 + 8 * (chunk ^ (4 * (i & 1))) + 8 <= K) v = *(const i32x4*)(arow[i] + (size_t)full * 64);
+            if (full * 64 + 8 * (chunk ^ (4 * (i & 1))) + 8 <= K) v = *(const anywhere*)(arow[i] + (size_t)full * 64);
             *(i32x4*)(buf0 + 1024 * (wave * NA + i) + 16 * lane) = v;
         }
 #pragma unroll
@@ -226,6 +228,7 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
 // 1536, 32 of 1024 x 768: 96 rows per expert 99 / 120, 53 / 75; 128 rows 142 / 120, 78 / 76; 384 rows 229 / 189, 126 / 124;
 // 2048 rows 942 / 734, 634 / 514).
 static int tile_rows(int64_t T, int top, int E) { return T * top >= (int64_t)128 * E ? 256 : 128; }
+static int tile_count(int64_t T, int top, int E, int rows) { return (int)((T * top + rows - 1) / rows + E); }
 
 // Units of work that a launch makes at least, by cutting the column tiles of its pairs of row tiles into parts: a pair of row tiles is
 // one die's, so few of them left dies without any (us, 128-row tiles, weights not in a cache, whole pairs / parts: one expert of 4096 x
@@ -235,17 +238,16 @@ static int tile_rows(int64_t T, int top, int E) { return T * top >= (int64_t)128
 constexpr int kUnits = 16;
 
 template <int MODE>
-static void launch_tiles(int rows, const void* a, const void* w, const int32_t* row_pair, const int32_t* tile_expert, void* out, int top,
+static void launch_tiles(int rows, bool dma, const void* a, const void* w, const int32_t* row_pair, const int32_t* tile_expert, void* out, int top,
                          int tiles, int N, int K, float limit, float alpha, int act_kind, const float* in_wts, hipStream_t s) {
     const int nct = MODE == 1 ? (N + 127) / 128 : (N + 255) / 256, pairs = (tiles + 1) / 2;
     const int want = (kUnits + pairs - 1) / pairs, cols = (nct + want - 1) / want, segs = (nct + cols - 1) / cols;
     dim3 grid((unsigned)((pairs * segs + 7) / 8 * 8 * 2 * cols));
-    if (rows == 256)
-        hipLaunchKernelGGL((moe_tiles_kernel<MODE, 4>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, row_pair,
-                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts);
-    else
-        hipLaunchKernelGGL((moe_tiles_kernel<MODE, 2>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, row_pair,
-                           tile_expert, (unsigned short*)out, top, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts);
+#define SM_TILES(MB_, DMA_)                                                                                                             \
+    hipLaunchKernelGGL((moe_tiles_kernel<MODE, MB_, DMA_>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, \
+                       row_pair, tile_expert, (unsigned short*)out, top, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts)
+    if (!dma) SM_TILES(2, false); else if (rows == 256) SM_TILES(4, true); else SM_TILES(2, true);
+#undef SM_TILES
 }
 
 }  // namespace sm
@@ -256,7 +258,7 @@ using namespace sm;
 extern "C" int sm_moe_tiles128_count(int64_t T, int top, int E) {
     if (T <= 0 || top <= 0 || E <= 0) return 0;
     const int rows = tile_rows(T, top, E);
-    return (int)((T * top + rows - 1) / rows + E) * (rows / kBigRows);
+    return tile_count(T, top, E, rows) * (rows / kBigRows);
 }
 
 extern "C" int sm_moe_tiles128(const void* h, const int32_t* idx, const float* wts, const void* w_gu, const void* w_down,
@@ -272,16 +274,18 @@ extern "C" int sm_moe_tiles128(const void* h, const int32_t* idx, const float* w
         return SM_ESHAPE;
     }
     if (T == 0) return SM_OK;
-    const int rows = tile_rows(T, top, E), tiles = sm_moe_tiles128_count(T, top, E) / (rows / kBigRows);
+    // (operands off 16 bytes go through registers, in tiles of 128 rows, which need no more room)
+    const bool dma = ((uintptr_t)h | (uintptr_t)act | (uintptr_t)w_gu | (uintptr_t)w_down) % 16 == 0;
+    const int rows = dma ? tile_rows(T, top, E) : kBigRows, tiles = tile_count(T, top, E, rows);
     hipStream_t s = as_stream(stream);
     if (int rc = launch_moe_align(idx, T * top, E, rows, tiles, row_pair, tile_expert, pair_row, s)) return rc;
     const float* in_wts = weight_in ? wts : nullptr;
     if (act_is_gated(act_kind))
-        launch_tiles<1>(rows, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
+        launch_tiles<1>(rows, dma, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
     else
-        launch_tiles<2>(rows, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
+        launch_tiles<2>(rows, dma, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
     SM_CHECK_LAUNCH("sm_moe_tiles128 (gate/up)");
-    launch_tiles<0>(rows, act, w_down, row_pair, tile_expert, prod, top, tiles, W, F, 0.f, 0.f, 0, nullptr, s);
+    launch_tiles<0>(rows, dma, act, w_down, row_pair, tile_expert, prod, top, tiles, W, F, 0.f, 0.f, 0, nullptr, s);
     SM_CHECK_LAUNCH("sm_moe_tiles128 (down)");
     if (y == nullptr) return SM_OK;               // the caller sums a token's pairs itself
     return sm_moe_combine(prod, pair_row, weight_in ? nullptr : wts, shared, shared_scale, y, T, top, W, stream);
