@@ -60,13 +60,17 @@ __global__ __launch_bounds__(64 * WAVES, SLIM && WAVES > 1 ? 2 : 1) void latent_
             for (int e = 0; e < 4; ++e) part[2 + 32 * d + 8 * rq + 4 * hi + e] = oacc[d][4 * rq + e];
 }
 
-// A workgroup per (sequence, head), four waves: a wave adds up every fourth split, two columns per lane, and the waves' sums meet
-// in LDS.  The splits' maxima and sums are read a split per lane in front of the outputs.  (One wave walking the splits one
+// A workgroup per (sequence, head), one wave or four: of four each adds up every fourth split, two columns per lane, and the waves'
+// sums meet in LDS.  The splits' maxima and sums are read a split per lane in front of the outputs.  (One wave walking the splits one
 // after another, a column per lane, three dependent rounds of loads per split: 17 us for 64 sequences of 16 heads and up to
 // 11 splits, against 21 of the attention itself.)
-__global__ __launch_bounds__(256) void latent_decode_merge_kernel(const float* __restrict__ ws, unsigned short* __restrict__ o, int H,
-                                                                  int R, int splits, int stride, const float* __restrict__ sink) {
-    __shared__ float2 part[4][64];
+// One wave where four have nothing to share out, up to five splits, and where the rows fill the chip several times over, from 6400 (us of
+// the whole step with four / one): 256 sequences of about 450 keys, 64 heads of 32 columns, 4 splits 33.5 / 22.6; 512 of 300, 64 heads of
+// 192 + 64, 2 splits 82 / 52; 128 of 1000, 64 heads, 8 splits 14 % more with four; 16 heads of 100 sequences, 8 splits 13 % less.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void latent_decode_merge_kernel(const float* __restrict__ ws, unsigned short* __restrict__ o, int H,
+                                                                         int R, int splits, int stride, const float* __restrict__ sink) {
+    __shared__ float2 part[WAVES][64];
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2), aligned(2)));      // (workspace and output as the caller has them)
     typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
     const size_t row = blockIdx.x;                          // b * H + h
@@ -91,21 +95,23 @@ __global__ __launch_bounds__(256) void latent_decode_merge_kernel(const float* _
         const int c = c0 + 2 * lane;
         float2 acc = make_float2(0.f, 0.f);
 #pragma unroll 4
-        for (int s = wave; s < splits; s += 4) {
+        for (int s = wave; s < splits; s += WAVES) {
             const float* p = first + s * step;
             const f32x2 ml = *(const f32x2*)p, x = *(const f32x2*)(p + 2 + min(c, R - 2));
             const float f = __builtin_amdgcn_exp2f(ml.x - M);
             if (ml.y > 0.f) { acc.x += f * x.x; acc.y += f * x.y; }
         }
-        part[wave][lane] = acc;
-        __syncthreads();
+        if (WAVES > 1) {
+            part[wave][lane] = acc;
+            __syncthreads();
+        }
         if (wave == 0 && c < R) {
 #pragma unroll
-            for (int v = 1; v < 4; ++v) { acc.x += part[v][lane].x; acc.y += part[v][lane].y; }
+            for (int v = 1; v < WAVES; ++v) { acc.x += part[v][lane].x; acc.y += part[v][lane].y; }
             const u16x2 o2 = {__builtin_bit_cast(unsigned short, (bf16_t)(acc.x * inv)), __builtin_bit_cast(unsigned short, (bf16_t)(acc.y * inv))};
             *(u16x2*)(o + row * R + c) = o2;
         }
-        __syncthreads();
+        if (WAVES > 1) __syncthreads();
     }
 }
 
@@ -162,8 +168,11 @@ extern "C" int sm_latent_attn_decode(const void* q, const void* cache, const int
 #undef SM_DEC_
 #undef SM_DEC
     SM_CHECK_LAUNCH("sm_latent_attn_decode");
-    hipLaunchKernelGGL(latent_decode_merge_kernel, dim3((unsigned)(B * H)), dim3(256), 0, s, (const float*)workspace,
-                       (unsigned short*)o, H, RV, splits, part_stride(padded_nbv(R, RV)), sink);
+#define SM_MERGE(WAVES_)                                                                                                       \
+    hipLaunchKernelGGL(latent_decode_merge_kernel<WAVES_>, dim3((unsigned)(B * H)), dim3(64 * WAVES_), 0, s, (const float*)workspace, \
+                       (unsigned short*)o, H, RV, splits, part_stride(padded_nbv(R, RV)), sink)
+    if (splits <= 5 || B * H >= 6400) SM_MERGE(1); else SM_MERGE(4);
+#undef SM_MERGE
     SM_CHECK_LAUNCH("sm_latent_attn_decode (merge)");
     return SM_OK;
 }

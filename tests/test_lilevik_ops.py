@@ -271,6 +271,52 @@ def test_matrix_core_latent_decode_equals_portable(B, H, R, RV):
         near(a, b.double().cpu(), dt, bf16=2e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,R,RV", [(257, 3, 64, 64), (300, 22, 192, 128), (600, 2, 32, 32), (128, 50, 40, 36)])
+def test_latent_decode_merge_in_one_wave_equals_portable(B, H, R, RV):
+    """One to five splits, and more of them over many rows, contexts that leave splits empty (the bound as above)."""
+    g = gen(B + R)
+    dev, dt = "cuda", torch.bfloat16
+    lens = [1, 64, 65, 129, 300, 700]
+    ctx, blocks = batch([(lens[i % 6] - 1, 1) for i in range(B)], device=dev, seed=B)
+    cache = (torch.randn(blocks, 64, R, generator=g) * 0.7).to(dt).to(dev)
+    q = (torch.randn(B, H, R, generator=g) * 0.7).to(dt).to(dev)
+    sink = torch.randn(H, generator=g).to(dev)
+    for kw in (dict(), dict(sink=sink), dict(window=64, sink=sink)):
+        a = seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=RV, **kw)
+        b = seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=RV, force_rows=True, **kw)
+        near(a, b.double().cpu(), dt, bf16=2e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,R,keys,most", [(256, 64, 32, 450, 28.), (512, 64, 256, 300, 67.)])
+def test_latent_decode_of_many_sequences_is_not_held_up_by_the_merge(B, H, R, keys, most):
+    """Four and two splits of many rows: 22.5 and 52 us; with a merge of four waves per row, which have one split each or none, 33.5 and
+    82 us."""
+    g = gen(1)
+    ctx, blocks = batch([(keys - 1, 1)] * B, device="cuda", seed=2)
+    cache = torch.randn(blocks, 64, R, generator=g).bfloat16().cuda()
+    q = torch.randn(B, H, R, generator=g).bfloat16().cuda()
+
+    def step():
+        return seq_ops.latent_attention(q, cache, ctx, 0.2, value_cols=min(R, 192))
+    for _ in range(3):
+        step()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(10):
+            step()
+    best = float("inf")
+    for _ in range(8):
+        s, e = torch.cuda.Event(True), torch.cuda.Event(True)
+        s.record()
+        graph.replay()
+        e.record()
+        torch.cuda.synchronize()
+        best = min(best, s.elapsed_time(e) * 100)
+    assert best <= most, best
+
+
 # ------------------------------------------------------------------------------------------ latent attention with a query latent
 @pytest.mark.parametrize("device,dtype", CASES)
 @pytest.mark.parametrize("H,D,Rd,V,R,Q", [(3, 8, 8, 16, 24, 20), (1, 4, 2, 4, 8, 4), (2, 40, 24, 72, 136, 56), (4, 24, 8, 40, 112, 64),
