@@ -9,9 +9,10 @@ namespace sm {
 // floats per (sequence, split, head) in the workspace: scaled maximum, sum, RP outputs
 __host__ __device__ constexpr int part_stride(int nb) { return 32 * nb + 2; }
 
-// SLIM: rows of exactly 32 NB columns on 16 bytes, in the loop of 32-key tiles (latent_slim_loop), which goes straight to LDS.  A split is a few
-// tiles behind the latency of its first loads, so what counts is how many workgroups run beside each other; the other loop, with a
-// tile in registers on its way, spills in one wave of 256 columns.  Microseconds with the merge, other loop / this one, rows of
+// SLIM: rows of exactly 32 NB columns on 16 bytes, in the loop of 32-key tiles (latent_slim_loop), which goes straight to LDS.  A split is
+// a few tiles behind the latency of its first loads, so what counts is how many workgroups run beside each other; the other loop, with a
+// tile in registers on its way, spills in one wave of 256 columns.  Below 96 columns it has registers enough, and its tiles of 64 keys half
+// the steps (us, 32 heads of 64 columns, other loop / this one: 64 sequences of 1000 keys 13.6 / 14.2, 600 46 / 49).  Microseconds with the merge, other loop / this one, rows of
 // 192 + 64: 64 sequences of about 1000 keys 28 / 22 (16 heads), 42 / 35 (64 heads), 8 sequences 21 / 18, 256 of about 450 41 / 31, 16 of
 // 3500 with 128 heads 49 / 40.  256 registers, so that two waves share a SIMD, where a workgroup has two or four waves:
 // 35 against 42 at 64 heads; one wave alone holds more than that and would spill (30 against 22).
@@ -157,7 +158,7 @@ extern "C" int sm_latent_attn_decode(const void* q, const void* cache, const int
     dim3 grid((unsigned)splits, (unsigned)B);
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
-#define SM_DEC(NB_, NBV_, W_) do { if (R == 32 * NB_ && (uintptr_t)cache % 16 == 0) SM_DEC_(NB_, NBV_, W_, true); else SM_DEC_(NB_, NBV_, W_, false); } while (0)
+#define SM_DEC(NB_, NBV_, W_) do { if (R == 32 * NB_ && (uintptr_t)cache % 16 == 0) SM_DEC_(NB_, NBV_, W_, (NB_ >= 3)); else SM_DEC_(NB_, NBV_, W_, false); } while (0)
 #define SM_DEC_(NB_, NBV_, W_, SLIM_)                                                                                      \
     hipLaunchKernelGGL((latent_attn_decode_kernel<NB_, NBV_, W_, SLIM_>), grid, dim3(64 * W_), 0, s, (const unsigned short*)q, \
                        (const unsigned short*)cache, block_tables, ctx, (float*)workspace, c, H, R, block_size, max_blocks, \
