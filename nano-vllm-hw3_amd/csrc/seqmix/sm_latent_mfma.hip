@@ -87,7 +87,17 @@ extern "C" int sm_latent_attn_tiles(const void* q, const void* cache, const int3
     const float c = scale * 1.4426950408889634f;
     hipStream_t s = as_stream(stream);
     const int nb = (R + 31) / 32, nbv = (RV + 31) / 32;
-#define SM_TILES(NB_, NBV_) do { if (R == 32 * NB_ && (uintptr_t)cache % 16 == 0) SM_TILES_(NB_, NBV_, true); else SM_TILES_(NB_, NBV_, false); } while (0)
+    // Rows whose 256 columns are all values need more than the 256 registers of two waves per SIMD and spill: that pays only where two
+    // workgroups share a CU.  Where a CU has one, the other loop's steps of 64 keys are half as many (us, other loop / this one, 16
+    // heads: 6 prompts of 195 to 411 tokens 34 / 42, 1 x 2000 115 / 151, 8 x 300 30 / 38, 1 x 4096 (512 tiles) 243 / 304; 16 x 300
+    // (608 tiles) 56 / 45, 8 x 1000 150 / 126; 8 heads, 8 x 1000 (504 tiles) 82 / 95).
+    const bool shared_cus = tiles * B > 512;
+    const bool aligned = (uintptr_t)cache % 16 == 0;
+#define SM_TILES(NB_, NBV_)                                                                                             \
+    do {                                                                                                                \
+        if (R == 32 * NB_ && aligned && (NBV_ < 8 || shared_cus)) SM_TILES_(NB_, NBV_, true);                          \
+        else SM_TILES_(NB_, NBV_, false);                                                                               \
+    } while (0)
 #define SM_TILES_(NB_, NBV_, SLIM_)                                                                                       \
     hipLaunchKernelGGL((latent_attn_tiles_kernel<NB_, NBV_, SLIM_>), grid, block, 0, s, (const unsigned short*)q,                 \
                        (const unsigned short*)cache, block_tables, qstart, seq_pos0, (unsigned short*)o, c, H, R, block_size, \

@@ -272,6 +272,36 @@ def test_matrix_core_latent_decode_equals_portable(B, H, R, RV):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("lens,H", [([195, 411, 271, 205, 213, 295], 16), ([2000], 16), ([64] * 16, 16), ([300] * 32, 16)])
+def test_latent_prompts_of_whole_rows_take_the_faster_loop(lens, H):
+    """Rows of 256 columns that are all values, on few and on many row tiles.  The kernel's two loops are told apart by the alignment of
+    the cache (off 16 bytes: tiles in registers); on few tiles the aligned call takes that one too (the other took up to 1.3 times as
+    long), on many the other, and both agree."""
+    g = gen(len(lens))
+    ctx, blocks = batch([(0, n) for n in lens], device="cuda", seed=3)
+    buf = torch.randn(blocks * 64 * 256 + 8, generator=g).bfloat16().cuda()
+    off, cache = buf[4:-4].view(blocks, 64, 256), buf[4:-4].view(blocks, 64, 256).clone()
+    q = torch.randn(ctx.num_tokens, H, 256, generator=g).bfloat16().cuda()
+
+    def us(c):
+        for _ in range(5):
+            y = seq_ops.latent_attention(q, c, ctx, 0.06)
+        best = float("inf")
+        for _ in range(6):
+            s, e = torch.cuda.Event(True), torch.cuda.Event(True)
+            s.record()
+            for _ in range(20):
+                seq_ops.latent_attention(q, c, ctx, 0.06)
+            e.record()
+            torch.cuda.synchronize()
+            best = min(best, s.elapsed_time(e) * 50)
+        return best, y
+    (t, y), (t_off, y_off) = us(cache), us(off)
+    near(y, y_off.double().cpu(), torch.bfloat16, bf16=2e-2)
+    assert t <= 1.1 * t_off, (t, t_off)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,H,R,RV", [(257, 3, 64, 64), (300, 22, 192, 128), (600, 2, 32, 32), (128, 50, 40, 36)])
 def test_latent_decode_merge_in_one_wave_equals_portable(B, H, R, RV):
     """One to five splits, and more of them over many rows, contexts that leave splits empty (the bound as above)."""
