@@ -24,7 +24,9 @@ OUT_DIR = os.path.join(HERE, "nanovllm", "_lib")
 LIB = os.path.join(OUT_DIR, "libqlinear.so")
 SEQMIX_LIB = os.path.join(OUT_DIR, "libseqmix.so")
 HYMIX_LIB = os.path.join(OUT_DIR, "libhymix.so")
-# the packed-f32 VALU forms stay off (plain f32 code only): some of them have given wrong results on this hardware
+# The packed-f32 VALU forms stay off (plain f32 code only): some of them have given wrong results on this hardware.  Without them
+# products and sums that were a packed multiply and a packed add, in the norms and the rotation among others, become fused
+# multiply-adds: one rounding less, so their results differ from a build with the packed forms by up to a bf16 rounding.
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-fno-gpu-rdc", "-Xclang", "-target-feature", "-Xclang",
          "-packed-fp32-ops"]
 TARGETS = {

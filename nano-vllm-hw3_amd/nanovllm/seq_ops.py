@@ -281,7 +281,7 @@ def moe_experts(h, idx, wts, w_gu, w_down, limit, alpha=1.702, shared=None, form
     """y[t] = sum_k wts[t, k] * expert_{idx[t, k]}(h[t]) (+ shared[t]); w_gu [E, 2F, W] (gate rows then up rows),
     w_down [E, W, F]; an expert is a clamped GLU between its two products.  ``form``: "pairs" | "grouped" | "tiles128"
     forces one; by default float32 runs pair by pair and bf16 grouped by expert on the matrix cores, in tiles of 32 rows
-    for small groups (decode) and of 128 rows for large ones (prefill).  ``tiled`` = (tile_expert_weights(w_gu, 2),
+    for small groups (decode) and of 128 or 256 rows for large ones (prefill; ``experts_form``).  ``tiled`` = (tile_expert_weights(w_gu, 2),
     tile_expert_weights(w_down)), what the grouped forms read (made here when the caller does not keep them).
     ``act_kind`` = ACT_GELU / ACT_GELU_TANH: an expert is down(gelu(up h)) instead, w_gu is [E, F, W] (tiled in one part);
     ACT_SILU_GLU: the gated form g sigmoid(alpha g) u without the one and, with limit = inf and alpha = 1, silu(gate) * up;
