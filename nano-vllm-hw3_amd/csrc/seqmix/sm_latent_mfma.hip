@@ -92,10 +92,17 @@ extern "C" int sm_latent_attn_tiles(const void* q, const void* cache, const int3
     // heads: 6 prompts of 195 to 411 tokens 34 / 42, 1 x 2000 115 / 151, 8 x 300 30 / 38, 1 x 4096 (512 tiles) 243 / 304; 16 x 300
     // (608 tiles) 56 / 45, 8 x 1000 150 / 126; 8 heads, 8 x 1000 (504 tiles) 82 / 95).
     const bool shared_cus = tiles * B > 512;
+    // Rows of 32 to 96 columns with up to 64 values: the other loop has registers enough for the tile on its way, and without a window a
+    // row tile's chain of steps is what counts as long as all of them run beside each other (us, other / this one: 8 heads, rows of 32
+    // columns, 1 x 6000 97 / 106, 40 x 70 8.7 / 9.7; of 64, 1 x 2000 44 / 47, 2 x 1500 34 / 36; 16 heads, 8 x 300 12.0 / 11.9; of 64 + 32,
+    // 32 heads, 1 x 2000 54 / 58).  Up to 512 row tiles, 768 where a sequence has half as many as fit (of 64, 16 heads, 1 x 6000 135 /
+    // 141; of 64 + 32 152 / 164; short ones, 32 heads, 40 x 70 14.0 / 10.4); above, throughput counts (16 heads, 8 x 1100 42 / 36; 64
+    // heads, 1 x 2000 70 / 60), and with a window, whose few steps do not lie in the loads' way (1 x 2000, window 256 17 / 13).
+    const bool chain = window <= 0 && tiles * B <= (tiles >= 256 ? 768 : 512);
     const bool aligned = (uintptr_t)cache % 16 == 0;
 #define SM_TILES(NB_, NBV_)                                                                                             \
     do {                                                                                                                \
-        if (R == 32 * NB_ && aligned && (NBV_ < 8 || shared_cus)) SM_TILES_(NB_, NBV_, true);                          \
+        if (R == 32 * NB_ && aligned && (NBV_ < 8 || shared_cus) && !(NB_ <= 3 && NBV_ <= 2 && chain)) SM_TILES_(NB_, NBV_, true); \
         else SM_TILES_(NB_, NBV_, false);                                                                               \
     } while (0)
 #define SM_TILES_(NB_, NBV_, SLIM_)                                                                                       \
