@@ -22,8 +22,9 @@ constexpr int kBigRows = 128;                 // tiles are one or two times as m
 // unrolled by two, so that the compiler sees that a read of one does not wait for the loads into the other.)
 //
 // Bound by the matrix cores: 128 x 128 per wave needs half of what LDS delivers (smaller wave tiles need all of it).  32768
-// rows over 16 experts: gate and up of 2 x 1536 x 2048 in 449 us (0.92 PFLOP/s), down in 252 us (0.82), against 950 and 434 us
-// of tiles of 128 rows with one LDS buffer, two barriers per step and the weights loaded to registers by every wave.  What is
+// rows over 16 experts: gate and up of 2 x 1536 x 2048 in about 470 us (0.88 PFLOP/s; 449 with the gate's quotient by the hardware's reciprocal,
+// which is less exact), down in 252 us (0.82), against 950 and 434 us of tiles of 128 rows with one LDS buffer, two barriers
+// per step and the weights loaded to registers by every wave.  What is
 // left: a first load and a last store per tile that no other workgroup of the CU covers, and a last round of tiles that does
 // not fill the chip.
 template <int MODE, int MB, bool DMA>
