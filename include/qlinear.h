@@ -275,7 +275,9 @@ int ql_gemm_force_config(int mt, int wn, int wk, int cp, int split_k);
  * each workgroup taking one contiguous range, and tiles that several workgroups share are combined like split-K
  * tiles (ascending k order, bit-reproducible); it keeps every CU busy when the tile count does not fill whole
  * rounds of the chip (152 tiles of 128 x 256 for a Qwen3-4B gate/up projection at 256 rows).  ql_gemm_workspace_bytes / _max_bytes see the table, so set entries before sizing a
- * workspace.  ql_gemm_plan_query writes {mt, wn, wk, cp, split_k} of the plan a call would run to out[5]. */
+ * workspace.  ql_gemm_plan_query writes {mt, wn, wk, cp, split_k} of the plan a call would run to out[5];
+ * {mt, 8, 1, 8, 1} is the 32 mt x 256 tile of prefill-sized problems (operands on 16 bytes, groups of 128), which needs
+ * no workspace and gives way to a table entry or a forced configuration. */
 #define QL_PLAN_GROUP 1    /* per-group scales */
 #define QL_PLAN_SILU 2     /* ql_gemm_*_silu */
 #define QL_PLAN_ROPE 4     /* ql_gemm_*_rope */

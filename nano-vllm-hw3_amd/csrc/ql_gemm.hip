@@ -38,6 +38,7 @@ struct Plan {
     // stream-K schedule (sk_G > 0; `split` is then reported as -sk_G): workgroups, row tiles walked side by side,
     // k chunks per output tile, column / row tiles of the problem
     int sk_G = 0, sk_R = 1, sk_C = 0, sk_nb = 0, sk_mb = 0;
+    bool wide = false;                                       // tiles of 32 mt x 256 of ql_gemm_wide.h (reported as mt, 8, 1, 8)
 };
 
 // tiles built with the stream-K schedule (QL_TILE_LIST_SK*, ql_gemm_kernel.h)
@@ -94,7 +95,40 @@ static bool plan_lookup(int form, int64_t M, int64_t N, int64_t K, PlanEntry* ou
     return false;
 }
 
-static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = false, bool rope = false, bool w8a8 = false) {
+// Row fragments of the wide tile (ql_gemm_wide.h) a problem runs on, 0: one of the other tiles is faster or the form is not built.
+// Its kernels take whole steps of 256 bytes of an activation row, whole 32-column strips (whole gate/up pairs of them) and
+// groups of 64 or a multiple of 128 k.  Two of its workgroups share a CU, so a launch takes ceil(tiles / 256) times what a tile costs
+// beside another one, or what it costs alone (from four rounds on the rounds run into each other); the height with the least is
+// within 1 % of the best of them over 64..8192 rows of the Qwen3 0.6B, 4B and 8B shapes.  Costs: microseconds per 1000 k, measured there.
+// The line to the other tiles: 140 tiles of 64 rows, 200 with int8 groups, whose sums and widening keep the vector unit busy on
+// low tiles.  Above it the wide tile is faster in nearly all problems (weight-only per row 1.15 x at the median and 1.5 x at most, per
+// group 1.15 and 1.4, 8-bit activations 1.4 and 2.0; the worst 0.97, 0.91 and 0.98 x); below it most of the chip's CUs have no tile, and
+// slices of K or smaller tiles win.  Groups also go by the tile of 128 x 256, which costs 20.3 whatever shares its CU: 8192 x
+// 1024 outputs are one whole round of it.
+static int wide_rows(int64_t M, int64_t N, int64_t K, int group, bool fp8, bool silu, bool w8a8) {
+    static const double pair[3][5] = {{0, 0, 7.5, 11.1, 13.5}, {0, 0, 10.8, 13.4, 0}, {0, 0, 4.6, 6.8, 8.0}};
+    static const double alone[3][5] = {{0, 0, 9.2, 12.2, 15.1}, {0, 0, 13.7, 16.6, 0}, {0, 0, 6.7, 8.3, 10.2}};
+    if (K % (w8a8 ? 256 : 128) || N % (silu ? 64 : 32) || (group && group != 64 && group % 128)) return 0;
+    const int64_t cols = (N + 255) / 256;
+    if ((M + 63) / 64 * cols < (group && !fp8 ? 200 : 140)) return 0;
+    const int kind = w8a8 ? 2 : group ? 1 : 0;
+    auto rounds = [&](int mt) -> double {
+        const double n = (double)((M + 32 * mt - 1) / (32 * mt) * cols) / 256;
+        return n < 4 ? (double)(int64_t)(n + 255. / 256) : n + 0.5;
+    };
+    int best = 0;
+    double least = 0;
+    for (int mt = 2; mt <= (group ? 3 : 4); ++mt) {
+        const double n = rounds(mt), cost = n > 1 ? n * pair[kind][mt] : alone[kind][mt];
+        if (!best || cost < least) { best = mt; least = cost; }
+    }
+    if (group && (M + 127) / 128 * cols >= 256 && least > rounds(4) * 20.3) return 0;
+    return best;
+}
+
+// wide_group: the group size of a call that may run on the wide tile (0: no groups), -1: it may not
+static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = false, bool rope = false, bool w8a8 = false,
+                      int wide_group = -1, bool fp8 = false) {
     Plan pl;
     // Tile ladder, smallest to largest output tile.  On a 256-CU chip these GEMMs are bound by
     // instruction issue and L2->LDS traffic per workgroup, not by HBM or MFMA peak, so the measured
@@ -165,6 +199,12 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
     if (plan_lookup((group ? QL_PLAN_GROUP : 0) | (silu ? QL_PLAN_SILU : 0) | (rope ? QL_PLAN_ROPE : 0) | (w8a8 ? QL_PLAN_W8A8 : 0),
                     M, N, K, &te)) {
         mt = te.mt; wn = te.wn; wk = te.wk; cp = te.cp; t_split = te.split;
+    } else if (const int rows = wide_group >= 0 && f_mt == 0 && f_split == 0 ? wide_rows(M, N, K, wide_group, fp8, silu, w8a8) : 0) {
+        pl.wide = true;
+        pl.mt = rows; pl.wn = 8; pl.wk = 1; pl.cp = kWideCP; pl.split = 1; pl.k_per_split = (int)K;
+        const int64_t tiles = (M + 32 * rows - 1) / (32 * rows) * ((N + 255) / 256);
+        pl.grid = dim3((unsigned)((tiles + 7) / 8 * 8));
+        return pl;
     }
     if (f_mt > 0 && f_wn > 0 && f_wk > 0 && f_cp > 0 && tile_built(f_mt, f_wn, f_wk, f_cp, group) && !(silu && (f_wn & 1)) &&
         !(rope && !rope_tile_built(f_mt, f_wn, f_wk, f_cp))) {
@@ -291,6 +331,12 @@ static int check_common(const char* fn, int64_t M, int64_t N, int64_t K) {
 static int run(kern_t k, GemmParams& p, const Plan& pl, void* ws, size_t ws_bytes, hipStream_t s, const char* fn) {
     if (!k) { set_error("%s: tile (%d,%d,%d,%d) not built", fn, pl.mt, pl.wn, pl.wk, pl.cp); return QL_EINVAL; }
     p.k_per_split = pl.k_per_split;
+    if (pl.wide) {
+        p.ntile_n = (int)((p.N + 255) / 256);
+        hipLaunchKernelGGL(k, pl.grid, dim3(256), 0, s, p);
+        QL_CHECK_LAUNCH(fn);
+        return QL_OK;
+    }
     if (pl.sk_G > 0) {
         const size_t need = plan_workspace(pl);
         if (!ws || ws_bytes < need) {
@@ -522,7 +568,7 @@ int ql_gemm_plan_query(int form, int64_t M, int64_t N, int64_t K, int* out) {
     const bool group = (form & QL_PLAN_GROUP) != 0;
     const Plan pl = (form & QL_PLAN_PARTIAL) ? make_plan_partial(M, N, K, group)
                                              : make_plan(M, N, K, group, (form & QL_PLAN_SILU) != 0, (form & QL_PLAN_ROPE) != 0,
-                                                         (form & QL_PLAN_W8A8) != 0);
+                                                         (form & QL_PLAN_W8A8) != 0, group ? 128 : 0);
     out[0] = pl.mt; out[1] = pl.wn; out[2] = pl.wk; out[3] = pl.cp; out[4] = pl.split;
     return QL_OK;
 }
@@ -590,10 +636,14 @@ static int gemm_w8a16(const char* fn, bool silu, int wdtype, int granularity, co
     p.silu = silu ? 1 : 0;
     p.wtiled = tiled ? 1 : 0;
     if (rope) { p.rope_on = 1; p.rope = *rope; }
-    const Plan pl = make_plan(M, N, K, grp, silu, rope != nullptr);
+    // (the wide tile loads activations and stores results 16 bytes at a time)
+    const bool aligned = (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
+    const Plan pl = make_plan(M, N, K, grp, silu, rope != nullptr, false, aligned ? p.group : -1, wdtype == QL_FP8);
     kern_t k;
     const bool rp = rope != nullptr;
-    if (pl.sk_G > 0) {
+    if (pl.wide) {
+        k = wdtype == QL_INT8 ? pick_wide_bf16_i8(pl.mt, p.group, rp) : pick_wide_bf16_fp8(pl.mt, p.group, rp);
+    } else if (pl.sk_G > 0) {
         if (wdtype == QL_INT8) k = grp ? pick_sk_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_sk_bf16_i8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);
         else k = grp ? pick_sk_bf16_fp8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_sk_bf16_fp8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);
     } else if (wdtype == QL_INT8) k = grp ? pick_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_bf16_i8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);
@@ -629,9 +679,11 @@ static int gemm_w8a8(const char* fn, bool silu, int dtype, const void* qx, const
     if (rope) { p.rope_on = 1; p.rope = *rope; }
     p.rowmax_part = rowmax_part; p.nparts = nparts;
     p.rowmax_out = silu ? rowmax_out : nullptr; p.nparts_out = (int)(N / 64);
-    const Plan pl = make_plan(M, N, K, false, silu, rope != nullptr, true);
+    const bool aligned = (((uintptr_t)qx | (uintptr_t)y) & 15) == 0;
+    const Plan pl = make_plan(M, N, K, false, silu, rope != nullptr, true, aligned && !dynq && !p.rowmax_out ? 0 : -1);
     kern_t k;
-    if (dynq) k = dtype == QL_INT8 ? pick_i8_i8_dynq(pl.mt, pl.wn, pl.wk, pl.cp) : pick_fp8_fp8_dynq(pl.mt, pl.wn, pl.wk, pl.cp);
+    if (pl.wide) k = dtype == QL_INT8 ? pick_wide_i8_i8(pl.mt, rope != nullptr) : pick_wide_fp8_fp8(pl.mt, rope != nullptr);
+    else if (dynq) k = dtype == QL_INT8 ? pick_i8_i8_dynq(pl.mt, pl.wn, pl.wk, pl.cp) : pick_fp8_fp8_dynq(pl.mt, pl.wn, pl.wk, pl.cp);
     else k = dtype == QL_INT8 ? pick_i8_i8(pl.mt, pl.wn, pl.wk, pl.cp, rope != nullptr) : pick_fp8_fp8(pl.mt, pl.wn, pl.wk, pl.cp, rope != nullptr);
     return run(k, p, pl, workspace, workspace_bytes, as_stream(stream), fn);
 }
