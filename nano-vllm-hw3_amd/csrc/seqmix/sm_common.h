@@ -5,6 +5,8 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "../../../include/seqmix.h"
 
 namespace sm {
@@ -63,6 +65,26 @@ __host__ __device__ __forceinline__ bool act_is_gated(int act) {
 __device__ __forceinline__ float plain_act(float z, int act) {
     if (act == SM_ACT_RELU_SQ) { z = fmaxf(z, 0.f); return z * z; }
     return act == SM_ACT_GELU_TANH ? gelu_tanh(z) : gelu_erf(z);
+}
+
+// f(kind as a constant) for the kinds that a kernel's mode can meet (0: none, 1: the gated forms, 2: the plain ones), so that a loop over
+// outputs holds the code of one kind and no branches around it
+template <int MODE, typename F>
+__device__ __forceinline__ void with_act(int act, F f) {
+    auto is = [&](auto kind) {
+        if (act == decltype(kind)::value) f(kind);
+    };
+    if constexpr (MODE == 0) {
+        f(std::integral_constant<int, 0>{});
+    } else if constexpr (MODE == 1) {
+        is(std::integral_constant<int, SM_ACT_CLAMPED_GLU>{});
+        is(std::integral_constant<int, SM_ACT_SILU_GLU>{});
+        is(std::integral_constant<int, SM_ACT_GELU_TANH_GLU>{});
+    } else {
+        is(std::integral_constant<int, SM_ACT_GELU>{});
+        is(std::integral_constant<int, SM_ACT_GELU_TANH>{});
+        is(std::integral_constant<int, SM_ACT_RELU_SQ>{});
+    }
 }
 
 // the grouping of (token, choice) pairs by expert into tiles of `unit` rows (sm_moe_align.hip); SM_OK or an error code

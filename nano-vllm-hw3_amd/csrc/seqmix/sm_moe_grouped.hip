@@ -6,9 +6,9 @@
 // A row of the result depends only on its own inputs: which other pairs share its tile does not change it, so the
 // (arbitrary) order of pairs inside an expert's group leaves every value as it is.
 //
-// Operands go from global memory straight to the MFMA registers: both matrices are K-contiguous, a lane owns one row
-// and 32 consecutive k of a 64-k step (four 16-byte loads, four MFMA steps; the k order inside a step is free as
-// long as both operands agree).
+// Both matrices are K-contiguous and a lane multiplies 32 consecutive k of one row in a 64-k step (four MFMA steps; the k order
+// inside a step is free as long as both operands agree).  Weights go from global memory straight to the MFMA registers, in the
+// order that their layout gives them; activations go through registers and LDS.
 #include <algorithm>
 
 #include "sm_common.h"
@@ -34,8 +34,9 @@ __device__ __forceinline__ bf16x8 load8(const unsigned short* p, int k, int K) {
 // in_wts != NULL (modes 1, 2): pair p's products are scaled by in_wts[p] before the activation (a weight on the expert's input)
 //
 // A wave is a workgroup: sixteen tiles by 48 column blocks are three waves for every CU, where workgroups of four waves left a
-// quarter of the CUs without work (64 tokens, top 4 of 16 experts of 2048 x 1536: gate and up 76 -> 43 us, 4.6 TB/s of weights;
-// down 43 -> 37).
+// quarter of the CUs without work.  Bound by the weights, read once, and by what a short kernel takes to begin and end (64 tokens,
+// top 4 of 16 experts of 2048 x 1536: gate and up 44 us, 4.6 TB/s; down 23, 4.4).  Lanes that read their own rows of the activations from
+// global memory touched 64 cache lines with every load, and rows without a pair as many as the others: 46 and 37 us.
 template <int MODE>
 __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                           const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
@@ -47,14 +48,26 @@ __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* _
     if (e < 0) return;
     const int lane = threadIdx.x, l31 = lane & 31, hi = lane >> 5;
     const int n0 = blockIdx.y * 32;
-    const int row = tile * kRowsPerTile + l31;
-    const int pair = row_pair[row];
-    const unsigned short* ap = FROM_TOKENS ? a + (size_t)(pair < 0 ? 0 : pair / top) * K : a + (size_t)row * K;
+    // The tile's rows come 128 bytes at a time, eight lanes to a row, and go through LDS to the lanes that multiply them (chunk c
+    // of row r at place c ^ (r / 2 & 7)): a lane reading its own row would touch a cache line of its own with every load.  Rows
+    // without a pair repeat one that has a place in memory; nobody reads their sums.
+    __shared__ __attribute__((aligned(1024))) unsigned char rows[2][kRowsPerTile * 128];
+    __shared__ __attribute__((aligned(16))) int pairs[kRowsPerTile];
+    const int sub = lane >> 3, chunk = lane & 7;
+    const unsigned short* arow[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = tile * kRowsPerTile + 8 * j + sub, pair = row_pair[row];
+        if (chunk == 0) pairs[8 * j + sub] = pair;
+        arow[j] = (FROM_TOKENS ? a + (size_t)(pair < 0 ? 0 : pair / top) * K : a + (size_t)(pair < 0 ? tile * kRowsPerTile : row) * K) + 8 * chunk;
+    }
     // weights in the tiled layout of sm_moe_tile_weights: block (expert, 32-row block, 64-k step) = 4 KB, chunk s of
     // lane L at 16 (64 s + L): a wave's load is one contiguous KB
     const int nb32 = (N + 31) / 32, ksteps = (K + 63) / 64;
     const unsigned short* bp = w + (((size_t)e * (GATE_UP ? 2 : 1) * nb32 + n0 / 32) * ksteps) * 2048 + 8 * lane;
     const unsigned short* bp2 = bp + (size_t)nb32 * ksteps * 2048;      // the up blocks follow the gate blocks
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
     f32x16 acc = {0}, acc2 = {0};
     // A ring of 64-k steps in flight: with a handful of rows per expert (decode) a wave's few MFMAs per step hide nothing, so
     // the weight stream has to be kept busy by outstanding loads: three steps of gate and up (36 KB per wave), six of a single
@@ -65,17 +78,27 @@ __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* _
     auto request = [&](Stage& st, int step) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            st.a[s] = *(const bf16x8*)(ap + (size_t)step * 64 + 32 * hi + 8 * s);
+            st.a[s] = *(const bf16x8*)(arow[s] + (size_t)step * 64);
             st.b[s] = *(const bf16x8*)(bp + (size_t)step * 2048 + 512 * s);
             if (GATE_UP) st.b2[s] = *(const bf16x8*)(bp2 + (size_t)step * 2048 + 512 * s);
         }
     };
-    auto consume = [&](const Stage& st) {
+    const int put = sub * 128 + 16 * (chunk ^ (sub >> 1)), get = l31 * 128, swz = (l31 >> 1) & 7;
+    auto consume = [&](const Stage& st, unsigned char* lds) {
+        // (one wave, whose LDS accesses are carried out in their order: nothing to wait for but the order itself)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(bf16x8*)(lds + 1024 * j + (put ^ (64 * (j & 1)))) = st.a[j];
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        bf16x8 av[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) av[s] = *(const bf16x8*)(lds + get + 16 * ((4 * hi + s) ^ swz));
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(st.a[s], st.b[s], acc, 0, 0, 0);
-            if (GATE_UP) acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(st.a[s], st.b2[s], acc2, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s], st.b[s], acc, 0, 0, 0);
+            if (GATE_UP) acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s], st.b2[s], acc2, 0, 0, 0);
         }
+        asm volatile("" ::: "memory");
     };
     const int full = K / 64;
     if (full > 0) {
@@ -86,34 +109,42 @@ __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* _
         for (; step + RING <= full; step += RING)
 #pragma unroll
             for (int i = 0; i < RING; ++i) {
-                consume(st[i]);
+                consume(st[i], rows[i & 1]);
                 request(st[i], min(step + RING + i, full - 1));
             }
 #pragma unroll
         for (int i = 0; i < RING; ++i)
-            if (step + i < full) consume(st[i]);
+            if (step + i < full) consume(st[i], rows[i & 1]);
     }
     if (K % 64 != 0) {                                        // zeros past the end of a row (the weights end in zeros)
         Stage st;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            st.a[s] = load8(ap, full * 64 + 32 * hi + 8 * s, K);
+            st.a[s] = load8(arow[s] - 8 * chunk, full * 64 + 8 * chunk, K);
             st.b[s] = *(const bf16x8*)(bp + (size_t)full * 2048 + 512 * s);
             if (GATE_UP) st.b2[s] = *(const bf16x8*)(bp2 + (size_t)full * 2048 + 512 * s);
         }
-        consume(st);
+        consume(st, rows[0]);
     }
     if (n0 + l31 >= N) return;
+    int p[16];
+    float iw[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        const int orow = tile * kRowsPerTile + (r & 3) + 8 * (r >> 2) + 4 * hi;
-        const int p = row_pair[orow];
-        if (p < 0) continue;
-        const float iw = FROM_TOKENS && in_wts ? in_wts[p] : 1.f;
-        const float v = GATE_UP ? glu_bf16(acc[r] * iw, acc2[r] * iw, limit, alpha, act_kind)
-                                : (MODE == 2 ? plain_act((float)(bf16_t)(acc[r] * iw), act_kind) : acc[r]);
-        out[(size_t)orow * N + n0 + l31] = __builtin_bit_cast(unsigned short, (bf16_t)v);
+        p[r] = pairs[(r & 3) + 8 * (r >> 2) + 4 * hi];
+        iw[r] = FROM_TOKENS && in_wts && p[r] >= 0 ? in_wts[p[r]] : 1.f;
     }
+    with_act<MODE>(act_kind, [&](auto kind) {
+        constexpr int ACT = decltype(kind)::value;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            if (p[r] < 0) continue;
+            const int orow = tile * kRowsPerTile + (r & 3) + 8 * (r >> 2) + 4 * hi;
+            const float v = GATE_UP ? glu_bf16(acc[r] * iw[r], acc2[r] * iw[r], limit, alpha, ACT)
+                                    : (MODE == 2 ? plain_act((float)(bf16_t)(acc[r] * iw[r]), ACT) : acc[r]);
+            out[(size_t)orow * N + n0 + l31] = __builtin_bit_cast(unsigned short, (bf16_t)v);
+        }
+    });
 }
 
 // A token's pairs summed with their weights, in a fixed order, V channels per thread: 8 where rows and pointers allow 16-byte
