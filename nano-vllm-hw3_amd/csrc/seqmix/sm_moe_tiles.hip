@@ -21,16 +21,15 @@ constexpr int kBigRows = 128;                 // tiles are one or two times as m
 // fragments are read from LDS one 16-k product ahead, across the barrier too.  (The buffers are two arrays and the loop is
 // unrolled by two, so that the compiler sees that a read of one does not wait for the loads into the other.)
 //
-// Bound by the matrix cores: 128 x 128 per wave needs half of what LDS delivers (smaller wave tiles need all of it).  32768
-// rows over 16 experts: gate and up of 2 x 1536 x 2048 in about 470 us (0.88 PFLOP/s; 449 with the gate's quotient by the hardware's reciprocal,
-// which is less exact), down in 252 us (0.82), against 950 and 434 us of tiles of 128 rows with one LDS buffer, two barriers
-// per step and the weights loaded to registers by every wave.  What is
-// left: a first load and a last store per tile that no other workgroup of the CU covers, and a last round of tiles that does
-// not fill the chip.
+// Bound by the matrix cores and the power they may draw (with weights of zeros the same products take 10 % less): 128 x 128 per wave
+// needs half of what LDS delivers (smaller wave tiles need all of it).  32768 rows over 16 experts: gate and up of 2 x 1536 x 2048
+// in 435 us (0.95 PFLOP/s), down in 252 us (0.82).  A tile takes about 8 us beside its products: nothing covers its first loads and its
+// last stores.  Of 20 us that it was in gate and up, 4 were the pairs of its rows, fetched and divided one behind the other, and
+// 9 the activation's kind, asked for at every output.
 template <int MODE, int MB, bool DMA>
 __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                            const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
-                                                           unsigned short* __restrict__ out, int top, int N, int K, int tiles, int nct, int cols, int segs,
+                                                           unsigned short* __restrict__ out, int top, unsigned top_inv, int N, int K, int tiles, int nct, int cols, int segs,
                                                            float limit, float alpha, int act_kind, const float* __restrict__ in_wts) {
     constexpr bool GATE_UP = MODE == 1, FROM_TOKENS = MODE != 0;
     constexpr int ROWS = 64 * MB, A_BYTES = ROWS * 128, BUF = A_BYTES + 8 * 4096;
@@ -43,10 +42,16 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
     const int unit = turn * 8 + (blockIdx.x & 7), rows2 = unit / segs;
     const int tile = rows2 * 2 + (in_unit & 1), ct = (unit - rows2 * segs) * cols + (in_unit >> 1);
     if (tile >= tiles || ct >= nct) return;
-    const int e = tile_expert[tile];
-    if (e < 0) return;                                        // (uniform over the workgroup)
     const int lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // (the pairs of a lane's rows all at once, beside the expert: one behind the other they took longer than a tile's 12 first steps)
+    int pair[NA];
+    if (FROM_TOKENS) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) pair[i] = row_pair[tile * ROWS + 8 * (wave * NA + i) + (lane >> 3)];
+    }
+    const int e = tile_expert[tile];
+    if (e < 0) return;                                        // (uniform over the workgroup)
     const int wr = wave >> 1, wc = wave & 1;
     const int nb32 = (N + 31) / 32, ksteps = (K + 63) / 64;
 
@@ -56,9 +61,9 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
         const int row = tile * ROWS + 8 * (wave * NA + i) + (lane >> 3), ch = chunk ^ (4 * (i & 1));
-        if (FROM_TOKENS) {
-            const int p = row_pair[row];
-            arow[i] = a + (size_t)(p < 0 ? 0 : p / top) * K + 8 * ch;
+        if (FROM_TOKENS) {                                    // pair / top: the product with 1 / top is at most one too large
+            const unsigned p = (unsigned)max(pair[i], 0), q = top > 1 ? __umulhi(p, top_inv) : p;
+            arow[i] = a + (size_t)(q - (q * (unsigned)top > p ? 1u : 0u)) * K + 8 * ch;
         } else {
             arow[i] = a + (size_t)row * K + 8 * ch;
         }
@@ -206,23 +211,27 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_kernel(const unsigned short*
     }
     __syncthreads();
     constexpr int CH = GATE_UP ? 16 : 32;                     // finished chunks per row
+    // (the activation's kind is chosen once, not at every output)
+    auto finish = [&](auto kind) {
+        constexpr int ACT = decltype(kind)::value;
 #pragma unroll 4
-    for (int i = threadIdx.x; i < ROWS * CH; i += 256) {          // (rows without a pair too: nobody reads what they leave)
-        const int row = i / CH, c = i % CH, lrow = row & (32 * MB - 1);
-        const int col = (GATE_UP ? 128 : 256) * ct + 8 * c;
-        if (col >= N) continue;                               // (N % 8 == 0)
-        const unsigned char* src = (row >= 32 * MB ? buf1 : buf0) + lrow * 512;
-        bf16x8 x = *(const bf16x8*)(src + 16 * (c ^ (row & 31)));
-        if (GATE_UP) {
-            const bf16x8 u = *(const bf16x8*)(src + 16 * ((c + 16) ^ (row & 31)));
+        for (int i = threadIdx.x; i < ROWS * CH; i += 256) {      // (rows without a pair too: nobody reads what they leave)
+            const int row = i / CH, c = i % CH, lrow = row & (32 * MB - 1);
+            const int col = (GATE_UP ? 128 : 256) * ct + 8 * c;
+            const unsigned char* src = (row >= 32 * MB ? buf1 : buf0) + lrow * 512;
+            bf16x8 x = *(const bf16x8*)(src + 16 * (c ^ (row & 31)));
+            if (GATE_UP) {
+                const bf16x8 u = *(const bf16x8*)(src + 16 * ((c + 16) ^ (row & 31)));
 #pragma unroll
-            for (int r = 0; r < 8; ++r) x[r] = (bf16_t)gated_act((float)x[r], (float)u[r], limit, alpha, act_kind);
-        } else if (MODE == 2) {
+                for (int r = 0; r < 8; ++r) x[r] = (bf16_t)gated_act((float)x[r], (float)u[r], limit, alpha, ACT);
+            } else if (MODE == 2) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) x[r] = (bf16_t)plain_act((float)x[r], act_kind);
+                for (int r = 0; r < 8; ++r) x[r] = (bf16_t)plain_act((float)x[r], ACT);
+            }
+            if (col < N) *(bf16x8*)(out + ((size_t)tile * ROWS + row) * N + col) = x;      // (N % 8 == 0)
         }
-        *(bf16x8*)(out + ((size_t)tile * ROWS + row) * N + col) = x;
-    }
+    };
+    with_act<MODE>(act_kind, finish);
 }
 
 // Rows of a tile: 256 from 128 rows per expert on average, else 128 (us with 128 / 256 rows, two sizes: 16 experts of 2048 x
@@ -243,10 +252,11 @@ static void launch_tiles(int rows, bool dma, const void* a, const void* w, const
                          int tiles, int N, int K, float limit, float alpha, int act_kind, const float* in_wts, hipStream_t s) {
     const int nct = MODE == 1 ? (N + 127) / 128 : (N + 255) / 256, pairs = (tiles + 1) / 2;
     const int want = (kUnits + pairs - 1) / pairs, cols = (nct + want - 1) / want, segs = (nct + cols - 1) / cols;
+    const unsigned top_inv = top > 1 ? (unsigned)((((uint64_t)1 << 32) + top - 1) / top) : 0;
     dim3 grid((unsigned)((pairs * segs + 7) / 8 * 8 * 2 * cols));
 #define SM_TILES(MB_, DMA_)                                                                                                             \
     hipLaunchKernelGGL((moe_tiles_kernel<MODE, MB_, DMA_>), grid, dim3(256), 0, s, (const unsigned short*)a, (const unsigned short*)w, \
-                       row_pair, tile_expert, (unsigned short*)out, top, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts)
+                       row_pair, tile_expert, (unsigned short*)out, top, top_inv, N, K, tiles, nct, cols, segs, limit, alpha, act_kind, in_wts)
     if (!dma) SM_TILES(2, false); else if (rows == 256) SM_TILES(4, true); else SM_TILES(2, true);
 #undef SM_TILES
 }
