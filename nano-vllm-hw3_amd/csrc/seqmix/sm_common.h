@@ -89,7 +89,7 @@ __device__ __forceinline__ void with_act(int act, F f) {
 
 // the grouping of (token, choice) pairs by expert into tiles of `unit` rows (sm_moe_align.hip); SM_OK or an error code
 int launch_moe_align(const int32_t* idx, int64_t P, int E, int unit, int max_tiles, int32_t* row_pair, int32_t* tile_expert,
-                     int32_t* pair_row, hipStream_t s);
+                     int32_t* pair_row, int32_t* counts, hipStream_t s);
 
 static inline hipStream_t as_stream(void* s) { return (hipStream_t)s; }
 

@@ -23,92 +23,16 @@ __device__ __forceinline__ void fold_wave(float (&d)[M], int lane) {
     }
 }
 
-// kRouteTokens = tokens per workgroup: every router row read serves all of them
-template <typename T, int kRouteTokens>
-__global__ __launch_bounds__(256, kRouteTokens == 8 ? 3 : 4) void moe_route_kernel(const T* __restrict__ h, const float* __restrict__ router_w,
-                                                        int32_t* __restrict__ idx, float* __restrict__ wts, int64_t T_all, int W,
-                                                        int E, int top, int groups, int keep, int score,
-                                                        const float* __restrict__ correction, int group_top, int renorm,
-                                                        int staged, const float* __restrict__ bias,
-                                                        const float* __restrict__ gate_w, float* __restrict__ gate_out) {
-    // per token: E scores, `groups` group scores and, with gate_w, the gate's logit; then the staged rows
-    extern __shared__ float z_all[];
-    const int RS = E + groups + (gate_w ? 1 : 0), rows = E + (gate_w ? 1 : 0);     // the gate's row follows the experts'
-    const int64_t t0 = (int64_t)blockIdx.x * kRouteTokens;
-    const int nt = (int)min((int64_t)kRouteTokens, T_all - t0);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (staged) {
-        // the workgroup's token rows (one contiguous piece of h) go to LDS once; every expert's row is then read once per
-        // workgroup in 16-byte pieces and meets all the tokens there
-        T* h_lds = (T*)(z_all + (kRouteTokens * RS + 3) / 4 * 4);
-        const T* src = h + (size_t)t0 * W;
-        struct alignas(sizeof(T) * 4) Pack4 { T v[4]; };
-        for (int i0 = threadIdx.x * 4; i0 < nt * W; i0 += 8 * 1024) {     // W % 4 == 0; eight pieces of a thread in flight
-            Pack4 piece[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) piece[j] = *(const Pack4*)(src + min(i0 + 1024 * j, nt * W - 4));
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (i0 + 1024 * j < nt * W) *(Pack4*)(h_lds + i0 + 1024 * j) = piece[j];
-        }
-        __syncthreads();
-        // four experts at a time: a token's piece read from LDS and widened meets four router rows (one row at a time, the
-        // LDS reads and the 6 lane moves of every single sum were most of the kernel: 8192 tokens of 2048 channels, 16
-        // experts: 53 -> 29 us; 64 tokens 16 -> 9)
-        for (int e0 = 4 * wave; e0 < rows; e0 += 16) {
-            const float* wr[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = min(e0 + j, rows - 1);
-                wr[j] = e < E ? router_w + (size_t)e * W : gate_w;
-            }
-            constexpr int N = 4 * kRouteTokens;
-            float d[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) d[i] = 0.f;
-            float4 nxt[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) nxt[j] = *(const float4*)(wr[j] + min(lane * 4, W - 4));
-#pragma unroll 1
-            for (int c = lane * 4; c < W; c += 256) {
-                float4 wv[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    wv[j] = nxt[j];
-                    nxt[j] = *(const float4*)(wr[j] + min(c + 256, W - 4));
-                }
-#pragma unroll
-                for (int i = 0; i < kRouteTokens; ++i) {           // (rows past nt: whatever LDS holds, nobody reads their sums)
-                    const Pack4 hv = *(const Pack4*)(h_lds + (size_t)i * W + c);
-                    const float x0 = to_f(hv.v[0]), x1 = to_f(hv.v[1]), x2 = to_f(hv.v[2]), x3 = to_f(hv.v[3]);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) d[4 * i + j] += x0 * wv[j].x + x1 * wv[j].y + x2 * wv[j].z + x3 * wv[j].w;
-                }
-            }
-            fold_wave<N, 32>(d, lane);
-            const int v = lane / (64 / N), e = e0 + v % 4;
-            if (lane % (64 / N) == 0 && e < rows) z_all[v / 4 * RS + (e < E ? e : RS - 1)] = d[0];
-        }
-    } else {
-        for (int e = wave; e < rows; e += 4) {
-            const float* wr = e < E ? router_w + (size_t)e * W : gate_w;
-            float d[kRouteTokens];
-            for (int i = 0; i < kRouteTokens; ++i) d[i] = 0.f;
-            for (int c = lane; c < W; c += 64) {
-                const float wv = wr[c];
-                for (int i = 0; i < kRouteTokens; ++i)
-                    if (i < nt) d[i] += to_f(h[(size_t)(t0 + i) * W + c]) * wv;
-            }
-            for (int i = 0; i < kRouteTokens; ++i) {
-                const float sum = wave_sum(d[i]);
-                if (lane == 0) z_all[i * RS + (e < E ? e : RS - 1)] = sum;
-            }
-        }
-    }
-    __syncthreads();
+// From the logits to the choice: tokens t0 .. t0 + nt - 1, token i's E logits at z_all + i RS, then room for its group scores, then (with
+// gate_w) the gate's logit.  Called by all `waves` waves of a workgroup behind a barrier.
+__device__ __forceinline__ void finish_routes(float* z_all, int RS, int64_t t0, int nt, int wave, int waves, int32_t* __restrict__ idx,
+                                              float* __restrict__ wts, int E, int top, int groups, int keep, int score,
+                                              const float* __restrict__ correction, int group_top, int renorm,
+                                              const float* __restrict__ bias, const float* __restrict__ gate_w, float* __restrict__ gate_out) {
+    const int lane = threadIdx.x & 63;
     if (groups <= 1 && E <= 256) {
         // no groups: a wave finishes a token, lane l holding the scores of the experts l, l + 64, ...
-        for (int i = wave; i < nt; i += 4) {
+        for (int i = wave; i < nt; i += waves) {
             const int64_t t = t0 + i;
             const float* z = z_all + i * RS;
             if (gate_w != nullptr && lane == 0) gate_out[t] = 1.f / (1.f + expf(-z[RS - 1]));
@@ -271,6 +195,167 @@ __global__ __launch_bounds__(256, kRouteTokens == 8 ? 3 : 4) void moe_route_kern
     leave(tot);
 }
 
+// kRouteTokens = tokens per workgroup: every router row read serves all of them
+template <typename T, int kRouteTokens>
+__global__ __launch_bounds__(256, kRouteTokens == 8 ? 3 : 4) void moe_route_kernel(const T* __restrict__ h, const float* __restrict__ router_w,
+                                                        int32_t* __restrict__ idx, float* __restrict__ wts, int64_t T_all, int W,
+                                                        int E, int top, int groups, int keep, int score,
+                                                        const float* __restrict__ correction, int group_top, int renorm,
+                                                        int staged, const float* __restrict__ bias,
+                                                        const float* __restrict__ gate_w, float* __restrict__ gate_out) {
+    // per token: E scores, `groups` group scores and, with gate_w, the gate's logit; then the staged rows
+    extern __shared__ float z_all[];
+    const int RS = E + groups + (gate_w ? 1 : 0), rows = E + (gate_w ? 1 : 0);     // the gate's row follows the experts'
+    const int64_t t0 = (int64_t)blockIdx.x * kRouteTokens;
+    const int nt = (int)min((int64_t)kRouteTokens, T_all - t0);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (staged) {
+        // the workgroup's token rows (one contiguous piece of h) go to LDS once; every expert's row is then read once per
+        // workgroup in 16-byte pieces and meets all the tokens there
+        T* h_lds = (T*)(z_all + (kRouteTokens * RS + 3) / 4 * 4);
+        const T* src = h + (size_t)t0 * W;
+        struct alignas(sizeof(T) * 4) Pack4 { T v[4]; };
+        for (int i0 = threadIdx.x * 4; i0 < nt * W; i0 += 8 * 1024) {     // W % 4 == 0; eight pieces of a thread in flight
+            Pack4 piece[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) piece[j] = *(const Pack4*)(src + min(i0 + 1024 * j, nt * W - 4));
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (i0 + 1024 * j < nt * W) *(Pack4*)(h_lds + i0 + 1024 * j) = piece[j];
+        }
+        __syncthreads();
+        // four experts at a time: a token's piece read from LDS and widened meets four router rows (one row at a time, the
+        // LDS reads and the 6 lane moves of every single sum were most of the kernel: 8192 tokens of 2048 channels, 16
+        // experts: 53 -> 29 us; 64 tokens 16 -> 9)
+        for (int e0 = 4 * wave; e0 < rows; e0 += 16) {
+            const float* wr[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int e = min(e0 + j, rows - 1);
+                wr[j] = e < E ? router_w + (size_t)e * W : gate_w;
+            }
+            constexpr int N = 4 * kRouteTokens;
+            float d[N];
+#pragma unroll
+            for (int i = 0; i < N; ++i) d[i] = 0.f;
+            float4 nxt[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) nxt[j] = *(const float4*)(wr[j] + min(lane * 4, W - 4));
+#pragma unroll 1
+            for (int c = lane * 4; c < W; c += 256) {
+                float4 wv[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    wv[j] = nxt[j];
+                    nxt[j] = *(const float4*)(wr[j] + min(c + 256, W - 4));
+                }
+#pragma unroll
+                for (int i = 0; i < kRouteTokens; ++i) {           // (rows past nt: whatever LDS holds, nobody reads their sums)
+                    const Pack4 hv = *(const Pack4*)(h_lds + (size_t)i * W + c);
+                    const float x0 = to_f(hv.v[0]), x1 = to_f(hv.v[1]), x2 = to_f(hv.v[2]), x3 = to_f(hv.v[3]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) d[4 * i + j] += x0 * wv[j].x + x1 * wv[j].y + x2 * wv[j].z + x3 * wv[j].w;
+                }
+            }
+            fold_wave<N, 32>(d, lane);
+            const int v = lane / (64 / N), e = e0 + v % 4;
+            if (lane % (64 / N) == 0 && e < rows) z_all[v / 4 * RS + (e < E ? e : RS - 1)] = d[0];
+        }
+    } else {
+        for (int e = wave; e < rows; e += 4) {
+            const float* wr = e < E ? router_w + (size_t)e * W : gate_w;
+            float d[kRouteTokens];
+            for (int i = 0; i < kRouteTokens; ++i) d[i] = 0.f;
+            for (int c = lane; c < W; c += 64) {
+                const float wv = wr[c];
+                for (int i = 0; i < kRouteTokens; ++i)
+                    if (i < nt) d[i] += to_f(h[(size_t)(t0 + i) * W + c]) * wv;
+            }
+            for (int i = 0; i < kRouteTokens; ++i) {
+                const float sum = wave_sum(d[i]);
+                if (lane == 0) z_all[i * RS + (e < E ? e : RS - 1)] = sum;
+            }
+        }
+    }
+    __syncthreads();
+    finish_routes(z_all, RS, t0, nt, wave, 4, idx, wts, E, top, groups, keep, score, correction, group_top, renorm, bias, gate_w, gate_out);
+}
+
+// The logits on the matrix cores, in float32: sixteen tokens by 16 NT rows of the router (the gate's row follows the experts') per
+// workgroup, whose waves share the width among them, 32 channels a wave in turn; their sums meet in LDS and are added in wave order.  A lane
+// holds eight consecutive channels of one token and of one router row per 32 channels (the instruction's four k are channels 8 apart,
+// which both operands agree on), so everything comes in 16-byte loads, U steps of them at once, and a router row is read once
+// for sixteen tokens.  For many tokens: it is then bound by the reads of h, where staging the tokens in LDS and multiplying on the vector
+// unit spent its time in LDS reads and widening (16 experts, us: 8192 tokens of 2048 channels 28 -> 19, 4096 21 -> 13; 64 experts,
+// 8192 tokens of 4096 channels, which did not fit LDS, 2255 -> 88).  Below 2048 tokens a workgroup per token is as fast or faster (64
+// tokens 9.5 and 12.5: sixteen waves in few workgroups begin and end later), from 65 rows on the products of sixteen tokens are.
+template <typename T, int NT>
+__global__ __launch_bounds__(1024, NT == 1 && sizeof(T) == 2 ? 8 : 4) void moe_route_mfma_kernel(const T* __restrict__ h, const float* __restrict__ router_w,
+                                                              int32_t* __restrict__ idx, float* __restrict__ wts, int64_t T_all, int W,
+                                                              int E, int top, int groups, int keep, int score,
+                                                              const float* __restrict__ correction, int group_top, int renorm,
+                                                              const float* __restrict__ bias, const float* __restrict__ gate_w,
+                                                              float* __restrict__ gate_out) {
+    constexpr int WAVES = 16, U = NT <= 2 ? 4 : 2;
+    __shared__ float part[WAVES][NT][4][64];
+    __shared__ float z_all[16 * (32 * NT + 1)];                 // (as many groups as experts at most)
+    const int RS = E + groups + (gate_w ? 1 : 0), rows = E + (gate_w ? 1 : 0);
+    const int64_t t0 = (int64_t)blockIdx.x * 16;
+    const int nt = (int)min((int64_t)16, T_all - t0);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l15 = lane & 15, c0 = 8 * (lane >> 4);
+    struct alignas(16) Eight { T v[8]; };
+    struct alignas(16) Eight32 { float v[8]; };
+    const T* src = h + (size_t)(t0 + min(l15, nt - 1)) * W + c0;
+    const float* wr[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int e = min(16 * n + l15, rows - 1);
+        wr[n] = (e < E ? router_w + (size_t)e * W : gate_w) + c0;
+    }
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    f32x4 acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int left = (W / 32 - wave + WAVES - 1) / WAVES, k = 32 * wave;
+    auto some = [&](auto count) {                              // the next steps of this wave, all their loads in front
+        constexpr int C = decltype(count)::value;
+        Eight x[C];
+        Eight32 w[C][NT];
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            x[u] = *(const Eight*)(src + k + 32 * WAVES * u);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) w[u][n] = *(const Eight32*)(wr[n] + k + 32 * WAVES * u);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f(x[u].v[j]), w[u][n].v[j], acc[n], 0, 0, 0);
+        left -= C;
+        k += 32 * WAVES * C;
+    };
+    while (left >= U) some(std::integral_constant<int, U>{});
+    if (left >= 2) some(std::integral_constant<int, 2>{});
+    if (left >= 1) some(std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wave][n][r][lane] = acc[n][r];
+    __syncthreads();
+    for (int i = threadIdx.x; i < NT * 256; i += 1024) {        // token 4 (l / 16) + r, row 16 n + l % 16
+        const int n = i >> 8, r = (i >> 6) & 3, l = i & 63, token = 4 * (l >> 4) + r, e = 16 * n + (l & 15);
+        float sum = 0.f;
+#pragma unroll
+        for (int v = 0; v < WAVES; ++v) sum += part[v][n][r][l];
+        if (e < rows) z_all[token * RS + (e < E ? e : RS - 1)] = sum;
+    }
+    __syncthreads();
+    finish_routes(z_all, RS, t0, nt, wave, WAVES, idx, wts, E, top, groups, keep, score, correction, group_top, renorm, bias, gate_w, gate_out);
+}
+
 // workgroup = one (token, expert) pair; every wave produces outputs f = wave, wave + 4, ...
 template <typename T>
 __global__ __launch_bounds__(256) void moe_pairs_gate_up_kernel(const T* __restrict__ h, const int32_t* __restrict__ idx,
@@ -365,11 +450,22 @@ extern "C" int sm_moe_route(int dtype, const void* h, const float* router_w, int
         return SM_ESHAPE;
     }
     if (T == 0) return SM_OK;
+    const int router_rows = E + (gate_w ? 1 : 0);
+    const bool wide = ((uintptr_t)h | (uintptr_t)router_w | (uintptr_t)gate_w) % 16 == 0;
+    if (wide && W % 32 == 0 && router_rows <= 64 && T >= 2048) {
+#define SM_ROUTE(NT_)                                                                                                           \
+    hipLaunchKernelGGL((moe_route_mfma_kernel<DT, NT_>), dim3((unsigned)((T + 15) / 16)), dim3(1024), 0, as_stream(stream), (const DT*)h, \
+                       router_w, idx, wts, T, W, E, top, groups, keep, score, correction, group_top, renorm, bias, gate_w, gate_out)
+        SM_DISPATCH(dtype, "sm_moe_route", if (router_rows <= 16) SM_ROUTE(1); else if (router_rows <= 32) SM_ROUTE(2); else SM_ROUTE(4));
+#undef SM_ROUTE
+        SM_CHECK_LAUNCH("sm_moe_route");
+        return SM_OK;
+    }
     // the token rows of a workgroup are staged in LDS when they fit and the rows can be moved in pieces of four channels
     const int tok = T >= 4096 ? 8 : (T >= 1024 ? 4 : 1);       // enough workgroups for a small step
     const size_t scores = ((size_t)tok * (E + groups + (gate_w ? 1 : 0)) * 4 + 15) / 16 * 16;
     const size_t rows = (size_t)tok * W * (dtype == SM_F32 ? 4 : 2);
-    const int staged = W % 4 == 0 && scores + rows <= 60 * 1024 && ((uintptr_t)h | (uintptr_t)router_w | (uintptr_t)gate_w) % 16 == 0;
+    const int staged = W % 4 == 0 && scores + rows <= 60 * 1024 && wide;
 #define SM_ROUTE(TOK_)                                                                                                          \
     hipLaunchKernelGGL((moe_route_kernel<DT, TOK_>), dim3((unsigned)((T + TOK_ - 1) / TOK_)), dim3(256), scores + (staged ? rows : 0), \
                        as_stream(stream), (const DT*)h, router_w, idx, wts, T, W, E, top, groups, keep, score, correction, group_top, \

@@ -208,7 +208,7 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     if (T == 0) return SM_OK;
     const int tiles = sm_moe_grouped_tiles(T, top, E);
     hipStream_t s = as_stream(stream);
-    if (int rc = launch_moe_align(idx, T * top, E, kRowsPerTile, tiles, row_pair, tile_expert, pair_row, s)) return rc;
+    if (int rc = launch_moe_align(idx, T * top, E, kRowsPerTile, tiles, row_pair, tile_expert, pair_row, nullptr, s)) return rc;
     if (act_is_gated(act_kind))
         hipLaunchKernelGGL(moe_grouped_kernel<1>, dim3((unsigned)tiles, (unsigned)((F + 31) / 32)), dim3(64), 0, s,
                            (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, top, F,
@@ -236,7 +236,7 @@ extern "C" int sm_moe_align(const int32_t* idx, int64_t T, int top, int E, int32
     }
     if (T == 0) return SM_OK;
     return launch_moe_align(idx, T * top, E, kRowsPerTile, sm_moe_grouped_tiles(T, top, E), row_pair, tile_expert, pair_row,
-                            as_stream(stream));
+                            nullptr, as_stream(stream));
 }
 
 extern "C" int sm_moe_combine(const void* prod, const int32_t* pair_row, const float* wts, const void* shared,

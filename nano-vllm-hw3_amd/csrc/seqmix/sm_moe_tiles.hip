@@ -289,7 +289,9 @@ extern "C" int sm_moe_tiles128(const void* h, const int32_t* idx, const float* w
     const bool dma = ((uintptr_t)h | (uintptr_t)act | (uintptr_t)w_gu | (uintptr_t)w_down) % 16 == 0;
     const int rows = dma ? tile_rows(T, top, E) : kBigRows, tiles = tile_count(T, top, E, rows);
     hipStream_t s = as_stream(stream);
-    if (int rc = launch_moe_align(idx, T * top, E, rows, tiles, row_pair, tile_expert, pair_row, s)) return rc;
+    // (the counts of the grouping lie where the down product's results come later: 64 E numbers of 4 bytes, if that many fit)
+    int32_t* counts = (int64_t)tiles * rows * W * 2 >= (int64_t)64 * E * 4 && (uintptr_t)prod % 4 == 0 ? (int32_t*)prod : nullptr;
+    if (int rc = launch_moe_align(idx, T * top, E, rows, tiles, row_pair, tile_expert, pair_row, counts, s)) return rc;
     const float* in_wts = weight_in ? wts : nullptr;
     if (act_is_gated(act_kind))
         launch_tiles<1>(rows, dma, h, w_gu, row_pair, tile_expert, act, top, tiles, F, W, limit, alpha, act_kind, in_wts, s);
