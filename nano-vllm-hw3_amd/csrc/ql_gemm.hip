@@ -101,7 +101,7 @@ static bool plan_lookup(int form, int64_t M, int64_t N, int64_t K, PlanEntry* ou
 // beside another one, or what it costs alone (from four rounds on the rounds run into each other); the height with the least is
 // within 1 % of the best of them over 64..8192 rows of the Qwen3 0.6B, 4B and 8B shapes.  Costs: microseconds per 1000 k, measured there.
 // The line to the other tiles: 140 tiles of 64 rows, 200 with int8 groups, whose sums and widening keep the vector unit busy on
-// low tiles.  Above it the wide tile is faster in nearly all problems (weight-only per row 1.15 x at the median and 1.5 x at most, per
+// low tiles, and with groups of long K, which slices shorten (512 x 6144 of 4096 k in fp8, 192 tiles: 64 us, in slices 50).  Above it the wide tile is faster in nearly all problems (weight-only per row 1.15 x at the median and 1.5 x at most, per
 // group 1.15 and 1.4, 8-bit activations 1.4 and 2.0; the worst 0.97, 0.91 and 0.98 x); below it most of the chip's CUs have no tile, and
 // slices of K or smaller tiles win.  Groups also go by the tile of 128 x 256, which costs 20.3 whatever shares its CU: 8192 x
 // 1024 outputs are one whole round of it.
@@ -110,7 +110,7 @@ static int wide_rows(int64_t M, int64_t N, int64_t K, int group, bool fp8, bool 
     static const double alone[3][5] = {{0, 0, 9.2, 12.2, 15.1}, {0, 0, 13.7, 16.6, 0}, {0, 0, 6.7, 8.3, 10.2}};
     if (K % (w8a8 ? 256 : 128) || N % (silu ? 64 : 32) || (group && group != 64 && group % 128)) return 0;
     const int64_t cols = (N + 255) / 256;
-    if ((M + 63) / 64 * cols < (group && !fp8 ? 200 : 140)) return 0;
+    if ((M + 63) / 64 * cols < (group && (!fp8 || K >= 4096) ? 200 : 140)) return 0;
     const int kind = w8a8 ? 2 : group ? 1 : 0;
     auto rounds = [&](int mt) -> double {
         const double n = (double)((M + 32 * mt - 1) / (32 * mt) * cols) / 256;
