@@ -17,7 +17,7 @@
 //
 // Bound by the matrix cores in 16 bits (1.15 to 1.2 PFLOP/s, what a library product of 8192 reaches too), by the vector unit beside
 // them with int8 groups (widening 50 %, folds 25 % of the time), by both and LDS in 8 bits.  4099 rows, Qwen3-4B shapes,
-// microseconds of the 128 x 256 tile with one strip per wave / here: weight-only int8 qkv 158 / 134, o 113 / 84, gate_up 398 / 349,
+// microseconds of the 128 x 256 tile with one strip per wave / here (without the waits by position, see load_a): weight-only int8 qkv 158 / 134, o 113 / 84, gate_up 398 / 349,
 // down 223 / 191; groups of 128 178 / 154, 136 / 97, 500 / 405, 269 / 218; fp8 x fp8 106 / 71, 82 / 44, 311 / 180, 158 / 93.
 #pragma once
 #include "ql_gemm_kernel.h"
@@ -32,9 +32,8 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
     constexpr bool INT = ACT == ACT_I8, GROUP = FG > 0;
     constexpr int AB = ACT == ACT_BF16 ? 2 : 1, KS = 256 / AB, SUB = KS / 32, BM = 32 * MT, BUF = BM * 256;
     constexpr int NA = 2 * MT;                                // 1 KB pieces of activations a wave loads per step
-    constexpr int FS = GROUP ? SUB / FG : 0;                  // folds per step
+    constexpr int FS = GROUP ? SUB / (FG + !FG) : 0;                  // folds per step
     using acc_t = typename std::conditional<INT, i32x16, f32x16>::type;
-    typedef __attribute__((address_space(1))) const void gvoid;
     typedef __attribute__((address_space(3))) void lvoid;
     typedef __attribute__((address_space(1))) const unsigned char* gbytes;    // (global from the start: uniform base + 32-bit offset)
     __shared__ __attribute__((aligned(1024))) unsigned char buf0[BUF];
@@ -60,13 +59,19 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
         const int row = 8 * MT * wave + 4 * i + (lane >> 4);
         aoff[i] = (unsigned)min(m0 + row, p.M - 1) * (unsigned)p.K * AB + 16u * (unsigned)((lane & 15) ^ (row & 15));
     }
+    // (as buffer loads: behind a global load to LDS the compiler lets no load's registers be read before every load has arrived, so the
+    // first weights of a step, or the third with groups, waited for activations just asked for.  With waits by position 4099 rows of
+    // the Qwen3-4B projections take 857 us with groups of 128, not 914)
+    // (the host's pass over a kernel knows no buffer resources)
+#ifdef __HIP_DEVICE_COMPILE__
+    const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, (unsigned)p.M * (unsigned)p.K * AB, 0x00020000);
+#endif
     auto load_a = [&](unsigned char* buf, int t) {
-        gbytes src = (gbytes)p.x + (size_t)t * 256;
+#ifdef __HIP_DEVICE_COMPILE__
 #pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            asm volatile("" : "+v"(aoff[i]));                 // (widened to 64 bits at the load, where the address takes it as it is)
-            __builtin_amdgcn_global_load_lds((gvoid*)(src + aoff[i]), (lvoid*)(buf + (8 * MT * wave + 4 * i) * 256), 16, 0, 0);
-        }
+        for (int i = 0; i < NA; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lvoid*)(buf + (8 * MT * wave + 4 * i) * 256), 16, aoff[i], t * 256, 0, 0);
+#endif
     };
     // weights: as in the other tiles (columns past N: the last strip or row, never stored)
     const unsigned kmul = p.wtiled ? 32u : 1u;
@@ -130,12 +135,14 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
         asm volatile("" : "+v"(place[c]));                    // (one register each, whatever the buffer and the fragment)
     }
     // One step.  The wait counter is positional: behind a step's activation loads come its 2 SUB weight loads and 2 FS scales, so
-    // at most that many outstanding means that the activations are in LDS; behind the barrier everybody's are, and nobody reads
-    // the other buffer any more.
+    // at most that many outstanding means that the activations are in LDS (the weights of the step behind go on); behind the barrier
+    // everybody's are, and nobody reads the other buffer any more.
+    constexpr int AFTER = 2 * SUB + 2 * FS;
+    static_assert(AFTER < 64, "the wait counter's range");
     auto step = [&](unsigned char* cur, unsigned char* nxt, int t) __attribute__((always_inline)) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0070);                   // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(0x0070 | (AFTER & 15) | (AFTER >> 4) << 14);      // vmcnt(AFTER) lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -253,6 +260,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    __builtin_amdgcn_s_waitcnt(0x0F70);                       // vmcnt(0): fewer loads than AFTER follow the first activations
     {
         int t = 0;
         for (; t + 1 < steps; t += 2) {
@@ -310,6 +318,21 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
         }
         return;
     }
+    // (ROPE: the tile's columns are two whole 128-wide heads, eight lanes per (row, head), as in the other tiles.  A thread has one head
+    // and 2 MT rows; their cache slots and positions are requested in front of the image, their cosines and sines behind it, all at
+    // once: one row behind the other, each a chain of two trips to memory, took 6076 x 4096 outputs of 1024 k 85 us instead of 70)
+    constexpr int NR = ROPE ? 2 * MT : 1;
+    const int rc = threadIdx.x & 7, rhead = (int)bx * 2 + (((int)threadIdx.x >> 3) & 1), rrow = (int)threadIdx.x >> 4;
+    int64_t rpos[NR];
+    RopePre pre[NR];
+    if constexpr (ROPE) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int t = min(m0 + rrow + 16 * i, p.M - 1);
+            pre[i].slot = p.rope.slot_mapping ? p.rope.slot_mapping[t] : -1;
+            rpos[i] = p.rope.positions ? p.rope.positions[t] : (int64_t)t;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -317,15 +340,27 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 put(512, i, r, 8 * wave + 4 * j + (l31 >> 3), __builtin_bit_cast(unsigned short, outv(i, j, r)));
+    if constexpr (ROPE) {
+        const unsigned short* nw = rhead < p.rope.Hq ? p.rope.qw : p.rope.kw;
+        u16x8 w1 = {0, 0, 0, 0, 0, 0, 0, 0}, w2 = w1;
+        if (nw) { w1 = *(const u16x8*)(nw + 8 * rc); w2 = *(const u16x8*)(nw + 64 + 8 * rc); }
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {                        // (value heads too, which leave them unused)
+            const float* cs = p.rope.cos_sin + rpos[i] * 128 + 8 * rc;
+            pre[i].w1 = w1;
+            pre[i].w2 = w2;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { pre[i].c[e] = cs[e]; pre[i].sn[e] = cs[64 + e]; }
+        }
+    }
     __syncthreads();
     if constexpr (ROPE) {
-        // the tile's columns are two whole 128-wide heads: eight lanes per (row, head), as in the other tiles
-        for (int e = threadIdx.x; e < BM * 16; e += 256) {
-            const int c = e & 7, hh = (e >> 3) & 1, row = e >> 4, head = (int)bx * 2 + hh;
-            if (m0 + row >= p.M) break;                       // (rows ascend with e; whole 8-lane groups leave together)
-            if (head >= p.rope.Hq + 2 * p.rope.Hkv) continue;
-            const RopePre pre = rope_prefetch(m0 + row, head, 8 * c, p.rope);
-            rope_store_piece(piece(512, row, 16 * hh + c), piece(512, row, 16 * hh + 8 + c), m0 + row, head, 8 * c, p.rope, pre);
+        if (rhead >= p.rope.Hq + 2 * p.rope.Hkv) return;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int row = rrow + 16 * i;
+            if (m0 + row >= p.M) break;                       // (whole 8-lane groups leave together)
+            rope_store_piece(piece(512, row, 16 * (rhead & 1) + rc), piece(512, row, 16 * (rhead & 1) + 8 + rc), m0 + row, rhead, 8 * rc, p.rope, pre[i]);
         }
     } else {
 #pragma unroll 4
