@@ -193,8 +193,38 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
             pick = -1;
         }
     }
-    // a measured plan for this shape, if the table holds one (entries were checked when they were set)
+    // 33 to 256 rows over long K: the double-buffered 32 x 64 tile of 512-k chunks, four waves along K, in as many slices as give
+    // the chip two workgroups per CU (a slice of 1300 k at least; one round more from 8192 k on).  The tiles above wait for
+    // activations at every chunk, and 64 rows of them leave CUs idle.  Us with the ladder's tile / this one (w8a8 fp8 with the
+    // quantizer, weight-only int8), outputs x K: 6144 x 2560 64 rows 12.1 / 11.5, 10.9 / 9.9, 128 rows 15.1 / 12.7, 15.1 / 12.4; 2560 x 9728
+    // 64 rows 21.2 / 18.2, 15.0 / 13.4, 128 rows 25.6 / 20.2, 21.2 / 18.4, 256 rows 36.5 / 27.9 (w8a8); 4096 x 4096 128 rows 14.5 / 13.8,
+    // 13.6 / 12.8; 4096 x 12288 192 rows 49.3 / 42.2 (w8a8).  Fewer than 160 tiles of up to 4096 k (2560 x 4096 at 96 rows 11.1 / 12.2) and
+    // more than 576 tiles (6144 x 2560 at 256 rows 18.5 / 18.8) stay with it, and K up to 2048, which is one chunk there.
+    // With groups up to 128 rows, 64 rows of it from 65 on, in slices for one workgroup per CU: 6144 x 2560 64 rows 10.5 / 9.5, 128
+    // rows 20.6 / 13.0; 6144 x 4096 128 rows 26.7 / 18.2; 2560 x 9728 64 rows 14.9 / 14.1, 128 rows 21.5 / 19.4; not with fewer than 64
+    // tiles (1024 x 3072, 64 rows: 6.8 / 8.5).
     int t_split = 0;
+    if (!silu && !rope && M > 32 && M <= 256 && K > 2048) {
+        const int64_t cols = (N + 63) / 64;
+        if (!group) {
+            const int64_t t = (M + 31) / 32 * cols;
+            if (t <= 576 && (t >= 160 || K > 4096)) {
+                mt = 1; wn = 2; wk = 4; cp = 4;
+                t_split = (int)std::max<int64_t>(1, std::min<int64_t>((K >= 8192 && t > 240 ? 960 : 480) / t, K / 1300));
+            }
+        } else if (M <= 128) {
+            const int rows = M <= 64 ? 1 : 2;
+            const int64_t t = (M + 32 * rows - 1) / (32 * rows) * cols;
+            if (t >= 64) {
+                mt = rows; wn = 2; wk = 4; cp = 4;
+                t_split = (int)std::max<int64_t>(1, std::min<int64_t>(260 / t, K / 1300));
+            }
+        }
+    }
+    // 33 to 64 rows of 8-bit activations under the SiLU epilogue, K of 2048 and more: 64 x 64 tiles, so that the weights are read once
+    // (19456 x 2560 24.5 -> 22.3 us with the quantizer, 24576 x 4096 35.0 -> 30.3)
+    if (silu && w8a8 && M > 32 && M <= 64 && K >= 2048) { mt = 2; wn = 2; wk = 2; cp = 8; }
+    // a measured plan for this shape, if the table holds one (entries were checked when they were set)
     PlanEntry te;
     if (plan_lookup((group ? QL_PLAN_GROUP : 0) | (silu ? QL_PLAN_SILU : 0) | (rope ? QL_PLAN_ROPE : 0) | (w8a8 ? QL_PLAN_W8A8 : 0),
                     M, N, K, &te)) {

@@ -1,0 +1,67 @@
+"""Products of 33 to 256 rows over long K in slices of the double-buffered 32 x 64 and 64 x 64 tiles, at ragged rows, columns and last
+chunks: int8 x int8 against another tile (whole numbers: the same bits), the others against 64 bits."""
+import pytest
+import torch
+
+from tests.util import TDT
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def NQ():
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    from nanovllm import _qlinear as Q
+    from nanovllm.utils import quantization as NQ
+    Q.load()
+    return NQ
+
+
+# rows, columns, k, plan (tile, slices) without and with groups of 64
+SHAPES = [(33, 5136, 2112, (1, 2, 4, 4, 1), (1, 2, 4, 4, 1)), (64, 640, 8256, (1, 2, 4, 4, 6), None), (65, 4104, 4160, (1, 2, 4, 4, 2), (2, 2, 4, 4, 2)),
+          (128, 2560, 4160, (1, 2, 4, 4, 3), (2, 2, 4, 4, 3)), (129, 7200, 2112, (1, 2, 4, 4, 1), None), (256, 2312, 9024, (1, 2, 4, 4, 3), None)]
+
+
+@pytest.mark.parametrize("form", ["row_int8", "row_fp8", "w8a8_int8", "w8a8_fp8", "g64_int8", "g64_fp8"])
+@pytest.mark.parametrize("M,N,K,plan,group_plan", SHAPES)
+def test_mid_sizes(NQ, M, N, K, plan, group_plan, form):
+    from nanovllm import _qlinear as Q
+    kind, dt = form.split("_")
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    group = 64 if kind == "g64" else 0
+    m = NQ.QGroupLinear(TDT[dt], w, None, group) if group else NQ.QLinear(TDT[dt], w, None, weight_only=kind == "row")
+    want = group_plan if group else plan
+    if want:
+        assert Q.plan_query(Q.QL_PLAN_GROUP if group else Q.QL_PLAN_W8A8 if kind == "w8a8" else 0, M, N, K) == want
+    y, again = m(x), m.tile()(x)
+    assert torch.equal(y, again)
+    lib = Q.load()
+    assert lib.ql_gemm_force_config(2, 4, 1, 4, 1) == 0
+    try:
+        other = m(x)
+    finally:
+        lib.ql_gemm_force_config(0, 0, 0, 0, 0)
+    if form == "w8a8_int8":
+        assert torch.equal(y, other)
+        return
+    # sums of K float32 products in another order: each within K 2^-24 of the sum of their sizes (which is below 2 |x| |w|: codes times
+    # scales are at most 2^-4 off the weights in fp8, and half a step in int8), and one rounding to bf16 on either side
+    size = x.float().abs() @ w.float().abs().t() * 2
+    assert ((y.float() - other.float()).abs() <= 2.0 ** -7 * other.float().abs() + 2 * K * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("dt", ["int8", "fp8"])
+@pytest.mark.parametrize("M,N,K", [(33, 1984, 2048), (64, 19456, 2560), (40, 4160, 4128)])
+def test_silu_of_8_bit_activations(NQ, M, N, K, dt):
+    from nanovllm import ops
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    y = NQ.QLinear(TDT[dt], w, None).enable_silu_mul().tile()(x)
+    ref = ops.silu_mul(NQ.QLinear(TDT[dt], w, None)(x))
+    if dt == "int8":                                          # (whole numbers: whatever tile the plain product takes)
+        assert torch.equal(y, ref)
+    else:                                                     # gate and up may round to neighbouring bf16 numbers: 2^-8 of each, |silu'| <= 1.1
+        assert ((y.float() - ref.float()).abs() <= 0.02 * ref.float().abs() + 0.02).all()
