@@ -1,6 +1,6 @@
 // Quantizer kernels: per-row (dynamic, also used on activations), per-group, per-tensor and the
 // quantize-dequantize ("fake") forms.  All are HBM-bound byte movers: 16-byte loads per lane,
-// one pass for the row/group maxima and one for the conversion (the second pass hits L2).
+// one pass for the row/group maxima and one for the conversion (the second pass hits L2, or registers).
 #include "ql_common.h"
 
 namespace ql {
@@ -37,6 +37,23 @@ __device__ __forceinline__ float block_max_256(float v, float* sh) {
 
 // ---- per-row: one 256-thread block per row ---------------------------------------------------
 template <int DT>
+__device__ __forceinline__ unsigned long long quant8(const u16x8& v, float sc_inv) {
+    unsigned long long out = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float y = bf16_bits_to_f32(v[j]) * sc_inv;
+        unsigned b;
+        if (DT == QL_INT8) b = (unsigned)(unsigned char)(signed char)(int)roundf(y);
+        else b = f32_to_e4m3fn(y);
+        out |= (unsigned long long)b << (8 * j);
+    }
+    return out;
+}
+
+// NC > 0: a row of at most 2048 NC elements, which is read once, all of it requested at the start.  A few rows take what their chain of
+// waits takes (64 rows of 4096 elements 3.5 -> 3.0 us to int8, 4.2 -> 3.6 to fp8, of 9728 4.5 -> 3.9 and 6.1 -> 5.0, against a loop that
+// waits at every 2048 elements and reads the row again); many rows the time of their bytes.  NC == 0: longer rows, in that loop.
+template <int DT, int NC>
 __global__ __launch_bounds__(256) void quant_per_row_kernel(const unsigned short* __restrict__ x,
                                                             unsigned char* __restrict__ q,
                                                             float* __restrict__ scale, int64_t H) {
@@ -44,25 +61,29 @@ __global__ __launch_bounds__(256) void quant_per_row_kernel(const unsigned short
     const int64_t row = blockIdx.x;
     const unsigned short* xr = x + row * H;
     float m = 0.f;
-    for (int64_t c = threadIdx.x * 8; c < H; c += 256 * 8) m = fmaxf(m, absmax8(*(const u16x8*)(xr + c)));
+    u16x8 v[NC > 0 ? NC : 1];
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[i] = *(const u16x8*)(xr + min(8 * (int)threadIdx.x + 2048 * i, (int)H - 8));     // (past the end: its end again)
+#pragma unroll
+        for (int i = 0; i < NC; ++i) m = fmaxf(m, absmax8(v[i]));
+    } else {
+        for (int64_t c = threadIdx.x * 8; c < H; c += 256 * 8) m = fmaxf(m, absmax8(*(const u16x8*)(xr + c)));
+    }
     m = block_max_256(m, sh);
     const float row_max = fmaxf(m, 1e-8f);
     const float sc = row_max / QMax<DT>::v;
     const float sc_inv = QMax<DT>::v / row_max;
     if (threadIdx.x == 0) scale[row] = sc;
     unsigned char* qr = q + row * H;
-    for (int64_t c = threadIdx.x * 8; c < H; c += 256 * 8) {
-        const u16x8 v = *(const u16x8*)(xr + c);
-        unsigned long long out = 0;
+    if constexpr (NC > 0) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float y = bf16_bits_to_f32(v[j]) * sc_inv;
-            unsigned b;
-            if (DT == QL_INT8) b = (unsigned)(unsigned char)(signed char)(int)roundf(y);
-            else b = f32_to_e4m3fn(y);
-            out |= (unsigned long long)b << (8 * j);
+        for (int i = 0; i < NC; ++i) {
+            const int c = 8 * (int)threadIdx.x + 2048 * i;
+            if (c < (int)H) *(unsigned long long*)(qr + c) = quant8<DT>(v[i], sc_inv);
         }
-        *(unsigned long long*)(qr + c) = out;
+    } else {
+        for (int64_t c = threadIdx.x * 8; c < H; c += 256 * 8) *(unsigned long long*)(qr + c) = quant8<DT>(*(const u16x8*)(xr + c), sc_inv);
     }
 }
 
@@ -374,12 +395,14 @@ int ql_quant_per_row(int dtype, const void* x, int64_t T, int64_t H, void* q, fl
     if (T == 0) return QL_OK;
     if (T > 0x7FFFFFFF) { set_error("ql_quant_per_row: T too large"); return QL_ESHAPE; }
     dim3 grid((unsigned)T), block(256);
-    if (dtype == QL_INT8)
-        hipLaunchKernelGGL(quant_per_row_kernel<QL_INT8>, grid, block, 0, as_stream(stream),
-                           (const unsigned short*)x, (unsigned char*)q, scale, H);
-    else
-        hipLaunchKernelGGL(quant_per_row_kernel<QL_FP8>, grid, block, 0, as_stream(stream),
-                           (const unsigned short*)x, (unsigned char*)q, scale, H);
+#define QL_QR(DT_, NC_)                                                                                                            \
+    hipLaunchKernelGGL((quant_per_row_kernel<DT_, NC_>), grid, block, 0, as_stream(stream), (const unsigned short*)x, (unsigned char*)q, \
+                       scale, H)
+#define QL_QR_(DT_) do { if (H <= 2048) QL_QR(DT_, 1); else if (H <= 4096) QL_QR(DT_, 2); else if (H <= 6144) QL_QR(DT_, 3); \
+                         else if (H <= 10240) QL_QR(DT_, 5); else if (H <= 14336) QL_QR(DT_, 7); else QL_QR(DT_, 0); } while (0)
+    if (dtype == QL_INT8) QL_QR_(QL_INT8); else QL_QR_(QL_FP8);
+#undef QL_QR_
+#undef QL_QR
     QL_CHECK_LAUNCH("ql_quant_per_row");
     return QL_OK;
 }
