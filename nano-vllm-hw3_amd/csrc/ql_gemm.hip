@@ -31,6 +31,8 @@ static bool rope_tile_built(int mt, int wn, int wk, int cp) {
     return false;
 }
 
+int launch_head_rows(const void* x, const void* w, void* y, int64_t M, int64_t V, int64_t K, hipStream_t s);      // ql_head.hip
+
 struct Plan {
     int mt, wn, wk, cp, split, k_per_split;
     dim3 grid;
@@ -967,6 +969,9 @@ int ql_lmhead_logits(const void* x, const void* w, void* logits, int64_t M, int6
     if (int rc = head_common(fn, x, w, M, V, K)) return rc;
     if (M > 0 && !logits) { set_error("%s: bad argument", fn); return QL_EINVAL; }
     if (M == 0) return QL_OK;
+    // (up to 32 rows: a wave can bring the activations itself; more rows share them in the tiles' LDS)
+    if (M <= 32 && K % 64 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && f_mt == 0)
+        return launch_head_rows(x, w, logits, M, V, K, as_stream(stream));
     const Plan pl = make_plan_head(M, V, K);
     GemmParams p = head_params(x, w, M, V, K);
     p.y = (unsigned short*)logits;
