@@ -209,7 +209,44 @@ __global__ __launch_bounds__(256, kRouteTokens == 8 ? 3 : 4) void moe_route_kern
     const int64_t t0 = (int64_t)blockIdx.x * kRouteTokens;
     const int nt = (int)min((int64_t)kRouteTokens, T_all - t0);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (staged) {
+    if (staged && kRouteTokens == 1) {
+        // one token: its row and four router rows, 1024 channels of them at once, go to registers side by side (through LDS and 256
+        // channels at a time, 64 tokens of 2048 channels and 16 experts took 9.6 us, not 8.2)
+        constexpr int U = 4;
+        struct alignas(sizeof(T) * 4) Pack4 { T v[4]; };
+        const T* src = h + (size_t)t0 * W;
+        for (int e0 = 4 * wave; e0 < rows; e0 += 16) {
+            const float* wr[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int e = min(e0 + j, rows - 1);
+                wr[j] = e < E ? router_w + (size_t)e * W : gate_w;
+            }
+            float d[4] = {0.f, 0.f, 0.f, 0.f};
+            for (int c0 = lane * 4; c0 < W; c0 += 256 * U) {
+                Pack4 hv[U];
+                float4 wv[U][4];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int c = min(c0 + 256 * u, W - 4);
+                    hv[u] = *(const Pack4*)(src + c);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) wv[u][j] = *(const float4*)(wr[j] + c);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (c0 + 256 * u < W) {
+                        const float x0 = to_f(hv[u].v[0]), x1 = to_f(hv[u].v[1]), x2 = to_f(hv[u].v[2]), x3 = to_f(hv[u].v[3]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) d[j] += x0 * wv[u][j].x + x1 * wv[u][j].y + x2 * wv[u][j].z + x3 * wv[u][j].w;
+                    }
+            }
+            fold_wave<4, 32>(d, lane);
+            const int e = e0 + lane / 16;
+            if (lane % 16 == 0 && e < rows) z_all[e < E ? e : RS - 1] = d[0];
+        }
+    } else if (staged) {
         // the workgroup's token rows (one contiguous piece of h) go to LDS once; every expert's row is then read once per
         // workgroup in 16-byte pieces and meets all the tokens there
         T* h_lds = (T*)(z_all + (kRouteTokens * RS + 3) / 4 * 4);
@@ -288,7 +325,7 @@ __global__ __launch_bounds__(256, kRouteTokens == 8 ? 3 : 4) void moe_route_kern
 // for sixteen tokens.  For many tokens: it is then bound by the reads of h, where staging the tokens in LDS and multiplying on the vector
 // unit spent its time in LDS reads and widening (16 experts, us: 8192 tokens of 2048 channels 28 -> 19, 4096 21 -> 13; 64 experts,
 // 8192 tokens of 4096 channels, which did not fit LDS, 2255 -> 88).  Below 2048 tokens a workgroup per token is as fast or faster (64
-// tokens 9.5 and 12.5: sixteen waves in few workgroups begin and end later), from 65 rows on the products of sixteen tokens are.
+// tokens 8.2 and 12.5: sixteen waves in few workgroups begin and end later), from 65 rows on the products of sixteen tokens are.
 template <typename T, int NT>
 __global__ __launch_bounds__(1024, NT == 1 && sizeof(T) == 2 ? 8 : 4) void moe_route_mfma_kernel(const T* __restrict__ h, const float* __restrict__ router_w,
                                                               int32_t* __restrict__ idx, float* __restrict__ wts, int64_t T_all, int W,

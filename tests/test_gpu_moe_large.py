@@ -1,4 +1,4 @@
-"""Routing and grouping of many tokens: the router on the matrix cores and the grouping by several workgroups."""
+"""Routing (on the matrix cores for many tokens, a workgroup per token for few) and the grouping by several workgroups."""
 import os
 import sys
 
@@ -18,8 +18,9 @@ def gen(seed):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,W,E,top,groups,keep,gate", [
     (2048, 32, 16, 4, 1, 1, False), (2049, 544, 15, 3, 1, 1, True), (2063, 1024, 16, 2, 1, 1, True), (2050, 2048, 32, 4, 4, 2, False),
-    (2101, 1056, 33, 5, 1, 1, False), (2048, 4096, 64, 8, 8, 3, False), (2055, 1568, 63, 1, 1, 1, True), (2047, 96, 1, 1, 1, 1, False)])
-def test_route_of_many_tokens(dtype, T, W, E, top, groups, keep, gate):
+    (2101, 1056, 33, 5, 1, 1, False), (2048, 4096, 64, 8, 8, 3, False), (2055, 1568, 63, 1, 1, 1, True), (2047, 96, 1, 1, 1, 1, False),
+    (1, 4100, 17, 4, 1, 1, True), (300, 1028, 16, 2, 1, 1, False), (77, 2052, 6, 2, 3, 2, True), (1023, 4, 5, 1, 1, 1, False)])
+def test_route(dtype, T, W, E, top, groups, keep, gate):
     """Against 64-bit logits.  The sum of W products in float32 is off by at most W 2^-24 of the sum of their sizes (about sqrt(2 W / pi)
     times the spread of a logit, which is 1): below 4096 * 2^-24 * 51 = 0.013 at worst, some sqrt(W) 2^-24 = 4e-6 in fact.  So a chosen
     score lies within 1e-4 of the one the reference chooses in its place, and the weights likewise."""
@@ -40,7 +41,7 @@ def test_route_of_many_tokens(dtype, T, W, E, top, groups, keep, gate):
         c = c.masked_fill(drop.repeat_interleave(E // groups, 1), -1.0)
     else:
         sure = torch.ones(T, dtype=torch.bool)
-    assert sure.float().mean() > 0.99
+    assert sure.float().mean() > 0.95
     ref = c.topk(top, -1).values
     got = c.gather(1, idx)
     assert (got - ref).abs()[sure].max() < 1e-4
