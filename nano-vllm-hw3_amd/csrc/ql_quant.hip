@@ -38,13 +38,27 @@ __device__ __forceinline__ float block_max_256(float v, float* sh) {
 // ---- per-row: one 256-thread block per row ---------------------------------------------------
 template <int DT>
 __device__ __forceinline__ unsigned long long quant8(const u16x8& v, float sc_inv) {
+    float y[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y[j] = bf16_bits_to_f32(v[j]) * sc_inv;
+    if constexpr (DT == QL_FP8) {
+        // two at a time by the conversion instruction, which rounds as f32_to_e4m3fn does (a row's numbers are at most 448 here), in a
+        // tenth of its instructions (64 rows of 4096 elements 3.6 -> 3.0 us, of 9728 5.0 -> 4.2); NaNs by the latter
+        if (const float all = ((y[0] + y[1]) + (y[2] + y[3])) + ((y[4] + y[5]) + (y[6] + y[7])); all == all) {
+            int lo = 0, hi = 0;
+            lo = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], lo, false);
+            lo = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], lo, true);
+            hi = __builtin_amdgcn_cvt_pk_fp8_f32(y[4], y[5], hi, false);
+            hi = __builtin_amdgcn_cvt_pk_fp8_f32(y[6], y[7], hi, true);
+            return (unsigned long long)(unsigned)hi << 32 | (unsigned)lo;
+        }
+    }
     unsigned long long out = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        const float y = bf16_bits_to_f32(v[j]) * sc_inv;
         unsigned b;
-        if (DT == QL_INT8) b = (unsigned)(unsigned char)(signed char)(int)roundf(y);
-        else b = f32_to_e4m3fn(y);
+        if (DT == QL_INT8) b = (unsigned)(unsigned char)(signed char)(int)roundf(y[j]);
+        else b = f32_to_e4m3fn(y[j]);
         out |= (unsigned long long)b << (8 * j);
     }
     return out;

@@ -21,3 +21,25 @@ def test_row_lengths(H, dt):
     qo, so = O.per_row_quant(bits16(x), dt)
     assert np.array_equal(s.cpu().numpy(), so)
     assert np.array_equal(q.view(torch.uint8).cpu().numpy(), qo.view(np.uint8))
+
+
+@pytest.mark.parametrize("length", [8192, 65536])
+@pytest.mark.parametrize("top", [0x43E0, 0x3F80, 0x4049, 0x7F00, 0x0180])
+def test_every_number_to_fp8(length, top):
+    """All bf16 numbers up to a row's largest, negative ones, zeros and subnormals among them, under scales that are and are not powers of
+    two; a NaN leaves its neighbours alone."""
+    from nanovllm.utils import quantization as NQ
+    bits = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    bits = np.where((bits & 0x7FFF) > top, bits & 0x8000, bits).astype(np.uint16).reshape(-1, length)
+    bits[:, 5] = top
+    x = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
+    q, s = NQ.per_row_quant(x, torch.float8_e4m3fn)
+    qo, so = O.per_row_quant(bits, "fp8")
+    assert np.array_equal(s.cpu().numpy(), so)
+    assert np.array_equal(q.view(torch.uint8).cpu().numpy(), qo.view(np.uint8))
+    x[0, 9] = float("nan")
+    qn, _ = NQ.per_row_quant(x, torch.float8_e4m3fn)
+    qn, q = qn.view(torch.uint8), q.view(torch.uint8).clone()
+    assert (qn[0, 9].item() & 0x7F) == 0x7F
+    q[0, 9] = qn[0, 9]
+    assert torch.equal(q, qn)
