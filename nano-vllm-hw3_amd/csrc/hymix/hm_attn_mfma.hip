@@ -5,7 +5,7 @@
 //     list is split over workgroups, every (sequence, split, head) leaves an unnormalised partial state {m c, l, O} in the
 //     workspace, and a second launch merges the splits in order and adds the sink to the denominator.
 #include "../row_deal.h"
-#include "hm_attn_tile.h"
+#include "hm_attn_stream.h"
 
 namespace hm {
 
@@ -139,48 +139,56 @@ __global__ __launch_bounds__(64) void attn_decode_kernel(const unsigned short* _
             for (int e = 0; e < 4; ++e) part[2 + 32 * d + 8 * rq + 4 * hi + e] = oacc[d][4 * rq + e];
 }
 
-__global__ void attn_decode_merge_kernel(const float* __restrict__ ws, const float* __restrict__ sink,
-                                         unsigned short* __restrict__ o, int H, int V, int splits, int stride, int plain_sum,
-                                         OutArgs out) {
+// A wave per (sequence, head), two columns per lane; the splits' maxima and sums are read a split per lane in front of the outputs.
+__global__ __launch_bounds__(64) void attn_decode_merge_kernel(const float* __restrict__ ws, const float* __restrict__ sink,
+                                                               unsigned short* __restrict__ o, int H, int V, int splits, int stride,
+                                                               int plain_sum, OutArgs out) {
+    typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
     const size_t row = blockIdx.x;                          // b * H + h
     const size_t b = row / H, h = row % H;
-    unsigned short* orow = o + b * out.o_stride + h * V;
-    auto leave = [&](int c, float v) {
-        v *= out.scale;
-        if (out.gate) v *= fast_sigmoid((float)__builtin_bit_cast(bf16_t, out.gate[b * out.gate_stride + h * V + c]));
-        orow[c] = __builtin_bit_cast(unsigned short, (bf16_t)v);
-    };
-    if (plain_sum) {                                        // weights that are not normalised: the splits' outputs add up
-        for (int c = threadIdx.x; c < V; c += blockDim.x) {
-            float acc = 0.f;
-            for (int s = 0; s < splits; ++s) {
-                const float* p = ws + ((b * splits + s) * H + h) * stride;
-                if (p[1] > 0.f) acc += p[2 + c];
-            }
-            leave(c, acc);
+    const float* first = ws + (b * splits * H + h) * stride;
+    const size_t step = (size_t)H * stride;
+    const int c = 2 * threadIdx.x;                          // (V <= 128, a multiple of 8; a lane past it repeats the last pair)
+    // in log2 units, as the partial maxima; weights that are not normalised: the splits' outputs add up
+    const float sk = sink ? sink[h] * 1.4426950408889634f : -INFINITY;
+    float M = -INFINITY, L = 0.f;
+    if (!plain_sum) {
+        for (int s = threadIdx.x; s < splits; s += 64) {
+            const f32x2 ml = *(const f32x2*)(first + s * step);
+            if (ml.y > 0.f) M = fmaxf(M, ml.x);
         }
-        return;
-    }
-    const float sk = sink ? sink[h] * 1.4426950408889634f : -INFINITY;       // in log2 units, as the partial maxima
-    float M = sk;
-    for (int s = 0; s < splits; ++s) {
-        const float* p = ws + ((b * splits + s) * H + h) * stride;
-        if (p[1] > 0.f) M = fmaxf(M, p[0]);
-    }
-    float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;
-    for (int s = 0; s < splits; ++s) {
-        const float* p = ws + ((b * splits + s) * H + h) * stride;
-        if (p[1] > 0.f) L += __builtin_amdgcn_exp2f(p[0] - M) * p[1];
-    }
-    const float inv = 1.f / L;
-    for (int c = threadIdx.x; c < V; c += blockDim.x) {
-        float acc = 0.f;
-        for (int s = 0; s < splits; ++s) {
-            const float* p = ws + ((b * splits + s) * H + h) * stride;
-            if (p[1] > 0.f) acc += __builtin_amdgcn_exp2f(p[0] - M) * p[2 + c];
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) M = fmaxf(M, __shfl_xor(M, d));
+        M = fmaxf(M, sk);
+        for (int s = threadIdx.x; s < splits; s += 64) {
+            const f32x2 ml = *(const f32x2*)(first + s * step);
+            if (ml.y > 0.f) L += __builtin_amdgcn_exp2f(ml.x - M) * ml.y;
         }
-        leave(c, acc * inv);
+        L = wave_sum(L) + (sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f);
     }
+    f32x2 acc = {0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+        const float* p = first + s * step;
+        const f32x2 ml = *(const f32x2*)p, x = *(const f32x2*)(p + 2 + min(c, V - 2));
+        const float f = plain_sum ? 1.f : __builtin_amdgcn_exp2f(ml.x - M);
+        if (ml.y > 0.f) {                                   // (an empty split's outputs are not written)
+            acc.x += f * x.x;
+            acc.y += f * x.y;
+        }
+    }
+    if (c >= V) return;
+    const float inv = (plain_sum ? 1.f : 1.f / L) * out.scale;
+    float g0 = 1.f, g1 = 1.f;
+    if (out.gate) {
+        const u16x2 gt = *(const u16x2*)(out.gate + b * out.gate_stride + h * V + c);
+        g0 = fast_sigmoid((float)__builtin_bit_cast(bf16_t, (unsigned short)gt[0]));
+        g1 = fast_sigmoid((float)__builtin_bit_cast(bf16_t, (unsigned short)gt[1]));
+    }
+    const u16x2 y = {__builtin_bit_cast(unsigned short, (bf16_t)(acc.x * inv * g0)),
+                     __builtin_bit_cast(unsigned short, (bf16_t)(acc.y * inv * g1))};
+    *(u16x2*)(o + b * out.o_stride + h * V + c) = y;
 }
 
 static int padded_nb(int n) {
@@ -315,7 +323,24 @@ extern "C" int hm_attn_decode(const void* q, const void* k_cache, const void* v_
                        (const unsigned short*)v_cache, block_tables, ctx, window, keep_first, scale, (float*)workspace, H, G, D, \
                        V, block_size, max_blocks, splits, (const unsigned short*)kp_cache, (const unsigned short*)vp_cache, pool, \
                        pool_rows, chunk, head_bias, softcap)
-    HM_BY_HEAD_SIZE(nbk, nbv, sigmoid_w, softcap, HM_DEC);
+    // One, two or four query heads per group of 64 or 128 channels, softmax weights: the vector unit keeps up with the cache
+    // (hm_attn_stream.h has both forms' times; eight heads would need the registers of its loads, other widths other lane splits).
+    const int rep = H / G;
+    const bool stream_form = D == V && (D == 64 || D == 128) && (rep == 1 || rep == 2 || rep == 4) && !sigmoid_w && pool == 0 &&
+                             ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
+#define HM_STREAM(D_, R_, S_)                                                                                                  \
+    hipLaunchKernelGGL((attn_decode_stream_kernel<D_, R_, S_>), grid, dim3(256), 0, s, (const unsigned short*)q,                \
+                       (const unsigned short*)k_cache, (const unsigned short*)v_cache, block_tables, ctx, window, keep_first,   \
+                       (S_ == kSoftcap ? softcap : scale) * 1.4426950408889634f, S_ == kSoftcap ? 2.f * 1.4426950408889634f * scale / softcap : 0.f, \
+                       (float*)workspace, H, G, block_size, max_blocks, splits, chunk)
+#define HM_STREAM_R(D_, S_) do { if (rep == 1) HM_STREAM(D_, 1, S_); else if (rep == 2) HM_STREAM(D_, 2, S_); else HM_STREAM(D_, 4, S_); } while (0)
+#define HM_STREAM_D(S_) do { if (D == 64) HM_STREAM_R(64, S_); else HM_STREAM_R(128, S_); } while (0)
+    if (!stream_form) { HM_BY_HEAD_SIZE(nbk, nbv, sigmoid_w, softcap, HM_DEC); }
+    else if (softcap > 0.f) HM_STREAM_D(kSoftcap);
+    else HM_STREAM_D(kSoftmax);
+#undef HM_STREAM_D
+#undef HM_STREAM_R
+#undef HM_STREAM
 #undef HM_DEC
     HM_CHECK_LAUNCH("hm_attn_decode");
     hipLaunchKernelGGL(attn_decode_merge_kernel, dim3((unsigned)(B * H)), dim3(64), 0, s, (const float*)workspace, sink,
