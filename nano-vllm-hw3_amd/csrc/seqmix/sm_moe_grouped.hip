@@ -44,12 +44,15 @@ __device__ __forceinline__ bf16x8 load8(const unsigned short* p, int k, int K) {
 template <int MODE, bool FEW>
 __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                           const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
-                                                          unsigned short* __restrict__ out, int top, unsigned top_inv, int N, int K, float limit,
+                                                          unsigned short* __restrict__ out, int tiles, int top, unsigned top_inv, int N, int K, float limit,
                                                           float alpha, int act_kind, const float* __restrict__ in_wts) {
     constexpr bool GATE_UP = MODE == 1, FROM_TOKENS = MODE != 0;
-    const int tile = blockIdx.x;
+    // Workgroups go to the eight dies in turn: a die has every eighth column block, and its tiles one behind the other, so that the tiles of
+    // one expert meet its weights in one L2 (us of whole calls, tiles on neighbouring dies / here, weights not in a cache: 40 rows for each of
+    // 4 experts of 2048 x 4096 87 / 77, of 16 of 2048 x 1536 110 / 86, of one of 4096 x 11008 104 / 87; one tile per expert alike).
+    const int id = blockIdx.x >> 3, tile = id % tiles, n0 = ((id / tiles) * 8 + (blockIdx.x & 7)) * 32;
+    if (n0 >= N) return;
     const int lane = threadIdx.x, l31 = lane & 31, hi = lane >> 5;
-    const int n0 = blockIdx.y * 32;
     // The tile's rows come 128 bytes at a time, eight lanes to a row, and go through LDS to the lanes that multiply them (chunk c
     // of row r at place c ^ (r / 2 & 7)): a lane reading its own row would touch a cache line of its own with every load.  Rows
     // without a pair repeat one that has a place in memory; nobody reads their sums.
@@ -229,9 +232,10 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     hipStream_t s = as_stream(stream);
     if (int rc = launch_moe_align(idx, T * top, E, kRowsPerTile, tiles, row_pair, tile_expert, pair_row, nullptr, s)) return rc;
     const bool few = T <= 8 || (T <= 32 && std::min<int64_t>(T * top, E) * ((F + 31) / 32) <= 256);
+    auto grid = [&](int n) { return dim3((unsigned)((n + 255) / 256) * 8u * (unsigned)tiles); };
 #define SM_GROUPED(MODE_, FEW_)                                                                                                          \
-    hipLaunchKernelGGL((moe_grouped_kernel<MODE_, FEW_>), dim3((unsigned)tiles, (unsigned)((F + 31) / 32)), dim3(64), 0, s,              \
-                       (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, top, top_inv, \
+    hipLaunchKernelGGL((moe_grouped_kernel<MODE_, FEW_>), grid(F), dim3(64), 0, s,                                                     \
+                       (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, tiles, top, top_inv, \
                        F, W, limit, alpha, act_kind, weight_in ? wts : nullptr)
     if (act_is_gated(act_kind)) {
         if (few) SM_GROUPED(1, true); else SM_GROUPED(1, false);
@@ -240,8 +244,8 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     }
 #undef SM_GROUPED
     SM_CHECK_LAUNCH("sm_moe_grouped (gate/up)");
-    hipLaunchKernelGGL((moe_grouped_kernel<0, false>), dim3((unsigned)tiles, (unsigned)((W + 31) / 32)), dim3(64), 0, s,
-                       (const unsigned short*)act, (const unsigned short*)w_down, row_pair, tile_expert, (unsigned short*)prod, top, top_inv, W,
+    hipLaunchKernelGGL((moe_grouped_kernel<0, false>), grid(W), dim3(64), 0, s,
+                       (const unsigned short*)act, (const unsigned short*)w_down, row_pair, tile_expert, (unsigned short*)prod, tiles, top, top_inv, W,
                        F, 0.f, 0.f, 0, (const float*)nullptr);
     SM_CHECK_LAUNCH("sm_moe_grouped (down)");
     if (y == nullptr) return SM_OK;               // the caller sums a token's pairs itself
