@@ -51,13 +51,21 @@ __device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.f + er
 __device__ __forceinline__ float gelu_tanh(float z) {
     return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
+// n / d for d >= 1: a division's remainder step without its scaling (d 2^-32 and its reciprocal are never subnormal), the special cases
+// by the division's own last instruction.  7 instructions for 11: a gate's outputs are a sixth of the expert tiles' cycles.
+__device__ __forceinline__ float quotient(float n, float d) {
+    const float r = __builtin_amdgcn_rcpf(d * 0x1p-32f) * 0x1p-32f, q = n * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, n), r, q), d, n);
+}
 // the gated forms: g' = min(g, limit), u' = clamp(u, +-limit), g' sigmoid(alpha g') (u' + 1) (SM_ACT_CLAMPED_GLU), or with
 // SM_ACT_SILU_GLU the same without the one: silu(g) u for limit = +inf and alpha = 1; SM_ACT_GELU_TANH_GLU: gelu_tanh(g) u
 __device__ __forceinline__ float gated_act(float g, float u, float limit, float alpha, int act) {
     if (act == SM_ACT_GELU_TANH_GLU) return gelu_tanh(g) * u;
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return g / (1.f + __expf(-alpha * g)) * (u + (act == SM_ACT_SILU_GLU ? 0.f : 1.f));
+    // (minnum and maxnum as the hardware has them; the library's put a canonicalization in front of every operand)
+    asm("v_min_f32 %0, %1, %2" : "=v"(g) : "s"(limit), "v"(g));
+    u = __builtin_amdgcn_fmed3f(u, -limit, limit);
+    const float y = quotient(g, 1.f + __builtin_amdgcn_exp2f(g * (-1.4426950408889634f * alpha)));
+    return y * (act == SM_ACT_SILU_GLU ? u : u + 1.f);
 }
 __host__ __device__ __forceinline__ bool act_is_gated(int act) {
     return act == SM_ACT_CLAMPED_GLU || act == SM_ACT_SILU_GLU || act == SM_ACT_GELU_TANH_GLU;

@@ -1,0 +1,50 @@
+"""The expert tiles that a workgroup walks over (csrc/seqmix/sm_moe_tiles.hip) against the 32-row form, whose sums are the same bit for bit, where
+the walk can go wrong: one tile and none for most workgroups, a last round by halves and by whole tiles, odd numbers of row tiles, tiles
+of 128 and 256 rows, the fewest steps, outputs that end inside a tile, groups that end inside a block of 32 rows, weights on the input,
+and one of the two products whose k is no multiple of 128.  And the gate's quotient at the ends of its range."""
+import os
+import sys
+
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "nano-vllm-hw3_amd"))
+
+from nanovllm import seq_ops  # noqa: E402
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,top,E,W,F,act", [(1, 1, 1, 128, 128, "silu_glu"), (257, 1, 1, 128, 256, "silu_glu"), (300, 2, 3, 256, 136, "gelu"),
+                                             (700, 2, 5, 384, 1152, "clamped_glu"), (513, 3, 4, 1152, 384, "relu_sq"),
+                                             (4000, 2, 4, 256, 1536, "silu_glu"), (9001, 2, 3, 512, 1024, "clamped_glu"),
+                                             (6000, 2, 7, 200, 2048, "silu_glu"), (8300, 1, 32, 2048, 264, "gelu")])
+def test_walked_tiles_equal_the_small_ones(T, top, E, W, F, act):
+    g = torch.Generator().manual_seed(T + W)
+    parts = 2 if act.endswith("glu") else 1
+    kind = dict(silu_glu=seq_ops.ACT_SILU_GLU, clamped_glu=seq_ops.ACT_CLAMPED_GLU, gelu=seq_ops.ACT_GELU, relu_sq=seq_ops.ACT_RELU_SQ)[act]
+    h = torch.randn(T, W, generator=g).bfloat16().cuda()
+    w_gu, w_down = ((torch.randn(E, *s, generator=g) * s[1] ** -0.5).bfloat16().cuda() for s in ((parts * F, W), (W, F)))
+    # a last expert with few tokens, and the others as the numbers fall
+    bent = torch.rand(T, E, generator=g) + torch.tensor([0.0] * (E - 1) + [-0.6 if E > top else 0.0])
+    idx, wts = bent.topk(top, -1)[1].int().cuda(), torch.rand(T, top, generator=g).cuda()
+    for weight_in in (False, True):
+        a, b = (seq_ops.moe_experts(h, idx, wts, w_gu, w_down, 7.0, 1.702, form=f, act_kind=kind, weight_in=weight_in) for f in ("grouped", "tiles128"))
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_gate_at_the_ends_of_its_range():
+    """g / (1 + e^-g) * u in float32: quotients by more than 2^126 and by infinity, subnormal gates, infinities and NaN."""
+    g = torch.tensor([0.0, -0.0, 1e-40, -1e-40, 1e-30, 0.3, -0.3, 5.0, -5.0, 60.0, -60.0, -86.0, -87.5, -88.5, -90.0, -200.0, 2e38, -3e38, float("inf")])      # (1.5 g below 3.4e38)
+    u = torch.full_like(g, 1.5)
+    y = seq_ops.gated_act(torch.cat([g, u])[None].cuda(), seq_ops.ACT_SILU_GLU, float("inf"), 1.0)[0].cpu().double()
+    d = 1.0 + torch.exp(-g.double())
+    want = g.double() / d * 1.5
+    # float32: the exponential's argument is rounded (2^-24 of up to 90) and the hardware's exponential is good to 2 units; below the
+    # smallest normal number, and where e^-g has left float32's range, the result may be zero
+    assert torch.isinf(y[-1]) and y[-1] > 0
+    assert (y[:-1] - want[:-1]).abs().le(1.2e-5 * want[:-1].abs() + 2e-36).all()
+    for bad in (float("nan"), float("-inf")):
+        y = seq_ops.gated_act(torch.tensor([[1.0, bad, 2.0, 2.0]]).cuda(), seq_ops.ACT_SILU_GLU, 7.0, 1.0)[0].cpu()
+        assert abs(y[0].item() - 1.4621172) < 1e-6
