@@ -106,11 +106,13 @@ static bool wide_built(int64_t N, int64_t K, int group, bool silu, bool w8a8) {
 
 // Row fragments of the wide tile that a problem runs on; 0: the other tiles are faster; -1: the 128 x 256 tile of 64-k chunks is (groups).
 // Two of its workgroups share a CU, so a launch takes ceil(tiles / 256) times what a tile costs beside another one, or what it costs
-// alone (from four rounds on the rounds run into each other).  Costs: microseconds per 1000 k, measured over 64..8192 rows of the Qwen3
-// 0.6B, 1.7B, 4B and 8B shapes.  Groups of 64 fold twice as often; fp8 widens in less.
+// alone (from six rounds on the rounds run into each other).  Costs: microseconds of a tile and per 1000 k of it, fitted over 256..8192
+// rows of the Qwen3 0.6B, 1.7B, 4B and 8B shapes and eight others with weights that no cache holds (the rows that it picks are 0.1 to
+// 0.3 % slower than the best ones on average); 8-bit activations by k alone, over 64..8192 rows.
 // The line to the other tiles: 140 tiles of 64 rows, below which most of the chip's CUs have no tile and slices of K or smaller tiles
-// win; 150 with fp8 groups (140 x 12288 of 3584 k, 144 tiles: 39.9 / 43.8), 200 with int8 groups, whose sums and widening keep the vector unit busy on low tiles, and with groups of long K, which slices
-// shorten (512 x 6144 of 4096 k in fp8, 192 tiles: 64 us, in slices 50).
+// win.  Groups of 64: in int8 170 up to 4096 k, from there 160 (640 x 4096 of 4096 k: 63.2 there / 54.3 here), beyond 6144 k 190.  Longer
+// ones: 200 up to 1024 k and from 4096 on (512 x 6144 of 4096 k in fp8, 192 tiles: 50 in slices / 64 here), between those 140 in int8 (700
+// x 3584 of 1536 k, 154 tiles: 23.7 / 21.4), 150 beyond 1024 rows and in fp8 (140 x 12288 of 3584 k, 144 tiles: 39.9 / 43.8).
 // With other lines, us in the other tile / here:
 //   fp8 groups beyond 1024 rows, whose other tile is the 64 x 128 one of four waves: 200 (1280 x 2048 of 2048 k, 160 tiles: 22.2 / 24.7)
 //   int8 rows and groups of 128 over more than 10240 k, up to 1024 rows, whose other tile is the 64 x 128 one in three slices: 170 and 220 (640
@@ -119,35 +121,59 @@ static bool wide_built(int64_t N, int64_t K, int group, bool silu, bool w8a8) {
 //   up to 32 rows, whose other tile reads its weights past the caches and multiplies no padding: 200 tiles (36864 x 4096, 144 tiles, 1 row: 31.4 /
 //   39.1, 32 rows 38.9 / 37.4; 65536 x 2048, 256 tiles, 1 row: 40 / 29), 256 with groups under SiLU (51200 x 5120, 1 row: 61.6 / 67.9); 8-bit
 //   activations from 2048 k on (151936 x 1024, 1 row: 29.4 / 32.2)
-// Groups also go by the 128 x 256 tile of 64-k chunks, which costs 20.3 whatever shares its CU (8192 x 1024 outputs are one whole round of
-// it), and more with groups of 64 and those of 256 and more, whose folds it does not skip, and at short K, for its longer ends.
+// Groups also go by the 128 x 256 tile of 64-k chunks, which costs the same whatever shares its CU (8192 x 1024 outputs are one whole round of it).
 static int wide_rows(int64_t M, int64_t N, int64_t K, int group, bool fp8, bool silu, bool rope, bool w8a8) {
-    static const double pair[4][5] = {{0, 0, 7.5, 11.1, 13.5}, {0, 0, 10.8, 13.4, 0}, {0, 0, 4.6, 6.8, 8.0}, {0, 0, 12.3, 14.5, 0}};
-    static const double alone[4][5] = {{0, 0, 9.2, 12.2, 15.1}, {0, 0, 13.7, 16.6, 0}, {0, 0, 6.7, 8.3, 10.2}, {0, 0, 14.9, 18.0, 0}};
+    struct Cost { double tile, k; };
+    // 64, 96 and 128 rows: no groups in int8, fp8; groups of 128 and more; groups of 64; 8-bit activations
+    static const Cost pair[7][3] = {{{1.94, 6.25}, {3.08, 8.33}, {3.71, 10.95}}, {{1.83, 5.55}, {2.88, 7.75}, {3.46, 10.27}},
+                                 {{1.35, 7.82}, {2.29, 9.96}, {}}, {{0.89, 7.13}, {1.95, 9.47}, {}},
+                                 {{1.18, 9.42}, {2.30, 11.34}, {}}, {{0.84, 9.05}, {2.06, 10.81}, {}},
+                                 {{0, 4.6}, {0, 6.8}, {0, 8.0}}};
+    static const Cost alone[7][3] = {{{6.59, 6.40}, {8.48, 7.46}, {10.29, 9.54}}, {{6.37, 5.66}, {8.26, 6.74}, {12.00, 8.56}},
+                                  {{7.04, 8.09}, {8.09, 11.50}, {}}, {{6.16, 7.45}, {8.07, 11.04}, {}},
+                                  {{5.69, 10.81}, {8.29, 13.08}, {}}, {{4.77, 10.75}, {8.46, 12.59}, {}},
+                                  {{0, 6.7}, {0, 8.3}, {0, 10.2}}};
+    // the 128 x 256 tile of 64-k chunks: groups of 128, of 256 and more; groups of 64
+    static const Cost chunked[6] = {{}, {}, {4.85, 16.44}, {4.53, 15.62}, {5.22, 17.92}, {4.98, 17.11}};
+    // what a launch of several rounds takes beside them
+    const double start = w8a8 ? 0 : group ? 4 : 3;
     if (!wide_built(N, K, group, silu, w8a8)) return 0;
     const int64_t cols = (N + 255) / 256, low = (M + 63) / 64 * cols;
-    int64_t line = !group ? 140 : !fp8 || K >= 4096 || M > 1024 ? 200 : 150;
+    int64_t line = 140;
+    if (group == 64) line = K < 4096 ? (fp8 ? 140 : 170) : K <= 6144 ? 160 : 190;
+    else if (group && fp8) line = K >= 4096 || M > 1024 ? 200 : 150;
+    else if (group) line = K >= 4096 || K <= 1024 ? 200 : M > 1024 ? 150 : 140;
     if (K > 10240 && M <= 1024 && (group ? group == 128 : !fp8)) line = group ? 220 : 170;
     if (rope && K <= 1024 && M > 1024 && fp8 && !group && !w8a8) line = 400;
     if (M <= 32) line = group && silu ? 256 : 200;
     if (low < line || (M <= 32 && w8a8 && K < 2048)) return 0;
-    const int kind = w8a8 ? 2 : group == 64 ? 3 : group ? 1 : 0;
-    const double scale = group && fp8 ? 0.93 : 1;
+    const int kind = w8a8 ? 6 : (group == 64 ? 4 : group ? 2 : 0) + fp8;
+    const double k = K / 1000.;
     auto rounds = [&](int mt) -> double {
-        const double n = (double)((M + 32 * mt - 1) / (32 * mt) * cols) / 256;
-        return n < 4 ? (double)(int64_t)(n + 255. / 256) : n + (group ? 0.6 : 0.5);
+        const double n = (double)((M + 32 * mt - 1) / (32 * mt) * cols) / 256, whole = (double)(int64_t)(n + 255. / 256);
+        if (w8a8) return n < 4 ? whole : n + 0.5;
+        return n < 6 ? whole : std::min(whole, n + 0.7);
     };
-    int best = 0;
-    double least = 0;
-    for (int mt = 2; mt <= (group ? 3 : 4); ++mt) {
-        const double n = rounds(mt), cost = scale * (n > 1 ? n * pair[kind][mt] : alone[kind][mt]);
-        if (!best || cost < least) { best = mt; least = cost; }
-    }
+    auto cost = [&](int mt) -> double {
+        const double n = rounds(mt);
+        const Cost &p = pair[kind][mt - 2], &a = alone[kind][mt - 2];
+        if (n <= 1) return a.tile + a.k * k;
+        // (without groups the last of three rounds has its CU to itself, 6000 x 4096 of 1024 k in 128 rows 72 us, in 96 63)
+        if (!group && !w8a8 && n == 3) return 2 * (p.tile + p.k * k) + a.tile + a.k * k;
+        return start + n * (p.tile + p.k * k);
+    };
+    int best = 2;
+    for (int mt = 3; mt <= (group ? 3 : 4); ++mt)
+        if (cost(mt) < cost(best)) best = mt;
+    // (no shape of the fit: fewer rounds win, groups of 128 at 9000 x 1024 of 512 k 20.5 in 64 rows, 18.3 in 96, 4500 x 2048 of 768 k 25.6 / 22.7)
+    if (!w8a8 && K < 1024 && best == 2 && rounds(3) < rounds(2)) best = 3;
     if (group) {
-        // (up to 1024 rows and less than a round of it, groups of 128 and more are faster here at any count: 961 x 6144 of 2560 k 53 / 51)
-        const bool there = group == 64 || M > 1024 || (M + 127) / 128 * cols >= 256;
-        const double other = (group == 64 ? 22.2 : group == 128 ? 20.3 : 21.5) * (K <= 1024 ? 1.12 : 1);
-        if (there && least > rounds(4) * other) return -1;
+        // (up to 1024 rows and less than a round of it, groups of 128 and more are faster here at any count: 961 x 6144 of 2560 k 53 / 51.  With
+        // groups of 64 up to a round of it is faster than two here beyond 1024 k, unless its last row tile is more than half full, but not
+        // full: 1792 x 4096 of 4096 k 74 / 79, 961 x 6144 of 2560 k 54 / 55, 1000 x 6144 62 / 55; 1280 x 6144 of 1024 k 26 / 25)
+        const int64_t there = (M + 127) / 128 * cols;
+        if (group == 64 && there <= 256) return K > 1024 && M % 128 <= 64 && (M + 95) / 96 * cols > 256 ? -1 : best;
+        if ((group == 64 || M > 1024 || there >= 256) && cost(best) > start + rounds(4) * (chunked[kind].tile + chunked[kind].k * k)) return -1;
     }
     return best;
 }

@@ -5,20 +5,25 @@
 // for every 32 cycles of the matrix unit, which is all that LDS delivers to four SIMDs.)  Two workgroups share a CU, and one's
 // barriers, first loads and epilogue run under the other's products: up to 256 registers per lane, 128 of them sums.
 //   * Activations go from global memory straight to LDS (16 bytes per lane, no registers in between), 256 bytes of a row per step
-//     (128 k in 16 bits, 256 k in 8), two buffers: the loads of step t + 1 are issued behind the one barrier of step t.  16-byte
+//     (128 k in 16 bits, 256 k in 8), two buffers.  8 bits: the loads of step t + 1 are issued behind the one barrier of step t.  16 bits:
+//     those of step t + 2 behind the barrier in front of step t's last product, which is held in registers by then (step16).  16-byte
 //     chunk c of row r lies at place c ^ (r & 15): a lane reads its row's chunk, and 16 rows hit 16 places of the 256-byte bank row.
 //   * Weights go from global memory to the registers of the wave that multiplies them (16 bytes per lane and 32-k product), RW
 //     products ahead: a register is loaded again as soon as its weights are widened.  They are widened once for 32 MT rows.
-//   * Per-group sums take a second set of accumulators, so 96 rows are the most there, and weights are loaded 64 k ahead.
+//   * Per-group sums take a second set of accumulators, so 96 rows are the most there, and there weights are loaded 64 k ahead (64 rows
+//     have registers for 128 k: groups of 128, one tile per CU, 0.84 x the time of 64 k).
 //   * Tiles are dealt to the eight dies in contiguous runs of an order that goes through panels of eight row tiles, so that the
 //     tiles a die has at hand form a square and its L2 sees activations and weights several times.
 // The k order of a sum is that of the other tiles: results agree with theirs bit for bit (per-group scales: fused multiply-adds of
 // the same group sums in the same order).
 //
-// Bound by the matrix cores in 16 bits (1.15 to 1.2 PFLOP/s, what a library product of 8192 reaches too), by the vector unit beside
-// them with int8 groups (widening 50 %, folds 25 % of the time), by both and LDS in 8 bits.  4099 rows, Qwen3-4B shapes,
-// microseconds of the 128 x 256 tile with one strip per wave / here (without the waits by position, see load_a): weight-only int8 qkv 158 / 134, o 113 / 84, gate_up 398 / 349,
-// down 223 / 191; groups of 128 178 / 154, 136 / 97, 500 / 405, 269 / 218; fp8 x fp8 106 / 71, 82 / 44, 311 / 180, 158 / 93.
+// Bound by the matrix cores in 16 bits and by the power they take (random operands run at 1.7 to 2.0 GHz of 2.4; 1.15 to 1.25 PFLOP/s, what a
+// library product of 8192 reaches too), by the vector unit beside them with int8 groups, by both and LDS in 8 bits.  4099 rows, Qwen3-4B shapes,
+// microseconds of the 128 x 256 tile with one strip per wave / of this one with every product's weights widened in front of its matrix
+// instructions: weight-only int8 qkv 158 / 134, o 113 / 84, gate_up 398 / 349, down 223 / 191; groups of 128 178 / 154, 136 / 97, 500 / 405,
+// 269 / 218; fp8 x fp8 106 / 71, 82 / 44, 311 / 180, 158 / 93.  With step16, all four and groups of 128: 811, not 859.  256 to 8192 rows of
+// the Qwen3 shapes and others, times the figure before: 96 rows of a tile 0.90 in int8, 0.89 in fp8, 128 rows 0.95 and 0.94, groups of
+// 128 on 64 rows 0.87 (0.64 at best), on 96 rows 0.94; groups of 64 in fp8 on 96 rows that have their CUs to themselves 1.03.
 #pragma once
 #include "ql_gemm_kernel.h"
 
@@ -52,50 +57,57 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
     const int m0 = (int)by * BM, n0 = (int)bx * 256 + wave * 64;
     const int steps = p.K / KS;                               // (host: K % KS == 0)
 
-    // activations: piece i = rows 8 MT wave + 4 i .. + 3 of the tile (rows past M: the last one, never stored)
-    unsigned aoff[NA];
+    // activations: piece i = rows 8 MT wave + 4 i .. + 3 of the tile (rows past M lie behind the resource's end: zeros, never stored)
+    const int arow = 8 * MT * wave + (lane >> 4);
+    // (a row is a multiple of 256 bytes; 8 MT wave is one of 8 rows, so that 4 i only changes bits 2 and 3 of a row's number)
+    unsigned abase = (unsigned)(m0 + arow) * (unsigned)p.K * AB + 16u * (unsigned)((lane & 15) ^ (arow & 15));
+    auto aoff = [&](int i) -> unsigned {
+        return (abase ^ (16u * ((unsigned)((8 * MT * wave + 4 * i) ^ (8 * MT * wave)) & 12u))) + (unsigned)(4 * i) * (unsigned)p.K * AB;
+    };
+    // (8 bits have registers for the places, and are up to 6 % faster with them: 6000 x 4096 of 2048 k in fp8 66 us, not 70)
+    constexpr bool KEPT = ACT != ACT_BF16;
+    unsigned akept[KEPT ? NA : 1];
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-        const int row = 8 * MT * wave + 4 * i + (lane >> 4);
-        aoff[i] = (unsigned)min(m0 + row, p.M - 1) * (unsigned)p.K * AB + 16u * (unsigned)((lane & 15) ^ (row & 15));
-    }
+    for (int i = 0; i < (KEPT ? NA : 0); ++i) akept[i] = aoff(i);
     // (as buffer loads: behind a global load to LDS the compiler lets no load's registers be read before every load has arrived, so the
     // first weights of a step, or the third with groups, waited for activations just asked for.  With waits by position 4099 rows of
     // the Qwen3-4B projections take 857 us with groups of 128, not 914)
     // (the host's pass over a kernel knows no buffer resources)
 #ifdef __HIP_DEVICE_COMPILE__
-    const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, (unsigned)p.M * (unsigned)p.K * AB, 0x00020000);
+    const unsigned xbytes = (unsigned)p.M * (unsigned)p.K * AB;
 #endif
     auto load_a = [&](unsigned char* buf, int t) {
+        if constexpr (!KEPT) asm volatile("" : "+v"(abase));  // (worked out anew at every step, or each would keep its register)
 #ifdef __HIP_DEVICE_COMPILE__
+        // (a step past the last one finds an empty resource: nothing is read)
+        const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, KEPT || t < steps ? xbytes : 0u, 0x00020000);
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lvoid*)(buf + (8 * MT * wave + 4 * i) * 256), 16, aoff[i], t * 256, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lvoid*)(buf + (8 * MT * wave + 4 * i) * 256), 16, KEPT ? akept[i] : aoff(i), t * 256, 0, 0);
 #endif
     };
-    // weights: as in the other tiles (columns past N: the last strip or row, never stored)
+    // weights: as in the other tiles (strips past N: the last one, never stored; N is a multiple of 32).  A lane's place in a strip in a
+    // register, whatever the strip; what is uniform goes into the address
     const unsigned kmul = p.wtiled ? 32u : 1u;
-    unsigned woff[2];
+    unsigned wplace = p.wtiled ? (unsigned)lane * 16u : (unsigned)l31 * (unsigned)p.K + (unsigned)(16 * lh);
+    unsigned col[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int n = n0 + 32 * j;
-        woff[j] = p.wtiled ? min((unsigned)(n >> 5), (unsigned)((p.N + 31) / 32 - 1)) * (unsigned)p.K * 32u + (unsigned)lane * 16u
-                           : (unsigned)min(n + l31, p.N - 1) * (unsigned)p.K + (unsigned)(16 * lh);
-    }
+    for (int j = 0; j < 2; ++j) col[j] = (unsigned)min(n0 + 32 * j, p.N - 32);
+    unsigned wkept[2] = {col[0] * (unsigned)p.K + wplace, col[1] * (unsigned)p.K + wplace};
     auto load_w = [&](int k, int j) -> i32x4 {
-        asm volatile("" : "+v"(woff[j]));
-        return *(const __attribute__((address_space(1))) i32x4*)((gbytes)p.w + (unsigned)k * kmul + woff[j]);
+        if constexpr (KEPT) {
+            asm volatile("" : "+v"(wkept[j]));
+            return *(const __attribute__((address_space(1))) i32x4*)((gbytes)p.w + (unsigned)k * kmul + wkept[j]);
+        }
+        asm volatile("" : "+v"(wplace));
+        return *(const __attribute__((address_space(1))) i32x4*)((gbytes)p.w + (col[j] * (unsigned)p.K + (unsigned)k * kmul) + wplace);
     };
     // a group's scale (group k / group of the lane's columns; 4 N K / group bytes of them, so 32 bits hold an offset)
-    unsigned swoff[2];
-    if constexpr (GROUP) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) swoff[j] = (unsigned)min(n0 + 32 * j + l31, p.N - 1) * (unsigned)(p.K / p.group) * 4u;
-    }
+    unsigned splace = GROUP ? (unsigned)l31 * (unsigned)(p.K / p.group) * 4u : 0u;
     auto load_s = [&](int k, int j) -> float {
-        asm volatile("" : "+v"(swoff[j]));
+        asm volatile("" : "+v"(splace));
         const unsigned g = __umulhi((unsigned)k >> 5, p.gmagic);   // (groups of 64 and more: never 0)
-        return *(const __attribute__((address_space(1))) float*)((gbytes)p.sw + 4u * g + swoff[j]);
+        return *(const __attribute__((address_space(1))) float*)((gbytes)p.sw + 4u * (g + col[j] * (unsigned)(p.K / p.group)) + splace);
     };
 
     acc_t acc[MT][2], accg[GROUP ? MT : 1][2];
@@ -106,9 +118,11 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-    constexpr int RW = GROUP ? 2 : 4;                         // 32-k products that weights are loaded ahead
+    constexpr int RW = GROUP && MT > 2 ? 2 : 4;               // 32-k products that weights are loaded ahead
     i32x4 raw[RW][2];
-    float sc[GROUP ? FS : 1][2];
+    // a group's scales; groups of 64 on 64 rows are over before one group's way from memory: theirs are asked for a step ahead
+    constexpr int SD = GROUP && FG == 2 && MT == 2 ? 2 : 1;
+    float sc[SD][2] = {};
     load_a(buf0, 0);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
@@ -116,21 +130,15 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
     for (int s = 0; s < RW; ++s)
 #pragma unroll
         for (int j = 0; j < 2; ++j) raw[s][j] = load_w(32 * s, j);
-    if constexpr (GROUP) {
-#pragma unroll
-        for (int f = 0; f < FS; ++f)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) sc[f][j] = load_s(32 * FG * f, j);
-    }
     if constexpr (ACT != ACT_BF16) {
         if ((int)threadIdx.x < BM) sxs[threadIdx.x] = p.sx[min(m0 + (int)threadIdx.x, p.M - 1)];
     }
 
-    // the lane's places: chunk 4 s + 2 lh + q (16 bits) or 2 s + lh (8 bits) of its row in a fragment
+    // the lane's places, 8 bits: chunk 2 s + lh of its row in a fragment
     unsigned place[8];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const int chunk = ACT == ACT_BF16 ? 4 * (c >> 1) + 2 * lh + (c & 1) : 2 * c + lh;
+    for (int c = 0; c < (ACT == ACT_BF16 ? 0 : 8); ++c) {
+        const int chunk = 2 * c + lh;
         place[c] = (unsigned)(l31 * 256 + 16 * (chunk ^ (l31 & 15)));
         asm volatile("" : "+v"(place[c]));                    // (one register each, whatever the buffer and the fragment)
     }
@@ -153,71 +161,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
         const int kn = tn * KS;
         // the weights of the product RW behind product s of this step
         auto next_w = [&](int s, int j) -> i32x4 { return load_w(s + RW < SUB ? t * KS + 32 * (s + RW) : kn + 32 * (s + RW - SUB), j); };
-        if constexpr (ACT == ACT_BF16) {
-            if constexpr (GROUP) {
-#pragma unroll
-                for (int s = 0; s < SUB; ++s) {
-                    const int f = s / FG;
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        bf16x8 b[2];
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) {
-                            b[j] = widen8<FP8W>(raw[s % RW][j][2 * q], raw[s % RW][j][2 * q + 1]);
-                            if (q == 1) raw[s % RW][j] = next_w(s, j);
-                        }
-#pragma unroll
-                        for (int i = 0; i < MT; ++i) {
-                            const bf16x8 a = *(const bf16x8*)(cur + i * 8192 + place[2 * s + q]);
-#pragma unroll
-                            for (int j = 0; j < 2; ++j) {
-                                if (s % FG == 0 && q == 0) accg[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j], f32x16{}, 0, 0, 0);
-                                else accg[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j], accg[i][j], 0, 0, 0);
-                            }
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                    if (s % FG == FG - 1) {
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) {
-                            const float g = sc[f][j];
-                            sc[f][j] = load_s(kn + 32 * FG * f, j);
-#pragma unroll
-                            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                                for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(accg[i][j][r], g, acc[i][j][r]);
-#pragma unroll
-                            for (int i = 0; i < MT; ++i) asm volatile("" : "+v"(acc[i][j]));
-                        }
-                    }
-                }
-            } else {
-                bf16x8 b[2][2][2];
-                auto widen = [&](bf16x8 (&o)[2][2], int s) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const i32x4 w = raw[s][j];
-                        raw[s][j] = next_w(s, j);
-                        o[j][0] = widen8<FP8W>(w[0], w[1]);
-                        o[j][1] = widen8<FP8W>(w[2], w[3]);
-                    }
-                };
-                widen(b[0], 0);
-#pragma unroll
-                for (int s = 0; s < SUB; ++s) {
-                    if (s + 1 < SUB) widen(b[(s + 1) & 1], s + 1);
-#pragma unroll
-                    for (int i = 0; i < MT; ++i)
-#pragma unroll
-                        for (int q = 0; q < 2; ++q) {
-                            const bf16x8 a = *(const bf16x8*)(cur + i * 8192 + place[2 * s + q]);
-#pragma unroll
-                            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[s & 1][j][q], acc[i][j], 0, 0, 0);
-                        }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-        } else if constexpr (INT) {
+        if constexpr (INT) {
 #pragma unroll
             for (int s = 0; s < SUB; ++s) {
                 i32x4 w[2];
@@ -260,14 +204,135 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    __builtin_amdgcn_s_waitcnt(0x0F70);                       // vmcnt(0): fewer loads than AFTER follow the first activations
+    // 16 bits: a step is 2 SUB products of 16 k, 2 MT matrix instructions each; between them the widening of the next product's weights and
+    // the reads of its activations, each into the registers that the last of them has left, so that one wave of a SIMD keeps the matrix unit
+    // as busy as two (a wave issues up to five vector instructions in the 32 cycles of a matrix one; with all of a product's in front of its
+    // matrix instructions, two waves took the time of both units added up).  In front of a step's last product its activations are all
+    // read: the barrier stands there, behind it the next step's are in LDS and read, and those of the step after next take their place.
+    bf16x8 ga[MT], gb[2][2];
+    auto step16 = [&](unsigned char* cur, unsigned char* nxt, int t) __attribute__((always_inline)) {
+        const int kn = min(t + 1, steps - 1) * KS;
+        auto next_w = [&](int s, int j) -> i32x4 { return load_w(s + RW < SUB ? t * KS + 32 * (s + RW) : kn + 32 * (s + RW - SUB), j); };
+        int tid = threadIdx.x;                                // (worked out anew, as the activations' places: registers are short)
+        asm volatile("" : "+v"(tid));
+        // (chunk 4 s + 2 lh + q of the row lies at `at` ^ 16 (4 s + q))
+        const unsigned at = (unsigned)((tid & 31) * 256 + 16 * ((tid >> 4 & 2) ^ (tid & 15)));
+#pragma unroll
+        for (int p = 0; p < 2 * SUB; ++p) {
+            const int s = p >> 1, q = p & 1, pn = (p + 1) % (2 * SUB), sn = pn >> 1;
+            const bool last = p == 2 * SUB - 1, fold = GROUP && p % (2 * (FG + !FG)) == 0;
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            if (last) {                                       // vmcnt(AFTER) lgkmcnt(0), as below
+                __builtin_amdgcn_s_waitcnt(0x0070 | (AFTER & 15) | (AFTER >> 4) << 14);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                load_a(cur, t + 2);
+            }
+            const unsigned char* from = last ? nxt : cur;
+            const unsigned next = at ^ (64u * (pn >> 1) + 16u * (pn & 1));
+            float g[2] = {0.f, 0.f};
+            if constexpr (GROUP) {
+                if (fold) {                                   // the group in front of this one
+                    const int slot = SD == 2 && p == 0 ? 1 : 0;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        g[j] = p > 0 || t > 0 ? sc[slot][j] : 0.f;
+                        sc[slot][j] = load_s(SD == 1 ? t * KS + 32 * s : p == 0 ? t * KS + 32 * FG : kn, j);   // (this one's, for the next fold)
+                        if (MT == 2) continue;                // (its folds stand between the products)
+#pragma unroll
+                        for (int i = 0; i < MT; ++i)
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(accg[i][j][r], g[j], acc[i][j][r]);
+#pragma unroll
+                        for (int i = 0; i < MT; ++i) asm volatile("" : "+v"(acc[i][j]));
+                    }
+                    if (MT != 2) __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if constexpr (GROUP) {
+                        if (fold && MT == 2) {
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(accg[i][j][r], g[j], acc[i][j][r]);
+                            asm volatile("" : "+v"(acc[i][j]));
+                        }
+                        if (fold) accg[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga[i], gb[q][j], f32x16{}, 0, 0, 0);
+                        else accg[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga[i], gb[q][j], accg[i][j], 0, 0, 0);
+                    } else {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga[i], gb[q][j], acc[i][j], 0, 0, 0);
+                    }
+                }
+                ga[i] = *(const bf16x8*)(from + i * 8192 + next);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                gb[q ^ 1][j] = widen8<FP8W>(raw[sn % RW][j][2 * (q ^ 1)], raw[sn % RW][j][2 * (q ^ 1) + 1]);
+                if (q == 0) raw[s % RW][j] = next_w(s, j);
+            }
+            constexpr int V = ((FP8W ? 8 : 24) + 2 * MT) / (2 * MT);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (fold && MT == 2) __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, V, 0);
+                    if (j == 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    if (last) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                }
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (ACT == ACT_BF16) {
+        if constexpr (SD == 2)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) sc[0][j] = load_s(0, j);
+        load_a(buf1, 1);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0F70 | NA);              // vmcnt(NA): the first step's activations, and the weights
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if constexpr (GROUP) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) accg[i][j][r] = 0;
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) gb[0][j] = widen8<FP8W>(raw[0][j][0], raw[0][j][1]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) ga[i] = *(const bf16x8*)(buf0 + i * 8192 + l31 * 256 + 16 * ((2 * lh) ^ (l31 & 15)));
+    } else {
+        __builtin_amdgcn_s_waitcnt(0x0F70);                   // vmcnt(0): fewer loads than AFTER follow the first activations
+    }
     {
+        auto one = [&](unsigned char* cur, unsigned char* nxt, int t) __attribute__((always_inline)) {
+            if constexpr (ACT == ACT_BF16) step16(cur, nxt, t);
+            else step(cur, nxt, t);
+        };
         int t = 0;
         for (; t + 1 < steps; t += 2) {
-            step(buf0, buf1, t);
-            step(buf1, buf0, t + 1);
+            one(buf0, buf1, t);
+            one(buf1, buf0, t + 1);
         }
-        if (t < steps) step(buf0, buf1, t);
+        if (t < steps) one(buf0, buf1, t);
+    }
+    if constexpr (GROUP) {                                    // the last group
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][j][r] = __builtin_fmaf(accg[i][j][r], sc[SD - 1][j], acc[i][j][r]);
     }
 
     // ---- epilogue: scales, bias, one rounding; the tile as bf16 through LDS (rows of the first half in buf0, the others in buf1; a

@@ -51,6 +51,22 @@ def test_what_the_cost_rule_refuses_goes_to_the_tile_it_compared_with(no_table, 
     assert wide(p) or p == (4, 8, 1, 2, 1)
 
 
+@pytest.mark.parametrize("dtype", [I8, F8])
+@pytest.mark.parametrize("M,N,K,there", [(1792, 4096, 4096, True), (1024, 6144, 2560, True), (1088, 6144, 2560, True), (1089, 6144, 2560, False),
+                                         (1000, 6144, 2560, False), (1280, 6144, 1024, False), (900, 6144, 2560, False), (960, 4096, 4096, False)])
+def test_one_round_of_128_row_tiles_with_groups_of_64(no_table, dtype, M, N, K, there):
+    """Taken where two rounds of the prefill tile stand against it and its last row tile is whole, or at most half full."""
+    p = Q.plan_query(G, M, N, K, dtype, 64)
+    assert (p == (4, 8, 1, 2, 1)) == there and (there or wide(p))
+
+
+@pytest.mark.parametrize("form,group", [(0, 0), (G, 64), (G, 128)])
+@pytest.mark.parametrize("M,N,K,mt", [(4500, 1024, 512, 3), (9000, 1024, 512, 3), (4500, 2048, 768, 3), (3300, 1024, 512, 2), (16000, 480, 640, 2)])
+def test_fewer_rounds_of_taller_tiles_over_short_k(no_table, form, group, M, N, K, mt):
+    p = Q.plan_query(form, M, N, K, I8, group)
+    assert wide(p) and (p[0] >= mt if not group else p[0] == mt)
+
+
 MID, MID64 = (1, 2, 4, 4), (2, 2, 4, 4)
 
 
