@@ -45,12 +45,15 @@ template <int MODE, bool FEW>
 __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                           const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                           unsigned short* __restrict__ out, int tiles, int top, unsigned top_inv, int N, int K, float limit,
-                                                          float alpha, int act_kind, const float* __restrict__ in_wts) {
+                                                          float alpha, int act_kind, const float* __restrict__ in_wts, bool by_die) {
     constexpr bool GATE_UP = MODE == 1, FROM_TOKENS = MODE != 0;
-    // Workgroups go to the eight dies in turn: a die has every eighth column block, and its tiles one behind the other, so that the tiles of
-    // one expert meet its weights in one L2 (us of whole calls, tiles on neighbouring dies / here, weights not in a cache: 40 rows for each of
-    // 4 experts of 2048 x 4096 87 / 77, of 16 of 2048 x 1536 110 / 86, of one of 4096 x 11008 104 / 87; one tile per expert alike).
-    const int id = blockIdx.x >> 3, tile = id % tiles, n0 = ((id / tiles) * 8 + (blockIdx.x & 7)) * 32;
+    // Workgroups go to the eight dies in turn.  By die: a die has every eighth column block, and its tiles one behind the other, so that the
+    // tiles of one expert meet its weights in one L2 (us of whole calls, tiles on neighbouring dies / here, weights not in a cache: 40 rows
+    // for each of 4 experts of 2048 x 4096 87 / 77, of 16 of 2048 x 1536 110 / 86, of one of 4096 x 11008 104 / 87; one tile per expert alike).
+    // Up to 8 tokens no expert has a second tile, and what counts is how the few that are read lie in memory: 4 tokens, 16 experts of
+    // 2048 x 1536 68 / 63, 32 of them 79 / 91, 64 115 / 105, one token 51 / 63 and 58 / 65.  Those go by tiles.
+    const int id = blockIdx.x >> 3, tile = by_die ? id % tiles : (int)blockIdx.x % tiles;
+    const int n0 = (by_die ? (id / tiles) * 8 + (int)(blockIdx.x & 7) : (int)blockIdx.x / tiles) * 32;
     if (n0 >= N) return;
     const int lane = threadIdx.x, l31 = lane & 31, hi = lane >> 5;
     // The tile's rows come 128 bytes at a time, eight lanes to a row, and go through LDS to the lanes that multiply them (chunk c
@@ -236,7 +239,7 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
 #define SM_GROUPED(MODE_, FEW_)                                                                                                          \
     hipLaunchKernelGGL((moe_grouped_kernel<MODE_, FEW_>), grid(F), dim3(64), 0, s,                                                     \
                        (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, tiles, top, top_inv, \
-                       F, W, limit, alpha, act_kind, weight_in ? wts : nullptr)
+                       F, W, limit, alpha, act_kind, weight_in ? wts : nullptr, T > 8)
     if (act_is_gated(act_kind)) {
         if (few) SM_GROUPED(1, true); else SM_GROUPED(1, false);
     } else {
@@ -246,7 +249,7 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     SM_CHECK_LAUNCH("sm_moe_grouped (gate/up)");
     hipLaunchKernelGGL((moe_grouped_kernel<0, false>), grid(W), dim3(64), 0, s,
                        (const unsigned short*)act, (const unsigned short*)w_down, row_pair, tile_expert, (unsigned short*)prod, tiles, top, top_inv, W,
-                       F, 0.f, 0.f, 0, (const float*)nullptr);
+                       F, 0.f, 0.f, 0, (const float*)nullptr, T > 8);
     SM_CHECK_LAUNCH("sm_moe_grouped (down)");
     if (y == nullptr) return SM_OK;               // the caller sums a token's pairs itself
     return sm_moe_combine(prod, pair_row, weight_in ? nullptr : wts, shared, shared_scale, y, T, top, W, stream);
