@@ -24,11 +24,15 @@
 // same strengths, and give each other half of the results' rows at the next meeting, so that both have the same work.
 //
 // Against the walk that takes token after token, bound by the float32 vector unit and its chain of lane sums at two waves per
-// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 29 (prepare) + 143 (walk), 4 us per chunk at one wave
-// per SIMD: 1 us of vector work (the splits), 0.8 us of matrix work, the rest their chain K S -> R -> W -> S and its waits.  Four
-// waves of 32 keys: 195 us (the strengths worked out four times); results all in one wave, v read from global memory: 175 us.
+// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 29 (prepare) + 117 (walk), 3.1 us per chunk at one wave
+// per SIMD: 800 vector instructions, five cycles each (a third of them the splits), 0.8 us of matrix work, the rest their chain K S -> R -> W -> S
+// and its waits.  The walk took 143 with numbers split one at a time (each rounded once more to be packed), the waves' halves of the results chosen
+// element by element (through indexed moves) and the products' results in the accumulation registers (a copy for every number read).
+// Four waves of 32 keys: 195 us (the strengths worked out four times); results all in one wave, v read from global memory: 175 us.
 #include "hm_attn_tile.h"
 #include "hm_outer.h"
+
+#include <type_traits>
 
 namespace hm {
 
@@ -46,17 +50,23 @@ __device__ __forceinline__ size_t prepared_at(int q0, int b, int chunk, int h, i
 struct Terms { bf16x8 v[3]; };              // x = v[0] + v[1] + v[2], exactly
 
 __device__ __forceinline__ Terms split8(const float* x) {
-    Terms t;
+    // (two at a time: one conversion rounds and packs both; element by element the compiler rounds every number once more to pack it)
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 t[3];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const bf16_t a = (bf16_t)x[e];
-        const float ra = x[e] - (float)a;
-        const bf16_t b = (bf16_t)ra;
-        t.v[0][e] = a;
-        t.v[1][e] = b;
-        t.v[2][e] = (bf16_t)(ra - (float)b);
+    for (int e = 0; e < 4; ++e) {
+        float a = x[2 * e], b = x[2 * e + 1];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+            t[j][e] = u;
+            a -= __builtin_bit_cast(float, u << 16);
+            b -= __builtin_bit_cast(float, u & 0xFFFF0000u);
+        }
     }
-    return t;
+    return {__builtin_bit_cast(bf16x8, t[0]), __builtin_bit_cast(bf16x8, t[1]), __builtin_bit_cast(bf16x8, t[2])};
 }
 
 // big += a b of the leading terms, small += the five products down to 2^-24 of it: the large sums take few roundings
@@ -191,6 +201,8 @@ __device__ __forceinline__ int first_spoiled(float* x, int hi) {
     if (!__any(!(z == 0.f))) return kChunk;
     int first = kChunk;
 #pragma unroll
+    for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(x[r]));      // (or the comparisons are made in front of the branch)
+#pragma unroll
     for (int r = 15; r >= 0; --r)
         if (!(fabsf(x[r]) <= 3.402823466e38f)) {
             x[r] = 0.f;
@@ -302,6 +314,7 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
                 *(i32x4*)(buf + i) = i32x4{0, 0, 0, 0};
                 *(i32x4*)(buf + ROWS + i) = i32x4{0, 0, 0, 0};
             }
+            for (int i = left * 64 + 16 * (int)threadIdx.x; i < kChunk * 64; i += 2048) *(i32x4*)(buf + VAT + i) = i32x4{0, 0, 0, 0};
             meet();
         }
         const unsigned char* prep = buf + PREP;
@@ -339,7 +352,7 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
             const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 (s16x4 __attribute__((address_space(3)))*)(buf + VAT + v_at + 512 * r4));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * r4 + e] = e + 8 * r4 + 4 * hi < left ? to_f(__builtin_bit_cast(bf16_t, (short)x[e])) : 0.f;
+            for (int e = 0; e < 4; ++e) v[4 * r4 + e] = to_f(__builtin_bit_cast(bf16_t, (short)x[e]));
         }
         float w[16], wd[16], cq[16];
 #pragma unroll
@@ -375,10 +388,12 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) w[r] = big[r] + small[r];
-            if (first < kChunk)
+            if (__any(first < kChunk))
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
+                for (int r = 0; r < 16; ++r) {
+                    asm volatile("" : "+v"(w[r]));
                     if ((r & 3) + 8 * (r >> 2) + 4 * hi >= first) w[r] = __builtin_nanf("");
+                }
         }
         const float end = *(const float*)(prep + kEndAt);
 #pragma unroll
@@ -403,34 +418,37 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
             }
         }
         {                                                     // P W of the wave's half of the strengths, and the parts of the results
-            f32x16 big = zeros(), small = zeros();
-            float x[8];
-            bf16x8 m[3];
             const int first = first_spoiled(w, hi);
-            if (first < kChunk)
+            if (__any(first < kChunk))
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
+                for (int r = 0; r < 16; ++r) {
+                    asm volatile("" : "+v"(cq[r]));
                     if ((r & 3) + 8 * (r >> 2) + 4 * hi >= first) cq[r] = __builtin_nanf("");
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = wave ? w[8 + e] : w[e];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) m[j] = *(const bf16x8*)(prep + j * kTermBytes + wave * 1024 + 16 * lane);
-            mul_terms(m, split8(x), big, small);
-#pragma unroll
-            for (int r4 = 0; r4 < 2; ++r4) {
-                f32x4 y;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = 4 * r4 + e;
-                    const int g = 8 + r;                      // given to the other wave if this is the first, kept if it is the second
-                    y[e] = wave ? cq[r] * (qsb[r] + qss[r]) + (big[r] + small[r]) : cq[g] * (qsb[g] + qss[g]) + (big[g] + small[g]);
-                    const double c = wave ? cq[g] : cq[r], qb = wave ? qsb[g] : qsb[r], qs = wave ? qss[g] : qss[r],
-                                pb = wave ? big[g] : big[r], ps = wave ? small[g] : small[r];
-                    part[r] = c * (qb + qs) + (pb + ps);
-                    if (!DELTA) part[r] += (double)skip * (double)(wave ? v[g] : v[r]);
                 }
-                swap_o[DELTA ? 0 : turn][wave ^ 1][r4][lane] = y;
-            }
+            // (one form per wave: chosen element by element, the halves go through indexed register moves)
+            auto results = [&](auto second) __attribute__((always_inline)) {
+                constexpr int KEPT = second ? 8 : 0, GIVEN = 8 - KEPT;
+                f32x16 big = zeros(), small = zeros();
+                bf16x8 m[3];
+#pragma unroll
+                for (int j = 0; j < 3; ++j) m[j] = *(const bf16x8*)(prep + j * kTermBytes + (KEPT / 8) * 1024 + 16 * lane);
+                mul_terms(m, split8(w + KEPT), big, small);
+#pragma unroll
+                for (int r4 = 0; r4 < 2; ++r4) {
+                    f32x4 y;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int r = 4 * r4 + e, g = GIVEN + r, k = KEPT + r;
+                        y[e] = cq[g] * (qsb[g] + qss[g]) + (big[g] + small[g]);
+                        const double c = cq[k], qb = qsb[k], qs = qss[k], pb = big[k], ps = small[k];
+                        part[r] = c * (qb + qs) + (pb + ps);
+                        if (!DELTA) part[r] += (double)skip * (double)v[k];
+                    }
+                    swap_o[DELTA ? 0 : turn][wave ^ 1][r4][lane] = y;
+                }
+            };
+            if (wave) results(std::true_type{});
+            else results(std::false_type{});
         }
 #pragma unroll
         for (int blk = 0; blk < NB; ++blk)
