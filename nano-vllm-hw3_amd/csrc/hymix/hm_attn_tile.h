@@ -61,6 +61,19 @@ __device__ __forceinline__ TileWalk<TK> make_walk(int min_pos, int max_pos, int 
     return w;
 }
 
+// The mask of a tile of 32 PARTS keys, counted from a lane's first: a row sees the last `near` keys up to its own, key `ahead`, and those up to
+// `kept`.  Without && and ||: with them the compiler branches lane by lane, 626 instructions per tile of 64.
+template <int PARTS>
+__device__ __forceinline__ void mask_tile(f32x16 (&s)[PARTS], int ahead, int near, int kept) {
+#pragma unroll
+    for (int j = 0; j < PARTS; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int c = 32 * j + (r & 3) + 8 * (r >> 2);
+            s[j][r] = ((unsigned)ahead - (unsigned)c < (unsigned)near) | (c <= kept) ? s[j][r] : -INFINITY;
+        }
+}
+
 // Walks tiles [vt_lo, vt_hi) of `walk` for the calling lane's query row at position row_pos; wave_min_pos / wave_max_pos = the
 // smallest / largest position of the wave's rows.  Every wave of the workgroup must call this with the same tiles.  On return oacc holds the
 // unnormalised output (lane: query l & 31, columns 32 d + 8 (r >> 2) + 4 (l >> 5) + (r & 3)), m_run the row maximum of
@@ -162,6 +175,8 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
 
     const int my_pool = pooled_seen(row_pos, window, pool);   // pooled entries this row sees
     const int chunk_lo = chunk > 0 ? row_pos / chunk * chunk : 0;
+    const int near = window > 0 ? min(window, row_pos + 1 - chunk_lo) : row_pos + 1 - chunk_lo,
+              kept = window > 0 ? min(keep_first - 1, row_pos) : -1;    // (the last of the kept ones that the row sees)
     const int wave_chunk_lo = chunk > 0 ? wave_max_pos / chunk * chunk : 0;
     load_tile(vt_lo);
     store_tile();
@@ -208,15 +223,7 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
                 }
         } else if (kt0 + kTileKeys - 1 > wave_min_pos || (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo) {
             // (a tile that every row of the wave sees whole needs no mask)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi;
-                    const bool seen = key <= row_pos && key >= chunk_lo &&
-                                      (window <= 0 || row_pos - key < window || key < keep_first);
-                    if (!seen) s[j][r] = -INFINITY;
-                }
+            mask_tile(s, row_pos - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
         }
         bf16x8 pf[2][2];
         if (SIG) {
@@ -287,9 +294,10 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
 
 // The same walk for head sizes of exactly 32 NBK and 32 NBV channels, whose tiles go from global memory straight to LDS: two
 // buffers, one barrier per tile.  The loop above holds a tile in registers on its way (a wave then has 350 of them and its SIMD
-// to itself, with nothing to fill its waits; held to 256 it takes 110 us where this one takes 83 and the first took 174: eight
+// to itself, with nothing to fill its waits; held to 256 it takes 110 us where this one takes 73 and the first took 174: eight
 // prompts of about 1000 tokens, 16 / 8 heads of 128, a window of 512, capped scores).  What is left is the vector unit's:
-// three exponentials or reciprocals per capped score.  Tiles of 32 keys, which fit three waves, measured the same.
+// three exponentials or reciprocals per capped score.  (82 us with masks that branched lane by lane, two tiles of ten, and with every
+// piece's address worked out at every tile, 130 of a tile's 530 vector instructions.)  Tiles of 32 keys, which fit three waves, measured the same.
 // A row of 2 P bytes is kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows
 // that differ mod 16, one chunk) and the 32 of a transposed read (four rows, four chunks) then touch every bank once.  A
 // wave none of whose rows sees a tile leaves it out: a masked score would add an exact zero.
@@ -324,15 +332,30 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
 #pragma unroll
     for (int ks = 0; ks < 2 * NBK; ++ks) qf[ks] = *(const bf16x8*)(qrow + 16 * ks + 8 * hi);
 
-    // one tile: pieces of 1 KB, dealt to the four waves; lane l of a piece brings the chunk that belongs at 16 l
-    auto load_part = [&](auto geom, unsigned char* to, const unsigned short* src, const unsigned short* psrc, int vt, int kt0, size_t row0) {
+    // one tile: pieces of 1 KB, dealt to the four waves; lane l of a piece brings the chunk that belongs at 16 l.  A lane's pieces are a
+    // whole number of 16 rows apart, so its chunk is the same in all of them, and its place in a whole tile is one number.
+    auto lane_row = [&](auto geom) { return wave * (64 / decltype(geom)::CH) + lane / decltype(geom)::CH; };
+    auto lane_chunk = [&](auto geom) { return (lane % decltype(geom)::CH) ^ decltype(geom)::swz(lane_row(geom)); };
+    const unsigned k_place = 2u * ((unsigned)lane_row(GK()) * (unsigned)(G * GK::P) + 8u * (unsigned)lane_chunk(GK())),
+                   v_place = 2u * ((unsigned)lane_row(GV()) * (unsigned)(G * GV::P) + 8u * (unsigned)lane_chunk(GV()));
+    auto load_part = [&](auto geom, unsigned char* to, const unsigned short* src, const unsigned short* psrc, int vt, int kt0, size_t row0,
+                         unsigned place) {
         typedef decltype(geom) GG;
-        constexpr int LPR = GG::CH;                        // lanes per row
+        constexpr int RP = 64 / GG::CH;                    // rows of a piece
+        static_assert(64 % GG::CH == 0 && 4 * RP % 16 == 0 && GG::PIECES % 4 == 0, "pieces of whole rows");
+        typedef __attribute__((address_space(1))) const unsigned char* gbytes;
+        if (vt >= walk.pool_tiles && kt0 + kSlimKeys <= n_keys) {
+            const gbytes from = (gbytes)(src + (row0 * G + g) * GG::P);
+#pragma unroll
+            for (int i0 = 0; i0 < GG::PIECES; i0 += 4)
+                __builtin_amdgcn_global_load_lds((gvoid*)(from + (size_t)(i0 * RP) * (size_t)(2 * G * GG::P) + place),
+                                                 (lvoid*)(to + 1024 * (i0 + wave)), 16, 0, 0);
+            return;
+        }
+        const int ch = lane_chunk(geom);
 #pragma unroll
         for (int i0 = 0; i0 < GG::PIECES; i0 += 4) {
-            const int i = i0 + wave;
-            if (GG::PIECES < 4 && i >= GG::PIECES) break;
-            const int row = i * (64 / LPR) + lane / LPR, ch = (lane % LPR) ^ GG::swz(row);
+            const int row = lane_row(geom) + i0 * RP;
             const unsigned short* from;
             if (vt < walk.pool_tiles) {                    // pooled entries, each found through the block table
                 const int e = min(vt * kSlimKeys + row, walk.n_pool - 1);
@@ -340,7 +363,7 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
             } else {
                 from = src + ((row0 + min(row, n_keys - 1 - kt0)) * G + g) * GG::P;
             }
-            __builtin_amdgcn_global_load_lds((gvoid*)(from + 8 * ch), (lvoid*)(to + 1024 * i), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gvoid*)(from + 8 * ch), (lvoid*)(to + 1024 * (i0 + wave)), 16, 0, 0);
         }
     };
     auto load_tile = [&](unsigned char* buf, int vt) {
@@ -351,8 +374,8 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
             const int page = kt0 / block_size;
             row0 = (size_t)table[page] * block_size + (kt0 - page * block_size);
         }
-        load_part(GK(), buf, kc, kp, vt, kt0, row0);
-        load_part(GV(), buf + GK::BYTES, vc, vp, vt, kt0, row0);
+        load_part(GK(), buf, kc, kp, vt, kt0, row0, k_place);
+        load_part(GV(), buf + GK::BYTES, vc, vp, vt, kt0, row0, v_place);
     };
     auto landed = [&]() {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
@@ -371,6 +394,8 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
               v_at8 = GV::at(4 * hi + tq + 8, 2 * gq + (tp >> 1)) + 8 * (tp & 1);
     const int my_pool = pooled_seen(row_pos, window, pool);
     const int chunk_lo = chunk > 0 ? row_pos / chunk * chunk : 0;
+    const int near = window > 0 ? min(window, row_pos + 1 - chunk_lo) : row_pos + 1 - chunk_lo,
+              kept = window > 0 ? min(keep_first - 1, row_pos) : -1;    // (the last of the kept ones that the row sees)
     const int wave_chunk_lo = chunk > 0 ? wave_max_pos / chunk * chunk : 0, wave_chunk_first = chunk > 0 ? wave_min_pos / chunk * chunk : 0;
 
     auto work = [&](const unsigned char* buf, int vt) {
@@ -409,14 +434,7 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
                     if (kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi >= my_pool) s[j][r] = -INFINITY;
         } else if (kt1 > wave_min_pos || (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo) {
             // (a tile that every row of the wave sees whole needs no mask)
-#pragma unroll
-            for (int j = 0; j < kSlimParts; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi;
-                    const bool seen = key <= row_pos && key >= chunk_lo && (window <= 0 || row_pos - key < window || key < keep_first);
-                    if (!seen) s[j][r] = -INFINITY;
-                }
+            mask_tile(s, row_pos - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
         }
         bf16x8 pf[2 * kSlimParts];
         if (SIG) {

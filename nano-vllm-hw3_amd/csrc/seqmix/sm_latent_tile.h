@@ -33,6 +33,9 @@ struct TileGeom {
     static constexpr int RP = 32 * NB, CH = RP / 8, RS = RP * 2 + 16, LDS_BYTES = kTileKeys * RS;
 };
 
+// Whether a row at row_pos sees a key: the last `near` keys up to its own.  One comparison: with two and a || the compiler branches lane by lane.
+__device__ __forceinline__ bool visible(int key, int row_pos, int near) { return (unsigned)row_pos - (unsigned)key < (unsigned)near; }
+
 // Walks keys [k_lo, k_hi) (k_lo % 64 == 0, k_lo < k_hi) for the calling lane's query row, whose last visible key is
 // row_pos; wave_min_pos = the smallest row_pos of the wave (tiles wholly below it skip the mask).  Every wave of the
 // workgroup must call this with the same key range.  On return oacc holds the unnormalised output (lane: query
@@ -85,6 +88,7 @@ __device__ __forceinline__ void latent_tile_loop(const unsigned short* __restric
         for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
     m_run = -INFINITY;
     float l_run = 0.f;
+    const int near = window > 0 ? min(window, row_pos + 1) : row_pos + 1;
     const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;      // transposed-read address pieces
 
     load_tile(k_lo);
@@ -113,7 +117,7 @@ __device__ __forceinline__ void latent_tile_loop(const unsigned short* __restric
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int key = kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi;
-                    if (key > row_pos || (window > 0 && row_pos - key >= window)) s[j][r] = -INFINITY;
+                    s[j][r] = visible(key, row_pos, near) ? s[j][r] : -INFINITY;
                 }
         }
         float mx = s[0][0];
@@ -205,17 +209,31 @@ __device__ __forceinline__ void latent_slim_loop(const unsigned short* __restric
 #pragma unroll
     for (int ks = 0; ks < 2 * NB; ++ks) qf[ks] = *(const bf16x8*)(qrow + 16 * ks + 8 * hi);
 
-    // one tile: pieces of 1 KB, dealt to the waves; lane l of a piece brings the chunk that belongs at 16 l
+    // one tile: pieces of 1 KB, dealt to the waves; lane l of a piece brings the chunk that belongs at 16 l.  A lane's places in a whole tile
+    // are numbers worked out once
+    constexpr int NP = (G::PIECES + WAVES - 1) / WAVES;
+    unsigned place[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int c = 64 * (p * WAVES + wave) + lane, row = c / G::CH;
+        place[p] = (unsigned)(2 * row * G::P + 16 * ((c % G::CH) ^ G::swz(row)));
+    }
     auto load_tile = [&](unsigned char* buf, int kt0) {
         const int page = __builtin_amdgcn_readfirstlane(kt0 / block_size);             // (a tile lies in one cache block)
         const size_t row0 = (size_t)table[page] * block_size + (kt0 - page * block_size);
+        typedef __attribute__((address_space(1))) const unsigned char* gbytes;
+        const gbytes from = (gbytes)(cache + row0 * G::P);
+        const bool whole = kt0 + kSlimKeys <= k_hi;
 #pragma unroll
-        for (int i0 = 0; i0 < G::PIECES; i0 += WAVES) {
-            const int i = i0 + wave;
+        for (int p = 0; p < NP; ++p) {
+            const int i = p * WAVES + wave;
             if (G::PIECES % WAVES != 0 && i >= G::PIECES) break;
-            const int c = 64 * i + lane, row = c / G::CH, ch = (c % G::CH) ^ G::swz(row);
-            __builtin_amdgcn_global_load_lds((gvoid*)(cache + (row0 + min(row, k_hi - 1 - kt0)) * G::P + 8 * ch), (lvoid*)(buf + 1024 * i),
-                                             16, 0, 0);
+            unsigned at = place[p];
+            if (!whole) {                                  // (rows past the end: the last one's)
+                const int row = (int)(at / (unsigned)(2 * G::P));
+                at -= (unsigned)(row - min(row, k_hi - 1 - kt0)) * (unsigned)(2 * G::P);
+            }
+            __builtin_amdgcn_global_load_lds((gvoid*)(from + at), (lvoid*)(buf + 1024 * i), 16, 0, 0);
         }
     };
     auto landed = [&]() {
@@ -229,6 +247,7 @@ __device__ __forceinline__ void latent_slim_loop(const unsigned short* __restric
         for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
     m_run = -INFINITY;
     float l_run = 0.f;
+    const int near = window > 0 ? min(window, row_pos + 1) : row_pos + 1;
     const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;      // transposed-read address pieces
     // Where the chunk's bits that an address steps through are none that the row changes by addition, the reads' addresses are one
     // base each, changed by exclusive or.
@@ -251,7 +270,7 @@ __device__ __forceinline__ void latent_slim_loop(const unsigned short* __restric
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = kt0 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-                if (key > row_pos || (window > 0 && row_pos - key >= window)) s[r] = -INFINITY;
+                s[r] = visible(key, row_pos, near) ? s[r] : -INFINITY;
             }
         }
         float mx = s[0];
