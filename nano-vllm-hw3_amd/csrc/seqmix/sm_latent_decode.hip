@@ -76,32 +76,59 @@ __global__ __launch_bounds__(64 * WAVES) void latent_decode_merge_kernel(const f
     typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
     const size_t row = blockIdx.x;                          // b * H + h
     const size_t b = row / H, h = row % H;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const float* first = ws + (b * splits * H + h) * stride;
     const size_t step = (size_t)H * stride;
     // (an empty split has sum 0 and outputs that nobody wrote: it counts for nothing)
-    float M = -INFINITY, L = 0.f;
-    for (int s = lane; s < splits; s += 64) {
-        const f32x2 ml = *(const f32x2*)(first + s * step);
-        if (ml.y > 0.f) M = fmaxf(M, ml.x);
+    // A wave's first splits of the first two column blocks are asked for in front of the maximum, which they do not wait for: with one
+    // round of loads behind another the kernel took 6.9 us of 20.6 (64 sequences of 16 heads, 11 splits of 192 columns), so 4.5.
+    constexpr int U = WAVES == 1 ? 6 : 4;
+    const f32x2 ml = lane < splits ? *(const f32x2*)(first + lane * step) : f32x2{-INFINITY, 0.f};
+    f32x2 ahead[2][U];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            ahead[k][u] = *(const f32x2*)(first + min(wave + u * WAVES, splits - 1) * step + 2 + min(128 * k + 2 * lane, R - 2));
+    __builtin_amdgcn_sched_barrier(0);
+    float M = ml.y > 0.f ? ml.x : -INFINITY;
+    for (int s = lane + 64; s < splits; s += 64) {
+        const f32x2 more = *(const f32x2*)(first + s * step);
+        if (more.y > 0.f) M = fmaxf(M, more.x);
     }
     M = wave_max(M);
-    for (int s = lane; s < splits; s += 64) {
-        const f32x2 ml = *(const f32x2*)(first + s * step);
-        if (ml.y > 0.f) L += __builtin_amdgcn_exp2f(ml.x - M) * ml.y;
+    const float fl = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - M) : 0.f;
+    float L = ml.y > 0.f ? fl * ml.y : 0.f;
+    for (int s = lane + 64; s < splits; s += 64) {
+        const f32x2 more = *(const f32x2*)(first + s * step);
+        if (more.y > 0.f) L += __builtin_amdgcn_exp2f(more.x - M) * more.y;
     }
     L = wave_sum(L);
     const float inv = sink ? sink_inv(M, L, sink[h]) : 1.f / L;
-    for (int c0 = 0; c0 < R; c0 += 128) {                   // (R % 4 == 0)
+    const unsigned long long counts = __builtin_amdgcn_ballot_w64(ml.y > 0.f);
+    auto block = [&](int c0, const f32x2* have) __attribute__((always_inline)) {      // (R % 4 == 0)
         const int c = c0 + 2 * lane;
         float2 acc = make_float2(0.f, 0.f);
+        auto add = [&](int s, f32x2 x) __attribute__((always_inline)) {
+            if (s < 64) {
+                if (counts >> s & 1) {
+                    const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, fl), s));
+                    acc.x += f * x.x;
+                    acc.y += f * x.y;
+                }
+            } else {
+                const f32x2 more = *(const f32x2*)(first + s * step);
+                const float f = __builtin_amdgcn_exp2f(more.x - M);
+                if (more.y > 0.f) { acc.x += f * x.x; acc.y += f * x.y; }
+            }
+        };
+        int s = wave;
+        if (have)
+#pragma unroll
+            for (int u = 0; u < U; ++u, s += WAVES)
+                if (s < splits) add(s, have[u]);
 #pragma unroll 4
-        for (int s = wave; s < splits; s += WAVES) {
-            const float* p = first + s * step;
-            const f32x2 ml = *(const f32x2*)p, x = *(const f32x2*)(p + 2 + min(c, R - 2));
-            const float f = __builtin_amdgcn_exp2f(ml.x - M);
-            if (ml.y > 0.f) { acc.x += f * x.x; acc.y += f * x.y; }
-        }
+        for (; s < splits; s += WAVES) add(s, *(const f32x2*)(first + s * step + 2 + min(c, R - 2)));
         if (WAVES > 1) {
             part[wave][lane] = acc;
             __syncthreads();
@@ -113,7 +140,10 @@ __global__ __launch_bounds__(64 * WAVES) void latent_decode_merge_kernel(const f
             *(u16x2*)(o + row * R + c) = o2;
         }
         if (WAVES > 1) __syncthreads();
-    }
+    };
+    block(0, ahead[0]);
+    if (R > 128) block(128, ahead[1]);
+    for (int c0 = 256; c0 < R; c0 += 128) block(c0, nullptr);
 }
 
 // the padded value width the kernel SM_BY_LATENT_SIZE picks for (R, RV)

@@ -1,0 +1,42 @@
+"""Latent decode attention in any number of splits (csrc/seqmix/sm_latent_decode.hip: the merge asks for a wave's first splits of the first
+256 columns in front of their maximum) against plain float64 attention: splits around what is asked for ahead and around the 64 lanes,
+most of them empty, one wave and four per row, values narrower than a row, with and without a sink."""
+import os
+import sys
+
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "nano-vllm-hw3_amd"))
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+
+from test_hymix_ops import batch, gen, rnd  # noqa: E402
+
+from nanovllm import seq_ops  # noqa: E402
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H", [(6, 8), (50, 128)])                     # (four waves per row; one)
+@pytest.mark.parametrize("R,RV", [(64, 64), (136, 132), (256, 192), (256, 256)])
+@pytest.mark.parametrize("sink", [False, True])
+def test_merged_splits(monkeypatch, B, H, R, RV, sink):
+    bf, page, scale = torch.bfloat16, 64, 0.1
+    lens = [(1, 64, 65, 200, 700, 1100)[b % 6] for b in range(B)]
+    g = gen(B + R + RV)
+    ctx, _ = batch([(n - 1, 1) for n in lens], page, seed=B)
+    cache = rnd(g, (int(ctx.block_tables.max()) + 1) * page, R, dtype=bf)
+    q, sk = rnd(g, B, H, R, dtype=bf), rnd(g, H, s=2.0) if sink else None
+    want = torch.empty(B, H, RV, dtype=torch.float64)
+    for b, n in enumerate(lens):
+        rows = cache[ctx.block_tables[b].long()[torch.arange(n) // page] * page + torch.arange(n) % page].double()
+        s = q[b].double() @ rows.t() * scale
+        s = s if sk is None else torch.cat([s, sk[:, None].double()], 1)
+        want[b] = torch.softmax(s, -1)[:, :n] @ rows[:, :RV]
+    ctx, _ = batch([(n - 1, 1) for n in lens], page, device="cuda", seed=B)
+    qc, cc, sc = q.cuda(), cache.view(-1, page, R).cuda(), sk.cuda() if sink else None
+    for splits in (1, 4, 5, 6, 7, 16, 17, 64, 65, 130):
+        monkeypatch.setattr(seq_ops, "decode_splits", lambda *a: splits)
+        got = seq_ops.latent_attention(qc, cc, ctx, scale, value_cols=RV, sink=sc).double().cpu()
+        # one rounding to bf16 (2^-9 of the value) and the weights' own (2^-9 of each, so of the largest value at most), twice over
+        assert (got - want).abs().le(2.0 ** -8 * (want.abs() + 5.0)).all(), splits
