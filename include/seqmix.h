@@ -165,7 +165,7 @@ int sm_moe_grouped(const void* h, const int32_t* idx, const float* wts, const vo
                    const void* shared, const float* shared_scale, int weight_in, float limit, float alpha, int act_kind, void* y, int64_t T, int top, int E, int W, int F,
                    int32_t* row_pair, int32_t* tile_expert, int32_t* pair_row, void* act, void* prod, void* stream);
 
-/* sm_moe_grouped in tiles of 128 rows, or of 256 from 128 pairs per expert on average (both operands straight to LDS): the form
+/* sm_moe_grouped in tiles of 128 rows, or of 256 from 128 pairs per expert on average and with tiles enough (both operands straight to LDS): the form
  * for large groups.  Same arguments, scratch by n = sm_moe_tiles128_count(T, top, E), which is room in units of 128 rows and
  * not a number of tiles: row_pair int32 [128 n], tile_expert int32 [n], pair_row int32 [T * top], act bf16 [128 n, F], prod bf16
  * [128 n, W].  An expert's last tile is padded, so there are up to 128 E rows (256 E) more than pairs.  row_pair and tile_expert are
