@@ -26,6 +26,7 @@
 // 128 on 64 rows 0.87 (0.64 at best), on 96 rows 0.94; groups of 64 in fp8 on 96 rows that have their CUs to themselves 1.03.
 #pragma once
 #include "ql_gemm_kernel.h"
+#include "step_window.h"
 
 namespace ql {
 
@@ -79,11 +80,12 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
     auto load_a = [&](unsigned char* buf, int t) {
         if constexpr (!KEPT) asm volatile("" : "+v"(abase));  // (worked out anew at every step, or each would keep its register)
 #ifdef __HIP_DEVICE_COMPILE__
-        // (a step past the last one finds an empty resource: nothing is read)
-        const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, KEPT || t < steps ? xbytes : 0u, 0x00020000);
+        // (a step past the last one finds an empty resource, at its start: nothing is read; 8 bits have none)
+        const StepWindow win = KEPT ? StepWindow{xbytes, t * 256u} : step_window(t, steps, 256u, xbytes);
+        const auto xrsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, win.bytes, 0x00020000);
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lvoid*)(buf + (8 * MT * wave + 4 * i) * 256), 16, KEPT ? akept[i] : aoff(i), t * 256, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lvoid*)(buf + (8 * MT * wave + 4 * i) * 256), 16, KEPT ? akept[i] : aoff(i), win.at, 0, 0);
 #endif
     };
     // weights: as in the other tiles (strips past N: the last one, never stored; N is a multiple of 32).  A lane's place in a strip in a
