@@ -12,6 +12,7 @@
 #include <algorithm>
 
 #include "sm_common.h"
+#include "sm_moe_deal.h"
 
 namespace sm {
 
@@ -45,16 +46,11 @@ template <int MODE, bool FEW>
 __global__ __launch_bounds__(64) void moe_grouped_kernel(const unsigned short* __restrict__ a, const unsigned short* __restrict__ w,
                                                           const int32_t* __restrict__ row_pair, const int32_t* __restrict__ tile_expert,
                                                           unsigned short* __restrict__ out, int tiles, int top, unsigned top_inv, int N, int K, float limit,
-                                                          float alpha, int act_kind, const float* __restrict__ in_wts, bool by_die) {
+                                                          float alpha, int act_kind, const float* __restrict__ in_wts) {
     constexpr bool GATE_UP = MODE == 1, FROM_TOKENS = MODE != 0;
-    // Workgroups go to the eight dies in turn.  By die: a die has every eighth column block, and its tiles one behind the other, so that the
-    // tiles of one expert meet its weights in one L2 (us of whole calls, tiles on neighbouring dies / here, weights not in a cache: 40 rows
-    // for each of 4 experts of 2048 x 4096 87 / 77, of 16 of 2048 x 1536 110 / 86, of one of 4096 x 11008 104 / 87; one tile per expert alike).
-    // Up to 8 tokens no expert has a second tile, and what counts is how the few that are read lie in memory: 4 tokens, 16 experts of
-    // 2048 x 1536 68 / 63, 32 of them 79 / 91, 64 115 / 105, one token 51 / 63 and 58 / 65.  Those go by tiles.
-    const int id = blockIdx.x >> 3, tile = by_die ? id % tiles : (int)blockIdx.x % tiles;
-    const int n0 = (by_die ? (id / tiles) * 8 + (int)(blockIdx.x & 7) : (int)blockIdx.x / tiles) * 32;
-    if (n0 >= N) return;
+    const MoePlace place = moe_place(blockIdx.x, blockIdx.y, blockIdx.z);
+    const int tile = place.tile, n0 = place.block * 32;
+    if (n0 >= N || tile >= tiles) return;
     const int lane = threadIdx.x, l31 = lane & 31, hi = lane >> 5;
     // The tile's rows come 128 bytes at a time, eight lanes to a row, and go through LDS to the lanes that multiply them (chunk c
     // of row r at place c ^ (r / 2 & 7)): a lane reading its own row would touch a cache line of its own with every load.  Rows
@@ -235,11 +231,14 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     hipStream_t s = as_stream(stream);
     if (int rc = launch_moe_align(idx, T * top, E, kRowsPerTile, tiles, row_pair, tile_expert, pair_row, nullptr, s)) return rc;
     const bool few = T <= 8 || (T <= 32 && std::min<int64_t>(T * top, E) * ((F + 31) / 32) <= 256);
-    auto grid = [&](int n) { return dim3((unsigned)((n + 255) / 256) * 8u * (unsigned)tiles); };
+    auto grid = [&](int n) {
+        const MoeGrid g = moe_grid(tiles, n);
+        return dim3(g.x, g.y, g.z);
+    };
 #define SM_GROUPED(MODE_, FEW_)                                                                                                          \
     hipLaunchKernelGGL((moe_grouped_kernel<MODE_, FEW_>), grid(F), dim3(64), 0, s,                                                     \
                        (const unsigned short*)h, (const unsigned short*)w_gu, row_pair, tile_expert, (unsigned short*)act, tiles, top, top_inv, \
-                       F, W, limit, alpha, act_kind, weight_in ? wts : nullptr, T > 8)
+                       F, W, limit, alpha, act_kind, weight_in ? wts : nullptr)
     if (act_is_gated(act_kind)) {
         if (few) SM_GROUPED(1, true); else SM_GROUPED(1, false);
     } else {
@@ -249,7 +248,7 @@ extern "C" int sm_moe_grouped(const void* h, const int32_t* idx, const float* wt
     SM_CHECK_LAUNCH("sm_moe_grouped (gate/up)");
     hipLaunchKernelGGL((moe_grouped_kernel<0, false>), grid(W), dim3(64), 0, s,
                        (const unsigned short*)act, (const unsigned short*)w_down, row_pair, tile_expert, (unsigned short*)prod, tiles, top, top_inv, W,
-                       F, 0.f, 0.f, 0, (const float*)nullptr, T > 8);
+                       F, 0.f, 0.f, 0, (const float*)nullptr);
     SM_CHECK_LAUNCH("sm_moe_grouped (down)");
     if (y == nullptr) return SM_OK;               // the caller sums a token's pairs itself
     return sm_moe_combine(prod, pair_row, weight_in ? nullptr : wts, shared, shared_scale, y, T, top, W, stream);
