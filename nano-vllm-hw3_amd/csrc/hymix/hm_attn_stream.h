@@ -24,6 +24,7 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(const unsigned 
                                                                  int window, int keep_first, float c_log2, float pre,
                                                                  float* __restrict__ ws, int H, int G, int block_size, int max_blocks,
                                                                  int splits, int chunk) {
+    typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
     constexpr int NL = D / 64, U = REP == 4 ? 2 : 4, STRIDE = D + 2;       // 16-byte pieces of a key per lane; keys in flight per lane
     __shared__ float st_m[16][REP], st_l[16][REP];
     __shared__ __attribute__((aligned(16))) float st_acc[16][REP][D];
@@ -87,8 +88,7 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(const unsigned 
                     vv[u][p] = __builtin_nontemporal_load((const i32x4*)(vc + at + 64 * p));
                 }
             }
-            // Inline, kept in order and closed by a wait statement: the compiler does not see that these are dot-product
-            // instructions, whose result needs up to four wait states before another instruction reads it.
+            __builtin_amdgcn_sched_barrier(0);               // (all asked for first: left alone the compiler moves half of them to their use)
             float sc[U][REP];
 #pragma unroll
             for (int u = 0; u < U; ++u)
@@ -96,18 +96,11 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(const unsigned 
                 for (int h = 0; h < REP; ++h) {
                     sc[u][h] = 0.f;
 #pragma unroll
-                    for (int p = 0; p < NL; ++p)
-                        asm volatile("s_nop 0\n\tv_dot2c_f32_bf16 %0, %1, %5\n\tv_dot2c_f32_bf16 %0, %2, %6\n\t"
-                                     "v_dot2c_f32_bf16 %0, %3, %7\n\tv_dot2c_f32_bf16 %0, %4, %8"
-                                     : "+v"(sc[u][h])
-                                     : "v"(qp[h][4 * p]), "v"(qp[h][4 * p + 1]), "v"(qp[h][4 * p + 2]), "v"(qp[h][4 * p + 3]),
-                                       "v"(kk[u][p][0]), "v"(kk[u][p][1]), "v"(kk[u][p][2]), "v"(kk[u][p][3]));
+                    for (int j = 0; j < 4 * NL; ++j) {
+                        const int kd = kk[u][j >> 2][j & 3];   // (a value: a bit cast of the element itself reads the vector's first one)
+                        sc[u][h] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, qp[h][j]), __builtin_bit_cast(bf16x2, kd), sc[u][h], false);
+                    }
                 }
-            asm volatile("s_nop 3" : "+v"(sc[U - 1][REP - 1]));
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int h = 0; h < REP; ++h) asm volatile("" : "+v"(sc[u][h]));
             bool seen[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
