@@ -53,6 +53,10 @@ __device__ __forceinline__ float gelu_tanh(float z) {
 }
 // n / d for d >= 1: a division's remainder step without its scaling (d 2^-32 and its reciprocal are never subnormal), the special cases
 // by the division's own last instruction.  7 instructions for 11: a gate's outputs are a sixth of the expert tiles' cycles.
+// Not correctly rounded in every case, but nearly: the first quotient is off by 1.5 units at most (the reciprocal's one, the product's half), its
+// remainder is exact, and the reciprocal scales that with a relative error of 2^-21 (2^-20 where it is subnormal): 0.5 units + 2^-19.
+// Gates of 2^22 numbers each (normal ones, +-90, +-e^85, -86 to -89; alpha 1 and 8) have the errors of the division, largest and mean, to
+// every digit shown: the exponential's are 4 to 64 units.
 __device__ __forceinline__ float quotient(float n, float d) {
     const float r = __builtin_amdgcn_rcpf(d * 0x1p-32f) * 0x1p-32f, q = n * r;
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, n), r, q), d, n);
@@ -61,9 +65,10 @@ __device__ __forceinline__ float quotient(float n, float d) {
 // SM_ACT_SILU_GLU the same without the one: silu(g) u for limit = +inf and alpha = 1; SM_ACT_GELU_TANH_GLU: gelu_tanh(g) u
 __device__ __forceinline__ float gated_act(float g, float u, float limit, float alpha, int act) {
     if (act == SM_ACT_GELU_TANH_GLU) return gelu_tanh(g) * u;
-    // (minnum and maxnum as the hardware has them; the library's put a canonicalization in front of every operand)
+    // (minnum and maxnum as the hardware has them: the library's put a canonicalization in front of every operand, and a caller that has
+    // numbers from memory does so itself, since a signalling NaN would come through)
     asm("v_min_f32 %0, %1, %2" : "=v"(g) : "s"(limit), "v"(g));
-    u = __builtin_amdgcn_fmed3f(u, -limit, limit);
+    u = __builtin_amdgcn_fmed3f(u, -fabsf(limit), limit);     // (min(max(u, -limit), limit), which is the limit for negative ones)
     const float y = quotient(g, 1.f + __builtin_amdgcn_exp2f(g * (-1.4426950408889634f * alpha)));
     return y * (act == SM_ACT_SILU_GLU ? u : u + 1.f);
 }

@@ -53,7 +53,8 @@ __global__ void gated_act_kernel(const T* __restrict__ gu, int64_t row_stride, i
     const Pack g = *(const Pack*)(row + c), u = *(const Pack*)(row + F + c);
     Pack o;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) o.v[e] = from_f<T>(gated_act(to_f(g.v[e]), to_f(u.v[e]), limit, alpha, act));
+    for (int e = 0; e < VEC; ++e)
+        o.v[e] = from_f<T>(gated_act(__builtin_canonicalizef(to_f(g.v[e])), __builtin_canonicalizef(to_f(u.v[e])), limit, alpha, act));
     *(Pack*)(out + (size_t)t * out_stride + c) = o;
 }
 
