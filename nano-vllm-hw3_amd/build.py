@@ -32,9 +32,10 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-fno-gpu-rdc", 
 # Kernels of one wave per SIMD have 512 registers, and there the compiler puts the results of matrix instructions into the accumulation
 # half, from which the vector unit has to copy every number that it reads.  These files' kernels read them all (softmax, splits, folds)
 # and need few more than 256: results in the vector half take the copies out (the chunked recurrences' walk 1.09 x, latent decode
-# attention 1.14 x, its spills gone; the same bits).  Tiles that hold 256 sums per lane (sm_moe_tiles) need the other half.
+# attention 1.14 x; the same bits).  Tiles that hold 256 sums per lane (sm_moe_tiles) need the other half.
 VECTOR_RESULTS = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-FILE_FLAGS = {f: VECTOR_RESULTS for f in ("hm_outer_chunk.hip", "hm_attn_mfma.hip", "sm_latent_decode.hip", "sm_latent_mfma.hip")}
+FILE_FLAGS = {f: VECTOR_RESULTS for f in ("hm_outer_chunk.hip", "hm_attn_mfma.hip", "sm_latent_decode.hip", "sm_latent_mfma.hip",
+                                          "ql_gemm_inst_wide_bf16_i8.hip", "ql_gemm_inst_wide_bf16_fp8.hip")}
 TARGETS = {
     "qlinear": dict(src=CSRC, lib=LIB, header="qlinear.h", flags=FLAGS, obj=""),
     "seqmix": dict(src=os.path.join(CSRC, "seqmix"), lib=SEQMIX_LIB, header="seqmix.h", flags=FLAGS, obj="seqmix_"),

@@ -11,7 +11,10 @@
 //   * Weights go from global memory to the registers of the wave that multiplies them (16 bytes per lane and 32-k product), RW
 //     products ahead: a register is loaded again as soon as its weights are widened.  They are widened once for 32 MT rows.
 //   * Per-group sums take a second set of accumulators, so 96 rows are the most there, and there weights are loaded 64 k ahead (64 rows
-//     have registers for 128 k: groups of 128, one tile per CU, 0.84 x the time of 64 k).
+//     have registers for 128 k: groups of 128, one tile per CU, 0.84 x the time of 64 k).  With nothing beside it on its CU a workgroup
+//     takes a weight's way from memory for every 64 k, and has twice the registers: 96 rows of at most one tile per CU have weights 128 k
+//     ahead too (256 to 3000 rows, 512 to 12288 k: groups of 128 0.92 in int8, 0.94 in fp8, groups of 64 in fp8 0.90; in int8 the compiler
+//     moves a fold's sums through accumulation registers, 1.07: not built).
 //   * Tiles are dealt to the eight dies in contiguous runs of an order that goes through panels of eight row tiles, so that the
 //     tiles a die has at hand form a square and its L2 sees activations and weights several times.
 // The k order of a sum is that of the other tiles: results agree with theirs bit for bit (per-group scales: fused multiply-adds of
@@ -23,7 +26,7 @@
 // instructions: weight-only int8 qkv 158 / 134, o 113 / 84, gate_up 398 / 349, down 223 / 191; groups of 128 178 / 154, 136 / 97, 500 / 405,
 // 269 / 218; fp8 x fp8 106 / 71, 82 / 44, 311 / 180, 158 / 93.  With step16, all four and groups of 128: 811, not 859.  256 to 8192 rows of
 // the Qwen3 shapes and others, times the figure before: 96 rows of a tile 0.90 in int8, 0.89 in fp8, 128 rows 0.95 and 0.94, groups of
-// 128 on 64 rows 0.87 (0.64 at best), on 96 rows 0.94; groups of 64 in fp8 on 96 rows that have their CUs to themselves 1.03.
+// 128 on 64 rows 0.87 (0.64 at best), on 96 rows 0.94.
 #pragma once
 #include "ql_gemm_kernel.h"
 #include "step_window.h"
@@ -32,9 +35,9 @@ namespace ql {
 
 constexpr int kWidePanel = 8;                 // row tiles of a panel
 
-// FG: 32-k products behind which a group's sum is folded into the total with its scale (0: no groups)
-template <int ACT, bool FP8W, int FG, int MT, bool ROPE>
-__global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) {
+// FG: 32-k products behind which a group's sum is folded into the total with its scale (0: no groups).  ALONE: at most one workgroup for every CU
+template <int ACT, bool FP8W, int FG, int MT, bool ROPE, bool ALONE = false>
+__global__ __launch_bounds__(256, ALONE ? 1 : 2) void qgemm_wide_kernel(const GemmParams p) {
     constexpr bool INT = ACT == ACT_I8, GROUP = FG > 0;
     constexpr int AB = ACT == ACT_BF16 ? 2 : 1, KS = 256 / AB, SUB = KS / 32, BM = 32 * MT, BUF = BM * 256;
     constexpr int NA = 2 * MT;                                // 1 KB pieces of activations a wave loads per step
@@ -120,7 +123,7 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-    constexpr int RW = GROUP && MT > 2 ? 2 : 4;               // 32-k products that weights are loaded ahead
+    constexpr int RW = GROUP && MT > 2 && !ALONE ? 2 : 4;     // 32-k products that weights are loaded ahead
     i32x4 raw[RW][2];
     // a group's scales; groups of 64 on 64 rows are over before one group's way from memory: theirs are asked for a step ahead
     constexpr int SD = GROUP && FG == 2 && MT == 2 ? 2 : 1;
@@ -439,19 +442,22 @@ __global__ __launch_bounds__(256, 2) void qgemm_wide_kernel(const GemmParams p) 
 }
 
 template <int ACT, bool FP8W, int FG, bool ROPE>
-kern_t pick_wide_impl(int mt) {
+kern_t pick_wide_impl(int mt, bool alone = false) {
     switch (mt) {
         case 2: return (kern_t)qgemm_wide_kernel<ACT, FP8W, FG, 2, ROPE>;
-        case 3: return (kern_t)qgemm_wide_kernel<ACT, FP8W, FG, 3, ROPE>;
+        case 3:
+            if constexpr (FG > 2 || (FG == 2 && FP8W))
+                if (alone) return (kern_t)qgemm_wide_kernel<ACT, FP8W, FG, 3, ROPE, true>;
+            return (kern_t)qgemm_wide_kernel<ACT, FP8W, FG, 3, ROPE>;
         case 4: if constexpr (FG == 0) return (kern_t)qgemm_wide_kernel<ACT, FP8W, FG, 4, ROPE>; break;
     }
     return nullptr;
 }
 
 template <bool FP8W, bool ROPE>
-kern_t pick_wide_w16(int mt, int group) {
+kern_t pick_wide_w16(int mt, int group, bool alone) {
     if (group == 0) return pick_wide_impl<ACT_BF16, FP8W, 0, ROPE>(mt);
-    return group == 64 ? pick_wide_impl<ACT_BF16, FP8W, 2, ROPE>(mt) : pick_wide_impl<ACT_BF16, FP8W, 4, ROPE>(mt);
+    return group == 64 ? pick_wide_impl<ACT_BF16, FP8W, 2, ROPE>(mt, alone) : pick_wide_impl<ACT_BF16, FP8W, 4, ROPE>(mt, alone);
 }
 
 }  // namespace ql

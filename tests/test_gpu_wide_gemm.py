@@ -90,6 +90,30 @@ def check_silu(NQ, M, N, form, dt):
     return plan[0]
 
 
+@pytest.mark.parametrize("dt", ["int8", "fp8"])
+@pytest.mark.parametrize("form", ["g64", "g128", "g256"])
+@pytest.mark.parametrize("M,K", [(1819, 128), (1900, 256), (1920, 384), (1901, 640), (1825, 1152), (1920, 1280), (2000, 384)])
+def test_wide_tiles_that_have_their_cus_to_themselves(NQ, dt, form, M, K):
+    """96 rows of at most one tile for every CU hold weights for 128 k with up to 20 row tiles (all but the last): one step and more, odd
+    numbers of them, ragged rows and columns."""
+    from nanovllm import _qlinear as Q
+    group, N = int(form[1:]), 2400
+    K = (K + 255) // 256 * 256 if group == 256 else K
+    x, w, bias = tensors(M, N, K, M + K)
+    m = NQ.QGroupLinear(TDT[dt], w, bias, group)
+    if dt == "int8":
+        m.tile()
+    assert Q.plan_query(Q.QL_PLAN_GROUP, M, N, K, Q.dtype_code(TDT[dt]), group) == (3, 8, 1, 8, 1)
+    assert torch.equal(m(x), other_tile(lambda: m(x)))
+
+
+@pytest.mark.parametrize("dt", ["int8", "fp8"])
+@pytest.mark.parametrize("form", ["g64", "g128"])
+def test_wide_epilogues_that_have_their_cus_to_themselves(NQ, dt, form):
+    assert check_silu(NQ, 1901, 2432, form, dt) == 3
+    check_rope(NQ, 1901, 16, 2, 256, form, dt)
+
+
 @pytest.mark.parametrize("form", ["row", "g64", "g128", "w8a8"])
 @pytest.mark.parametrize("M,N", [(9000, 448), (12001, 320)])
 def test_wide_silu_epilogue(NQ, M, N, form):
