@@ -112,7 +112,8 @@ static bool wide_alone(int64_t row_tiles, int64_t col_tiles) { return row_tiles 
 // Two of its workgroups share a CU, so a launch takes ceil(tiles / 256) times what a tile costs beside another one, or what it costs
 // alone (from six rounds on the rounds run into each other).  Costs: microseconds of a tile and per 1000 k of it, fitted over 256..8192
 // rows of the Qwen3 0.6B, 1.7B, 4B and 8B shapes and eight others with weights that no cache holds (the rows that it picks are 0.1 to
-// 0.3 % slower than the best ones on average); 8-bit activations by k alone, over 64..8192 rows.
+// 0.3 % slower than the best ones on average; with groups, over 1399 calls that are not among those, 500 of them where the model has 64 and 96
+// rows within 6 %, 0.3 %, 57 by more than 3 % and 16 by more than 6 %); 8-bit activations by k alone, over 64..8192 rows.
 // The line to the other tiles: 140 tiles of 64 rows, below which most of the chip's CUs have no tile and slices of K or smaller tiles
 // win.  Groups of 64: in int8 170 up to 4096 k, from there 160 (640 x 4096 of 4096 k: 63.2 there / 54.3 here), beyond 6144 k 190.  Longer
 // ones: 200 up to 1024 k and from 4096 on (512 x 6144 of 4096 k in fp8, 192 tiles: 50 in slices / 64 here), between those 140 in int8 (700
@@ -169,8 +170,9 @@ static int wide_rows(int64_t M, int64_t N, int64_t K, int group, bool fp8, bool 
     int best = 2;
     for (int mt = 3; mt <= (group ? 3 : 4); ++mt)
         if (cost(mt) < cost(best)) best = mt;
-    // (no shape of the fit: fewer rounds win, groups of 128 at 9000 x 1024 of 512 k 20.5 in 64 rows, 18.3 in 96, 4500 x 2048 of 768 k 25.6 / 22.7)
-    if (!w8a8 && K < 1024 && best == 2 && rounds(3) < rounds(2)) best = 3;
+    // (fewer rounds win over short K, groups of 128 at 9000 x 1024 of 512 k 20.5 in 64 rows, 18.3 in 96, 4500 x 2048 of 768 k 25.6 / 22.7; without groups
+    // only up to three: of more they run into each other, int8 rows 1024 x 19456 of 512 k 28.5 / 30.4, 1500 x 13312 of 768 k 36.7 / 38.7)
+    if (!w8a8 && K < 1024 && best == 2 && rounds(3) < rounds(2) && (group || rounds(2) <= 3)) best = 3;
     if (group) {
         // (up to 1024 rows and less than a round of it, groups of 128 and more are faster here at any count: 961 x 6144 of 2560 k 53 / 51.  With
         // groups of 64 up to a round of it is faster than two here beyond 1024 k, unless its last row tile is more than half full, but not

@@ -67,6 +67,12 @@ def test_fewer_rounds_of_taller_tiles_over_short_k(no_table, form, group, M, N, 
     assert wide(p) and (p[0] >= mt if not group else p[0] == mt)
 
 
+@pytest.mark.parametrize("form,dtype,M,N,K", [(0, I8, 1024, 19456, 512), (0, I8, 1500, 13312, 768), (S, I8, 1500, 13312, 768), (S, F8, 1500, 13312, 768),
+                                              (S, I8, 769, 19456, 768)])
+def test_four_rounds_over_short_k_stay_in_low_tiles(no_table, form, dtype, M, N, K):
+    assert Q.plan_query(form, M, N, K, dtype) == (2, 8, 1, 8, 1)
+
+
 MID, MID64 = (1, 2, 4, 4), (2, 2, 4, 4)
 
 
