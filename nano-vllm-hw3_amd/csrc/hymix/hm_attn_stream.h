@@ -11,9 +11,13 @@
 // Microseconds with the merge, attn_decode_kernel / this one (caches not in L2; floor = the cache at 6.1 TB/s): 64 sequences of 700 to
 // 1300 keys, heads 16 / 8 of 128: 71 / 52 (floor 43), 16 / 4 of 128: 48 / 38 (22), 16 / 8 of 64: 43 / 32 (22), window 256 with capped
 // scores 34 / 22 (11); 64 of 1700 to 1800: 102 / 80 (75); 16 of 700 to 1300, 16 / 8 of 128: 36 / 22 (11); 4 of them 25 / 13; one of 100
-// keys 15 / 7.4.  512 to 3072 workgroups measured within 5 % of each other, so the splits stay those of the other form.
+// keys 15 / 7.4.  512 to 3072 workgroups measured within 5 % of each other, so the splits stay those of the other form.  Only waves with keys leave states:
+// with all four's merged whatever their keys, 256 sequences of 32 keys, 16 / 4 heads of 128, took 17.7 us, not 16.4, where the other form takes 15.5
+// (more than 768 workgroups of up to 64 keys and four heads of 128: the only ones that it is faster for, by up to 0.9 us).
 #pragma once
 #include "hm_attn_tile.h"
+
+#include <type_traits>
 
 namespace hm {
 
@@ -68,7 +72,8 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(const unsigned 
     // (32 U keys' worth of halves: with two keys per lane a half takes two steps)
     constexpr int STEPS = 4 / U;
     int half = 2 * vt_lo + wave;
-    const int end = 2 * vt_hi;
+    const int end = 2 * vt_hi - (first_key(2 * vt_hi - 1) >= n ? 1 : 0);    // (the last tile's second half may lie past the last key)
+    const int used = min(4, end - 2 * vt_lo);                // waves that have keys: short sequences have no states of the others to merge
     int key0 = half < end ? first_key(half) : 0;
     int64_t row0 = half < end ? page_row(key0) : 0;
     for (; half < end; half += 4) {
@@ -152,43 +157,52 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(const unsigned 
         return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, false));
     };
     const int state = 4 * wave + (lane >> 4);
+    if (wave < used)
 #pragma unroll
-    for (int h = 0; h < REP; ++h) {
-        const float mo = other(m[h]), lo = other(l[h]), mn = fmaxf(m[h], mo), mc = mn == -INFINITY ? 0.f : mn;
-        const float wa = __builtin_amdgcn_exp2f(m[h] - mc), wb = __builtin_amdgcn_exp2f(mo - mc);
-        if (lane % 16 == 0) { st_m[state][h] = mn; st_l[state][h] = l[h] * wa + lo * wb; }
+        for (int h = 0; h < REP; ++h) {
+            const float mo = other(m[h]), lo = other(l[h]), mn = fmaxf(m[h], mo), mc = mn == -INFINITY ? 0.f : mn;
+            const float wa = __builtin_amdgcn_exp2f(m[h] - mc), wb = __builtin_amdgcn_exp2f(mo - mc);
+            if (lane % 16 == 0) { st_m[state][h] = mn; st_l[state][h] = l[h] * wa + lo * wb; }
 #pragma unroll
-        for (int j = 0; j < 8 * NL; ++j) {
-            const float o = other(acc[h][j]);
-            acc[h][j] = acc[h][j] * wa + o * wb;
+            for (int j = 0; j < 8 * NL; ++j) {
+                const float o = other(acc[h][j]);
+                acc[h][j] = acc[h][j] * wa + o * wb;
+            }
+            if ((lane & 8) == 0) {
+#pragma unroll
+                for (int p = 0; p < NL; ++p)
+#pragma unroll
+                    for (int e = 0; e < 8; e += 4)
+                        *(float4*)&st_acc[state][h][64 * p + 8 * seg + e] =
+                            make_float4(acc[h][8 * p + e], acc[h][8 * p + e + 1], acc[h][8 * p + e + 2], acc[h][8 * p + e + 3]);
+            }
         }
-        if ((lane & 8) == 0) {
-#pragma unroll
-            for (int p = 0; p < NL; ++p)
-#pragma unroll
-                for (int e = 0; e < 8; e += 4)
-                    *(float4*)&st_acc[state][h][64 * p + 8 * seg + e] =
-                        make_float4(acc[h][8 * p + e], acc[h][8 * p + e + 1], acc[h][8 * p + e + 2], acc[h][8 * p + e + 3]);
-        }
-    }
     __syncthreads();
-    for (int o = threadIdx.x; o < REP * D; o += 256) {
-        const int h = o / D, d = o % D;
-        float M = st_m[0][h];
+    auto merge = [&](auto states) __attribute__((always_inline)) {
+        constexpr int S = decltype(states)::value;
+        for (int o = threadIdx.x; o < REP * D; o += 256) {
+            const int h = o / D, d = o % D;
+            float M = st_m[0][h];
 #pragma unroll
-        for (int s = 1; s < 16; ++s) M = fmaxf(M, st_m[s][h]);
-        const float mc = M == -INFINITY ? 0.f : M;
-        float num = 0.f, den = 0.f;
+            for (int s = 1; s < S; ++s) M = fmaxf(M, st_m[s][h]);
+            const float mc = M == -INFINITY ? 0.f : M;
+            float num = 0.f, den = 0.f;
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            const float w = __builtin_amdgcn_exp2f(st_m[s][h] - mc);
-            num += w * st_acc[s][h][d];
-            den += w * st_l[s][h];
+            for (int s = 0; s < S; ++s) {
+                const float w = __builtin_amdgcn_exp2f(st_m[s][h] - mc);
+                num += w * st_acc[s][h][d];
+                den += w * st_l[s][h];
+            }
+            float* p = part + h * STRIDE;
+            p[2 + d] = num;
+            if (d == 0) { p[0] = den > 0.f ? M : -INFINITY; p[1] = den; }
         }
-        float* p = part + h * STRIDE;
-        p[2 + d] = num;
-        if (d == 0) { p[0] = den > 0.f ? M : -INFINITY; p[1] = den; }
-    }
+    };
+    using std::integral_constant;
+    if (used == 4) merge(integral_constant<int, 16>{});
+    else if (used == 3) merge(integral_constant<int, 12>{});
+    else if (used == 2) merge(integral_constant<int, 8>{});
+    else merge(integral_constant<int, 4>{});
 }
 
 }  // namespace hm
