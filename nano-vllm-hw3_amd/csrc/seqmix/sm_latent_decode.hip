@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64 * WAVES, SLIM && WAVES > 1 ? 2 : 1) void latent_
 // One wave where four have nothing to share out, up to five splits, and where the rows fill the chip several times over, from 6400 (us of
 // the whole step with four / one): 256 sequences of about 450 keys, 64 heads of 32 columns, 4 splits 33.5 / 22.6; 512 of 300, 64 heads of
 // 192 + 64, 2 splits 82 / 52; 128 of 1000, 64 heads, 8 splits 14 % more with four; 16 heads of 100 sequences, 8 splits 13 % less.
-template <int WAVES>
+template <int WAVES, int U>
 __global__ __launch_bounds__(64 * WAVES) void latent_decode_merge_kernel(const float* __restrict__ ws, unsigned short* __restrict__ o, int H,
                                                                          int R, int splits, int stride, const float* __restrict__ sink) {
     __shared__ float2 part[WAVES][64];
@@ -80,9 +80,9 @@ __global__ __launch_bounds__(64 * WAVES) void latent_decode_merge_kernel(const f
     const float* first = ws + (b * splits * H + h) * stride;
     const size_t step = (size_t)H * stride;
     // (an empty split has sum 0 and outputs that nobody wrote: it counts for nothing)
-    // A wave's first splits of the first two column blocks are asked for in front of the maximum, which they do not wait for: with one
-    // round of loads behind another the kernel took 6.9 us of 20.6 (64 sequences of 16 heads, 11 splits of 192 columns), so 4.5.
-    constexpr int U = WAVES == 1 ? 6 : 4;
+    // A wave's first U splits of the first two column blocks are asked for in front of the maximum, which they do not wait for: with one
+    // round of loads behind another the kernel took 6.9 us of 20.6 (64 sequences of 16 heads, 11 splits of 192 columns), so 4.5.  (With six asked for
+    // where there is one, 400 sequences of 128 heads of 64 + 64 took 35.1 us, not 32.5.)
     const f32x2 ml = lane < splits ? *(const f32x2*)(first + lane * step) : f32x2{-INFINITY, 0.f};
     f32x2 ahead[2][U];
 #pragma unroll
@@ -127,8 +127,16 @@ __global__ __launch_bounds__(64 * WAVES) void latent_decode_merge_kernel(const f
 #pragma unroll
             for (int u = 0; u < U; ++u, s += WAVES)
                 if (s < splits) add(s, have[u]);
-#pragma unroll 4
-        for (; s < splits; s += WAVES) add(s, *(const f32x2*)(first + s * step + 2 + min(c, R - 2)));
+        // (four at a time: a lane's number cannot be read by another while the compiler has loads to move over the condition)
+        for (; s < splits; s += 4 * WAVES) {
+            f32x2 x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = *(const f32x2*)(first + min(s + u * WAVES, splits - 1) * step + 2 + min(c, R - 2));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (s + u * WAVES < splits) add(s + u * WAVES, x[u]);
+        }
         if (WAVES > 1) {
             part[wave][lane] = acc;
             __syncthreads();
@@ -199,10 +207,14 @@ extern "C" int sm_latent_attn_decode(const void* q, const void* cache, const int
 #undef SM_DEC_
 #undef SM_DEC
     SM_CHECK_LAUNCH("sm_latent_attn_decode");
-#define SM_MERGE(WAVES_)                                                                                                       \
-    hipLaunchKernelGGL(latent_decode_merge_kernel<WAVES_>, dim3((unsigned)(B * H)), dim3(64 * WAVES_), 0, s, (const float*)workspace, \
+#define SM_MERGE(WAVES_, U_)                                                                                                   \
+    hipLaunchKernelGGL((latent_decode_merge_kernel<WAVES_, U_>), dim3((unsigned)(B * H)), dim3(64 * WAVES_), 0, s, (const float*)workspace, \
                        (unsigned short*)o, H, RV, splits, part_stride(padded_nbv(R, RV)), sink)
-    if (splits <= 5 || B * H >= 6400) SM_MERGE(1); else SM_MERGE(4);
+    if (splits <= 5 || B * H >= 6400) {
+        if (splits <= 2) SM_MERGE(1, 2); else SM_MERGE(1, 6);
+    } else {
+        SM_MERGE(4, 4);
+    }
 #undef SM_MERGE
     SM_CHECK_LAUNCH("sm_latent_attn_decode (merge)");
     return SM_OK;

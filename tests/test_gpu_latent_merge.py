@@ -1,6 +1,6 @@
 """Latent decode attention in any number of splits (csrc/seqmix/sm_latent_decode.hip: the merge asks for a wave's first splits of the first
 256 columns in front of their maximum) against plain float64 attention: splits around what is asked for ahead and around the 64 lanes,
-most of them empty, one wave and four per row, values narrower than a row, with and without a sink."""
+most of them empty or, with one sequence of 130 tiles, all of them used, one wave and four per row, values narrower than a row, with and without a sink."""
 import os
 import sys
 
@@ -22,7 +22,7 @@ from nanovllm import seq_ops  # noqa: E402
 @pytest.mark.parametrize("sink", [False, True])
 def test_merged_splits(monkeypatch, B, H, R, RV, sink):
     bf, page, scale = torch.bfloat16, 64, 0.1
-    lens = [(1, 64, 65, 200, 700, 1100)[b % 6] for b in range(B)]
+    lens = [8320 if b == 5 else (1, 64, 65, 200, 700, 1100)[b % 6] for b in range(B)]      # (130 tiles: splits 65 and 130 are used to the last)
     g = gen(B + R + RV)
     ctx, _ = batch([(n - 1, 1) for n in lens], page, seed=B)
     cache = rnd(g, (int(ctx.block_tables.max()) + 1) * page, R, dtype=bf)
@@ -35,7 +35,7 @@ def test_merged_splits(monkeypatch, B, H, R, RV, sink):
         want[b] = torch.softmax(s, -1)[:, :n] @ rows[:, :RV]
     ctx, _ = batch([(n - 1, 1) for n in lens], page, device="cuda", seed=B)
     qc, cc, sc = q.cuda(), cache.view(-1, page, R).cuda(), sk.cuda() if sink else None
-    for splits in (1, 4, 5, 6, 7, 16, 17, 64, 65, 130):
+    for splits in (1, 2, 3, 4, 5, 6, 7, 16, 17, 64, 65, 130):
         monkeypatch.setattr(seq_ops, "decode_splits", lambda *a: splits)
         got = seq_ops.latent_attention(qc, cc, ctx, scale, value_cols=RV, sink=sc).double().cpu()
         # one rounding to bf16 (2^-9 of the value) and the weights' own (2^-9 of each, so of the largest value at most), twice over
