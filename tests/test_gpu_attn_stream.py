@@ -64,3 +64,28 @@ def test_streamed_decode_attention(monkeypatch, H, G, D, page, window, keep, chu
         # one rounding to bf16 (2^-9 of the value), and weights whose scores carry the float32 error of D products and the exponential's
         # (scores to 40, 2e-6 of them at most) times the largest value
         assert (got - want).abs().le(2.0 ** -8 * want.abs() + 1e-4 * top).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D", [(4, 2, 64), (16, 2, 128), (6, 2, 32)])            # (streamed; not)
+@pytest.mark.parametrize("sink", [False, True])
+def test_more_than_64_splits(monkeypatch, H, G, D, sink):
+    """The merge beyond its 64 lanes: 130 tiles, which are 65 used splits of 65 or 130 where a split takes pairs of them, else 130."""
+    bf, scale, page, lens = torch.bfloat16, 0.3, 64, [8320, 70, 8257]
+    g = gen(H + D)
+    ctx, _ = batch([(n - 1, 1) for n in lens], page, seed=H)
+    rows = (int(ctx.block_tables.max()) + 1) * page
+    kc, vc = (rnd(g, rows, G, D, dtype=bf) for _ in range(2))
+    q, sk = rnd(g, len(lens), H, D, dtype=bf), rnd(g, H, s=2.0) if sink else None
+    want = []
+    for b, n in enumerate(lens):
+        at = ctx.block_tables[b].long()[torch.arange(n) // page] * page + torch.arange(n) % page
+        want.append(reference(q[b].double(), kc[at].double(), vc[at].double(), n, scale, 0, 0, 0, 0.0, sk))
+    want, top = torch.stack(want), vc.double().abs().max()
+    ctx, _ = batch([(n - 1, 1) for n in lens], page, device="cuda", seed=H)
+    for splits in (64, 65, 130):
+        monkeypatch.setattr(hy_ops, "decode_splits", lambda *a: splits)
+        got = hy_ops.paged_attention(q.cuda(), kc.view(-1, page, G, D).cuda(), vc.view(-1, page, G, D).cuda(), ctx, scale,
+                                     sk.cuda() if sink else None).view(want.shape).double().cpu()
+        # a rounding to bf16; where the weights go through the matrix cores each is rounded too (2^-9 of it, so of the largest value at most)
+        assert (got - want).abs().le(2.0 ** -8 * want.abs() + (1e-4 if D == 64 else 2.0 ** -9) * top).all(), splits

@@ -74,15 +74,17 @@ def test_gate_takes_minimum_and_maximum_as_the_library_does(dtype, act, alpha, l
 @pytest.mark.parametrize("T,top,E", [(1, 1, 1), (16, 4, 3), (17, 4, 70), (1024, 4, 5), (1025, 4, 5), (4096, 1, 130), (4097, 1, 130), (63, 65, 200)])
 def test_pairs_sorted_by_expert(T, top, E):
     """The grouping of pairs that a workgroup keeps in registers (up to 4096) and of more, by what the experts make of it: every one of
-    them multiplies by a number of its own, a power of two, and a pair that went to another would be off by at least that factor."""
+    them moves the columns by a number of its own (and beyond as many experts as columns doubles them), so that a pair which went to
+    another would have its values elsewhere."""
     g = torch.Generator().manual_seed(T + E)
     W = F = 128
     idx = torch.randint(0, E, (T, top), generator=g).int()
-    scale = 2.0 ** (torch.arange(E) % 8 - 4).double()
-    one = torch.eye(W)
-    w_gu, w_down = one.repeat(E, 1, 1).bfloat16(), (one[None] * scale[:, None, None]).bfloat16()
+    one, e = torch.eye(W), torch.arange(E)
+    down = torch.stack([torch.roll(one, int(i) % W, 0) * 2.0 ** (int(i) // W) for i in e])
+    w_gu, w_down = one.repeat(E, 1, 1).bfloat16(), down.bfloat16()
     h, wts = torch.randn(T, W, generator=g).abs().bfloat16(), torch.rand(T, top, generator=g)
-    want = (h.double()[:, None] ** 2).bfloat16().double() * (wts.double() * scale[idx.long()])[..., None]
+    at = (torch.arange(W) - idx.long()[..., None] % W) % W
+    want = (h.double() ** 2).bfloat16().double()[:, None].expand(T, top, W).gather(2, at) * (wts.double() * 2.0 ** (idx // W).double())[..., None]
     y = seq_ops.moe_experts(h.cuda(), idx.cuda(), wts.cuda(), w_gu.cuda(), w_down.cuda(), 7.0, form="grouped", act_kind=seq_ops.ACT_RELU_SQ).double().cpu()
     # the products are exact, the square is rounded to bf16 here as there (a tie may fall either way) and the sum once: 2^-8 of each
     assert (y - want.sum(1)).abs().le(2.0 ** -8 * want.sum(1) * 1.01 + 1e-30).all()
