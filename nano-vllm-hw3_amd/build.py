@@ -71,7 +71,7 @@ def build(force=False, verbose=True, target="qlinear"):
     hipcc = _hipcc()
     shared = os.path.join(HERE, "csrc")                                   # headers of more than one library lie there
     headers = [os.path.join(d, f) for d in {CSRC, shared} for f in os.listdir(d) if f.endswith(".h")]
-    headers.append(os.path.join(HERE, "..", "include", spec["header"]))
+    headers += [os.path.join(HERE, "..", "include", spec["header"]), os.path.abspath(__file__)]       # (the flags are here)
     srcs = sorted(f for f in os.listdir(CSRC) if f.endswith(".hip"))      # every translation unit of the folder
 
     def compile_one(src):
