@@ -4,6 +4,7 @@
 // Row r of a group is the same sum whatever else shares its tile, so every form agrees bit for bit on a row's products
 // (same k order inside a 64-k step, same accumulation).
 #include "sm_common.h"
+#include "sm_moe_rows.h"
 
 namespace sm {
 
@@ -553,10 +554,6 @@ __global__ __launch_bounds__(256, 1) void moe_tiles_walk_kernel(const unsigned s
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // (nothing may land in LDS that is no longer this workgroup's)
 }
 
-// Rows of a tile: 256 from 128 rows per expert on average, else 128 (moe_tiles_kernel, us with 128 / 256 rows, two sizes: 16 experts of
-// 2048 x 1536, 32 of 1024 x 768: 96 rows per expert 99 / 120, 53 / 75; 128 rows 142 / 120, 78 / 76; 384 rows 229 / 189, 126 / 124;
-// 2048 rows 942 / 734, 634 / 514); walked over, 256 only where they are kWalk256 tiles of the first product at least.
-static int tile_rows(int64_t T, int top, int E) { return T * top >= (int64_t)128 * E ? 256 : 128; }
 static int tile_count(int64_t T, int top, int E, int rows) { return (int)((T * top + rows - 1) / rows + E); }
 
 // Units of work that a launch makes at least, by cutting the column tiles of its pairs of row tiles into parts: a pair of row tiles is
@@ -565,10 +562,6 @@ static int tile_count(int64_t T, int top, int E, int rows) { return (int)((T * t
 // 1024 x 768 58 / 59).  Two units per die: with one the largest of these is 30 % slower at 512 rows, with four the small ones lose up
 // to 3 % to activations read by more dies.
 constexpr int kUnits = 16;
-// Walked over by kWalkers workgroups, one per CU.  With fewer than one and a half tiles of 256 rows each, those of 128 share the work out better
-// (us with 128 / 256 rows: 4 experts of 2048 x 4096, 192 tiles 94 / 105, 320 131 / 130, 448 194 / 179; 8 of 1024 x 768, 216 77 / 81, 408
-// 122 / 130; 16 of 2048 x 1536, 288 132 / 152, 384 174 / 176, 864 377 / 359; 8 of 4096 x 14336, 896 729 / 700, 1344 1139 / 979).
-constexpr int kWalkers = 256, kWalk256 = 384;
 // (an even number of whole steps; 32 bits hold the offsets into the rows and into an expert's weights, and a tile's number)
 static bool walks(bool dma, int64_t a_rows, int K, int parts, int N, int64_t tiles) {
     return dma && K % 128 == 0 && a_rows * K * 2 < (int64_t)1 << 32 && (int64_t)parts * (N + 31) * K * 2 < (int64_t)1 << 32 &&
@@ -604,7 +597,7 @@ using namespace sm;
 // room for a call's rows, in units of 128 rows
 extern "C" int sm_moe_tiles128_count(int64_t T, int top, int E) {
     if (T <= 0 || top <= 0 || E <= 0) return 0;
-    const int rows = tile_rows(T, top, E);
+    const int rows = moe_tile_rows(T * top, E);
     return tile_count(T, top, E, rows) * (rows / kBigRows);
 }
 
@@ -623,10 +616,9 @@ extern "C" int sm_moe_tiles128(const void* h, const int32_t* idx, const float* w
     if (T == 0) return SM_OK;
     // (operands off 16 bytes go through registers, in tiles of 128 rows, which need no more room)
     const bool dma = ((uintptr_t)h | (uintptr_t)act | (uintptr_t)w_gu | (uintptr_t)w_down) % 16 == 0;
-    int rows = dma ? tile_rows(T, top, E) : kBigRows, tiles = tile_count(T, top, E, rows);
+    int rows = dma ? moe_tile_rows(T * top, E) : kBigRows, tiles = tile_count(T, top, E, rows);
     const bool gated = act_is_gated(act_kind);
-    const int64_t about = (T * top / 256 + E / 2) * (gated ? (F + 127) / 128 : (F + 255) / 256);      // (half a tile of every group is empty)
-    if (rows == 256 && about < kWalk256) {
+    if (rows == 256 && moe_walk_low(T * top, E, gated ? (F + 127) / 128 : (F + 255) / 256, W)) {
         const int tiles128 = tile_count(T, top, E, kBigRows);  // (no more room than twice as many of 256 rows)
         if (walks(dma, T, W, gated ? 2 : 1, F, tiles128) && walks(dma, (int64_t)tiles128 * kBigRows, F, 1, W, tiles128)) {
             rows = kBigRows;

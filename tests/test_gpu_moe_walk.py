@@ -18,7 +18,7 @@ from nanovllm import seq_ops  # noqa: E402
 @pytest.mark.parametrize("T,top,E,W,F,act", [(1, 1, 1, 128, 128, "silu_glu"), (257, 1, 1, 128, 256, "silu_glu"), (300, 2, 3, 256, 136, "gelu"),
                                              (700, 2, 5, 384, 1152, "clamped_glu"), (513, 3, 4, 1152, 384, "relu_sq"),
                                              (4000, 2, 4, 256, 1536, "silu_glu"), (9001, 2, 3, 512, 1024, "clamped_glu"),
-                                             (6000, 2, 7, 200, 2048, "silu_glu"), (8300, 1, 32, 2048, 264, "gelu")])
+                                             (6000, 2, 7, 200, 2048, "silu_glu"), (8300, 1, 32, 2048, 264, "gelu"), (1000, 1, 1, 2048, 8192, "silu_glu")])
 def test_walked_tiles_equal_the_small_ones(T, top, E, W, F, act):
     g = torch.Generator().manual_seed(T + W)
     parts = 2 if act.endswith("glu") else 1
