@@ -1,6 +1,7 @@
 // Host-side dispatch of the fused dequant GEMMs: tile selection, split-K planning, argument checks,
 // and the extern "C" entry points.  The kernels live in ql_gemm_kernel.h / ql_gemm_inst_*.hip.
 #include "ql_gemm_kernel.h"
+#include "wide_ring.h"
 #include <stdlib.h>
 #include <algorithm>
 #include <map>
@@ -104,10 +105,6 @@ static bool wide_built(int64_t N, int64_t K, int group, bool silu, bool w8a8) {
     return !(K % (w8a8 ? 256 : 128) || N % (silu ? 64 : 32) || (group && group != 64 && group % 128));
 }
 
-// Whether groups' tiles of 96 rows hold weights for 128 k: at most one tile for every CU, and few row tiles, whose weights come from memory (with
-// more they come from L2, and what the ring costs at a tile's start shows: 20 row tiles 0.92, 22 to 29 1.02 to 1.07, 2222 x 2048 of 1536 k 21.4 / 22.8).
-static bool wide_alone(int64_t row_tiles, int64_t col_tiles) { return row_tiles * col_tiles <= kCus && row_tiles <= 20; }
-
 // Row fragments of the wide tile that a problem runs on; 0: the other tiles are faster; -1: the 128 x 256 tile of 64-k chunks is (groups).
 // Two of its workgroups share a CU, so a launch takes ceil(tiles / 256) times what a tile costs beside another one, or what it costs
 // alone (from six rounds on the rounds run into each other).  Costs: microseconds of a tile and per 1000 k of it, fitted over 256..8192
@@ -135,9 +132,11 @@ static int wide_rows(int64_t M, int64_t N, int64_t K, int group, bool fp8, bool 
                                  {{1.18, 9.42}, {2.30, 11.34}, {}}, {{0.84, 9.05}, {2.06, 10.81}, {}},
                                  {{0, 4.6}, {0, 6.8}, {0, 8.0}}};
     static const Cost alone[7][3] = {{{6.59, 6.40}, {8.48, 7.46}, {10.29, 9.54}}, {{6.37, 5.66}, {8.26, 6.74}, {12.00, 8.56}},
-                                  {{7.04, 8.09}, {9.11, 9.80}, {}}, {{6.16, 7.45}, {8.71, 9.77}, {}},
-                                  {{5.69, 10.81}, {8.29, 13.08}, {}}, {{4.77, 10.75}, {8.32, 11.07}, {}},
+                                  {{7.04, 8.09}, {8.09, 11.50}, {}}, {{6.16, 7.45}, {8.07, 11.04}, {}},
+                                  {{5.69, 10.81}, {8.29, 13.08}, {}}, {{4.77, 10.75}, {8.46, 12.59}, {}},
                                   {{0, 6.7}, {0, 8.3}, {0, 10.2}}};
+    // 96 rows alone that hold weights for 128 k
+    static const Cost ring[6] = {{}, {}, {9.11, 9.80}, {8.71, 9.77}, {8.29, 13.08}, {8.32, 11.07}};
     // the 128 x 256 tile of 64-k chunks: groups of 128, of 256 and more; groups of 64
     static const Cost chunked[6] = {{}, {}, {4.85, 16.44}, {4.53, 15.62}, {5.22, 17.92}, {4.98, 17.11}};
     // what a launch of several rounds takes beside them
@@ -161,7 +160,8 @@ static int wide_rows(int64_t M, int64_t N, int64_t K, int group, bool fp8, bool 
     };
     auto cost = [&](int mt) -> double {
         const double n = rounds(mt);
-        const Cost &p = pair[kind][mt - 2], &a = alone[kind][mt - 2];
+        const bool long_ring = group && mt == 3 && wide_alone((M + 95) / 96, cols, K);
+        const Cost &p = pair[kind][mt - 2], &a = long_ring ? ring[kind] : alone[kind][mt - 2];
         if (n <= 1) return a.tile + a.k * k;
         // (without groups the last of three rounds has its CU to itself, 6000 x 4096 of 1024 k in 128 rows 72 us, in 96 63)
         if (!group && !w8a8 && n == 3) return 2 * (p.tile + p.k * k) + a.tile + a.k * k;
@@ -776,7 +776,7 @@ static int gemm_w8a16(const char* fn, bool silu, int wdtype, int granularity, co
     kern_t k;
     const bool rp = rope != nullptr;
     if (pl.wide) {
-        const bool alone = wide_alone((M + 32 * pl.mt - 1) / (32 * pl.mt), (N + 255) / 256);
+        const bool alone = wide_alone((M + 32 * pl.mt - 1) / (32 * pl.mt), (N + 255) / 256, K);
         k = wdtype == QL_INT8 ? pick_wide_bf16_i8(pl.mt, p.group, rp, alone) : pick_wide_bf16_fp8(pl.mt, p.group, rp, alone);
     } else if (pl.sk_G > 0) {
         if (wdtype == QL_INT8) k = grp ? pick_sk_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_sk_bf16_i8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);

@@ -1243,7 +1243,7 @@ kern_t pick_sk_bf16_fp8_row(int, int, int, int, bool rope);
 kern_t pick_sk_bf16_fp8_group(int, int, int, int, bool rope);
 kern_t pick_fp8_fp8_dynq(int, int, int, int);
 // the wide tiles (ql_gemm_wide.h), which a plan names by (mt, 8, 1, kWideCP)
-constexpr int kWideCP = 8, kCus = 256;
+constexpr int kWideCP = 8;
 kern_t pick_wide_bf16_i8(int mt, int group, bool rope, bool alone);      // (alone: at most one tile for every CU)
 kern_t pick_wide_bf16_fp8(int mt, int group, bool rope, bool alone);
 kern_t pick_wide_i8_i8(int mt, bool rope);

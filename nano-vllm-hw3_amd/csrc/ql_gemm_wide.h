@@ -13,8 +13,7 @@
 //   * Per-group sums take a second set of accumulators, so 96 rows are the most there, and there weights are loaded 64 k ahead (64 rows
 //     have registers for 128 k: groups of 128, one tile per CU, 0.84 x the time of 64 k).  With nothing beside it on its CU a workgroup
 //     takes a weight's way from memory for every 64 k, and has twice the registers: 96 rows of at most one tile per CU have weights 128 k
-//     ahead too (256 to 3000 rows, 512 to 12288 k: groups of 128 0.92 in int8, 0.94 in fp8, groups of 64 in fp8 0.90; in int8 the compiler
-//     moves a fold's sums through accumulation registers, 1.07: not built).
+//     ahead too where that pays (wide_ring.h; not groups of 64 in int8: the compiler moves a fold's sums through accumulation registers, 1.07).
 //   * Tiles are dealt to the eight dies in contiguous runs of an order that goes through panels of eight row tiles, so that the
 //     tiles a die has at hand form a square and its L2 sees activations and weights several times.
 // The k order of a sum is that of the other tiles: results agree with theirs bit for bit (per-group scales: fused multiply-adds of
