@@ -290,7 +290,7 @@ __global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* 
         asm volatile("" ::: "memory");
     };
     double part[8];                                          // the last chunk's results of tokens 16 wave..: this wave's part
-    // (in double: in float32 the state-space form's error was 1 to 5 % above the token-by-token walk's; 1 us of 142)
+    // (in double: in float32 the state-space form's error was 1 to 5 % above the token-by-token walk's; 1 us, measured when the walk took 142)
     // their sum with the other wave's part, written before the last meeting (turn: 0 for an even chunk of the portion, 1 for an odd one)
     auto store_rows = [&](int t0, bool whole, int turn) {
         float* orow = o + ((size_t)(q0 + t0 + 16 * wave + 4 * hi) * H + h) * V + col;

@@ -19,8 +19,9 @@
 // The k order of a sum is that of the other tiles: results agree with theirs bit for bit (per-group scales: fused multiply-adds of
 // the same group sums in the same order).
 //
-// Bound by the matrix cores in 16 bits and by the power they take (random operands run at 1.7 to 2.0 GHz of 2.4; 1.15 to 1.25 PFLOP/s, what a
-// library product of 8192 reaches too), by the vector unit beside them with int8 groups, by both and LDS in 8 bits.  4099 rows, Qwen3-4B shapes,
+// Bound by the matrix cores in 16 bits and by the power they take (random operands run at 1.7 to 2.0 GHz of 2.4; 1.15 to 1.25 PFLOP/s, where a
+// library product in bf16, which widens nothing, reaches 1.2 at these shapes and 1.5 to 1.6 at 8192 x 8192 of 8192 k), by the vector unit beside them
+// with int8 groups, by both and LDS in 8 bits.  4099 rows, Qwen3-4B shapes,
 // microseconds of the 128 x 256 tile with one strip per wave / of this one with every product's weights widened in front of its matrix
 // instructions: weight-only int8 qkv 158 / 134, o 113 / 84, gate_up 398 / 349, down 223 / 191; groups of 128 178 / 154, 136 / 97, 500 / 405,
 // 269 / 218; fp8 x fp8 106 / 71, 82 / 44, 311 / 180, 158 / 93.  With step16, all four and groups of 128: 811, not 859.  256 to 8192 rows of

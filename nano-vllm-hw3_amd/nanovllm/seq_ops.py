@@ -255,9 +255,11 @@ def experts_form(pairs, E, W, F):
     the waves per CU.  So the large ones win from 24 rows per expert on average and, as long as they leave CUs without a
     tile, only from about 3.5 waves per CU of the small ones (the two products' mean by what they take: their k, and 256 for the
     rest).  Microseconds, 32-row form / large tiles, weights not in a cache: 16 experts of 2048 x 1536 (4.3 waves at 24 rows) 16
-    rows 69 / 69, 24 rows 71 / 70, 48 rows 88 / 76; 128 of 2048 x 768 (22 at 24) 8 rows 247 / 246, 24 rows 292 / 248; 8 of 1024
-    x 768 (2.2 at 64, 3.8 at 127) 48 rows 28 / 32, 96 rows 32 / 32; 2 of 4096 x 4096 (2.5 at 64, 3.5 at 96) 64 rows 70 / 92, 96
-    rows 96 / 94; 4 of 2048 x 4096 (2.4 at 40, 4.7 at 96) 40 rows 77 / 83, 64 rows 74 / 82, 96 rows 99 / 83."""
+    rows 69 / 75, 48 rows 98 / 83; 16 of 2048 x 768 24 rows 48 / 50, 48 rows 60 / 54; 128 of 2048 x 768 (22 at 24) 8 rows 241 / 244, 24
+    rows 270 / 248; 8 of 1024 x 768 (2.2 at 64, 3.8 at 127) 96 rows 35 / 36, 127 rows 39 / 36; 8 of 1024 x 1536 64 rows 43 / 45, 96
+    rows 48 / 45; 4 of 2048 x 4096 (2.4 at 40, 4.7 at 96) 64 rows 76 / 85, 96 rows 88 / 87; one of 4096 x 11008 127 rows 135 / 163.
+    Where the line is wrong: 16 of 2048 x 1536 at 24 rows 73 / 79 and 2 of 4096 x 4096 (3.5 at 96) at 96 rows 85 / 100 go to the large
+    tiles, 16 of 2048 x 768 at 32 rows 54 / 53 to the small ones."""
     mean = ((W + 256) * F + (F + 256) * W) / (W + F + 512)
     waves_per_cu = (pairs / 32 + E / 2) * mean / 32 / 256
     return "tiles128" if pairs >= 24 * E and waves_per_cu >= 3.5 else "grouped"
