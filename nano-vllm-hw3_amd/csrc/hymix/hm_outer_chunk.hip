@@ -6,41 +6,53 @@
 // (state-space form: W = beta v), and then
 //   o_t = rq_t (G_t S^T q_t + sum_{i <= t} D_ti rk_i (q_t . k_i) w_i) + skip v_t,   S <- G_31 S + sum_i D_31,i rk_i k_i w_i^T.
 // Everything that does not depend on the state is worked out for all chunks at once (prepare): P_ti = rq_t rk_i (q_t . k_i) D_ti,
-// T = (I + A)^-1 by forward substitution, and four numbers per token.  The walk over a sequence's chunks is left with five
-// products per chunk: K S, Q S, T R, P W and K^T W.
+// N = (I + A)^-1 - I by forward substitution, and four numbers per token.  The walk over a sequence's chunks is left with five
+// products per chunk: K S, Q S, N R (W = R + N R), P W and K^T W.
 //
-// Precision: the stored q, k are bf16 and enter the products exactly; every float32 operand (S, T, R, P, W) enters as the sum of
+// Precision: the stored q, k are bf16 and enter the products exactly; every float32 operand (S, N, R, P, W) enters as the sum of
 // three bf16 numbers, which is the number itself, and of the nine products of two such sums the six above 2^-24 of the result
-// are kept, the leading one in a sum of its own; sums are float32, products of decays double.  Against float64 the results are as near
-// as the token-by-token walk's: 8 prompts of 900 to 1100 tokens, 16 heads: gated delta 128 x 128 o 2.7e-7 of its norm (walk 2.95e-7),
-// state 4.4e-7 (4.8e-7); state space 128 x 64 o 1.68e-7 (1.68e-7), state 3.19e-7 (3.25e-7).  A token that is not finite spoils
+// are kept, the leading one in a sum of its own; sums are float32, products of decays double.  Against float64 the results are nearer
+// than the token-by-token walk's: 8 prompts of 900 to 1100 tokens, 16 heads: gated delta 128 x 128 o 2.6e-7 of its norm (walk 2.95e-7),
+// state 4.2e-7 (4.8e-7); state space 128 x 64 o 1.68e-7 (1.68e-7), state 3.19e-7 (3.25e-7).  A token that is not finite spoils
 // its own and later tokens, as in the walk, and none in front of it.
 //
-// The walk is one workgroup of two waves per (sequence, head, 32 value channels), half of the keys each, the state in the
-// accumulators of the products: lane l holds column l & 31 and the keys 32 blk + 16 (r >> 3) + 8 (l >> 5) + (r & 7) of its wave's,
-// register r.  That is the order in which a lane's eight numbers of a B operand come (8 keys in a row: a row of K or Q is read from
-// LDS in 16-byte pieces as the A operand), so the state never moves; strengths and results keep tokens (r & 3) + 8 (r >> 2) +
-// 4 (l >> 5) per lane, and the prepared A operands are stored in that order.  The waves add up their parts of K S in LDS, work out the
-// same strengths, and give each other half of the results' rows at the next meeting, so that both have the same work.
+// The walk is one workgroup of 2 NW waves per (sequence, head, 16 NW value channels).  Wave w < NW keeps 16 columns of the state in the
+// accumulators of its products: lane l holds column l & 15 and of every 32 keys 8 (l >> 4) + 0..7.  That is the order in which a lane's
+// eight numbers of a B operand come (a row of K or Q is read from LDS in 16-byte pieces as the A operand), so the state never moves; the
+// 32 tokens' strengths lie in the lanes as 4 (l >> 4) + 0..3 and 16 further, and the prepared A operands are stored in that order.
+// Its partner w + NW, on the same SIMD with four columns' waves, asks for the chunks two ahead and makes the results of the chunk before
+// from the strengths that it is handed through LDS.  One meeting per chunk.
 //
 // Against the walk that takes token after token, bound by the float32 vector unit and its chain of lane sums at two waves per
-// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 29 (prepare) + 117 (walk), 3.1 us per chunk at one wave
-// per SIMD: 800 vector instructions, five cycles each (a third of them the splits), 0.8 us of matrix work, the rest their chain K S -> R -> W -> S
-// and its waits.  The walk took 143 with numbers split one at a time (each rounded once more to be packed), the waves' halves of the results chosen
-// element by element (through indexed moves) and the products' results in the accumulation registers (a copy for every number read).
-// Four waves of 32 keys: 195 us (the strengths worked out four times); results all in one wave, v read from global memory: 175 us.
+// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 29 (prepare) + 74 (walk); one such prompt 49 us (walk).
+// What is left of a chunk's 3800 cycles: the chain S -> K S -> R -> W -> S of one wave, 380 vector instructions of 4.5 cycles (8 for a
+// conversion to bf16) and 85 matrix ones of 16, next to 3300 cycles of its partner, and LDS (58 KB per chunk and 16 columns).
+// With two waves of half the keys each on 32 columns, which both work out the strengths and give each other parts of the results in
+// LDS, the walk took 118 (one prompt: 90); one wave per SIMD with all of a chunk's work 99 (75); the state's terms handed on
+// through LDS so that the partner makes Q S too 85 (63: LDS is then the bound); results in double here as well 78 (57).
 #include "hm_attn_tile.h"
 #include "hm_outer.h"
-
-#include <type_traits>
 
 namespace hm {
 
 constexpr int kChunk = 32;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-// bytes of a prepared (chunk, head): P as three terms of an A operand, the tokens' coefficients, T as P
-constexpr int kTermBytes = 2 * 64 * 16, kOperand = 3 * kTermBytes, kCoefAt = kOperand, kEndAt = kCoefAt + kChunk * 16, kTAt = kOperand + 1024,
-              kPrepared = kTAt + kOperand;
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
+typedef bf16_t bf16x4 __attribute__((ext_vector_type(4)));
+
+// A prepared (chunk, head): P, and T with the delta form, as A operands of 16 rows (tokens): three terms each, of rows 0..15 the
+// columns 0..15 (the others are zero), of rows 16..31 all; four coefficients per token; the whole chunk's decay.  Column 8 g + e of a
+// lane's eight stands for token 4 g + e, or 16 + 4 g + e - 4 from e = 4 on: the order in which a lane holds strengths.
+constexpr int kTermLow = 64 * 8, kTermBytes = kTermLow + 64 * 16, kOperand = 3 * kTermBytes, kPrepared = 10240;
+constexpr int kBeta = 0, kOldKey = kChunk, kOldQuery = 2 * kChunk, kLeft = 3 * kChunk;       // beta, beta G rk, G rq, D_31 rk (state space: D_31 beta)
+template <bool DELTA>
+struct Prepared {
+    static constexpr int kTAt = kOperand, kCoefAt = DELTA ? 2 * kOperand : kOperand, kEndAt = kCoefAt + kChunk * 16,
+                         kPieces = (kEndAt + 4 + 1023) / 1024;
+    static_assert(1024 * kPieces <= kPrepared, "whole pieces are read");
+};
 
 // chunks are numbered q0 / 32 + b + chunk: numbers of different sequences never meet
 __device__ __forceinline__ size_t prepared_at(int q0, int b, int chunk, int h, int H) {
@@ -49,42 +61,97 @@ __device__ __forceinline__ size_t prepared_at(int q0, int b, int chunk, int h, i
 
 struct Terms { bf16x8 v[3]; };              // x = v[0] + v[1] + v[2], exactly
 
-__device__ __forceinline__ Terms split8(const float* x) {
-    // (two at a time: one conversion rounds and packs both; element by element the compiler rounds every number once more to pack it)
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef bf16_t bf16x2 __attribute__((ext_vector_type(2)));
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+// a - u[0], b - u[1] (exact): a product with (-1, 0) and (0, -1) added up.  The factors are kept from the compiler, which would take
+// them for the inline constant -1.0 and that for both halves.
+struct Minus {
+    bf16x2 lo, hi;
+    __device__ __forceinline__ Minus() {
+        unsigned l = 0x0000BF80u, h = 0xBF800000u;
+        asm volatile("" : "+s"(l), "+s"(h));
+        lo = __builtin_bit_cast(bf16x2, l);
+        hi = __builtin_bit_cast(bf16x2, h);
+    }
+};
+
+// each term the nearest bf16 to what the terms in front of it leave: products of two such sums may drop what is below 2^-24 of them
+// (here and below all numbers term by term: a dot product's result may be read three instructions later)
+__device__ __forceinline__ Terms split8(const float* x, const Minus& minus) {
     u32x4 t[3];
+    float a[8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        float a = x[2 * e], b = x[2 * e + 1];
+    for (int e = 0; e < 8; ++e) a[e] = x[e];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
-            t[j][e] = u;
-            a -= __builtin_bit_cast(float, u << 16);
-            b -= __builtin_bit_cast(float, u & 0xFFFF0000u);
-        }
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[j][e] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a[2 * e], a[2 * e + 1]}), bf16x2));
+        if (j < 2)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const unsigned u = t[j][e / 2];
+                a[e] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, u), e & 1 ? minus.hi : minus.lo, a[e], false);
+            }
     }
     return {__builtin_bit_cast(bf16x8, t[0]), __builtin_bit_cast(bf16x8, t[1]), __builtin_bit_cast(bf16x8, t[2])};
 }
 
-// big += a b of the leading terms, small += the five products down to 2^-24 of it: the large sums take few roundings
-__device__ __forceinline__ void mul_terms(const bf16x8* a, const Terms& b, f32x16& big, f32x16& small) {
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b.v[0], small, 0, 0, 0);
-    big = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b.v[0], big, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b.v[2], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b.v[1], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b.v[1], small, 0, 0, 0);
-    small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b.v[0], small, 0, 0, 0);
+// each term the upper 16 bits of what the terms in front of it leave (the conversion takes twice as long): for products with numbers
+// that are bf16 themselves, of which none is dropped
+__device__ __forceinline__ Terms cut8(const float* x, const Minus& minus) {
+    u32x4 t[3];
+    float a[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = x[e];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            t[j][e] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, a[2 * e + 1]), __builtin_bit_cast(unsigned, a[2 * e]), 0x07060302u);
+        if (j < 2)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const unsigned u = t[j][e / 2];
+                a[e] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, u), e & 1 ? minus.hi : minus.lo, a[e], false);
+            }
+    }
+    return {__builtin_bit_cast(bf16x8, t[0]), __builtin_bit_cast(bf16x8, t[1]), __builtin_bit_cast(bf16x8, t[2])};
 }
 
-__device__ __forceinline__ f32x16 zeros() {
-    f32x16 z;
+__device__ __forceinline__ f32x4 zeros4() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
+
+// A lower triangular prepared operand (32 x 32), a lane's part
+struct Lower {
+    s16x4 a0[3];
+    bf16x8 a1[3];
+    __device__ __forceinline__ void read(const unsigned char* op, int lane) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) z[r] = 0.f;
-    return z;
-}
+        for (int j = 0; j < 3; ++j) {
+            a0[j] = *(const s16x4*)(op + j * kTermBytes + 8 * lane);
+            a1[j] = *(const bf16x8*)(op + j * kTermBytes + kTermLow + 16 * lane);
+        }
+    }
+    // times 16 columns of strengths: rows 0..15 in [0], 16..31 in [1].  big has the products of the leading terms (of rows 16..31 and columns
+    // 16..31: more), small the five down to 2^-24 of them: the large sums take few roundings.
+    __device__ __forceinline__ void times(const Terms& b, f32x4 (&big)[2], f32x4& more, f32x4 (&small)[2]) const {
+        s16x4 b0[3], b1;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const s16x8 x = __builtin_bit_cast(s16x8, b.v[j]);
+            b0[j] = s16x4{x[0], x[1], x[2], x[3]};
+            if (j == 0) b1 = s16x4{x[4], x[5], x[6], x[7]};
+        }
+        const s16x8 a = __builtin_bit_cast(s16x8, a1[0]);
+        constexpr int A[5] = {2, 0, 1, 0, 1}, B[5] = {0, 2, 1, 1, 0};
+        big[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0[0], b0[0], zeros4(), 0, 0, 0);
+        big[1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(s16x4{a[0], a[1], a[2], a[3]}, b0[0], zeros4(), 0, 0, 0);
+        more = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(s16x4{a[4], a[5], a[6], a[7]}, b1, zeros4(), 0, 0, 0);
+        small[0] = small[1] = zeros4();
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            small[0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0[A[i]], b0[B[i]], small[0], 0, 0, 0);
+            small[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[A[i]], b.v[B[i]], small[1], 0, 0, 0);
+        }
+    }
+};
 
 __device__ __forceinline__ float lane_value(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -141,16 +208,32 @@ __global__ __launch_bounds__(64) void outer_chunk_prepare_kernel(const bf16_t* _
         p[r] = i <= l31 ? rq * (qk[r] * m) : 0.f;             // (chosen, not multiplied: a later token's NaN stays out)
         if (DELTA) a[r] = i < l31 ? beta * rk * (kk[r] * m) : 0.f;
     }
+    // row l31 of an operand from its columns 4 hi.., 16 + 4 hi.. (quarter hi) and 8 + 4 hi.., 24 + 4 hi.. (quarter 2 + hi)
+    const Minus minus;
+    auto put = [&](unsigned char* op, const float* lo, const float* up) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        const Terms t = split8(p + 8 * ks);
+        for (int u = 0; u < 2; ++u) {
+            const float y[8] = {lo[4 * u], lo[4 * u + 1], lo[4 * u + 2], lo[4 * u + 3], up[4 * u], up[4 * u + 1], up[4 * u + 2], up[4 * u + 3]};
+            const Terms t = split8(y, minus);
+            const int at = 16 * (2 * u + hi) + (l31 & 15);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) *(bf16x8*)(out + j * kTermBytes + ks * 1024 + 16 * lane) = t.v[j];
+            for (int j = 0; j < 3; ++j) {
+                const i32x4 x = __builtin_bit_cast(i32x4, t.v[j]);
+                typedef int i32x2 __attribute__((ext_vector_type(2)));
+                if (l31 < 16) *(i32x2*)(op + j * kTermBytes + 8 * at) = i32x2{x[0], x[1]};
+                else *(i32x4*)(op + j * kTermBytes + kTermLow + 16 * at) = x;
+            }
+        }
+    };
+    put(out, p, p + 8);
+    if (hi == 0) {
+        float* coef = (float*)(out + Prepared<DELTA>::kCoefAt);
+        coef[kBeta + l31] = beta;
+        coef[kOldKey + l31] = (float)(Gt * (double)(beta * rk));
+        coef[kOldQuery + l31] = (float)(Gt * (double)rq);
+        coef[kLeft + l31] = (float)(DELTA ? dend * (double)rk : dend * (double)beta);
     }
-    if (hi == 0)
-        *(float4*)(out + kCoefAt + 16 * l31) =
-            make_float4(beta, (float)(Gt * (double)(beta * rk)), (float)(Gt * (double)rq), (float)(dend * (double)rk));
-    if (lane == 0) *(float*)(out + kEndAt) = (float)end;
+    if (lane == 0) *(float*)(out + Prepared<DELTA>::kEndAt) = (float)end;
     if constexpr (DELTA) {
         // a token's row that is not finite is left out here (the rows of earlier tokens would multiply it by zero) and put in below
         float z = 0.f;
@@ -177,295 +260,335 @@ __global__ __launch_bounds__(64) void outer_chunk_prepare_kernel(const bf16_t* _
             }
             x[j] = j == l31 ? 1.f : j < l31 ? -((s[0] + s[1]) + (s[2] + s[3])) : 0.f;
         }
+        float lo[8], up[8];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            float y[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int i = 16 * ks + (e & 3) + 8 * (e >> 2);
-                y[e] = (hi ? x[i + 4] : x[i]) + z;
-            }
-            const Terms t = split8(y);
-#pragma unroll
-            for (int j = 0; j < 3; ++j) *(bf16x8*)(out + kTAt + j * kTermBytes + ks * 1024 + 16 * lane) = t.v[j];
+        for (int e = 0; e < 8; ++e) {
+            const int i = (e & 3) + 8 * (e >> 2);
+            const int t = i + 4 * hi;                         // (the diagonal's ones stay out: W = R + N R)
+            lo[e] = (t == l31 ? 0.f : hi ? x[i + 4] : x[i]) + z;
+            up[e] = (t + 16 == l31 ? 0.f : hi ? x[16 + i + 4] : x[16 + i]) + z;
         }
+        put(out + Prepared<DELTA>::kTAt, lo, up);
     }
 }
 
-// The first of a column's 32 tokens (16 in this lane, 16 in the one 32 further) whose x is not finite, its non-finite x made zero; 32
-// where there is none.  The triangular products multiply a token by zeros above the diagonal, and zero times infinity is not zero.
-__device__ __forceinline__ int first_spoiled(float* x, int hi) {
-    float z = 0.f;
+__device__ __forceinline__ bool spoiled(const float* x) {
+    float z0 = 0.f, z1 = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) z = __builtin_fmaf(x[r], 0.f, z);
-    if (!__any(!(z == 0.f))) return kChunk;
+    for (int r = 0; r < 4; ++r) {
+        z0 = __builtin_fmaf(x[r], 0.f, z0);
+        z1 = __builtin_fmaf(x[4 + r], 0.f, z1);
+    }
+    const float z = z0 + z1;
+    return __builtin_expect(__any(!(z == 0.f)), 0);
+}
+
+// The first of a column's 32 tokens (8 in this lane, the others in those 16, 32 and 48 further) whose x is not finite, its non-finite x
+// made zero; 32 where there is none.  The triangular products multiply a token by zeros above the diagonal, and zero times infinity is not zero.
+__device__ __forceinline__ int first_spoiled(float* x, int g) {
     int first = kChunk;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(x[r]));      // (or the comparisons are made in front of the branch)
+    for (int r = 0; r < 8; ++r) asm volatile("" : "+v"(x[r]));       // (or the comparisons are made in front of the caller's branch)
 #pragma unroll
-    for (int r = 15; r >= 0; --r)
+    for (int r = 7; r >= 0; --r)
         if (!(fabsf(x[r]) <= 3.402823466e38f)) {
             x[r] = 0.f;
-            first = (r & 3) + 8 * (r >> 2) + 4 * hi;
+            first = (r & 3) + 16 * (r >> 2) + 4 * g;
         }
+    first = min(first, __shfl_xor(first, 16));
     return min(first, __shfl_xor(first, 32));
 }
 
-template <int DK, bool DELTA>
-__global__ __launch_bounds__(128, 1) void outer_chunk_walk_kernel(const bf16_t* __restrict__ rows, int64_t stride, int q_off, int k_off,
-                                                                  int v_off, const unsigned char* __restrict__ work,
-                                                                  const float* __restrict__ skip_w, float* __restrict__ state,
-                                                                  const int32_t* __restrict__ qstart, const int32_t* __restrict__ seq_pos0,
-                                                                  const int32_t* __restrict__ seq_slot, float* __restrict__ o, int H, int G,
-                                                                  int V) {
-    constexpr int NB = DK / 64;                               // blocks of 32 keys of a wave
+template <int DK, int NW, bool DELTA>
+__global__ __launch_bounds__(128 * NW) void outer_chunk_walk_kernel(const bf16_t* __restrict__ rows, int64_t stride, int q_off, int k_off,
+                                                                    int v_off, const unsigned char* __restrict__ work,
+                                                                    const float* __restrict__ skip_w, float* __restrict__ state,
+                                                                    const int32_t* __restrict__ qstart, const int32_t* __restrict__ seq_pos0,
+                                                                    const int32_t* __restrict__ seq_slot, float* __restrict__ o, int H, int G,
+                                                                    int V) {
+    constexpr int KS = DK / 32;                               // steps of 32 keys
     typedef SlimGeom<DK / 32> GM;
+    typedef Prepared<DELTA> PR;
     typedef __attribute__((address_space(1))) const void gvoid;
     typedef __attribute__((address_space(3))) void lvoid;
     constexpr int ROWS = kChunk * GM::RB, PREP = 2 * ROWS;    // bytes of a chunk's K (and Q); where its prepared part lies
-    constexpr int KQ = ROWS / 2048, NP = (DELTA ? kPrepared : kTAt) / 1024, VAT = PREP + 1024 * NP;
-    __shared__ __attribute__((aligned(1024))) unsigned char buf0[VAT + kChunk * 64];
-    __shared__ __attribute__((aligned(1024))) unsigned char buf1[VAT + kChunk * 64];
-    // Either wave's part of K S, and of the other's rows of results.  swap_k: written between a chunk's first and second meeting, read
-    // behind the second one.  swap_o: wave w reads swap_o[.][w] of chunk c behind the first meeting of chunk c + 1, and the other wave
-    // writes the place again at the end of a chunk.  The delta form's second meeting lies between the two; the state-space form
-    // has one meeting per chunk, so its chunks take two places in turn, and the first meeting of chunk c + 2 lies between.
-    __shared__ __attribute__((aligned(16))) f32x4 swap_k[2][4][64], swap_o[DELTA ? 1 : 2][2][2][64];
-    const int b = blockIdx.x, h = blockIdx.y, gr = h / (H / G), lane = threadIdx.x & 63, l31 = lane & 31, hi = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int col = blockIdx.z * 32 + l31;
+    constexpr int KQ = ROWS / (1024 * NW), VAT = PREP + 1024 * PR::kPieces, VP = 32 * NW;         // (VP: bytes of a row of V)
+    constexpr int LOADS = 2 * KQ + 1 + PR::kPieces / NW;      // a wave's per chunk, at least
+    __shared__ __attribute__((aligned(1024))) unsigned char buf0[VAT + kChunk * VP];
+    __shared__ __attribute__((aligned(1024))) unsigned char buf1[VAT + kChunk * VP];
+    __shared__ __attribute__((aligned(1024))) unsigned char buf2[VAT + kChunk * VP];
+    // what a chunk's results are made of: the strengths and the state's part (state space: a double in two numbers), read behind the next
+    // meeting while the next chunk's are written to the other half
+    constexpr int GIVEN = DELTA ? 4 : 6;
+    __shared__ __attribute__((aligned(16))) f32x4 given[2][NW][GIVEN][64];
+    const int b = blockIdx.x, h = blockIdx.y, gr = h / (H / G), lane = threadIdx.x & 63, l15 = lane & 15, g = lane >> 4;
+    const int warp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = warp % NW;
+    const int col = (blockIdx.z * NW + wave) * 16 + l15;
     const int q0 = qstart[b], n = qstart[b + 1] - q0;
     if (n <= 0) return;
-    float* st = state + ((size_t)seq_slot[b] * H + h) * (size_t)DK * V + (size_t)(32 * NB * wave + 8 * hi) * V + col;
-    const bool fresh = seq_pos0[b] == 0;
-    const float skip = DELTA ? 0.f : skip_w[h];
-    f32x16 S[NB];
-#pragma unroll
-    for (int blk = 0; blk < NB; ++blk)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) S[blk][r] = fresh ? 0.f : st[(size_t)(32 * blk + 16 * (r >> 3) + (r & 7)) * V];
+    const int r_at = GM::at(l15, g);                          // row l15, chunk g (8 keys), as the A operand of K S and Q S
+    const int v_at = VP * (4 * g + (l15 >> 2)) + 32 * wave + 8 * (l15 & 3);        // the wave's columns of V, by the transposing read
+    const Minus minus;
 
-    const bf16_t *ks0 = rows + (size_t)q0 * stride + k_off + (size_t)gr * DK, *qs0 = rows + (size_t)q0 * stride + q_off + (size_t)gr * DK;
-    const bf16_t* vs0 = rows + (size_t)q0 * stride + v_off + (size_t)h * V + blockIdx.z * 32;
-    // a chunk's K, Q, V (rows past the end: the last one, cleared before use) and prepared part: 1 KB pieces to the two waves in turn
-    int row_of[KQ], ch_of[KQ];
-    size_t off_of[KQ];
-#pragma unroll
-    for (int j = 0; j < KQ; ++j) {
-        const int c = 64 * (2 * j + wave) + lane;
-        row_of[j] = c / GM::CH;
-        ch_of[j] = 8 * ((c % GM::CH) ^ GM::swz(row_of[j]));
-        off_of[j] = (size_t)row_of[j] * stride + ch_of[j];
-    }
-    const int v_row = 16 * wave + (lane >> 2);
-    auto load_chunk = [&](unsigned char* buf, int t0) {
-        const unsigned char* prep = work + prepared_at(q0, b, t0 / kChunk, h, H) + 1024 * wave + 16 * lane;
-        const bool whole = t0 + kChunk <= n;
-        __builtin_amdgcn_global_load_lds((gvoid*)(vs0 + (size_t)min(t0 + v_row, n - 1) * stride + 8 * (lane & 3)),
-                                         (lvoid*)(buf + VAT + 1024 * wave), 16, 0, 0);
-#pragma unroll
-        for (int j = 0; j < KQ; ++j) {
-            const size_t off = whole ? (size_t)t0 * stride + off_of[j] : (size_t)min(t0 + row_of[j], n - 1) * stride + ch_of[j];
-            const int at = 1024 * (2 * j + wave);
-            __builtin_amdgcn_global_load_lds((gvoid*)(ks0 + off), (lvoid*)(buf + at), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((gvoid*)(qs0 + off), (lvoid*)(buf + ROWS + at), 16, 0, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < NP / 2; ++j)
-            __builtin_amdgcn_global_load_lds((gvoid*)(prep + 2048 * j), (lvoid*)(buf + PREP + 1024 * (2 * j + wave)), 16, 0, 0);
-        if (NP % 2 && wave == 0)
-            __builtin_amdgcn_global_load_lds((gvoid*)(prep + 1024 * (NP - 1)), (lvoid*)(buf + PREP + 1024 * (NP - 1)), 16, 0, 0);
-    };
-    // row l31, chunk 2 (16 keys) + hi, as the A operand of K S and Q S; columns of K for K^T W by the transposing read, the two
-    // middle quads of 16 keys exchanged (the state's order of keys)
-    const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, pq = ((ti & 1) << 1) | ((ti >> 1) & 1);
-    const int r_at = GM::at(l31, hi) ^ (64 * NB * wave), c_at = (GM::at(4 * hi + tq, 2 * gq + (pq >> 1)) + 8 * (pq & 1)) ^ (64 * NB * wave),
-              v_at = 64 * (4 * hi + tq) + 32 * gq + 8 * (ti & 3),
-              c_at8 = (GM::at(4 * hi + tq + 8, 2 * gq + (pq >> 1)) + 8 * (pq & 1)) ^ (64 * NB * wave);
-
-    // LDS accesses of both waves in front of it are done; loads from global memory go on (__syncthreads would wait for them)
+    // LDS accesses of all waves in front of it are done; loads from global memory go on (__syncthreads would wait for them)
     auto meet = [&]() {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    double part[8];                                          // the last chunk's results of tokens 16 wave..: this wave's part
-    // (in double: in float32 the state-space form's error was 1 to 5 % above the token-by-token walk's; 1 us, measured when the walk took 142)
-    // their sum with the other wave's part, written before the last meeting (turn: 0 for an even chunk of the portion, 1 for an odd one)
-    auto store_rows = [&](int t0, bool whole, int turn) {
-        float* orow = o + ((size_t)(q0 + t0 + 16 * wave + 4 * hi) * H + h) * V + col;
-#pragma unroll
-        for (int r4 = 0; r4 < 2; ++r4) {
-            const f32x4 y = swap_o[DELTA ? 0 : turn][wave][r4][lane];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = e + 8 * r4;
-                if (whole || t0 + 16 * wave + 4 * hi + t < n) orow[(size_t)t * H * V] = (float)(part[4 * r4 + e] + (double)y[e]);
-            }
+    auto clear_absent = [&](unsigned char* buf, int left) {   // an absent token's row: zeros, whatever the one in its place holds
+        for (int i = left * GM::RB + 16 * (int)threadIdx.x; i < ROWS; i += 2048 * NW) {
+            *(i32x4*)(buf + i) = i32x4{0, 0, 0, 0};
+            *(i32x4*)(buf + ROWS + i) = i32x4{0, 0, 0, 0};
+        }
+        for (int i = left * VP + 16 * (int)threadIdx.x; i < kChunk * VP; i += 2048 * NW) *(i32x4*)(buf + VAT + i) = i32x4{0, 0, 0, 0};
+        meet();
+    };
+    auto transposed = [&](const unsigned char* at) {
+        return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)at));
+    };
+    auto in_turn = [&](auto&& chunk) {
+        for (int t0 = 0, turn = 0; t0 < n; t0 += 3 * kChunk, turn ^= 1) {
+            chunk(buf0, buf2, t0, turn);
+            if (t0 + kChunk < n) chunk(buf1, buf0, t0 + kChunk, turn ^ 1);
+            if (t0 + 2 * kChunk < n) chunk(buf2, buf1, t0 + 2 * kChunk, turn);
         }
     };
-    auto chunk = [&](unsigned char* buf, unsigned char* nxt, int t0, int turn) {
-        const int left = n - t0;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the chunk has landed (and rows of results a whole chunk old)
-        meet();
-        if (t0 > 0) store_rows(t0 - kChunk, true, turn ^ 1);
-        if (left < kChunk) {                                  // an absent token's row: zeros, whatever the one in its place holds
-            for (int i = left * GM::RB + 16 * (int)threadIdx.x; i < ROWS; i += 2048) {
-                *(i32x4*)(buf + i) = i32x4{0, 0, 0, 0};
-                *(i32x4*)(buf + ROWS + i) = i32x4{0, 0, 0, 0};
-            }
-            for (int i = left * 64 + 16 * (int)threadIdx.x; i < kChunk * 64; i += 2048) *(i32x4*)(buf + VAT + i) = i32x4{0, 0, 0, 0};
+
+    if (warp < NW) {                                          // the state and the strengths
+        float* st = state + ((size_t)seq_slot[b] * H + h) * (size_t)DK * V + (size_t)(8 * g) * V + col;
+        const bool fresh = seq_pos0[b] == 0;
+        const float skip = DELTA ? 0.f : skip_w[h];
+        f32x4 S[KS][2];
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) S[ks][e >> 2][e & 3] = fresh ? 0.f : st[(size_t)(32 * ks + e) * V];
+        // columns of K for K^T W by the transposing read: rows 4 g.., of 32 keys those 8 i + 0..3, i = 0..3
+        const int c_at = GM::at(4 * g + (l15 >> 2), l15 & 3);
+        in_turn([&](unsigned char* buf, unsigned char*, int t0, int turn) __attribute__((always_inline)) {
             meet();
-        }
-        const unsigned char* prep = buf + PREP;
-        Terms s[2 * NB];                                      // the wave's part of the state, 16 keys at a time
+            if (n - t0 < kChunk) clear_absent(buf, n - t0);
+            const unsigned char* prep = buf + PREP;
+            // everything that the chunk brings is asked for before the first product
+            bf16x8 kf[KS][2], qf[KS][2];
 #pragma unroll
-        for (int ks = 0; ks < 2 * NB; ++ks) {
-            float x[8];
+            for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = S[ks >> 1][8 * (ks & 1) + e];
-            s[ks] = split8(x);
-        }
-        f32x16 ksb = zeros(), kss = zeros(), qsb = zeros(), qss = zeros();
-        if (DELTA) {                                          // each wave has its keys' part of K S
-#pragma unroll
-            for (int ks = 0; ks < 2 * NB; ++ks) {
-                const bf16x8 kf = *(const bf16x8*)(buf + (r_at ^ (32 * ks)));
-                kss = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, s[ks].v[2], kss, 0, 0, 0);
-                ksb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, s[ks].v[0], ksb, 0, 0, 0);
-                kss = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, s[ks].v[1], kss, 0, 0, 0);
-            }
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                f32x4 x;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = ksb[4 * r4 + e] += kss[4 * r4 + e];
-                swap_k[wave][r4][lane] = x;
-            }
-            meet();
-        }
-        if (t0 + kChunk < n) load_chunk(nxt, t0 + kChunk);    // (the other buffer was last read in front of the first meeting)
-        __builtin_amdgcn_sched_barrier(0);
-        float v[16];                                          // column l31 of V, by the transposing read
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (s16x4 __attribute__((address_space(3)))*)(buf + VAT + v_at + 512 * r4));
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * r4 + e] = to_f(__builtin_bit_cast(bf16_t, (short)x[e]));
-        }
-        float w[16], wd[16], cq[16];
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            f32x4 x = {0.f, 0.f, 0.f, 0.f};
-            if (DELTA) x = swap_k[wave ^ 1][r4][lane];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = 4 * r4 + e;
-                const float4 cf = *(const float4*)(prep + kCoefAt + 16 * ((r & 3) + 8 * (r >> 2) + 4 * hi));      // beta, beta G rk, G rq, D_31 rk
-                w[r] = cf.x * v[r];
-                if (DELTA) w[r] -= cf.y * (ksb[r] + x[e]);
-                cq[r] = cf.z;
-                wd[r] = cf.w;
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2 * NB; ++ks) {                 // and of Q S (independent of what surrounds it)
-            const bf16x8 qf = *(const bf16x8*)(buf + ROWS + (r_at ^ (32 * ks)));
-            qss = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, s[ks].v[2], qss, 0, 0, 0);
-            qsb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, s[ks].v[0], qsb, 0, 0, 0);
-            qss = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf, s[ks].v[1], qss, 0, 0, 0);
-        }
-        if (DELTA) {
-            f32x16 big = zeros(), small = zeros();
-            const int first = first_spoiled(w, hi);
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                bf16x8 m[3];
-#pragma unroll
-                for (int j = 0; j < 3; ++j) m[j] = *(const bf16x8*)(prep + kTAt + j * kTermBytes + ks * 1024 + 16 * lane);
-                mul_terms(m, split8(w + 8 * ks), big, small);
-            }
-#pragma unroll
-            for (int r = 0; r < 16; ++r) w[r] = big[r] + small[r];
-            if (__any(first < kChunk))
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    asm volatile("" : "+v"(w[r]));
-                    if ((r & 3) + 8 * (r >> 2) + 4 * hi >= first) w[r] = __builtin_nanf("");
+                for (int tb = 0; tb < 2; ++tb) {
+                    if (DELTA) kf[ks][tb] = *(const bf16x8*)(buf + (r_at ^ (64 * ks)) + 16 * GM::RB * tb);
+                    else qf[ks][tb] = *(const bf16x8*)(buf + ROWS + (r_at ^ (64 * ks)) + 16 * GM::RB * tb);
                 }
-        }
-        const float end = *(const float*)(prep + kEndAt);
+            const f32x4* coef = (const f32x4*)(prep + PR::kCoefAt) + g;
+            f32x4 beta[2], ck[2], cq[2], left[2];
+            bf16x4 vx[2];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) wd[r] *= w[r];
-        f32x16 ib[NB], is[NB];
-#pragma unroll
-        for (int blk = 0; blk < NB; ++blk) ib[blk] = is[blk] = zeros();
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const Terms d = split8(wd + 8 * ks);
-#pragma unroll
-            for (int blk = 0; blk < NB; ++blk) {
-                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (s16x4 __attribute__((address_space(3)))*)(buf + (c_at ^ (64 * blk)) + 16 * GM::RB * ks));
-                const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (s16x4 __attribute__((address_space(3)))*)(buf + (c_at8 ^ (64 * blk)) + 16 * GM::RB * ks));
-                const s16x8 kt8 = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
-                const bf16x8 kt = __builtin_bit_cast(bf16x8, kt8);
-                is[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, d.v[2], is[blk], 0, 0, 0);
-                ib[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, d.v[0], ib[blk], 0, 0, 0);
-                is[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, d.v[1], is[blk], 0, 0, 0);
+            for (int tb = 0; tb < 2; ++tb) {
+                vx[tb] = transposed(buf + VAT + v_at + 16 * VP * tb);
+                beta[tb] = coef[kBeta / 4 + 4 * tb];
+                if (DELTA) ck[tb] = coef[kOldKey / 4 + 4 * tb];
+                cq[tb] = coef[kOldQuery / 4 + 4 * tb];
+                left[tb] = coef[kLeft / 4 + 4 * tb];
             }
-        }
-        {                                                     // P W of the wave's half of the strengths, and the parts of the results
-            const int first = first_spoiled(w, hi);
-            if (__any(first < kChunk))
+            const float end = *(const float*)(prep + PR::kEndAt);
+            Lower N;
+            if (DELTA) N.read(prep + PR::kTAt, lane);
+            float w[8], wd[8];
+            f32x4 kb[2] = {zeros4(), zeros4()}, kl[2] = {zeros4(), zeros4()}, qb[2] = {zeros4(), zeros4()}, qc[2] = {zeros4(), zeros4()},
+                  ql[2] = {zeros4(), zeros4()};
+            Terms s[KS];                                      // the wave's columns of the state, 32 keys at a time
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    asm volatile("" : "+v"(cq[r]));
-                    if ((r & 3) + 8 * (r >> 2) + 4 * hi >= first) cq[r] = __builtin_nanf("");
+            for (int ks = 0; ks < KS; ++ks) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = S[ks][e >> 2][e & 3];
+                s[ks] = cut8(x, minus);
+                if (DELTA) {
+#pragma unroll
+                    for (int tb = 0; tb < 2; ++tb) kl[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks][tb], s[ks].v[2], kl[tb], 0, 0, 0);
+#pragma unroll
+                    for (int tb = 0; tb < 2; ++tb) kb[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks][tb], s[ks].v[0], kb[tb], 0, 0, 0);
+#pragma unroll
+                    for (int tb = 0; tb < 2; ++tb) kl[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks][tb], s[ks].v[1], kl[tb], 0, 0, 0);
                 }
-            // (one form per wave: chosen element by element, the halves go through indexed register moves)
-            auto results = [&](auto second) __attribute__((always_inline)) {
-                constexpr int KEPT = second ? 8 : 0, GIVEN = 8 - KEPT;
-                f32x16 big = zeros(), small = zeros();
-                bf16x8 m[3];
+            }
+            if (DELTA)
 #pragma unroll
-                for (int j = 0; j < 3; ++j) m[j] = *(const bf16x8*)(prep + j * kTermBytes + (KEPT / 8) * 1024 + 16 * lane);
-                mul_terms(m, split8(w + KEPT), big, small);
+                for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-                for (int r4 = 0; r4 < 2; ++r4) {
-                    f32x4 y;
+                    for (int tb = 0; tb < 2; ++tb) qf[ks][tb] = *(const bf16x8*)(buf + ROWS + (r_at ^ (64 * ks)) + 16 * GM::RB * tb);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const float v = to_f(vx[r >> 2][r & 3]);
+                w[r] = beta[r >> 2][r & 3] * v;
+                if (!DELTA) wd[r] = left[r >> 2][r & 3] * v;
+            }
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) ql[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks][tb], s[ks].v[2], ql[tb], 0, 0, 0);
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) {
+                    f32x4& q = ks < KS / 2 ? qb[tb] : qc[tb];
+                    q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks][tb], s[ks].v[0], q, 0, 0, 0);
+                }
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) ql[tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[ks][tb], s[ks].v[1], ql[tb], 0, 0, 0);
+            }
+            bf16x8 kt[KS][2];
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+                    kt[ks][half] = __builtin_shufflevector(transposed(buf + (c_at ^ (64 * ks)) + 8 * half),
+                                                           transposed(buf + (c_at ^ (64 * ks)) + 8 * half + 16 * GM::RB), 0, 1, 2, 3, 4, 5, 6, 7);
+            if (DELTA) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) w[r] -= ck[r >> 2][r & 3] * (kb[r >> 2][r & 3] + kl[r >> 2][r & 3]);
+                auto solve = [&](float* x) {
+                    f32x4 big[2], more, small[2];
+                    N.times(split8(x, minus), big, more, small);
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) x[r] += (r < 4 ? big[0][r & 3] : big[1][r & 3] + more[r & 3]) + small[r >> 2][r & 3];
+                };
+                float r0[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) r0[r] = w[r];
+                solve(w);
+                if (spoiled(w)) {                             // (a row that is not finite leaves none of its column finite)
+                    const int first = first_spoiled(r0, g);
+                    solve(r0);
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) w[r] = (r & 3) + 16 * (r >> 2) + 4 * g >= first ? __builtin_nanf("") : r0[r];
+                }
+            }
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb) {
+                f32x4* to = &given[turn][wave][tb][lane];
+                to[0] = f32x4{w[4 * tb], w[4 * tb + 1], w[4 * tb + 2], w[4 * tb + 3]};
+                if (DELTA) {
+                    to[128] = cq[tb] * (qb[tb] + (qc[tb] + ql[tb]));
+                } else {
+                    // (in double, here and where P W is added: in float32 the error was 1 to 5 % above the token-by-token walk's)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const int r = 4 * r4 + e, g = GIVEN + r, k = KEPT + r;
-                        y[e] = cq[g] * (qsb[g] + qss[g]) + (big[g] + small[g]);
-                        const double c = cq[k], qb = qsb[k], qs = qss[k], pb = big[k], ps = small[k];
-                        part[r] = c * (qb + qs) + (pb + ps);
-                        if (!DELTA) part[r] += (double)skip * (double)v[k];
+                        const double z = (double)cq[tb][e] * ((double)qb[tb][e] + (double)qc[tb][e] + (double)ql[tb][e]) +
+                                         (double)skip * (double)to_f(vx[tb][e]);
+                        to[128][e] = (float)z;
+                        to[256][e] = (float)(z - (double)(float)z);
                     }
-                    swap_o[DELTA ? 0 : turn][wave ^ 1][r4][lane] = y;
                 }
-            };
-            if (wave) results(std::true_type{});
-            else results(std::false_type{});
+            }
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+                if (DELTA) wd[r] = left[r >> 2][r & 3] * w[r];
+            const Terms d = cut8(wd, minus);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    f32x4 ib = zeros4(), is = zeros4();
+                    is = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[2], is, 0, 0, 0);
+                    ib = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[0], ib, 0, 0, 0);
+                    is = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[1], is, 0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) S[ks][half][e] = end * S[ks][half][e] + (ib[e] + is[e]);
+                }
+        });
+        meet();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) st[(size_t)(32 * ks + e) * V] = S[ks][e >> 2][e & 3];
+        return;
+    }
+
+    // the loads and the results
+    const bf16_t *ks0 = rows + (size_t)q0 * stride + k_off + (size_t)gr * DK, *qs0 = rows + (size_t)q0 * stride + q_off + (size_t)gr * DK;
+    const bf16_t* vs0 = rows + (size_t)q0 * stride + v_off + (size_t)h * V + blockIdx.z * 16 * NW;
+    // a chunk's K, Q, V (rows past the end: the last one, cleared before use) and prepared part: 1 KB pieces to the waves in turn
+    int row_of[KQ], ch_of[KQ];
+    size_t off_of[KQ];
+#pragma unroll
+    for (int j = 0; j < KQ; ++j) {
+        const int c = 64 * (NW * j + wave) + lane;
+        row_of[j] = c / GM::CH;
+        ch_of[j] = 8 * ((c % GM::CH) ^ GM::swz(row_of[j]));
+        off_of[j] = (size_t)row_of[j] * stride + ch_of[j];
+    }
+    const int v_row = (64 * wave + lane) / (2 * NW), v_ch = 8 * (lane % (2 * NW));
+    auto load_chunk = [&](unsigned char* buf, int t0) {
+        const unsigned char* prep = work + prepared_at(q0, b, t0 / kChunk, h, H) + 1024 * wave + 16 * lane;
+        const bool whole = t0 + kChunk <= n;
+        __builtin_amdgcn_global_load_lds((gvoid*)(vs0 + (size_t)min(t0 + v_row, n - 1) * stride + v_ch),
+                                         (lvoid*)(buf + VAT + 1024 * wave), 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < KQ; ++j) {
+            const size_t off = whole ? (size_t)t0 * stride + off_of[j] : (size_t)min(t0 + row_of[j], n - 1) * stride + ch_of[j];
+            const int at = 1024 * (NW * j + wave);
+            __builtin_amdgcn_global_load_lds((gvoid*)(ks0 + off), (lvoid*)(buf + at), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((gvoid*)(qs0 + off), (lvoid*)(buf + ROWS + at), 16, 0, 0);
         }
 #pragma unroll
-        for (int blk = 0; blk < NB; ++blk)
+        for (int j = 0; j < PR::kPieces / NW; ++j)
+            __builtin_amdgcn_global_load_lds((gvoid*)(prep + 1024 * NW * j), (lvoid*)(buf + PREP + 1024 * (NW * j + wave)), 16, 0, 0);
+        if (PR::kPieces % NW != 0 && wave < PR::kPieces % NW) {
+            constexpr int J = PR::kPieces / NW;
+            __builtin_amdgcn_global_load_lds((gvoid*)(prep + 1024 * NW * J), (lvoid*)(buf + PREP + 1024 * (NW * J + wave)), 16, 0, 0);
+        }
+    };
+    // what the chunk leaves in registers for its results, which are worked out behind the next meeting
+    Lower P;
+    auto results = [&](int t0, bool whole, int turn) {
+        float w[8];
+        f32x4 q[2][2];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) S[blk][r] = end * S[blk][r] + (ib[blk][r] + is[blk][r]);
+        for (int tb = 0; tb < 2; ++tb) {
+            const f32x4* from = &given[turn][wave][tb][lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[4 * tb + e] = from[0][e];
+#pragma unroll
+            for (int i = 0; i < (DELTA ? 1 : 2); ++i) q[i][tb] = from[128 * (i + 1)];
+        }
+        int first = kChunk;
+        if (spoiled(w)) first = first_spoiled(w, g);
+        f32x4 pb[2], pm, pl[2];
+        P.times(split8(w, minus), pb, pm, pl);
+        float* orow = o + ((size_t)(q0 + t0 + 4 * g) * H + h) * V + col;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int i = r & 3, tb = r >> 2, t = i + 16 * tb;
+            float y;
+            if (DELTA) {
+                y = q[0][tb][i] + (r < 4 ? pb[0][i] + pl[0][i] : pb[1][i] + (pm[i] + pl[1][i]));
+            } else {
+                double z = ((double)q[0][tb][i] + (double)q[1][tb][i]) + ((double)pb[tb][i] + (double)pl[tb][i]);
+                if (r >= 4) z += (double)pm[i];
+                y = (float)z;
+            }
+            if (t + 4 * g >= first) y = __builtin_nanf("");
+            if (whole || t0 + 4 * g + t < n) orow[(size_t)t * H * V] = y;
+        }
     };
     load_chunk(buf0, 0);
-    for (int t0 = 0; t0 < n; t0 += 2 * kChunk) {
-        chunk(buf0, buf1, t0, 0);
-        if (t0 + kChunk < n) chunk(buf1, buf0, t0 + kChunk, 1);
-    }
+    if (n > kChunk) load_chunk(buf1, kChunk);
+    in_turn([&](unsigned char* buf, unsigned char* nxt, int t0, int turn) __attribute__((always_inline)) {
+        const int left = n - t0;
+        // the chunk has landed: what was asked for behind it are the next chunk's loads and, from the third chunk on, eight rows of results
+        if (t0 > kChunk && left > kChunk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + 8) : "memory");
+        else if (t0 > kChunk) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else if (left > kChunk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        meet();
+        if (left < kChunk) clear_absent(buf, left);
+        if (left > 2 * kChunk) load_chunk(nxt, t0 + 2 * kChunk);      // (its buffer was last read in front of this meeting)
+        if (t0 > 0) results(t0 - kChunk, true, turn ^ 1);
+        const unsigned char* prep = buf + PREP;
+        P.read(prep, lane);
+    });
     meet();
-    store_rows((n - 1) / kChunk * kChunk, false, (n - 1) / kChunk & 1);
-#pragma unroll
-    for (int blk = 0; blk < NB; ++blk)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) st[(size_t)(32 * blk + 16 * (r >> 3) + (r & 7)) * V] = S[blk][r];
+    const int last = (n - 1) / kChunk;
+    results(last * kChunk, false, last & 1);
 }
 
 template <bool DELTA>
@@ -476,15 +599,20 @@ static void launch_chunks(const void* rows_, int64_t stride, int q_off, int k_of
     const int64_t items = T * G;
     hipLaunchKernelGGL((outer_gates_kernel<bf16_t, 8, DELTA>), dim3((unsigned)((items + 15) / 16)), dim3(256), 0, s, rows, stride, q_off,
                        k_off, ga, gates, items, H, G, D);
-    const dim3 pg((unsigned)((max_q + kChunk - 1) / kChunk), (unsigned)B, (unsigned)H), wg((unsigned)B, (unsigned)H, (unsigned)(V / 32));
-#define HM_CHUNKS(DK)                                                                                                              \
+    // Four waves of columns share a chunk's K, Q and prepared part, two have a SIMD each and LDS to themselves: where every CU has at most one
+    // workgroup of two, those (one prompt of 900 tokens, 16 heads of 128 x 128: 49.5 us, four 52.2; 32 heads of 128 x 64 state space 39 and
+    // 48); beyond, a CU has room for one workgroup of either and four take half the rounds.
+    const int nw = V % 64 == 0 && (int64_t)B * H * (V / 32) > 256 ? 4 : 2;
+    const dim3 pg((unsigned)((max_q + kChunk - 1) / kChunk), (unsigned)B, (unsigned)H), wg((unsigned)B, (unsigned)H, (unsigned)(V / (16 * nw)));
+#define HM_CHUNKS(DK, NW)                                                                                                              \
     do {                                                                                                                           \
         hipLaunchKernelGGL((outer_chunk_prepare_kernel<DK, DELTA>), pg, dim3(64), 0, s, rows, stride, q_off, k_off, gates, qstart,   \
                            (unsigned char*)work, H, G);                                                                            \
-        hipLaunchKernelGGL((outer_chunk_walk_kernel<DK, DELTA>), wg, dim3(128), 0, s, rows, stride, q_off, k_off, v_off,             \
+        hipLaunchKernelGGL((outer_chunk_walk_kernel<DK, NW, DELTA>), wg, dim3(128 * NW), 0, s, rows, stride, q_off, k_off, v_off,             \
                            (const unsigned char*)work, ga.skip, state, qstart, seq_pos0, seq_slot, o, H, G, V);                    \
     } while (0)
-    if (D == 64) HM_CHUNKS(64); else HM_CHUNKS(128);
+    if (nw == 4) { if (D == 64) HM_CHUNKS(64, 4); else HM_CHUNKS(128, 4); }
+    else { if (D == 64) HM_CHUNKS(64, 2); else HM_CHUNKS(128, 2); }
 #undef HM_CHUNKS
 }
 

@@ -281,6 +281,33 @@ def test_long_portions_by_chunks_keep_every_chunks_results(monkeypatch, kind, H,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["delta", "space"])
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 64), (128, 128)])
+def test_chunk_walks_of_two_and_four_waves_agree(kind, D, V):
+    """Workgroups have 32 value channels up to 256 of them and 64 beyond: a column's sums are the same, so the bits are.  Portions of one,
+    two, three and four chunks, the last ones whole and of a single token (each takes another turn of the buffers)."""
+    g = gen(D + V)
+    H, lens = 4, [128, 65, 96, 64, 97, 33, 128, 32]
+    n = sum(lens)
+    rows, pre = rnd(g, n, 2 * D + H * V, dtype=torch.bfloat16).cuda(), rnd(g, n, 2 * H, s=2.0, dtype=torch.bfloat16).cuda()
+    A, bias, skip = (t.cuda() for t in (*forget(g, H), rnd(g, H)))
+    outs = []
+    few = 256 // (H * (V // 32) * len(lens))                            # copies of the batch that 256 workgroups of two hold
+    for copies in (1, few, few + 1):
+        ctx, _ = batch([(0, m) for m in lens] * copies, device="cuda", seed=2)
+        st = torch.full((max(int(s) for s in ctx.seq_slot) + 1, H, D, V), 7.0, device="cuda")
+        x, p = rows.repeat(copies, 1), pre.repeat(copies, 1)
+        assert hy_ops._outer_chunked(x, (0, D, 2 * D), D, V, ctx)
+        if kind == "delta":
+            o = hy_ops.gated_delta(x, 0, D, 2 * D, p, 0, H, A, bias, H, 1, D, V, st, ctx)
+        else:
+            o = hy_ops.state_space(x, 2 * D, 0, D, p, 0, A, bias, skip, H, 1, D, V, st, ctx)
+        outs.append((o.view(copies, n, H, V), st[ctx.seq_slot.long()].view(copies, len(lens), H, D, V)))
+    for o, st in outs:
+        assert torch.isfinite(o).all() and (o == outs[0][0]).all() and (st == outs[0][1]).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("D,V", [(32, 64), (64, 128), (128, 64), (256, 72)])
 def test_recurrence_forms_agree(dtype, D, V):
