@@ -24,7 +24,7 @@
 // from the strengths that it is handed through LDS.  One meeting per chunk.
 //
 // Against the walk that takes token after token, bound by the float32 vector unit and its chain of lane sums at two waves per
-// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 29 (prepare) + 74 (walk); one such prompt 49 us (walk).
+// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 22 (prepare) + 72 (walk); one such prompt 9 + 49 us.
 // What is left of a chunk's 3800 cycles: the chain S -> K S -> R -> W -> S of one wave, 380 vector instructions of 4.5 cycles (8 for a
 // conversion to bf16) and 85 matrix ones of 16, next to 3300 cycles of its partner, and LDS (58 KB per chunk and 16 columns).
 // With two waves of half the keys each on 32 columns, which both work out the strengths and give each other parts of the results in
@@ -75,23 +75,29 @@ struct Minus {
 
 // each term the nearest bf16 to what the terms in front of it leave: products of two such sums may drop what is below 2^-24 of them
 // (here and below all numbers term by term: a dot product's result may be read three instructions later)
-__device__ __forceinline__ Terms split8(const float* x, const Minus& minus) {
-    u32x4 t[3];
-    float a[8];
+template <int N>
+__device__ __forceinline__ void split(const float* x, const Minus& minus, unsigned (&t)[3][N / 2]) {
+    float a[N];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) a[e] = x[e];
+    for (int e = 0; e < N; ++e) a[e] = x[e];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[j][e] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a[2 * e], a[2 * e + 1]}), bf16x2));
+        for (int e = 0; e < N / 2; ++e) t[j][e] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a[2 * e], a[2 * e + 1]}), bf16x2));
         if (j < 2)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const unsigned u = t[j][e / 2];
-                a[e] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, u), e & 1 ? minus.hi : minus.lo, a[e], false);
-            }
+            for (int e = 0; e < N; ++e)
+                a[e] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, t[j][e / 2]), e & 1 ? minus.hi : minus.lo, a[e], false);
     }
-    return {__builtin_bit_cast(bf16x8, t[0]), __builtin_bit_cast(bf16x8, t[1]), __builtin_bit_cast(bf16x8, t[2])};
+}
+
+__device__ __forceinline__ Terms split8(const float* x, const Minus& minus) {
+    unsigned t[3][4];
+    split<8>(x, minus, t);
+    Terms r;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) r.v[j] = __builtin_bit_cast(bf16x8, (u32x4{t[j][0], t[j][1], t[j][2], t[j][3]}));
+    return r;
 }
 
 // each term the upper 16 bits of what the terms in front of it leave (the conversion takes twice as long): for products with numbers
@@ -153,122 +159,235 @@ struct Lower {
     }
 };
 
-__device__ __forceinline__ float lane_value(float v, int lane) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+template <int CTRL>
+__device__ __forceinline__ float of_quad(float v) {            // the value of lane CTRL / 0x55 of each four
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
-// One wave per (chunk, sequence, head).  Lane l stands for token l & 31.
+// One wave per (chunk, sequence, head), from the rows and the gates' pre-activations.  Lane (l15, g4) has the products of tokens t = l15
+// and 16 + l15 with the tokens i = 4 g4 + 0..3 and 16 + 4 g4 + 0..3: as the 16-row products leave them and as the walk reads them, so
+// they are stored as they lie.
+//
+// The decays D_ti are products in double, put together from quads of tokens: t's part of its quad, the quads between, the rest of
+// i's quad; a product of up to 32 decays is the one place where the chunk would round more often than the token-by-token walk does.
+// (I + A)^-1 by blocks of 16: T11 and T22 by forward substitution, a column per lane, T21 = -T22 A21 T11 by the float32 matrix products.
+//
+// 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 22 us (state space, 32 heads of 128 x 64: 26) of which the stores are 5, 4096 waves of
+// 990 vector instructions and a way of 6 us each (one prompt: 9 us).  With a kernel of its own for the gates in front, products of
+// decays token by token and the whole of (I + A)^-1 by substitution in 32 lanes of 64 it was 32 + 11 (27 + 12; 11 + 5).  Four chunks
+// per workgroup, or a group's heads side by side on one die: no difference.
 template <int DK, bool DELTA>
 __global__ __launch_bounds__(64) void outer_chunk_prepare_kernel(const bf16_t* __restrict__ rows, int64_t stride, int q_off, int k_off,
-                                                                 const float* __restrict__ gates, const int32_t* __restrict__ qstart,
+                                                                 GateArgs<bf16_t> ga, const int32_t* __restrict__ qstart,
                                                                  unsigned char* __restrict__ work, int H, int G) {
-    constexpr int PITCH = 36;
-    __shared__ __attribute__((aligned(16))) float at[kChunk * PITCH];          // column j of A, row by row
+    constexpr int AP = 36, TP = 20;                           // floats between rows of A, columns of T: whole 16 bytes, every bank once
+    typedef Prepared<DELTA> PR;
+    __shared__ double own[kChunk], rest[kChunk], quad[8], between[8][8];
+    __shared__ f32x4 inside[kChunk], token[kChunk];
+    __shared__ __attribute__((aligned(16))) float row_a[DELTA ? kChunk * AP : 4], col_t[DELTA ? 2 : 1][DELTA ? 16 * TP : 4];
     const int b = blockIdx.y, h = blockIdx.z, gr = h / (H / G);
     const int q0 = qstart[b], n = qstart[b + 1] - q0;
     const int c = blockIdx.x, t0 = c * kChunk;
     if (t0 >= n) return;
-    const int lane = threadIdx.x, l31 = lane & 31, hi = lane >> 5;
-    const bool valid = t0 + l31 < n;                          // past the portion's end: the identity step
-    const size_t tok = q0 + min(t0 + l31, n - 1);
-    const bf16_t *q = rows + tok * stride + q_off + (size_t)gr * DK + 8 * hi, *k = rows + tok * stride + k_off + (size_t)gr * DK + 8 * hi;
-    const float4 *gp = (const float4*)(gates + (tok * H + h) * 8);
-    const float4 ga = gp[0], gb = gp[1];
-    const float g = valid ? ga.x : 1.f, beta = valid ? ga.y : 0.f, rk = valid ? ga.w : 0.f, rq = valid ? gb.w : 0.f;
-    f32x16 kk, qk;                                            // [i, t]: lane: token t, register r: i = (r & 3) + 8 (r >> 2) + 4 hi
-#pragma unroll
-    for (int r = 0; r < 16; ++r) kk[r] = qk[r] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < DK / 16; ++ks) {
-        i32x4 kv = *(const i32x4*)(k + 16 * ks), qv = *(const i32x4*)(q + 16 * ks);
-        if (!valid) { kv = i32x4{0, 0, 0, 0}; qv = kv; }
-        const bf16x8 kf = __builtin_bit_cast(bf16x8, kv), qf = __builtin_bit_cast(bf16x8, qv);
-        if (DELTA) kk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, kf, kk, 0, 0, 0);
-        qk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf, qk, 0, 0, 0);
-    }
-    // D_ti rk_i, from i = t down (zero for i > t); and the products over the whole chunk.  In double: a product of up to 32 decays
-    // is the one place where the chunk would round more often than the token-by-token walk does.
-    float m0[16], m1[16];
-    double cur = 0., end = 1., dend = 0.;
-#pragma unroll
-    for (int i = kChunk - 1; i >= 0; --i) {
-        if (i < kChunk - 1) cur *= (double)lane_value(g, i + 1);
-        if (l31 == i) { cur = 1.; dend = end; }
-        end *= (double)lane_value(g, i);
-        const float m = (float)(cur * (double)lane_value(rk, i));
-        if (i & 4) m1[(i & 3) + 4 * (i >> 3)] = m; else m0[(i & 3) + 4 * (i >> 3)] = m;
-    }
-    const double Gt = cur * (double)lane_value(g, 0);         // (cur is D_t0 now)
-    unsigned char* out = work + prepared_at(q0, b, c, h, H);
-    float p[16], a[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float m = hi ? m1[r] : m0[r];
-        const int i = (r & 3) + 8 * (r >> 2) + 4 * hi;
-        p[r] = i <= l31 ? rq * (qk[r] * m) : 0.f;             // (chosen, not multiplied: a later token's NaN stays out)
-        if (DELTA) a[r] = i < l31 ? beta * rk * (kk[r] * m) : 0.f;
-    }
-    // row l31 of an operand from its columns 4 hi.., 16 + 4 hi.. (quarter hi) and 8 + 4 hi.., 24 + 4 hi.. (quarter 2 + hi)
+    const int lane = threadIdx.x, l31 = lane & 31, l15 = lane & 15, g4 = lane >> 4;
     const Minus minus;
-    auto put = [&](unsigned char* op, const float* lo, const float* up) {
+    f32x4 kk00 = zeros4(), kk10 = zeros4(), kk11 = zeros4(), qk00 = zeros4(), qk10 = zeros4(), qk11 = zeros4();
+    float qq = 0.f, ksq = 0.f;                                // of token l31
+    {
+        bf16x8 k[2][DK / 32], q[2][DK / 32];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const float y[8] = {lo[4 * u], lo[4 * u + 1], lo[4 * u + 2], lo[4 * u + 3], up[4 * u], up[4 * u + 1], up[4 * u + 2], up[4 * u + 3]};
-            const Terms t = split8(y, minus);
-            const int at = 16 * (2 * u + hi) + (l31 & 15);
+        for (int tb = 0; tb < 2; ++tb) {
+            const int t = t0 + 16 * tb + l15;
+            const bf16_t* row = rows + (size_t)(q0 + min(t, n - 1)) * stride + (size_t)gr * DK + 8 * g4;
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const i32x4 x = __builtin_bit_cast(i32x4, t.v[j]);
-                typedef int i32x2 __attribute__((ext_vector_type(2)));
-                if (l31 < 16) *(i32x2*)(op + j * kTermBytes + 8 * at) = i32x2{x[0], x[1]};
-                else *(i32x4*)(op + j * kTermBytes + kTermLow + 16 * at) = x;
+            for (int ks = 0; ks < DK / 32; ++ks) {
+                k[tb][ks] = *(const bf16x8*)(row + k_off + 32 * ks);
+                q[tb][ks] = *(const bf16x8*)(row + q_off + 32 * ks);
             }
+        }
+        if (t0 + kChunk > n)                                  // past the portion's end: the identity step
+#pragma unroll
+            for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+                for (int ks = 0; ks < DK / 32; ++ks)
+                    if (t0 + 16 * tb + l15 >= n) {
+                        asm volatile("" : "+v"(k[tb][ks]), "+v"(q[tb][ks]));      // (or every chunk makes the choice)
+                        k[tb][ks] = q[tb][ks] = __builtin_bit_cast(bf16x8, (i32x4{0, 0, 0, 0}));
+                    }
+#pragma unroll
+        for (int ks = 0; ks < DK / 32; ++ks) {
+            if (DELTA) {
+                kk00 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[0][ks], k[0][ks], kk00, 0, 0, 0);
+                kk11 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[1][ks], k[1][ks], kk11, 0, 0, 0);
+                kk10 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[0][ks], k[1][ks], kk10, 0, 0, 0);
+            }
+            qk00 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[0][ks], q[0][ks], qk00, 0, 0, 0);
+            qk11 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[1][ks], q[1][ks], qk11, 0, 0, 0);
+            qk10 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[0][ks], q[1][ks], qk10, 0, 0, 0);
+        }
+        if (DELTA) {                                          // the squared lengths (on the products' diagonals they have larger errors)
+            auto square = [&](const bf16x8 (&x)[2][DK / 32]) {
+                float sum[2];
+#pragma unroll
+                for (int tb = 0; tb < 2; ++tb) {
+                    float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int ks = 0; ks < DK / 32; ++ks)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const bf16x2 u = {x[tb][ks][2 * e], x[tb][ks][2 * e + 1]};
+                            s[e] = __builtin_amdgcn_fdot2_f32_bf16(u, u, s[e], false);
+                        }
+                    sum[tb] = (s[0] + s[1]) + (s[2] + s[3]);
+                    sum[tb] += __shfl_xor(sum[tb], 16);
+                    sum[tb] += __shfl_xor(sum[tb], 32);
+                }
+                return lane & 16 ? sum[1] : sum[0];
+            };
+            qq = square(q);
+            ksq = square(k);
+        }
+    }
+    // ---- lane l31 (either half): the gates of that token, and its quad's decays
+    Gates gt = make_gates<bf16_t, DELTA>(ga, q0 + min(t0 + l31, n - 1), h, qq, ksq, 0.f);
+    if (t0 + l31 >= n) {
+        gt.g = 1.f;
+        gt.a1 = gt.rk = gt.rq = 0.f;
+    }
+    const int e4 = lane & 3;
+    {
+        const double g0 = of_quad<0x00>(gt.g), g1 = of_quad<0x55>(gt.g), g2 = of_quad<0xAA>(gt.g), g3 = of_quad<0xFF>(gt.g);
+        const double r0 = of_quad<0x00>(gt.rk), r1 = of_quad<0x55>(gt.rk), r2 = of_quad<0xAA>(gt.rk), r3 = of_quad<0xFF>(gt.rk);
+        const double g12 = g1 * g2, g23 = g2 * g3, g123 = g1 * g23;
+        const double x0 = e4 == 0 ? 1. : e4 == 1 ? g1 : e4 == 2 ? g12 : g123, x1 = e4 == 1 ? 1. : e4 == 2 ? g2 : g23, x2 = e4 == 2 ? 1. : g3;
+        own[l31] = g0 * x0;
+        rest[l31] = (e4 == 0 ? g123 : e4 == 1 ? g23 : e4 == 2 ? g3 : 1.) * (double)gt.rk;
+        inside[l31] = f32x4{(float)(x0 * r0), (float)(x1 * r1), (float)(x2 * r2), (float)r3};       // (of tokens behind t: not used)
+        token[l31] = f32x4{gt.a1, gt.rk, gt.rq, 0.f};
+        if (e4 == 3) quad[l31 >> 2] = g0 * x0;
+    }
+    __syncthreads();
+    {
+        double r = 1.;                                        // the quads between q = lane & 7 and lane >> 3
+#pragma unroll
+        for (int s = 1; s < 7; ++s)
+            if (s > (lane & 7) && s < lane >> 3) r *= quad[s];
+        between[lane >> 3][lane & 7] = r;
+    }
+    __syncthreads();
+    unsigned char* out = work + prepared_at(q0, b, c, h, H);
+    if (lane < kChunk) {
+        const int q = lane >> 2;
+        const double first = quad[0], last = quad[7], in_front = q > 0 ? first * between[q][0] : 1., behind = q < 7 ? between[7][q] * last : 1.;
+        const double Gt = own[lane] * in_front;
+        float* coef = (float*)(out + PR::kCoefAt);
+        coef[kBeta + lane] = gt.a1;
+        coef[kOldKey + lane] = (float)(Gt * (double)(gt.a1 * gt.rk));
+        coef[kOldQuery + lane] = (float)(Gt * (double)gt.rq);
+        coef[kLeft + lane] = (float)(rest[lane] * behind * (DELTA ? 1. : (double)gt.a1));
+        if (lane == 0) *(float*)(out + PR::kEndAt) = (float)(first * between[7][0] * last);
+    }
+    // D_ti rk_i for t and the quad q of i; of later tokens anything
+    auto decay = [&](int t, int q) {
+        const double d = own[t] * between[t >> 2][q];
+        const f32x4 in = inside[t];
+        f32x4 m;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m[e] = (t >> 2) == q ? in[e] : (float)(d * rest[4 * q + e]);
+        return m;
+    };
+    const f32x4 m00 = decay(l15, g4), m10 = decay(16 + l15, g4), m11 = decay(16 + l15, 4 + g4), tk0 = token[l15], tk1 = token[16 + l15];
+    // three terms of rows 0..15 (columns 4 g4..) and of rows 16..31 (columns 4 g4.. and 16 + 4 g4..)
+    auto put = [&](unsigned char* op, const f32x4& x00, const f32x4& x10, const f32x4& x11) {
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        const float low[4] = {x00[0], x00[1], x00[2], x00[3]}, up[8] = {x10[0], x10[1], x10[2], x10[3], x11[0], x11[1], x11[2], x11[3]};
+        unsigned tl[3][2], tu[3][4];
+        split<4>(low, minus, tl);
+        split<8>(up, minus, tu);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            *(u32x2*)(op + j * kTermBytes + 8 * lane) = u32x2{tl[j][0], tl[j][1]};
+            *(u32x4*)(op + j * kTermBytes + kTermLow + 16 * lane) = u32x4{tu[j][0], tu[j][1], tu[j][2], tu[j][3]};
         }
     };
-    put(out, p, p + 8);
-    if (hi == 0) {
-        float* coef = (float*)(out + Prepared<DELTA>::kCoefAt);
-        coef[kBeta + l31] = beta;
-        coef[kOldKey + l31] = (float)(Gt * (double)(beta * rk));
-        coef[kOldQuery + l31] = (float)(Gt * (double)rq);
-        coef[kLeft + l31] = (float)(DELTA ? dend * (double)rk : dend * (double)beta);
+    {
+        f32x4 p00, p10, p11;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {                         // (chosen, not multiplied: a later token's NaN stays out)
+            const bool seen = 4 * g4 + e <= l15;
+            p00[e] = seen ? tk0[2] * (qk00[e] * m00[e]) : 0.f;
+            p10[e] = tk1[2] * (qk10[e] * m10[e]);
+            p11[e] = seen ? tk1[2] * (qk11[e] * m11[e]) : 0.f;
+        }
+        put(out, p00, p10, p11);
     }
-    if (lane == 0) *(float*)(out + Prepared<DELTA>::kEndAt) = (float)end;
     if constexpr (DELTA) {
+        const float s0 = tk0[0] * tk0[1], s1 = tk1[0] * tk1[1];
+        f32x4 a00, a10, a11;
+        float z0 = 0.f, z1 = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool seen = 4 * g4 + e < l15;
+            a00[e] = seen ? s0 * (kk00[e] * m00[e]) : 0.f;
+            a10[e] = s1 * (kk10[e] * m10[e]);
+            a11[e] = seen ? s1 * (kk11[e] * m11[e]) : 0.f;
+            z0 = __builtin_fmaf(a00[e], 0.f, z0);
+            z1 = __builtin_fmaf(a10[e], 0.f, __builtin_fmaf(a11[e], 0.f, z1));
+        }
         // a token's row that is not finite is left out here (the rows of earlier tokens would multiply it by zero) and put in below
-        float z = 0.f;
+        z0 += __shfl_xor(z0, 16);
+        z1 += __shfl_xor(z1, 16);
+        z0 += __shfl_xor(z0, 32);
+        z1 += __shfl_xor(z1, 32);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) z = __builtin_fmaf(a[r], 0.f, z);
-        z += __shfl_xor(z, 32);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a[r] = z == 0.f ? a[r] : 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) at[((r & 3) + 8 * (r >> 2) + 4 * hi) * PITCH + l31] = a[r];
+        for (int e = 0; e < 4; ++e) {
+            a00[e] = z0 == 0.f ? a00[e] : 0.f;
+            a10[e] = z1 == 0.f ? a10[e] : 0.f;
+            a11[e] = z1 == 0.f ? a11[e] : 0.f;
+        }
+        *(f32x4*)(row_a + l15 * AP + 4 * g4) = a00;
+        *(f32x4*)(row_a + (16 + l15) * AP + 16 + 4 * g4) = a11;
         __syncthreads();
-        // row t of (I + A)^-1, from its diagonal down: x (I + A) = e_t
-        float x[kChunk];
+        // column l15 of the block's inverse: (I + A) x = e
+        const int tb = l31 >> 4;
+        const float* rows_a = row_a + 16 * tb * (AP + 1);
+        float x[16];
 #pragma unroll
-        for (int j = kChunk - 1; j >= 0; --j) {
+        for (int t = 0; t < 16; ++t) {
             float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i4 = (j + 1) / 4; i4 < kChunk / 4; ++i4) {
-                const float4 v = *(const float4*)(at + j * PITCH + 4 * i4);
-                const float e[4] = {v.x, v.y, v.z, v.w};
+            for (int i4 = 0; i4 < (t + 3) / 4; ++i4) {
+                const f32x4 v = *(const f32x4*)(rows_a + t * AP + 4 * i4);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
-                    if (4 * i4 + u > j) s[u] += x[4 * i4 + u] * e[u];
+                    if (4 * i4 + u < t) s[u] += v[u] * x[4 * i4 + u];
             }
-            x[j] = j == l31 ? 1.f : j < l31 ? -((s[0] + s[1]) + (s[2] + s[3])) : 0.f;
+            x[t] = t == l15 ? 1.f : t > l15 ? -((s[0] + s[1]) + (s[2] + s[3])) : 0.f;
         }
-        float lo[8], up[8];
+        if (lane < kChunk)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int i = (e & 3) + 8 * (e >> 2);
-            const int t = i + 4 * hi;                         // (the diagonal's ones stay out: W = R + N R)
-            lo[e] = (t == l31 ? 0.f : hi ? x[i + 4] : x[i]) + z;
-            up[e] = (t + 16 == l31 ? 0.f : hi ? x[16 + i + 4] : x[16 + i]) + z;
+            for (int i = 0; i < 4; ++i) *(f32x4*)(col_t[tb] + l15 * TP + 4 * i) = f32x4{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]};
+        __syncthreads();
+        // T21: the order of the sums is the lanes', k = 4 g4 + s in step s
+        const f32x4 t11 = *(const f32x4*)(col_t[0] + l15 * TP + 4 * g4);
+        f32x4 t22, u = zeros4(), t21 = zeros4(), n00, n10, n11;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            t22[s] = col_t[1][(4 * g4 + s) * TP + l15];
+            u = __builtin_amdgcn_mfma_f32_16x16x4f32(a10[s], t11[s], u, 0, 0, 0);
         }
-        put(out + Prepared<DELTA>::kTAt, lo, up);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) t21 = __builtin_amdgcn_mfma_f32_16x16x4f32(t22[s], u[s], t21, 0, 0, 0);
+        *(f32x4*)(row_a + l15 * TP + 4 * g4) = t21;            // (A's rows are done with)
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {                         // (the diagonal's ones stay out: W = R + N R)
+            const bool one = 4 * g4 + e == l15;
+            n00[e] = (one ? 0.f : col_t[0][(4 * g4 + e) * TP + l15]) + z0;
+            n10[e] = z1 - row_a[(4 * g4 + e) * TP + l15];
+            n11[e] = (one ? 0.f : t22[e]) + z1;
+        }
+        put(out + PR::kTAt, n00, n10, n11);
     }
 }
 
@@ -592,13 +711,9 @@ __global__ __launch_bounds__(128 * NW) void outer_chunk_walk_kernel(const bf16_t
 }
 
 template <bool DELTA>
-static void launch_chunks(const void* rows_, int64_t stride, int q_off, int k_off, int v_off, const GateArgs<bf16_t>& ga, float* gates,
-                          void* work, float* state, const int32_t* qstart, const int32_t* seq_pos0, const int32_t* seq_slot, float* o,
-                          int B, int64_t T, int H, int G, int D, int V, int max_q, hipStream_t s) {
+static void launch_chunks(const void* rows_, int64_t stride, int q_off, int k_off, int v_off, const GateArgs<bf16_t>& ga, void* work, float* state, const int32_t* qstart, const int32_t* seq_pos0, const int32_t* seq_slot, float* o,
+                          int B, int H, int G, int D, int V, int max_q, hipStream_t s) {
     const bf16_t* rows = (const bf16_t*)rows_;
-    const int64_t items = T * G;
-    hipLaunchKernelGGL((outer_gates_kernel<bf16_t, 8, DELTA>), dim3((unsigned)((items + 15) / 16)), dim3(256), 0, s, rows, stride, q_off,
-                       k_off, ga, gates, items, H, G, D);
     // Four waves of columns share a chunk's K, Q and prepared part, two have a SIMD each and LDS to themselves: where every CU has at most one
     // workgroup of two, those (one prompt of 900 tokens, 16 heads of 128 x 128: 49.5 us, four 52.2; 32 heads of 128 x 64 state space 39 and
     // 48); beyond, a CU has room for one workgroup of either and four take half the rounds.
@@ -606,7 +721,7 @@ static void launch_chunks(const void* rows_, int64_t stride, int q_off, int k_of
     const dim3 pg((unsigned)((max_q + kChunk - 1) / kChunk), (unsigned)B, (unsigned)H), wg((unsigned)B, (unsigned)H, (unsigned)(V / (16 * nw)));
 #define HM_CHUNKS(DK, NW)                                                                                                              \
     do {                                                                                                                           \
-        hipLaunchKernelGGL((outer_chunk_prepare_kernel<DK, DELTA>), pg, dim3(64), 0, s, rows, stride, q_off, k_off, gates, qstart,   \
+        hipLaunchKernelGGL((outer_chunk_prepare_kernel<DK, DELTA>), pg, dim3(64), 0, s, rows, stride, q_off, k_off, ga, qstart,      \
                            (unsigned char*)work, H, G);                                                                            \
         hipLaunchKernelGGL((outer_chunk_walk_kernel<DK, NW, DELTA>), wg, dim3(128 * NW), 0, s, rows, stride, q_off, k_off, v_off,             \
                            (const unsigned char*)work, ga.skip, state, qstart, seq_pos0, seq_slot, o, H, G, V);                    \
@@ -645,13 +760,12 @@ extern "C" int hm_gated_delta_chunks(const void* rows, int64_t stride, int q_off
                                      const int32_t* seq_pos0, const int32_t* seq_slot, float* o, int B, int64_t T, int H, int G, int D,
                                      int V, int max_q, void* stream) {
     int rc = outer_args_bad("hm_gated_delta_chunks", stride, q_off, k_off, v_off, pre_stride, b_off, a_off, rows, pre, A, dt_bias, gates,
-                            state, qstart, seq_pos0, seq_slot, o, B, T, H, G, D, V, max_q < 2 ? 2 : max_q);
+                            state, qstart, seq_pos0, seq_slot, o, B, T, H, G, D, V, max_q < 1 ? max_q : 1);
     if (!rc) rc = chunk_args_bad("hm_gated_delta_chunks", stride, q_off, k_off, v_off, rows, work, B, T, D, V);
     if (rc) return rc;
     if (B == 0 || T == 0 || max_q == 0) return HM_OK;
     GateArgs<bf16_t> ga = {(const bf16_t*)pre, pre_stride, b_off, a_off, A, dt_bias, nullptr, unit_eps, q_scale};
-    launch_chunks<true>(rows, stride, q_off, k_off, v_off, ga, gates, work, state, qstart, seq_pos0, seq_slot, o, B, T, H, G, D, V, max_q,
-                        as_stream(stream));
+    launch_chunks<true>(rows, stride, q_off, k_off, v_off, ga, work, state, qstart, seq_pos0, seq_slot, o, B, H, G, D, V, max_q, as_stream(stream));
     HM_CHECK_LAUNCH("hm_gated_delta_chunks");
     return HM_OK;
 }
@@ -661,14 +775,13 @@ extern "C" int hm_state_space_chunks(const void* rows, int64_t stride, int x_off
                                      float* state, const int32_t* qstart, const int32_t* seq_pos0, const int32_t* seq_slot, float* y, int B,
                                      int64_t T, int H, int G, int N, int V, int max_q, void* stream) {
     int rc = outer_args_bad("hm_state_space_chunks", stride, c_off, b_off, x_off, pre_stride, 0, dt_off, rows, pre, A, dt_bias, gates,
-                            state, qstart, seq_pos0, seq_slot, y, B, T, H, G, N, V, max_q < 2 ? 2 : max_q);
+                            state, qstart, seq_pos0, seq_slot, y, B, T, H, G, N, V, max_q < 1 ? max_q : 1);
     if (!rc) rc = chunk_args_bad("hm_state_space_chunks", stride, c_off, b_off, x_off, rows, work, B, T, N, V);
     if (rc) return rc;
     if (B > 0 && T > 0 && !D) { set_error("hm_state_space_chunks: bad argument"); return HM_EINVAL; }
     if (B == 0 || T == 0 || max_q == 0) return HM_OK;
     GateArgs<bf16_t> ga = {(const bf16_t*)pre, pre_stride, 0, dt_off, A, dt_bias, D, 0.f, 1.f};
-    launch_chunks<false>(rows, stride, c_off, b_off, x_off, ga, gates, work, state, qstart, seq_pos0, seq_slot, y, B, T, H, G, N, V, max_q,
-                         as_stream(stream));
+    launch_chunks<false>(rows, stride, c_off, b_off, x_off, ga, work, state, qstart, seq_pos0, seq_slot, y, B, H, G, N, V, max_q, as_stream(stream));
     HM_CHECK_LAUNCH("hm_state_space_chunks");
     return HM_OK;
 }

@@ -357,15 +357,18 @@ def _outer_work(rows, H, ctx):
 
 
 def _outer_args(rows, pre, state, o_shape, H, D, V, ctx):
-    """Checks of the outer-product recurrences; (output, gates scratch or None)."""
+    """Checks of the outer-product recurrences; the output."""
     _rows(rows, "rows")
     _rows(pre, "pre")
     T = rows.shape[0]
     assert pre.shape[0] == T and pre.dtype == rows.dtype
     assert state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (H, D, V)
-    o = torch.empty(o_shape, dtype=torch.float32, device=rows.device)
-    gates = torch.empty((T, H, 8), dtype=torch.float32, device=rows.device) if ctx.max_q > 1 else None
-    return o, gates
+    return torch.empty(o_shape, dtype=torch.float32, device=rows.device)
+
+
+def _outer_gates(rows, H, ctx):
+    """Scratch for the gates of a walk that takes token after token."""
+    return torch.empty((rows.shape[0], H, 8), dtype=torch.float32, device=rows.device) if ctx.max_q > 1 else None
 
 
 def gated_delta(rows, q_off, k_off, v_off, pre, b_off, a_off, A, dt_bias, H, G, D, V, state, ctx: StepContext, q_scale=1.0,
@@ -379,15 +382,16 @@ def gated_delta(rows, q_off, k_off, v_off, pre, b_off, a_off, A, dt_bias, H, G, 
     if not rows.is_cuda:
         return cpu_ops.gated_delta(rows, q_off, k_off, v_off, pre, b_off, a_off, A, dt_bias, H, G, D, V, unit_eps, q_scale, state, ctx)
     assert A.dtype == dt_bias.dtype == torch.float32 and A.numel() == dt_bias.numel() == H
-    o, gates = _outer_args(rows, pre, state, (rows.shape[0], H, V), H, D, V, ctx)
+    o = _outer_args(rows, pre, state, (rows.shape[0], H, V), H, D, V, ctx)
     if _outer_chunked(rows, (q_off, k_off, v_off), D, V, ctx):
         work = _outer_work(rows, H, ctx)
         HM.check(HM.load().hm_gated_delta_chunks(rows.data_ptr(), rows.stride(0), q_off, k_off, v_off, pre.data_ptr(), pre.stride(0), b_off,
                                                  a_off, A.data_ptr(), dt_bias.data_ptr(), float(unit_eps), float(q_scale),
-                                                 gates.data_ptr(), work.data_ptr(), state.data_ptr(), ctx.qstart.data_ptr(),
+                                                 None, work.data_ptr(), state.data_ptr(), ctx.qstart.data_ptr(),
                                                  ctx.seq_pos0.data_ptr(), ctx.seq_slot.data_ptr(), o.data_ptr(), ctx.num_seqs,
                                                  rows.shape[0], H, G, D, V, int(ctx.max_q), _dev(rows)))
         return o
+    gates = _outer_gates(rows, H, ctx)
     HM.check(HM.load().hm_gated_delta(HM.dtype_code(rows.dtype), rows.data_ptr(), rows.stride(0), q_off, k_off, v_off, pre.data_ptr(),
                                       pre.stride(0), b_off, a_off, A.data_ptr(), dt_bias.data_ptr(), float(unit_eps), float(q_scale),
                                       HM.ptr(gates), state.data_ptr(), ctx.qstart.data_ptr(), ctx.seq_pos0.data_ptr(),
@@ -405,15 +409,16 @@ def state_space(rows, x_off, b_off, c_off, pre, dt_off, A, dt_bias, D, H, G, N, 
     if not rows.is_cuda:
         return cpu_ops.state_space(rows, x_off, b_off, c_off, pre, dt_off, A, dt_bias, D, H, G, N, V, state, ctx)
     assert A.dtype == dt_bias.dtype == D.dtype == torch.float32 and A.numel() == dt_bias.numel() == D.numel() == H
-    y, gates = _outer_args(rows, pre, state, (rows.shape[0], H, V), H, N, V, ctx)
+    y = _outer_args(rows, pre, state, (rows.shape[0], H, V), H, N, V, ctx)
     if _outer_chunked(rows, (x_off, b_off, c_off), N, V, ctx):
         work = _outer_work(rows, H, ctx)
         HM.check(HM.load().hm_state_space_chunks(rows.data_ptr(), rows.stride(0), x_off, b_off, c_off, pre.data_ptr(), pre.stride(0), dt_off,
-                                                 A.data_ptr(), dt_bias.data_ptr(), D.data_ptr(), gates.data_ptr(), work.data_ptr(),
+                                                 A.data_ptr(), dt_bias.data_ptr(), D.data_ptr(), None, work.data_ptr(),
                                                  state.data_ptr(), ctx.qstart.data_ptr(), ctx.seq_pos0.data_ptr(),
                                                  ctx.seq_slot.data_ptr(), y.data_ptr(), ctx.num_seqs, rows.shape[0], H, G, N, V,
                                                  int(ctx.max_q), _dev(rows)))
         return y
+    gates = _outer_gates(rows, H, ctx)
     HM.check(HM.load().hm_state_space(HM.dtype_code(rows.dtype), rows.data_ptr(), rows.stride(0), x_off, b_off, c_off, pre.data_ptr(),
                                       pre.stride(0), dt_off, A.data_ptr(), dt_bias.data_ptr(), D.data_ptr(), HM.ptr(gates),
                                       state.data_ptr(), ctx.qstart.data_ptr(), ctx.seq_pos0.data_ptr(), ctx.seq_slot.data_ptr(),
