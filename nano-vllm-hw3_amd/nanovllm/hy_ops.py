@@ -337,10 +337,10 @@ def delta_gate_norm(o, g, norm_w, eps, dtype, act=GATE_SIGMOID, gate_first=False
 
 
 # Tokens of the longest portion from which a step takes 32 tokens at a time, by key channels, where the portions have half of that on
-# average: below, the chunks cost more than they save (microseconds, chunks / walk, 16 heads of 128 x 128: 1 portion of 32 21 / 17,
-# of 64 22 / 27, of 256 44 / 88; 64 portions of 16 67 / 59, of 32 72 / 94, of 64 107 / 166; 4 heads of 64 x 64: 1 portion of 64
-# 21 / 20, of 128 25 / 33; 64 of 64 25 / 22, of 128 35 / 36).
-CHUNKS_MIN_TOKENS = {64: 128, 128: 64}
+# average: below, the chunks cost more than they save (microseconds, chunks / walk, 16 heads of 128 x 128: 1 portion of 16 10.6 / 11.7,
+# of 32 10.6 / 16.7, of 128 15.7 / 46.6; 64 portions of 16 43 / 59, of 32 48 / 97; 4 heads of 64 x 64: 1 portion of 16 9.5 / 8.9, of
+# 32 9.5 / 12.5; 64 of 16 10.8 / 10.7, of 32 11.0 / 14.5; state space, 16 heads of 128 x 64, 1 portion of 16 8.2 / 10.6).
+CHUNKS_MIN_TOKENS = {64: 32, 128: 16}
 
 
 def _outer_chunked(rows, offsets, D, V, ctx):
