@@ -307,10 +307,10 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
         const int64_t t = (M + 32 * mt - 1) / (32 * mt) * ((N + 63) / 64), room = group ? 260 : K >= 8192 && t > 240 ? 960 : 480;
         t_split = (int)std::max<int64_t>(1, std::min<int64_t>(room / t, K / 1300));
     }
-    // 33 to 64 rows of 8-bit activations under the SiLU epilogue, K of 2048 and more, where the ladder ends in 64 x 128 tiles: 64 x 64
-    // tiles, so that the weights are read once and more workgroups share them (fp8, us: 19456 x 2048 17.7 -> 15.2, 24576 x 4096 34.4 -> 25.9; the ladder's
-    // own 64 x 64 tile of 12288 x 2048 takes 10.1 there, this one 11.9)
-    if (silu && w8a8 && pick == nladder - 1 && M > 32 && M <= 64 && K >= 2048) { mt = 2; wn = 2; wk = 2; cp = 8; }
+    // 33 to 64 rows of 8-bit activations under the SiLU epilogue, K of 2048 and more, where the ladder ends in 64 x 128 tiles: the same in one buffer of
+    // 512-k chunks, whose weights run on from chunk to chunk (19456 x 2560 in fp8 at 64 rows 19.3 us in 64 x 64 tiles, 16.1 here; 24576 x 4096 28.9 /
+    // 26.6; the ladder's own double-buffered tile 20.7 and 34.8)
+    if (silu && w8a8 && pick == nladder - 1 && M > 32 && M <= 64 && K >= 2048) { mt = 2; wn = 4; wk = 2; cp = 8; }
     // a measured plan for this shape, if the table holds one (entries were checked when they were set); for calls that the wide tile is
     // not built for, one of theirs as well
     const int form = (group ? QL_PLAN_GROUP : 0) | (silu ? QL_PLAN_SILU : 0) | (rope ? QL_PLAN_ROPE : 0) | (w8a8 ? QL_PLAN_W8A8 : 0);

@@ -337,7 +337,7 @@ void qgemm_kernel(const GemmParams p) {
     // A-fragment reads: row 32*i + l31; the XOR swizzle only involves lane-constant bits
     const int a_g4 = ((((l31 / SWZ_RPB) & SWZ_MASK) ^ (ACT == ACT_BF16 ? 2 * lh : lh)) & SWZ_MASK) << 4;
     const int a_hi = (ACT == ACT_BF16 ? 2 * lh : lh) & ~SWZ_MASK;   // 0 unless a row has < 4 pieces (never)
-    const int a_row = l31 * RB + (a_hi << 4);
+    int a_row = l31 * RB + (a_hi << 4);
 
     // qkv epilogue: what the thread's first (row, head, piece) needs from memory (cache slot, cos/sin of the token's
     // position, norm weights) is requested NOW, so that this chain of dependent reads is over long before the tail
@@ -722,15 +722,20 @@ void qgemm_kernel(const GemmParams p) {
     // RUN_ON: the same without a pause between chunks.  Chunk `it`'s activations are in LDS and its first D weight loads in flight;
     // if another chunk follows (MORE), its activations are requested in front of this one's steps and wait in registers until
     // everybody is through with the buffer, and the ring of weight loads runs on into it, so that a slice waits for memory once
-    // and not once per chunk (1 to 16 rows, the four projections of a layer: Qwen3-4B with fp8 weights 39.5 -> 38 us, with groups
-    // 46 -> 44.5, Qwen3-8B with groups 62.5 -> 59.5).  Built where the registers that this takes cost no workgroup per CU and no
-    // spills: one row fragment, fp8 weights or groups beside bf16 activations, chunk parts of up to 8 steps (with groups, chunks of
-    // 1024 k).  With int8 rows and with 8-bit activations it gained nothing or lost up to 4 %.
+    // and not once per chunk.  One row fragment of bf16 activations with fp8 weights or groups (1 to 16 rows, the four projections of a layer:
+    // Qwen3-4B with fp8 weights 39.5 -> 38 us, with groups 46 -> 44.5), up to chunks of 1024 k with groups.  Int8 rows and 8-bit activations
+    // need the steps' addresses worked out chunk by chunk (LEAN: kept over the loop they take 15 to 30 registers, and a workgroup per CU with them; that way
+    // they gained nothing or lost up to 20 %): 0.84 to 0.93 of the time in the 32 x 64 and 64 x 64 tiles over three chunks and more,
+    // 0.95 to 0.98 in the 32 x 32 ones (936 calls, 1 to 256 rows, weights that no cache holds).  Not in the 32 x 32 tile of 1024-k chunks with
+    // fp8 activations, which loses its third workgroup per CU (512 and more of them: 1.08), nor in the 64 x 64 tile with groups, which spills.
     // (an address past the slice's end is the last step's: step() skips what it brings)
-    constexpr bool RUN_ON = !DB && ACT == ACT_BF16 && MT == 1 && (FP8W || GROUP) && CP <= 8 && (!GROUP || CP * WK <= 32);
+    constexpr bool LEAN = !DB && CP <= 8 && !GROUP && !DYNQ && !W16 && !SK &&
+                          (ACT == ACT_BF16 ? !ROPE && (!FP8W || MT == 2) : !(ACT == ACT_FP8 && WN == 1 && WK == 8 && CP == 4));
+    constexpr bool RUN_ON = LEAN || (!DB && ACT == ACT_BF16 && MT == 1 && (FP8W || GROUP) && CP <= 8 && (!GROUP || CP * WK <= 32));
     auto chunk_on = [&](auto chk, auto gmc, auto morec, int it) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(morec)::value;
         const int kc = k0 + it * C::KB;
+        if constexpr (LEAN) asm volatile("" : "+v"(a_row));
         if constexpr (MORE) load_x(TrueT{}, kc + C::KB);
 #pragma unroll
         for (int c = 0; c < CP; ++c) {                               // (CP <= 8 = D)
@@ -1144,7 +1149,7 @@ struct TileCfg { int mt, wn, wk, cp, db; };
     X(1, 2, 4, 8, false) X(1, 2, 4, 4, true) X(2, 2, 4, 8, false) X(2, 2, 4, 4, true) X(1, 1, 8, 4, false)     \
     X(2, 4, 2, 4, true) X(4, 4, 2, 4, true)                                                          \
     X(1, 4, 1, 32, false) X(1, 4, 2, 16, false) X(2, 4, 2, 16, false) X(1, 2, 4, 16, false) X(1, 1, 8, 8, false) \
-    X(4, 8, 1, 2, true) X(4, 8, 1, 4, true)
+    X(4, 8, 1, 2, true) X(4, 8, 1, 4, true) X(2, 4, 2, 8, false)
 #define QL_TILE_LIST_TALL(X) X(8, 4, 1, 4, true)
 // tiles also built with the qkv (q/k norm + RoPE + KV store) epilogue: 128- or 256-column tiles
 #define QL_TILE_LIST_ROPE(X) X(1, 4, 2, 16, false) X(1, 4, 1, 4, true) X(2, 4, 2, 4, true) X(2, 4, 1, 4, true) X(4, 8, 1, 2, true) X(4, 8, 1, 4, true)
