@@ -592,13 +592,26 @@ void qgemm_kernel(const GemmParams p) {
                 // scales, e4m3 operands), which runs 64 k in the cycles the K = 16 instruction pair above takes for
                 // 32.  A lane's 32 operand bytes are its 16 of the even step and its 16 of the odd step, for A and
                 // B alike, so the contraction is again a permutation of the k sum.  The even step only parks its
-                // weights; a lone last step (K slice not a multiple of 64) takes the K = 16 path below.
+                // weights; a lone last step (K slice not a multiple of 64) has zeros for its odd half.  It must not
+                // take the K = 16 pair: with products of both latencies in front of a join, the compiler counts the
+                // wait of the short one for the results of the long one, which were then read before they were
+                // whole (32 x 32 tile of 1024-k chunks, 33 x 100 x 544: about one call in a thousand wrong).
                 typedef int i32x8 __attribute__((ext_vector_type(8)));
-                if ((c & 1) == 0 && (!decltype(chk)::value || kb + 32 < kend)) {
-                    w_even = w;
+                if ((c & 1) == 0) {
+                    if (!decltype(chk)::value || kb + 32 < kend) {
+                        w_even = w;
+                        return;
+                    }
+                    const i32x8 bb = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) {
+                        const i32x4 ae = *(const i32x4*)(smem + a0 + i * 32 * RB);
+                        const i32x8 aa = {ae[0], ae[1], ae[2], ae[3], 0, 0, 0, 0};
+                        acc[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aa, bb, acc[i], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+                    }
                     return;
                 }
-                if (c & 1) {
+                {
                     const int bc0 = base_c - APS;                  // the even step's first piece
                     const int a_ev = buf * C::XBYTES + a_row + ((bc0 & ~SWZ_MASK) << 4) + (((bc0 & SWZ_MASK) << 4) ^ a_g4);
                     const i32x8 bb = {w_even[0], w_even[1], w_even[2], w_even[3], w[0], w[1], w[2], w[3]};
