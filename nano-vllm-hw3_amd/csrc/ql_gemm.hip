@@ -231,11 +231,89 @@ static bool mid_tile(int pick, int64_t M, int64_t N, int64_t K, bool group, bool
     return (t > 128 && K > 4096) || (t >= 80 && K >= 8192) || (t >= 80 && t <= 120 && K >= 6144);
 }
 
+// What a call of up to 256 rows over more than 2048 k takes in microseconds (weights that no cache holds) on one of the tiles that read a weight
+// once per row tile, in `split` slices: a start, what slices cost, and for the workgroups that a CU runs (`q` of it in whole rounds, the rest
+// as they overlap) a part per workgroup and one per 1000 k of its slice, by how much of the tile's rows are asked for; and the weights' way.
+// Fitted over 7171 calls (600 shapes of 512..12288 columns by 2112..16384 k, 1 to 256 rows) of 20 forms each, 7 to 11 % off in the root mean
+// square.  Rows count by 32, so that the plan is one for every 32 rows.
+struct TileCost { double start, slices, slice, group, k, k_full, q, way; };
+constexpr int kCostTiles = 6;
+static const TileCfg kCostTile[kCostTiles] = {{1, 1, 8, 4, 0}, {1, 1, 8, 8, 0}, {1, 2, 4, 8, 0}, {1, 2, 4, 4, 1}, {2, 2, 4, 8, 0}, {2, 4, 2, 4, 1}};
+
+static double tile_cost(int tile, int64_t split, int64_t M, int64_t N, int64_t K, bool fp8, bool w8a8) {
+    static const TileCost cost[3][kCostTiles] = {             // int8, fp8 weights; 8-bit activations
+        {{3.662, 0, 0.397, 0.206, 0.887, 0.837, 0.569, 0},
+         {1.919, 0, 0.192, 2.269, 0.652, 0.919, 0.767, 0},
+         {1.548, 0.279, 0.484, 2.426, 1.421, 0.676, 0.813, 0.031},
+         {3.64, 0.72, 0.464, 0.165, 1.543, 0.764, 0.281, 0.062},
+         {1.572, 0.298, 0.569, 3.108, 2.358, 0.591, 0.805, 0.055},
+         {3.888, 0.926, 0.56, 1.309, 2.601, 2.785, 0.293, 0.101}},
+        {{3.337, 0.043, 0.407, 0.475, 0.92, 0.572, 0.544, 0},
+         {1.754, 0, 0.222, 2.345, 0.856, 0.562, 0.765, 0},
+         {1.693, 0.265, 0.427, 2.251, 1.316, 0.57, 0.819, 0.037},
+         {3.297, 0.878, 0.461, 0.176, 1.384, 0.698, 0.208, 0.073},
+         {1.982, 0, 0.653, 2.468, 2.822, 0.23, 0.639, 0.054},
+         {2.753, 1.316, 0.642, 1.657, 2.077, 2.6, 0.313, 0.108}},
+        {{3.534, 0.264, 0.409, 0.189, 0.836, 0.418, 0.522, 0.017},
+         {1.819, 0, 0.262, 2.375, 0.691, 0.304, 0.763, 0.028},
+         {2.934, 0.59, 0.446, 0.514, 1.172, 0.45, 0.866, 0.045},
+         {3.12, 0.89, 0.503, 0.063, 1.216, 0.591, 0.142, 0.087},
+         {2.361, 0.524, 0.537, 2.538, 1.572, 0.209, 0.758, 0.067},
+         {2.812, 1.477, 0.647, 1.911, 3.099, 0.865, 0.439, 0.123}}};
+    const TileCfg& t = kCostTile[tile];
+    const TileCost& c = cost[w8a8 ? 2 : fp8][tile];
+    const int64_t kb = 32 * t.cp * t.wk, chunks = (K + kb - 1) / kb, per = (chunks + split - 1) / split, mb = (M + 32 * t.mt - 1) / (32 * t.mt);
+    const double k = std::min(K, per * kb) / 1000., load = (double)(mb * ((N + 32 * t.wn - 1) / (32 * t.wn)) * split) / 256,
+                 full = (double)((M + 31) / 32) / (double)(mb * t.mt), rounds = (double)(int64_t)(load + 255. / 256);
+    return c.start + (split > 1 ? c.slices + c.slice * (double)(split - 1) : 0) + c.way * (double)(N * K) * 1e-6 +
+           (c.group + (c.k + c.k_full * full) * k) * ((1 - c.q) * std::max(1., load) + c.q * rounds);
+}
+
+// The tile and slices that the costs say are faster than the rules' (`tile` in `split` slices) by more than they are wrong by; false: keep those.
+// Lines: of the calls that change, 1 of 40 is slower than before by more than 4 %.  The double-buffered tiles stay: the 64 x 128 one's costs go up
+// and down with the number of tiles by more than the fit shows, and mid_tile's lines come from sweeps of their own.
+// us, rules / here: fp8 x fp8 33 x 8192 of 12288 k 38.1 / 24.1, 64 x 6144 of 8192 k 22.3 / 16.4; int8 64 x 2048 of 12288 k 17.4 / 13.3; over all calls
+// of 33 to 64 rows 0.92 (8-bit activations) and 0.95, up to 32 rows 0.96 and 0.98, from 65 rows on 0.95.
+static bool cheaper_tile(int tile, int64_t split, int64_t M, int64_t N, int64_t K, bool fp8, bool w8a8, int* best_tile, int* best_split) {
+    // (worked out once per thread for the last shapes that a place of the table has seen: up to 40 costs take a microsecond, as long as a launch)
+    struct Seen { int64_t rows = 0, N = 0, K = 0, split = 0; int tile = 0, kind = 0, best_tile = 0, best_split = 0; };
+    static thread_local Seen table[64];
+    const int64_t rows = (M + 31) / 32;
+    const int kind = w8a8 ? 2 : fp8;
+    Seen& seen = table[(uint64_t)(N * 5 + K * 3 + rows * 11 + kind) / 32 % 64];
+    auto answer = [&]() -> bool {
+        *best_tile = seen.best_tile;
+        if (seen.best_split) *best_split = seen.best_split;
+        return seen.best_split != 0;
+    };
+    if (seen.rows == rows && seen.N == N && seen.K == K && seen.split == split && seen.tile == tile && seen.kind == kind) return answer();
+    seen = Seen{rows, N, K, split, tile, kind, 0, 0};
+    const double line = M <= 32 ? 0.86 : M <= 64 ? 0.9 : 0.88;
+    double best = line * tile_cost(tile, split, M, N, K, fp8, w8a8);
+    for (int i = 0; i < kCostTiles; ++i) {
+        const TileCfg& t = kCostTile[i];
+        if (M <= 32 && t.mt > 1) continue;
+        const int64_t tiles = (M + 32 * t.mt - 1) / (32 * t.mt) * ((N + 32 * t.wn - 1) / (32 * t.wn)), kb = 32 * t.cp * t.wk, chunks = (K + kb - 1) / kb;
+        if (tiles > kMaxTiles) continue;
+        for (int64_t s = 1; s <= std::min<int64_t>(8, chunks); ++s) {
+            const int64_t per = (chunks + s - 1) / s;
+            if ((chunks + per - 1) / per != s || (s > 1 && tiles * s > 1100)) continue;        // (as many slices as are asked for)
+            const double c = tile_cost(i, s, M, N, K, fp8, w8a8);
+            if (c < best) {
+                best = c;
+                seen.best_tile = i;
+                seen.best_split = (int)s;
+            }
+        }
+    }
+    return answer();
+}
+
 // wide_group: the group size of a call that may run on the wide tile (0: no groups), -1: it may not (operands off 16 bytes, activations
 // quantized while they are staged, row maxima), kNoEntry: nor does it look for their entries (what a call that may takes in place of the wide tile)
 constexpr int kNoEntry = -2;
 static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = false, bool rope = false, bool w8a8 = false,
-                      int wide_group = -1, bool fp8 = false) {
+                      int wide_group = -1, bool fp8 = false, bool rules_only = false) {
     Plan pl;
     // Tile ladder, smallest to largest output tile.  On a 256-CU chip these GEMMs are bound by
     // instruction issue and L2->LDS traffic per workgroup, not by HBM or MFMA peak, so the measured
@@ -307,10 +385,39 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
         const int64_t t = (M + 32 * mt - 1) / (32 * mt) * ((N + 63) / 64), room = group ? 260 : K >= 8192 && t > 240 ? 960 : 480;
         t_split = (int)std::max<int64_t>(1, std::min<int64_t>(room / t, K / 1300));
     }
-    // 33 to 64 rows of 8-bit activations under the SiLU epilogue, K of 2048 and more, where the ladder ends in 64 x 128 tiles: the same in one buffer of
-    // 512-k chunks, whose weights run on from chunk to chunk (19456 x 2560 in fp8 at 64 rows 19.3 us in 64 x 64 tiles, 16.1 here; 24576 x 4096 28.9 /
-    // 26.6; the ladder's own double-buffered tile 20.7 and 34.8)
-    if (silu && w8a8 && pick == nladder - 1 && M > 32 && M <= 64 && K >= 2048) { mt = 2; wn = 4; wk = 2; cp = 8; }
+    // fewer tiles than CUs even at 32 x 32 (N = hidden size): split K so that each slice is one 1024-k
+    // chunk, combined in-kernel by the last arriver (measured: down_proj 11.1 -> 9.5 us at M = 64..128)
+    // (K >= 8192 is cut into 2048-k slices instead: two chunks per slice halve the slab traffic, measured on the
+    // Qwen3-4B down_proj shape; a grid of 144+ tiles of the 64 x 128 tile is not split at all)
+    auto rule_split = [&](int64_t tiles) -> int64_t {
+        if (tiles < 144) return K >= 8192 ? (K + 2047) / 2048 : (K + 1023) / 1024;
+        if (tiles < 160 && pick < nladder - 1) return (K + 1023) / 1024;
+        if (tiles < 512 && K >= 4096) return (K + 4095) / 4096;        // long K: at most four chunks per slice
+        return 1;
+    };
+    // (not in the allocation-free entry point, whose scratch array is sized for the rules' slices, nor for kernels that quantize while they
+    // stage, whose costs are others)
+    if (!silu && !rope && !group && M <= 256 && K > 2048 && !tl_skip_table && !rules_only) {
+        int tile = kCostTiles - 1;
+        while (tile >= 0 && !(kCostTile[tile].mt == mt && kCostTile[tile].wn == wn && kCostTile[tile].wk == wk && kCostTile[tile].cp == cp)) --tile;
+        const int64_t tiles = (M + 32 * mt - 1) / (32 * mt) * ((N + 32 * wn - 1) / (32 * wn)), kb0 = 32 * cp * wk, chunks = (K + kb0 - 1) / kb0;
+        int64_t slices = std::min(t_split ? t_split : rule_split(tiles), chunks);
+        slices = (chunks + (chunks + slices - 1) / slices - 1) / ((chunks + slices - 1) / slices);
+        int best = 0;
+        if (tile >= 0 && !kCostTile[tile].db && cheaper_tile(tile, slices, M, N, K, fp8, w8a8, &best, &t_split)) {
+            mt = kCostTile[best].mt; wn = kCostTile[best].wn; wk = kCostTile[best].wk; cp = kCostTile[best].cp;
+        }
+    }
+    // 33 to 64 rows of 8-bit activations under the SiLU epilogue, K of 2048 and more, where the ladder ends in 64 x 128 tiles: 64 x 64
+    // tiles, so that the weights are read once and more workgroups share them (fp8, us: 19456 x 2048 17.7 -> 15.2, 24576 x 4096 34.4 -> 25.9; the ladder's
+    // own 64 x 64 tile of 12288 x 2048 takes 10.1 there, this one 11.9)
+    if (silu && w8a8 && pick == nladder - 1 && M > 32 && M <= 64 && K >= 2048) {
+        mt = 2; wn = 2; wk = 2; cp = 8;
+        // beyond a round of those, 64 x 128 ones of 512-k chunks in one buffer, whose weights run on from chunk to chunk: 0.85 to 0.98 of the time at
+        // 17408..32768 columns by 2112..3072 k (19456 x 2560 in fp8, 64 rows 19.1 / 16.1), from 4096 k on 0.87 to 0.99 at 64 rows, 0.97 to 1.06 at 33;
+        // up to 16384 columns 1.02 to 1.32
+        if (N > 16384 && K > 2048 && (K < 4096 || M > 48)) { wn = 4; }
+    }
     // a measured plan for this shape, if the table holds one (entries were checked when they were set); for calls that the wide tile is
     // not built for, one of theirs as well
     const int form = (group ? QL_PLAN_GROUP : 0) | (silu ? QL_PLAN_SILU : 0) | (rope ? QL_PLAN_ROPE : 0) | (w8a8 ? QL_PLAN_W8A8 : 0);
@@ -339,14 +446,7 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
     const int64_t nblocks = (N + 32 * wn - 1) / (32 * wn);
     const int64_t kchunks = (K + kb - 1) / kb;
     const int64_t base = mblocks * nblocks;
-    // fewer tiles than CUs even at 32 x 32 (N = hidden size): split K so that each slice is one 1024-k
-    // chunk, combined in-kernel by the last arriver (measured: down_proj 11.1 -> 9.5 us at M = 64..128)
-    // (K >= 8192 is cut into 2048-k slices instead: two chunks per slice halve the slab traffic, measured on the
-    // Qwen3-4B down_proj shape; a grid of 144+ tiles of the 64 x 128 tile is not split at all)
-    int64_t split = 1;
-    if (base < 144) split = K >= 8192 ? (K + 2047) / 2048 : (K + 1023) / 1024;
-    else if (base < 160 && pick < nladder - 1) split = (K + 1023) / 1024;
-    else if (base < 512 && K >= 4096) split = (K + 4095) / 4096;   // long K: at most four chunks per slice
+    int64_t split = rule_split(base);
     // (gate/up with the SiLU epilogue: gate and up meet in the tile's LAST workgroup, which holds the whole reduced
     // tile; the heuristics were measured without slices there and keep one, a table entry may ask for more)
     if (silu) split = 1;
@@ -582,7 +682,7 @@ size_t ql_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int granularity)
     if (M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
     // (the qkv entry points with the RoPE epilogue may plan differently, and the W8A8 entry points may hold
     // plan-table entries of their own: cover them all)
-    // (and whether a call may run on the wide tile, and at 33 to 256 rows its weight type, decide too)
+    // (and whether a call may run on the wide tile, up to 256 rows its weight type, and whether its activations are quantized as they are staged)
     const bool grp = granularity == QL_PER_GROUP, heads = N % 128 == 0, strips = N % 64 == 0;
     size_t need = 0;
     auto see = [&](bool silu, bool rope, bool w8a8) {
@@ -590,7 +690,8 @@ size_t ql_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int granularity)
             const Plan pl = make_plan(M, N, K, grp, silu, rope, w8a8, -1, fp8);
             need = std::max(need, plan_workspace(pl));
             if (pl.narrow) need = std::max(need, plan_workspace(make_plan(M, N, K, grp, silu, rope, w8a8, kNoEntry, fp8)));
-            if (silu || rope || M <= 32 || M > 256) break;
+            if (silu || rope || M > 256) break;
+            if (w8a8) need = std::max(need, plan_workspace(make_plan(M, N, K, grp, silu, rope, w8a8, -1, fp8, true)));
         }
     };
     for (const bool w8a8 : {false, true}) {
@@ -816,7 +917,7 @@ static int gemm_w8a8(const char* fn, bool silu, int dtype, const void* qx, const
     p.rowmax_out = silu ? rowmax_out : nullptr; p.nparts_out = (int)(N / 64);
     const bool aligned = (((uintptr_t)qx | (uintptr_t)y) & 15) == 0;
     const Plan pl = make_plan(M, N, K, false, silu, rope != nullptr, true, aligned && !dynq && !p.rowmax_out ? 0 : -1,
-                              dtype == QL_FP8);
+                              dtype == QL_FP8, dynq);
     kern_t k;
     if (pl.wide) k = dtype == QL_INT8 ? pick_wide_i8_i8(pl.mt, rope != nullptr) : pick_wide_fp8_fp8(pl.mt, rope != nullptr);
     else if (dynq) k = dtype == QL_INT8 ? pick_i8_i8_dynq(pl.mt, pl.wn, pl.wk, pl.cp) : pick_fp8_fp8_dynq(pl.mt, pl.wn, pl.wk, pl.cp);

@@ -156,3 +156,18 @@ def test_scratch_covers_every_plan_of_a_row_count(N, K, table):
     finally:
         if not table:
             Q.load_plan_table(Q.PLAN_TABLE)
+
+
+@pytest.mark.parametrize("form,dtype", [(0, I8), (0, F8), (A, I8), (A, F8)])
+def test_costs_choose_one_plan_for_every_32_rows(no_table, form, dtype):
+    """Scratch is asked for by the last row count of 32: all of them have to run on its plan."""
+    for N, K in [(8192, 12288), (4096, 9728), (2048, 12288), (3072, 3072), (1344, 7104)]:
+        for last in (32, 64, 96, 160, 256):
+            assert len({Q.plan_query(form, M, N, K, dtype) for M in range(last - 31, last + 1)}) == 1
+
+
+@pytest.mark.parametrize("form,dtype,M,N,K,plan", [
+    (A, F8, 33, 8192, 12288, (2, 2, 4, 8, 2)), (A, I8, 64, 6144, 8192, (2, 2, 4, 8, 2)), (0, I8, 64, 2048, 12288, (1, 2, 4, 8, 4)),
+    (A | S, F8, 64, 19456, 2560, (2, 4, 2, 8, 1)), (A | S, F8, 64, 16384, 2560, (2, 2, 4, 8, 1))])
+def test_plans_that_costs_and_long_gates_take(no_table, form, dtype, M, N, K, plan):
+    assert Q.plan_query(form, M, N, K, dtype) == plan
