@@ -62,16 +62,27 @@ __device__ __forceinline__ TileWalk<TK> make_walk(int min_pos, int max_pos, int 
 }
 
 // The mask of a tile of 32 PARTS keys, counted from a lane's first: a row sees the last `near` keys up to its own, key `ahead`, and those up to
-// `kept`.  Without && and ||: with them the compiler branches lane by lane, 626 instructions per tile of 64.
-template <int PARTS>
-__device__ __forceinline__ void mask_tile(f32x16 (&s)[PARTS], int ahead, int near, int kept) {
+// `kept`.  LATER / EARLIER: whether the tile has keys behind some row's own, and keys in front of some row's window (or chunk); both are
+// uniform over a wave, and most masked tiles have one kind.  Without && and ||: with them the compiler branches lane by lane, 626 instructions
+// per tile of 64 (162 with both kinds in one comparison, 64 and 96 in two).
+template <bool LATER, bool EARLIER, int PARTS>
+__device__ __forceinline__ void mask_side(f32x16 (&s)[PARTS], int ahead, int near, int kept) {
+    asm volatile("");                                      // (a branch around it, not selects that every tile runs)
+    const int first = ahead - near;
 #pragma unroll
     for (int j = 0; j < PARTS; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int c = 32 * j + (r & 3) + 8 * (r >> 2);
-            s[j][r] = ((unsigned)ahead - (unsigned)c < (unsigned)near) | (c <= kept) ? s[j][r] : -INFINITY;
+            if (LATER) s[j][r] = c <= ahead ? s[j][r] : -INFINITY;
+            if (EARLIER) s[j][r] = ((c > first) | (c <= kept)) ? s[j][r] : -INFINITY;
         }
+}
+
+template <int PARTS>
+__device__ __forceinline__ void mask_tile(f32x16 (&s)[PARTS], bool later, bool earlier, int ahead, int near, int kept) {
+    if (later) mask_side<true, false>(s, ahead, near, kept);
+    if (earlier) mask_side<false, true>(s, ahead, near, kept);
 }
 
 // Walks tiles [vt_lo, vt_hi) of `walk` for the calling lane's query row at position row_pos; wave_min_pos / wave_max_pos = the
@@ -213,18 +224,9 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
                 for (int r = 0; r < 16; ++r)
                     s[j][r] = 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[j][r] * pre));
         }
-        if (pooled) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int e = kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi;
-                    if (e >= my_pool) s[j][r] = -INFINITY;
-                }
-        } else if (kt0 + kTileKeys - 1 > wave_min_pos || (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo) {
-            // (a tile that every row of the wave sees whole needs no mask)
-            mask_tile(s, row_pos - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
-        }
+        // (a tile that every row of the wave sees whole needs no mask; a pooled one hides what the row's window has not passed yet)
+        mask_tile(s, pooled | (kt0 + kTileKeys - 1 > wave_min_pos), !pooled & ((window > 0 & wave_max_pos - kt0 >= window) | (kt0 < wave_chunk_lo)),
+                  (pooled ? my_pool - 1 : row_pos) - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
         bf16x8 pf[2][2];
         if (SIG) {
 #pragma unroll
@@ -294,10 +296,12 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
 
 // The same walk for head sizes of exactly 32 NBK and 32 NBV channels, whose tiles go from global memory straight to LDS: two
 // buffers, one barrier per tile.  The loop above holds a tile in registers on its way (a wave then has 350 of them and its SIMD
-// to itself, with nothing to fill its waits; held to 256 it takes 110 us where this one takes 73 and the first took 174: eight
-// prompts of about 1000 tokens, 16 / 8 heads of 128, a window of 512, capped scores).  What is left is the vector unit's:
-// three exponentials or reciprocals per capped score.  (82 us with masks that branched lane by lane, two tiles of ten, and with every
-// piece's address worked out at every tile, 130 of a tile's 530 vector instructions.)  Tiles of 32 keys, which fit three waves, measured the same.
+// to itself, with nothing to fill its waits; held to 256 it takes 110 us where this one took 73 and the first 174: eight
+// prompts of about 1000 tokens, 16 / 8 heads of 128, a window of 512, capped scores).  What is left is the vector unit's: three
+// exponentials or reciprocals per capped score; 55 % of a SIMD's cycles are vector instructions, 20 % products, and a fifth of the time is
+// the last workgroups' (two rounds of unequal ones).  Masks of one side and the cap's last multiply-add folded into what a score is worth
+// took 32 such prompts from 225 to 211 us, two of 3000 to 4000 tokens from 71 to 65, heads of 64 from 56 to 50.  Tiles of 32 keys, which
+// fit three waves, and cache blocks looked up a tile ahead measured the same.
 // A row of 2 P bytes is kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows
 // that differ mod 16, one chunk) and the 32 of a transposed read (four rows, four chunks) then touch every bank once.  A
 // wave none of whose rows sees a tile leaves it out: a masked score would add an exact zero.
@@ -388,6 +392,7 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
         for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
     m_run = -INFINITY;
     float l_run = 0.f;
+    const float worth = MODE == kSoftcap ? 2.f * c_log2 : c_log2;
     const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;      // transposed-read address pieces
     // a chunk's number enters its place by exclusive or: the reads' addresses are one base each, changed in the chunk's bits
     const int k_at = GK::at(l31, hi), v_at = GV::at(4 * hi + tq, 2 * gq + (tp >> 1)) + 8 * (tp & 1),
@@ -420,21 +425,26 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[j][r] = __builtin_fmaf(s[j][r], c_log2, pre);
             }
-            if (MODE == kSoftcap) {                          // tanh(z) = 1 - 2 / (1 + e^2z); both infinities come out right
+            if (MODE == kSoftcap) {                          // tanh(z) = 1 - 2 / (1 + e^2z): its last term, the factor 2 in `worth`
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    s[j][r] = 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[j][r] * pre));
+                for (int r = 0; r < 16; ++r) s[j][r] = __builtin_amdgcn_rcpf(-1.f - __builtin_amdgcn_exp2f(s[j][r] * pre));
             }
         }
-        if (pooled) {
+        // (a tile that every row of the wave sees whole needs no mask; a pooled one hides what the row's window has not passed yet.  One form for
+        // both takes 40 registers less: 64 channels 47.8 -> 45.2 us, 128 under a cap 68.6 -> 66.7; but 128 without a cap 56.9 -> 58.0)
+        const bool later = kt1 > wave_min_pos, earlier = (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo;
+        if constexpr (MODE == kSoftmax && NBK == 4 && NBV == 4) {
+            if (pooled) {
 #pragma unroll
-            for (int j = 0; j < kSlimParts; ++j)
+                for (int j = 0; j < kSlimParts; ++j)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi >= my_pool) s[j][r] = -INFINITY;
-        } else if (kt1 > wave_min_pos || (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo) {
-            // (a tile that every row of the wave sees whole needs no mask)
-            mask_tile(s, row_pos - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
+                    for (int r = 0; r < 16; ++r)
+                        if (kt0 + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hi >= my_pool) s[j][r] = -INFINITY;
+            } else {
+                mask_tile(s, later, earlier, row_pos - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
+            }
+        } else {
+            mask_tile(s, pooled | later, !pooled & earlier, (pooled ? my_pool - 1 : row_pos) - kt0 - 4 * hi, near, kept - kt0 - 4 * hi);
         }
         bf16x8 pf[2 * kSlimParts];
         if (SIG) {
@@ -452,14 +462,14 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float m_new = fmaxf(m_run, mx);
             const bool none = m_new == -INFINITY;            // the row has seen nothing yet: no rescale, and every weight is zero
-            const float alpha = none ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_log2);
-            const float mc = none ? 0.f : m_new * c_log2;
+            const float alpha = none ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * worth);
+            const float mc = none ? 0.f : m_new * worth;
             float psum = 0.f;
 #pragma unroll
             for (int t = 0; t < 2 * kSlimParts; ++t)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t >> 1][8 * (t & 1) + e], c_log2, -mc));
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t >> 1][8 * (t & 1) + e], worth, -mc));
                     psum += p;
                     pf[t][e] = (bf16_t)p;
                 }
@@ -498,6 +508,7 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
     }
     l_tot = l_run + __shfl_xor(l_run, 32);
     if (SIG) { m_run = 0.f; l_tot = 1.f; }
+    if (MODE == kSoftcap) m_run = 1.f + 2.f * m_run;
 }
 
 }  // namespace hm
