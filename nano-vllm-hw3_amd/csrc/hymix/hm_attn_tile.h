@@ -299,9 +299,11 @@ __device__ __forceinline__ void kv_tile_loop(const unsigned short* __restrict__ 
 // to itself, with nothing to fill its waits; held to 256 it takes 110 us where this one took 73 and the first 174: eight
 // prompts of about 1000 tokens, 16 / 8 heads of 128, a window of 512, capped scores).  What is left is the vector unit's: three
 // exponentials or reciprocals per capped score; 55 % of a SIMD's cycles are vector instructions, 20 % products, and a fifth of the time is
-// the last workgroups' (two rounds of unequal ones).  Masks of one side and the cap's last multiply-add folded into what a score is worth
-// took 32 such prompts from 225 to 211 us, two of 3000 to 4000 tokens from 71 to 65, heads of 64 from 56 to 50.  Tiles of 32 keys, which
-// fit three waves, and cache blocks looked up a tile ahead measured the same.
+// the last workgroups' (two rounds of unequal ones).  Masks of one side, and pooled blocks in the same form, took 32 such prompts from 224 to
+// 213 us, two of 3000 to 4000 tokens from 71 to 66.5, heads of 64 without a cap from 50 to 44.  Scores are what the loop above makes of
+// them, bit for bit: with the cap's last multiply-add folded into what a score is worth, 1 to 4 % faster, the maximum that is taken off was
+// rounded to 2^-24 of the cap and not of itself, and with a cap of 50 one result in 650 differed by a bf16
+// rounding.  Tiles of 32 keys, which fit three waves, and cache blocks looked up a tile ahead measured the same.
 // A row of 2 P bytes is kept in 16-byte chunks, chunk c of row r at place c ^ swz(r): the 16 lanes of a 16-byte read (rows
 // that differ mod 16, one chunk) and the 32 of a transposed read (four rows, four chunks) then touch every bank once.  A
 // wave none of whose rows sees a tile leaves it out: a masked score would add an exact zero.
@@ -392,7 +394,6 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
         for (int r = 0; r < 16; ++r) oacc[d][r] = 0.f;
     m_run = -INFINITY;
     float l_run = 0.f;
-    const float worth = MODE == kSoftcap ? 2.f * c_log2 : c_log2;
     const int gq = (lane >> 4) & 1, ti = lane & 15, tq = ti >> 2, tp = ti & 3;      // transposed-read address pieces
     // a chunk's number enters its place by exclusive or: the reads' addresses are one base each, changed in the chunk's bits
     const int k_at = GK::at(l31, hi), v_at = GV::at(4 * hi + tq, 2 * gq + (tp >> 1)) + 8 * (tp & 1),
@@ -425,13 +426,14 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[j][r] = __builtin_fmaf(s[j][r], c_log2, pre);
             }
-            if (MODE == kSoftcap) {                          // tanh(z) = 1 - 2 / (1 + e^2z): its last term, the factor 2 in `worth`
+            if (MODE == kSoftcap) {                          // tanh(z) = 1 - 2 / (1 + e^2z); both infinities come out right
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[j][r] = __builtin_amdgcn_rcpf(-1.f - __builtin_amdgcn_exp2f(s[j][r] * pre));
+                for (int r = 0; r < 16; ++r)
+                    s[j][r] = 1.f - 2.f * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(s[j][r] * pre));
             }
         }
         // (a tile that every row of the wave sees whole needs no mask; a pooled one hides what the row's window has not passed yet.  One form for
-        // both takes 40 registers less: 64 channels 47.8 -> 45.2 us, 128 under a cap 68.6 -> 66.7; but 128 without a cap 56.9 -> 58.0)
+        // both takes 40 registers less: 64 channels 47.8 -> 45.2 us, 128 under a cap 70.5 -> 69.3; but 128 without a cap 56.9 -> 58.0)
         const bool later = kt1 > wave_min_pos, earlier = (window > 0 && wave_max_pos - kt0 >= window) || kt0 < wave_chunk_lo;
         if constexpr (MODE == kSoftmax && NBK == 4 && NBV == 4) {
             if (pooled) {
@@ -462,14 +464,14 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
             mx = fmaxf(mx, __shfl_xor(mx, 32));
             const float m_new = fmaxf(m_run, mx);
             const bool none = m_new == -INFINITY;            // the row has seen nothing yet: no rescale, and every weight is zero
-            const float alpha = none ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * worth);
-            const float mc = none ? 0.f : m_new * worth;
+            const float alpha = none ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * c_log2);
+            const float mc = none ? 0.f : m_new * c_log2;
             float psum = 0.f;
 #pragma unroll
             for (int t = 0; t < 2 * kSlimParts; ++t)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t >> 1][8 * (t & 1) + e], worth, -mc));
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t >> 1][8 * (t & 1) + e], c_log2, -mc));
                     psum += p;
                     pf[t][e] = (bf16_t)p;
                 }
@@ -508,7 +510,6 @@ __device__ __forceinline__ void kv_slim_loop(const unsigned short* __restrict__ 
     }
     l_tot = l_run + __shfl_xor(l_run, 32);
     if (SIG) { m_run = 0.f; l_tot = 1.f; }
-    if (MODE == kSoftcap) m_run = 1.f + 2.f * m_run;
 }
 
 }  // namespace hm
