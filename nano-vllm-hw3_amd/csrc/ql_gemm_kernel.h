@@ -420,10 +420,20 @@ void qgemm_kernel(const GemmParams p) {
         if constexpr (W16) return W2{i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}};
         else return i32x4{0, 0, 0, 0};
     };
-    auto load_x_to = [&](auto chk, int kc, xreg_t* sreg) {
+    constexpr bool PAIRS = ACT == ACT_FP8 && !W16 && !DYNQ && QL_FP8_K64;      // fp8 x fp8: two 32-k steps per instruction
+    constexpr bool LEAN = !DB && CP <= 8 && !GROUP && !DYNQ && !W16 && !SK &&
+                          (ACT == ACT_BF16 ? !ROPE && (!FP8W || MT == 2) : !(ACT == ACT_FP8 && WN == 1 && WK == 8 && CP == 4));
+    constexpr bool RUN_ON = LEAN || (!DB && ACT == ACT_BF16 && MT == 1 && (FP8W || GROUP) && CP <= 8 && (!GROUP || CP * WK <= 32));
+    // Pairs of fp8 steps that stop between chunks: the addresses of the staged rows and of the fragments are worked out chunk by chunk, and the
+    // ragged last chunk is behind the loop.  Kept over the loop, or with both forms in it, they take the 32 x 32 tile of 1024-k chunks from 80
+    // to 90 registers and with them its third workgroup per CU (6176 x 9216, 8 rows: 16.2 -> 18.1 us; 12288 x 12288, 16 rows 33.5 -> 37.4).
+    constexpr bool ANEW = PAIRS && !DB && !RUN_ON;
+    auto load_x_to = [&](auto chk, auto anew, int kc, xreg_t* sreg) {
         if (fullM) {
             const bool ok = !decltype(chk)::value || (kc + st_k < kend);
-            const unsigned off = ok ? xoff0 : (unsigned)(m0 * p.K) * XB;         // any valid address when past the slice
+            unsigned xoff = xoff0;
+            if constexpr (decltype(anew)::value) asm volatile("" : "+v"(xoff));
+            const unsigned off = ok ? xoff : (unsigned)(m0 * p.K) * XB;          // any valid address when past the slice
             const unsigned char* xs = p.x + (size_t)kc * XB;
 #pragma unroll
             for (int j = 0; j < C::NP; ++j)
@@ -431,9 +441,11 @@ void qgemm_kernel(const GemmParams p) {
         } else {
             // last row block: rows past M are not fetched (zeros: their outputs are never stored).  All lanes of a
             // wave hold pieces of the same row whenever a row has at least 64 pieces, so the branch is uniform.
+            int row0 = m0 + st_row0;
+            if constexpr (decltype(anew)::value) asm volatile("" : "+v"(row0));
 #pragma unroll
             for (int j = 0; j < C::NP; ++j) {
-                const int row = m0 + st_row0 + j * RS;
+                const int row = row0 + j * RS;
                 const int k = (kc + st_k < kend) ? kc + st_k : k0;
                 if (row < p.M) sreg[j] = xload(p.x + ((size_t)row * p.K + k) * XB);
                 else sreg[j] = xzero();
@@ -498,7 +510,7 @@ void qgemm_kernel(const GemmParams p) {
             }
         }
     };
-    auto load_x = [&](auto chk, int kc) { load_x_to(chk, kc, sreg); load_s(kc); };
+    auto load_x = [&](auto chk, int kc) { load_x_to(chk, FalseT{}, kc, sreg); load_s(kc); };
     auto store_x = [&](int buf, int kc) { store_x_from(buf, sreg); store_s(buf, kc); };
     // Double-buffered tiles: the scale of the group a wave is summing sits in a register, requested one fold ahead
     // (at the fold before it, for the group of the wave's next step).  Requested at the fold itself, the load's wait
@@ -558,7 +570,8 @@ void qgemm_kernel(const GemmParams p) {
         constexpr int GM = decltype(gmc)::value;
         const bool gstart = (GM == 1 && (ph & 3) == 0) || (GM == 2 && ph == 0);
         const int kb = kc + wk * C::KW + c * 32;   // first k of this step (wave-uniform)
-        if (decltype(chk)::value && kb >= kend) return;
+        // (a pair of fp8 steps is the odd one's to finish, also where the slice ends between them)
+        if (decltype(chk)::value && kb - (PAIRS && (c & 1) ? 32 : 0) >= kend) return;
         const int base_c = (wk * CP + c) * APS;    // first piece of the step in an LDS row (uniform)
         // piece index (base_c | lane part) with the low bits XOR-swizzled by the row; kept as an LDS byte OFFSET
         // (an integer), not a pointer: xor-ing a pointer through uintptr_t makes it generic and the read a flat load
@@ -587,38 +600,31 @@ void qgemm_kernel(const GemmParams p) {
                 }
             }
         } else {
-            if constexpr (ACT == ACT_FP8 && !W16 && !DYNQ && QL_FP8_K64) {
+            if constexpr (PAIRS) {
                 // fp8 x fp8 at the chip's full fp8 rate: two 32-k steps per v_mfma_scale_f32_32x32x64_f8f6f4 (unit
                 // scales, e4m3 operands), which runs 64 k in the cycles the K = 16 instruction pair above takes for
                 // 32.  A lane's 32 operand bytes are its 16 of the even step and its 16 of the odd step, for A and
                 // B alike, so the contraction is again a permutation of the k sum.  The even step only parks its
-                // weights; a lone last step (K slice not a multiple of 64) has zeros for its odd half.  It must not
-                // take the K = 16 pair: with products of both latencies in front of a join, the compiler counts the
-                // wait of the short one for the results of the long one, which were then read before they were
-                // whole (32 x 32 tile of 1024-k chunks, 33 x 100 x 544: about one call in a thousand wrong).
+                // weights; where the slice ends behind it (not a multiple of 64 k) the odd step stands for zeros: its weights are
+                // made zero, and its activations are the even step's again (what lies behind them in LDS need not be finite).
+                // A lone step must not take the K = 16 pair: with products of both latencies in front of a join, the
+                // compiler counts the wait of the short one for the results of the long one, which were then read before
+                // they were whole (32 x 32 tile of 1024-k chunks, 33 x 100 x 544: about one call in a thousand wrong).
                 typedef int i32x8 __attribute__((ext_vector_type(8)));
                 if ((c & 1) == 0) {
-                    if (!decltype(chk)::value || kb + 32 < kend) {
-                        w_even = w;
-                        return;
-                    }
-                    const i32x8 bb = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
-#pragma unroll
-                    for (int i = 0; i < MT; ++i) {
-                        const i32x4 ae = *(const i32x4*)(smem + a0 + i * 32 * RB);
-                        const i32x8 aa = {ae[0], ae[1], ae[2], ae[3], 0, 0, 0, 0};
-                        acc[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aa, bb, acc[i], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
-                    }
+                    w_even = w;
                     return;
                 }
                 {
+                    const bool lone = decltype(chk)::value && kb >= kend;
                     const int bc0 = base_c - APS;                  // the even step's first piece
                     const int a_ev = buf * C::XBYTES + a_row + ((bc0 & ~SWZ_MASK) << 4) + (((bc0 & SWZ_MASK) << 4) ^ a_g4);
-                    const i32x8 bb = {w_even[0], w_even[1], w_even[2], w_even[3], w[0], w[1], w[2], w[3]};
+                    const int a_od = lone ? a_ev : a0;
+                    const i32x8 bb = {w_even[0], w_even[1], w_even[2], w_even[3], lone ? 0 : w[0], lone ? 0 : w[1], lone ? 0 : w[2], lone ? 0 : w[3]};
 #pragma unroll
                     for (int i = 0; i < MT; ++i) {
                         const i32x4 ae = *(const i32x4*)(smem + a_ev + i * 32 * RB);
-                        const i32x4 ao = *(const i32x4*)(smem + a0 + i * 32 * RB);
+                        const i32x4 ao = *(const i32x4*)(smem + a_od + i * 32 * RB);
                         const i32x8 aa = {ae[0], ae[1], ae[2], ae[3], ao[0], ao[1], ao[2], ao[3]};
                         // (cbsz = blgp = 0: both operands e4m3; scale bytes 0x7F = 2^0)
                         acc[i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(aa, bb, acc[i], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
@@ -703,7 +709,7 @@ void qgemm_kernel(const GemmParams p) {
         using GMC = std::integral_constant<int, !decltype(gsel)::value ? 0 : (CP % 4 == 0) ? 1 : 2 + PAR>;
         const int kc = k0 + it * C::KB;
         wreg_t* wset = PAR ? wcur2 : wcur;
-        if (it + 2 < nchunks) load_x_to(TrueT{}, kc + 2 * C::KB, PAR ? sreg2 : sreg);
+        if (it + 2 < nchunks) load_x_to(TrueT{}, FalseT{}, kc + 2 * C::KB, PAR ? sreg2 : sreg);
 #pragma unroll
         for (int c = 0; c < CP; ++c) {
             const wreg_t w = wset[c];
@@ -717,9 +723,11 @@ void qgemm_kernel(const GemmParams p) {
         const int kc = k0 + it * C::KB;
         // activations first: the wait counter is positional, so staging them must not wait for the (slower,
         // HBM) weight loads issued behind them
-        load_x(chk, kc);
+        load_x_to(chk, std::integral_constant<bool, ANEW>{}, kc, sreg);
+        load_s(kc);
 #pragma unroll
         for (int j = 0; j < D; ++j) wcur[j] = load_w1(chk, kc, j);
+        if constexpr (ANEW) asm volatile("" : "+v"(a_row));
         store_x(0, kc);
         __syncthreads();
         for (int c0 = 0; c0 < CP; c0 += D) {
@@ -742,9 +750,6 @@ void qgemm_kernel(const GemmParams p) {
     // 0.95 to 0.98 in the 32 x 32 ones (936 calls, 1 to 256 rows, weights that no cache holds).  Not in the 32 x 32 tile of 1024-k chunks with
     // fp8 activations, which loses its third workgroup per CU (512 and more of them: 1.08), nor in the 64 x 64 tile with groups, which spills.
     // (an address past the slice's end is the last step's: step() skips what it brings)
-    constexpr bool LEAN = !DB && CP <= 8 && !GROUP && !DYNQ && !W16 && !SK &&
-                          (ACT == ACT_BF16 ? !ROPE && (!FP8W || MT == 2) : !(ACT == ACT_FP8 && WN == 1 && WK == 8 && CP == 4));
-    constexpr bool RUN_ON = LEAN || (!DB && ACT == ACT_BF16 && MT == 1 && (FP8W || GROUP) && CP <= 8 && (!GROUP || CP * WK <= 32));
     auto chunk_on = [&](auto chk, auto gmc, auto morec, int it) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(morec)::value;
         const int kc = k0 + it * C::KB;
@@ -771,10 +776,10 @@ void qgemm_kernel(const GemmParams p) {
     using GM1 = std::integral_constant<int, GS ? 1 : 0>;           // (the non-DEEP loops: whole groups per chunk part)
     if constexpr (DEEP) {
         if (nchunks > 0) {
-            load_x_to(TrueT{}, k0, sreg);                         // (before the weights: positional wait counter)
+            load_x_to(TrueT{}, FalseT{}, k0, sreg);               // (before the weights: positional wait counter)
 #pragma unroll
             for (int c = 0; c < CP; ++c) wcur[c] = load_w1(TrueT{}, k0, c);
-            if (nchunks > 1) load_x_to(TrueT{}, k0 + C::KB, sreg2);
+            if (nchunks > 1) load_x_to(TrueT{}, FalseT{}, k0 + C::KB, sreg2);
 #pragma unroll
             for (int c = 0; c < CP; ++c) wcur2[c] = load_w_ring(k0 + C::KB, c);
             store_x_from(0, sreg);
@@ -823,6 +828,10 @@ void qgemm_kernel(const GemmParams p) {
             for (; it + 1 < nchunks; ++it) chunk_on(FalseT{}, GM1{}, TrueT{}, it);
             if (k0 + (it + 1) * C::KB <= kend) chunk_on(FalseT{}, GM1{}, FalseT{}, it);
             else chunk_on(TrueT{}, GM1{}, FalseT{}, it);
+        } else if constexpr (ANEW) {
+            int it = 0;
+            for (; k0 + (it + 1) * C::KB <= kend; ++it) chunk_sb(FalseT{}, GM1{}, it);
+            if (it < nchunks) chunk_sb(TrueT{}, GM1{}, it);
         } else {
             for (int it = 0; it < nchunks; ++it) {
                 if (k0 + (it + 1) * C::KB <= kend) chunk_sb(FalseT{}, GM1{}, it);
