@@ -174,7 +174,7 @@ struct Cfg {
 };
 
 template <int ACT, bool FP8W, int MT, int WN, int WK, int CP, bool DB, bool GROUP, bool ROPE = false, bool W16 = false,
-          bool AMAX = false, bool DYNQ = false, bool SK = false>
+          bool AMAX = false, bool DYNQ = false, bool SK = false, bool STOP = false>
 // (second launch bound = waves per SIMD the register allocation must leave room for: the 128 x 256 weight-only tile
 // with 64-k chunks is held to 128 registers so that TWO of its 8-wave workgroups share a CU and one's prologue and
 // epilogue run under the other's MFMAs - worth more on the K <= 2048 shapes than the registers it gives up)
@@ -421,12 +421,12 @@ void qgemm_kernel(const GemmParams p) {
         else return i32x4{0, 0, 0, 0};
     };
     constexpr bool PAIRS = ACT == ACT_FP8 && !W16 && !DYNQ && QL_FP8_K64;      // fp8 x fp8: two 32-k steps per instruction
-    constexpr bool LEAN = !DB && CP <= 8 && !GROUP && !DYNQ && !W16 && !SK &&
+    constexpr bool LEAN = !STOP && !DB && CP <= 8 && !GROUP && !DYNQ && !W16 && !SK &&
                           (ACT == ACT_BF16 ? !ROPE && (!FP8W || MT == 2) : !(ACT == ACT_FP8 && WN == 1 && WK == 8 && CP == 4));
     constexpr bool RUN_ON = LEAN || (!DB && ACT == ACT_BF16 && MT == 1 && (FP8W || GROUP) && CP <= 8 && (!GROUP || CP * WK <= 32));
     // Pairs of fp8 steps that stop between chunks: the addresses of the staged rows and of the fragments are worked out chunk by chunk, and the
     // ragged last chunk is behind the loop.  Kept over the loop, or with both forms in it, they take the 32 x 32 tile of 1024-k chunks from 80
-    // to 90 registers and with them its third workgroup per CU (6176 x 9216, 8 rows: 16.2 -> 18.1 us; 12288 x 12288, 16 rows 33.5 -> 37.4).
+    // to 90 registers and with them its third workgroup per CU (6176 x 9216, 8 rows: 16.2 -> 18.3 us; 12288 x 12288, 16 rows 33.9 -> 37.2).
     constexpr bool ANEW = PAIRS && !DB && !RUN_ON;
     auto load_x_to = [&](auto chk, auto anew, int kc, xreg_t* sreg) {
         if (fullM) {
@@ -749,6 +749,7 @@ void qgemm_kernel(const GemmParams p) {
     // they gained nothing or lost up to 20 %): 0.84 to 0.93 of the time in the 32 x 64 and 64 x 64 tiles over three chunks and more,
     // 0.95 to 0.98 in the 32 x 32 ones (936 calls, 1 to 256 rows, weights that no cache holds).  Not in the 32 x 32 tile of 1024-k chunks with
     // fp8 activations, which loses its third workgroup per CU (512 and more of them: 1.08), nor in the 64 x 64 tile with groups, which spills.
+    // (STOP: int8 rows where stopping is the faster form all the same, see row_stops in ql_gemm.hip)
     // (an address past the slice's end is the last step's: step() skips what it brings)
     auto chunk_on = [&](auto chk, auto gmc, auto morec, int it) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(morec)::value;
@@ -1257,6 +1258,7 @@ int w8a16_dispatch(const char* fn, int wdtype, int granularity, const void* x, c
 size_t w8a16_workspace_need(int wdtype, int64_t M, int64_t N, int64_t K, int granularity, size_t* ticket_bytes);
 
 kern_t pick_bf16_i8_row(int, int, int, int, bool rope = false);
+kern_t pick_bf16_i8_row_stop(int wn);             // the tiles (1, 1, 8, 4) and (1, 2, 4, 8) that stop between chunks
 kern_t pick_bf16_i8_group(int, int, int, int, bool rope = false);
 kern_t pick_bf16_fp8_row(int, int, int, int, bool rope = false);
 kern_t pick_bf16_fp8_group(int, int, int, int, bool rope = false);

@@ -45,7 +45,7 @@ def registers(tmp_path_factory):
 
 
 def decode_kernel(act, fp8_weights, mt, wn, wk, cp):
-    return f"_ZN2ql12qgemm_kernelILi{act}ELb{fp8_weights}ELi{mt}ELi{wn}ELi{wk}ELi{cp}" + "ELb0" * 7 + "EEEvNS_10GemmParamsE"
+    return f"_ZN2ql12qgemm_kernelILi{act}ELb{fp8_weights}ELi{mt}ELi{wn}ELi{wk}ELi{cp}" + "ELb0" * 8 + "EEEvNS_10GemmParamsE"
 
 
 @pytest.mark.parametrize("act,fp8_weights,tile,most", [
