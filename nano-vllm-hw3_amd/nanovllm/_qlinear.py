@@ -126,7 +126,8 @@ def load():
 
 def load_plan_table(path, replace=False, strict=False):
     """Register the measured GEMM plans of a JSON file written by tools/autotune_plans.py:
-    {"plans": [{"form", "N", "K", "m_lo", "m_hi", "tile": [mt, wn, wk, cp], "split"}, ...]}.  Returns the number
+    {"plans": [{"form", "N", "K", "m_lo", "m_hi", "tile": [mt, wn, wk, cp], "split"}, ...]} (an entry's times, "us" and
+    "heuristic_us", are those of that tool, or with "timed": "alone" of tools/time_plans.py).  Returns the number
     of entries set; a missing file is no error (the built-in heuristics then apply to every shape).  An entry the
     library rejects (a tile this build does not have, an overlap) is skipped with a warning - a plan is an
     optimisation, never a reason not to start - unless ``strict``."""
