@@ -282,7 +282,8 @@ int ql_gemm_force_config(int mt, int wn, int wk, int cp, int split_k);
  * ql_gemm_plan_of_call writes {mt, wn, wk, cp, split_k} of the plan a call runs to out[5]: form with QL_PLAN_NARROW for operands off
  * 16 bytes, staged quantization or row maxima; dtype QL_INT8 or QL_FP8, the weights' (and 8-bit activations') type; group = the group
  * size with QL_PLAN_GROUP, else 0.  {mt, 8, 1, 8, 1} is a 32 mt x 256 tile, which needs no workspace.  ql_gemm_plan_query is the same for
- * QL_INT8 and groups of 128. */
+ * QL_INT8 and groups of 128.  ql_gemm_plans_costed counts the shapes that the calling thread has worked out tile costs for: none that
+ * the table holds, and none again among the last ones. */
 #define QL_PLAN_GROUP 1    /* per-group scales */
 #define QL_PLAN_SILU 2     /* ql_gemm_*_silu */
 #define QL_PLAN_ROPE 4     /* ql_gemm_*_rope */
@@ -295,6 +296,7 @@ void ql_gemm_plan_clear(void);
 int ql_gemm_plan_count(void);
 int ql_gemm_plan_query(int form, int64_t M, int64_t N, int64_t K, int* out);
 int ql_gemm_plan_of_call(int form, int dtype, int group, int64_t M, int64_t N, int64_t K, int* out);
+int64_t ql_gemm_plans_costed(void);
 
 /* ---- operators between the quantized GEMMs of a decoder layer (one launch each) ------------- */
 

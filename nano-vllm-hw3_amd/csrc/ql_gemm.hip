@@ -231,11 +231,11 @@ static bool mid_tile(int pick, int64_t M, int64_t N, int64_t K, bool group, bool
     return (t > 128 && K > 4096) || (t >= 80 && K >= 8192) || (t >= 80 && t <= 120 && K >= 6144);
 }
 
-// What a call of up to 256 rows over more than 2048 k takes in microseconds (weights that no cache holds) on one of the tiles that read a weight
-// once per row tile, in `split` slices: a start, what slices cost, and for the workgroups that a CU runs (`q` of it in whole rounds, the rest
-// as they overlap) a part per workgroup and one per 1000 k of its slice, by how much of the tile's rows are asked for; and the weights' way.
-// Fitted over 7171 calls (600 shapes of 512..12288 columns by 2112..16384 k, 1 to 256 rows) of 20 forms each, 7 to 11 % off in the root mean
-// square.  Rows count by 32, so that the plan is one for every 32 rows.
+// What a call of up to 256 rows over more than 2048 k takes in microseconds on one of the tiles that read a weight once per row tile, in
+// `split` slices: a start, what slices cost, and for the workgroups that a CU runs (`q` of it in whole rounds, the rest as they overlap) a part per
+// workgroup and one per 1000 k of its slice, by how much of the tile's rows are asked for; and the weights' way.  Fitted over 7171 calls (600 shapes
+// of 512..12288 columns by 2112..16384 k, 1 to 256 rows) of 20 forms each, 7 to 12 % off in the root mean square (tools/tile_costs.py; weights of up to
+// 16 MB came out of the memory-side cache).  Rows count by 32, so that the plan is one for every 32 rows.
 struct TileCost { double start, slices, slice, group, k, k_full, q, way; };
 constexpr int kCostTiles = 6;
 static const TileCfg kCostTile[kCostTiles] = {{1, 1, 8, 4, 0}, {1, 1, 8, 8, 0}, {1, 2, 4, 8, 0}, {1, 2, 4, 4, 1}, {2, 2, 4, 8, 0}, {2, 4, 2, 4, 1}};
@@ -270,23 +270,29 @@ static double tile_cost(int tile, int64_t split, int64_t M, int64_t N, int64_t K
 }
 
 // The tile and slices that the costs say are faster than the rules' (`tile` in `split` slices) by more than they are wrong by; false: keep those.
-// Lines: of the calls that change, 1 of 40 is slower than before by more than 4 %.  The double-buffered tiles stay: the 64 x 128 one's costs go up
-// and down with the number of tiles by more than the fit shows, and mid_tile's lines come from sweeps of their own.
+// On weights from memory 3978 random calls that change take 0.86 of the time, 43 of them more than 1.04 (the worst 1.19: 8-bit activations, 96 rows of
+// 8608 x 12608).  The double-buffered tiles stay: the 64 x 128 one's costs go up and down with the number of tiles by more than the fit
+// shows, and mid_tile's lines come from sweeps of their own.
 // us, rules / here: fp8 x fp8 33 x 8192 of 12288 k 38.1 / 24.1, 64 x 6144 of 8192 k 22.3 / 16.4; int8 64 x 2048 of 12288 k 17.4 / 13.3; over all calls
 // of 33 to 64 rows 0.92 (8-bit activations) and 0.95, up to 32 rows 0.96 and 0.98, from 65 rows on 0.95.
+static thread_local int64_t tl_costed = 0;                    // shapes that this thread has worked out costs for
 static bool cheaper_tile(int tile, int64_t split, int64_t M, int64_t N, int64_t K, bool fp8, bool w8a8, int* best_tile, int* best_split) {
-    // (worked out once per thread for the last shapes that a place of the table has seen: up to 40 costs take a microsecond, as long as a launch)
+    // (worked out once per thread for the last shape that a place of the table has seen: up to 40 costs take 0.3 us, a launch 2.  Shapes
+    // are multiples of large powers of two, so their bits are mixed: by (5 N + 3 K) / 32 all projections of Qwen3-8B met in one place)
     struct Seen { int64_t rows = 0, N = 0, K = 0, split = 0; int tile = 0, kind = 0, best_tile = 0, best_split = 0; };
-    static thread_local Seen table[64];
+    static thread_local Seen table[256];
     const int64_t rows = (M + 31) / 32;
     const int kind = w8a8 ? 2 : fp8;
-    Seen& seen = table[(uint64_t)(N * 5 + K * 3 + rows * 11 + kind) / 32 % 64];
+    uint64_t place = 0;
+    for (const int64_t v : {N, K, rows * 4 + kind}) place = (place ^ (uint64_t)v) * 0x9E3779B97F4A7C15u;
+    Seen& seen = table[place >> 56];
     auto answer = [&]() -> bool {
         *best_tile = seen.best_tile;
         if (seen.best_split) *best_split = seen.best_split;
         return seen.best_split != 0;
     };
     if (seen.rows == rows && seen.N == N && seen.K == K && seen.split == split && seen.tile == tile && seen.kind == kind) return answer();
+    ++tl_costed;
     seen = Seen{rows, N, K, split, tile, kind, 0, 0};
     const double line = M <= 32 ? 0.86 : M <= 64 ? 0.9 : 0.88;
     double best = line * tile_cost(tile, split, M, N, K, fp8, w8a8);
@@ -395,19 +401,6 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
         if (tiles < 512 && K >= 4096) return (K + 4095) / 4096;        // long K: at most four chunks per slice
         return 1;
     };
-    // (not in the allocation-free entry point, whose scratch array is sized for the rules' slices, nor for kernels that quantize while they
-    // stage, whose costs are others)
-    if (!silu && !rope && !group && M <= 256 && K > 2048 && !tl_skip_table && !rules_only) {
-        int tile = kCostTiles - 1;
-        while (tile >= 0 && !(kCostTile[tile].mt == mt && kCostTile[tile].wn == wn && kCostTile[tile].wk == wk && kCostTile[tile].cp == cp)) --tile;
-        const int64_t tiles = (M + 32 * mt - 1) / (32 * mt) * ((N + 32 * wn - 1) / (32 * wn)), kb0 = 32 * cp * wk, chunks = (K + kb0 - 1) / kb0;
-        int64_t slices = std::min(t_split ? t_split : rule_split(tiles), chunks);
-        slices = (chunks + (chunks + slices - 1) / slices - 1) / ((chunks + slices - 1) / slices);
-        int best = 0;
-        if (tile >= 0 && !kCostTile[tile].db && cheaper_tile(tile, slices, M, N, K, fp8, w8a8, &best, &t_split)) {
-            mt = kCostTile[best].mt; wn = kCostTile[best].wn; wk = kCostTile[best].wk; cp = kCostTile[best].cp;
-        }
-    }
     // 33 to 64 rows of 8-bit activations under the SiLU epilogue, K of 2048 and more, where the ladder ends in 64 x 128 tiles: 64 x 64
     // tiles, so that the weights are read once and more workgroups share them (fp8, us: 19456 x 2048 17.7 -> 15.2, 24576 x 4096 34.4 -> 25.9; the ladder's
     // own 64 x 64 tile of 12288 x 2048 takes 10.1 there, this one 11.9)
@@ -422,6 +415,8 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
     // not built for, one of theirs as well
     const int form = (group ? QL_PLAN_GROUP : 0) | (silu ? QL_PLAN_SILU : 0) | (rope ? QL_PLAN_ROPE : 0) | (w8a8 ? QL_PLAN_W8A8 : 0);
     const bool can_wide = wide_group >= 0 && wide_built(N, K, wide_group, silu, w8a8);
+    const bool forced = f_mt > 0 && f_wn > 0 && f_wk > 0 && f_cp > 0 && tile_built(f_mt, f_wn, f_wk, f_cp, group) && !(silu && (f_wn & 1)) &&
+                        !(rope && !rope_tile_built(f_mt, f_wn, f_wk, f_cp));
     PlanEntry te;
     if (plan_lookup(form, M, N, K, &te) ||
         (pl.narrow = !can_wide && wide_group != kNoEntry && plan_lookup(form | QL_PLAN_NARROW, M, N, K, &te))) {
@@ -435,9 +430,20 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
             return pl;
         }
         mt = 4; wn = 8; wk = 1; cp = 2; t_split = 1;
+    } else if (!silu && !rope && !group && M <= 256 && K > 2048 && !tl_skip_table && !rules_only && !forced) {
+        // (not in the allocation-free entry point, whose scratch array is sized for the rules' slices, nor for kernels that quantize while they
+        // stage, whose costs are others)
+        int tile = kCostTiles - 1;
+        while (tile >= 0 && !(kCostTile[tile].mt == mt && kCostTile[tile].wn == wn && kCostTile[tile].wk == wk && kCostTile[tile].cp == cp)) --tile;
+        const int64_t tiles = (M + 32 * mt - 1) / (32 * mt) * ((N + 32 * wn - 1) / (32 * wn)), kb0 = 32 * cp * wk, chunks = (K + kb0 - 1) / kb0;
+        int64_t slices = std::min(t_split ? t_split : rule_split(tiles), chunks);
+        slices = (chunks + (chunks + slices - 1) / slices - 1) / ((chunks + slices - 1) / slices);
+        int best = 0;
+        if (tile >= 0 && !kCostTile[tile].db && cheaper_tile(tile, slices, M, N, K, fp8, w8a8, &best, &t_split)) {
+            mt = kCostTile[best].mt; wn = kCostTile[best].wn; wk = kCostTile[best].wk; cp = kCostTile[best].cp;
+        }
     }
-    if (f_mt > 0 && f_wn > 0 && f_wk > 0 && f_cp > 0 && tile_built(f_mt, f_wn, f_wk, f_cp, group) && !(silu && (f_wn & 1)) &&
-        !(rope && !rope_tile_built(f_mt, f_wn, f_wk, f_cp))) {
+    if (forced) {
         mt = f_mt; wn = f_wn; wk = f_wk; cp = f_cp; t_split = 0;
     }
     pl.mt = mt; pl.wn = wn; pl.wk = wk; pl.cp = cp;
@@ -803,6 +809,8 @@ int ql_gemm_plan_of_call(int form, int dtype, int group, int64_t M, int64_t N, i
     out[0] = pl.mt; out[1] = pl.wn; out[2] = pl.wk; out[3] = pl.cp; out[4] = pl.split;
     return QL_OK;
 }
+
+int64_t ql_gemm_plans_costed(void) { return tl_costed; }
 
 int ql_gemm_plan_query(int form, int64_t M, int64_t N, int64_t K, int* out) {
     return ql_gemm_plan_of_call(form, QL_INT8, form >= 0 && (form & QL_PLAN_GROUP) ? 128 : 0, M, N, K, out);

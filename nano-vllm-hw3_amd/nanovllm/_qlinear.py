@@ -55,6 +55,7 @@ SIGNATURES = {
     "ql_gemm_plan_set": (_c_int, [_c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_int, _c_int, _c_int, _c_int, _c_int]),
     "ql_gemm_plan_clear": (None, []),
     "ql_gemm_plan_count": (_c_int, []),
+    "ql_gemm_plans_costed": (_c_i64, []),
     "ql_gemm_plan_query": (_c_int, [_c_int, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_int)]),
     "ql_gemm_plan_of_call": (_c_int, [_c_int, _c_int, _c_int, _c_i64, _c_i64, _c_i64, ctypes.POINTER(_c_int)]),
     "ql_add_rmsnorm": (_c_int, [_c_vp, _c_vp, _c_vp, ctypes.c_float, _c_vp, _c_vp, _c_i64, _c_i64, _c_vp]),

@@ -171,3 +171,36 @@ def test_costs_choose_one_plan_for_every_32_rows(no_table, form, dtype):
     (A | S, F8, 64, 19456, 2560, (2, 4, 2, 8, 1)), (A | S, F8, 64, 16384, 2560, (2, 2, 4, 8, 1))])
 def test_plans_that_costs_and_long_gates_take(no_table, form, dtype, M, N, K, plan):
     assert Q.plan_query(form, M, N, K, dtype) == plan
+
+
+MODELS = {"0.6b": [(4096, 1024), (1024, 2048), (1024, 3072)], "1.7b": [(4096, 2048), (2048, 2048), (2048, 6144)],
+          "4b": [(6144, 2560), (2560, 4096), (2560, 9728)], "8b": [(6144, 4096), (4096, 4096), (4096, 12288)]}
+
+
+@pytest.mark.parametrize("form,dtype", [(0, I8), (0, F8), (A, I8), (A, F8)])
+@pytest.mark.parametrize("model", MODELS)
+def test_costs_of_a_layers_shapes_are_worked_out_once(no_table, model, form, dtype):
+    """The linears of a layer in turn: each finds its answer of the step before."""
+    lib = Q.load()
+    for M in (1, 32, 33, 64, 100, 256):
+        def layer():
+            return [Q.plan_query(form, M, N, K, dtype) for N, K in MODELS[model]]
+        first, before = layer(), lib.ql_gemm_plans_costed()
+        for _ in range(3):
+            assert layer() == first
+        assert lib.ql_gemm_plans_costed() == before
+
+
+def test_costs_of_measured_and_forced_plans_are_not_worked_out(no_table):
+    lib = Q.load()
+    assert lib.ql_gemm_plan_set(A, 1, 32, 5024, 7072, 1, 2, 4, 8, 3) == 0
+    before = lib.ql_gemm_plans_costed()
+    assert Q.plan_query(A, 32, 5024, 7072, F8) == (1, 2, 4, 8, 3)
+    try:
+        assert lib.ql_gemm_force_config(1, 1, 8, 4, 1) == 0
+        assert Q.plan_query(A, 32, 5056, 7072, F8) == (1, 1, 8, 4, 1)
+    finally:
+        lib.ql_gemm_force_config(0, 0, 0, 0, 0)
+    assert lib.ql_gemm_plans_costed() == before
+    Q.plan_query(A, 32, 5056, 7072, F8)
+    assert lib.ql_gemm_plans_costed() == before + 1
