@@ -162,7 +162,8 @@ int ql_gemm_w8a8_silu(int dtype, const void* qx, const float* sx, const void* qw
  * K columns (what the workgroups of the producing kernel each see: ql_gemm_w8a8_silu and the attention kernels can
  * emit them; ql_row_absmax_parts computes them from x).  The kernel takes their maximum, clamps it at 1e-8 and
  * quantizes the activations while it stages them, with exactly the arithmetic of ql_quant_per_row; the result is
- * bit-identical to ql_quant_per_row followed by ql_gemm_w8a8.  Workspace as for ql_gemm_w8a8.
+ * bit-identical to ql_quant_per_row followed by ql_gemm_w8a8 (fp8: up to the order of its f32 sums, where the two run different plans: ql_gemm_plan_of_call
+ * with QL_PLAN_STAGED).  Workspace as for ql_gemm_w8a8.
  * ql_row_absmax_parts: out f32 [T, parts], out[t][i] = max |x[t, i*H/parts : (i+1)*H/parts]|; H % (8 * parts) == 0. */
 int ql_row_absmax_parts(const void* x_bf16, int64_t T, int64_t H, int parts, float* out, void* stream);
 /* ql_gemm_w8a8_silu that also emits what a ql_gemm_w8a8_dynq consumer of y needs: rowmax_part_out f32 [M, N/64],
@@ -280,7 +281,7 @@ int ql_gemm_force_config(int mt, int wn, int wk, int cp, int split_k);
  * K or N, operands off 16 bytes, activations quantized while they are staged, row maxima) also takes an entry of its form |
  * QL_PLAN_NARROW, behind one of its form.
  * ql_gemm_plan_of_call writes {mt, wn, wk, cp, split_k} of the plan a call runs to out[5]: form with QL_PLAN_NARROW for operands off
- * 16 bytes, staged quantization or row maxima; dtype QL_INT8 or QL_FP8, the weights' (and 8-bit activations') type; group = the group
+ * 16 bytes or row maxima, QL_PLAN_W8A8 | QL_PLAN_STAGED for ql_gemm_w8a8_dynq; dtype QL_INT8 or QL_FP8, the weights' (and 8-bit activations') type; group = the group
  * size with QL_PLAN_GROUP, else 0.  {mt, 8, 1, 8, 1} is a 32 mt x 256 tile, which needs no workspace.  ql_gemm_plan_query is the same for
  * QL_INT8 and groups of 128.  ql_gemm_plans_costed counts the shapes that the calling thread has worked out tile costs for: none that
  * the table holds, and none again among the last ones. */
@@ -290,6 +291,7 @@ int ql_gemm_force_config(int mt, int wn, int wk, int cp, int split_k);
 #define QL_PLAN_W8A8 8     /* ql_gemm_w8a8* (else ql_gemm_w8a16*) */
 #define QL_PLAN_PARTIAL 16 /* ql_gemm_*_partial */
 #define QL_PLAN_NARROW 32  /* calls that the 32 mt x 256 tiles are not built for */
+#define QL_PLAN_STAGED 64  /* ql_gemm_plan_of_call alone: activations quantized while they are staged (they share the entries of narrow calls) */
 int ql_gemm_plan_set(int form, int64_t m_lo, int64_t m_hi, int64_t N, int64_t K, int mt, int wn, int wk, int cp,
                      int split_k);
 void ql_gemm_plan_clear(void);

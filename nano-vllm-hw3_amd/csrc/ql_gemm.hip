@@ -796,16 +796,16 @@ int ql_gemm_plan_count(void) {
 }
 
 int ql_gemm_plan_of_call(int form, int dtype, int group, int64_t M, int64_t N, int64_t K, int* out) {
-    const int known = QL_PLAN_GROUP | QL_PLAN_SILU | QL_PLAN_ROPE | QL_PLAN_W8A8 | QL_PLAN_PARTIAL | QL_PLAN_NARROW;
-    const bool grp = (form & QL_PLAN_GROUP) != 0, partial = (form & QL_PLAN_PARTIAL) != 0;
-    if (!out || form < 0 || (form & ~known) || M <= 0 || N <= 0 || K <= 0 || K % 32 || (dtype != QL_INT8 && dtype != QL_FP8) ||
-        (grp ? group <= 0 : group != 0)) {
+    const int known = QL_PLAN_GROUP | QL_PLAN_SILU | QL_PLAN_ROPE | QL_PLAN_W8A8 | QL_PLAN_PARTIAL | QL_PLAN_NARROW | QL_PLAN_STAGED;
+    const bool grp = (form & QL_PLAN_GROUP) != 0, partial = (form & QL_PLAN_PARTIAL) != 0, staged = (form & QL_PLAN_STAGED) != 0;
+    if (!out || form < 0 || (form & ~known) || (staged && (form & ~QL_PLAN_NARROW) != (QL_PLAN_W8A8 | QL_PLAN_STAGED)) || M <= 0 ||
+        N <= 0 || K <= 0 || K % 32 || (dtype != QL_INT8 && dtype != QL_FP8) || (grp ? group <= 0 : group != 0)) {
         set_error("ql_gemm_plan_of_call: bad argument");
         return QL_EINVAL;
     }
     const Plan pl = partial ? make_plan_partial(M, N, K, grp)
                             : make_plan(M, N, K, grp, (form & QL_PLAN_SILU) != 0, (form & QL_PLAN_ROPE) != 0, (form & QL_PLAN_W8A8) != 0,
-                                        (form & QL_PLAN_NARROW) ? -1 : group, dtype == QL_FP8);
+                                        (form & (QL_PLAN_NARROW | QL_PLAN_STAGED)) ? -1 : group, dtype == QL_FP8, staged);
     out[0] = pl.mt; out[1] = pl.wn; out[2] = pl.wk; out[3] = pl.cp; out[4] = pl.split;
     return QL_OK;
 }

@@ -14,7 +14,7 @@ LIB_PATH = os.environ.get("QLINEAR_LIB") or os.path.join(_HERE, "_lib", "libqlin
 QL_INT8, QL_FP8 = 0, 1
 QL_TILED = 16
 QL_PER_ROW, QL_PER_TENSOR, QL_PER_GROUP = 0, 1, 2
-QL_PLAN_GROUP, QL_PLAN_SILU, QL_PLAN_ROPE, QL_PLAN_W8A8, QL_PLAN_PARTIAL, QL_PLAN_NARROW = 1, 2, 4, 8, 16, 32
+QL_PLAN_GROUP, QL_PLAN_SILU, QL_PLAN_ROPE, QL_PLAN_W8A8, QL_PLAN_PARTIAL, QL_PLAN_NARROW, QL_PLAN_STAGED = 1, 2, 4, 8, 16, 32, 64
 PLAN_TABLE = os.environ.get("QLINEAR_PLANS") or os.path.join(_HERE, "_plans", "gfx950.json")
 
 _c_vp, _c_i64, _c_int, _c_sz = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_size_t

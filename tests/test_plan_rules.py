@@ -1,6 +1,7 @@
 """Where the GEMM planner's lines lie, at the sizes on either side of each (host only): the plans that sweeps over cold weights
 found faster, and scratch that covers whatever a call may run."""
 import itertools
+import re
 
 import pytest
 
@@ -204,3 +205,31 @@ def test_costs_of_measured_and_forced_plans_are_not_worked_out(no_table):
     assert lib.ql_gemm_plans_costed() == before
     Q.plan_query(A, 32, 5056, 7072, F8)
     assert lib.ql_gemm_plans_costed() == before + 1
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 8192, 12288), (64, 6144, 8192), (8, 4096, 9728), (48, 1344, 7104), (16, 5120, 8192), (200, 1024, 5120)])
+@pytest.mark.parametrize("dtype", [I8, F8])
+@pytest.mark.parametrize("entry", [None, A, A | NARROW])
+def test_a_query_of_staged_quantization_answers_for_the_call(no_table, entry, dtype, M, N, K):
+    """The call says what scratch its plan needs, and launches nothing without it."""
+    import ctypes
+    lib = Q.load()
+    if entry is not None:
+        assert lib.ql_gemm_plan_set(entry, M, M, N, K, 1, 2, 4, 4, 4) == 0
+    mt, wn, wk, cp, split = Q.plan_query(A | Q.QL_PLAN_STAGED, M, N, K, dtype)
+    assert split > 1 and (entry is None) != ((mt, wn, wk, cp, split) == (1, 2, 4, 4, 4))
+    here = ctypes.create_string_buffer(64)
+    at = ctypes.addressof(here)
+    assert lib.ql_gemm_w8a8_dynq(dtype, at, at, 1, at, at, None, at, M, N, K, None, 0, None) != 0
+    tiles = -(-M // (32 * mt)) * -(-N // (32 * wn))
+    slabs = tiles * split * wn * mt * 16 * 64 * 4
+    need, slices = re.search(r"workspace of (\d+) bytes needed for split-K=(\d+)", lib.ql_last_error().decode()).groups()
+    assert int(slices) == split and int(need) == 65536 + slabs              # (a ticket for each of 16384 tiles in front)
+
+
+def test_what_a_query_of_staged_quantization_refuses(no_table):
+    import ctypes
+    lib, out = Q.load(), (ctypes.c_int * 5)()
+    for form in (Q.QL_PLAN_STAGED, A | S | Q.QL_PLAN_STAGED, A | R | Q.QL_PLAN_STAGED, A | Q.QL_PLAN_PARTIAL | Q.QL_PLAN_STAGED):
+        assert lib.ql_gemm_plan_of_call(form, I8, 0, 33, 8192, 12288, out) != 0
+    assert lib.ql_gemm_plan_set(A | Q.QL_PLAN_STAGED, 1, 32, 8192, 12288, 1, 2, 4, 4, 1) != 0
