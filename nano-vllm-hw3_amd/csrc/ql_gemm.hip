@@ -270,7 +270,7 @@ static double tile_cost(int tile, int64_t split, int64_t M, int64_t N, int64_t K
 }
 
 // The tile and slices that the costs say are faster than the rules' (`tile` in `split` slices) by more than they are wrong by; false: keep those.
-// On weights from memory 3978 random calls that change take 0.86 of the time, 43 of them more than 1.04 (the worst 1.19: 8-bit activations, 96 rows of
+// On weights from memory 3978 random calls that change take 0.86 of the time, 49 of them more than 1.04 (the worst 1.18: 8-bit activations, 96 rows of
 // 8608 x 12608).  The double-buffered tiles stay: the 64 x 128 one's costs go up and down with the number of tiles by more than the fit
 // shows, and mid_tile's lines come from sweeps of their own.
 // us, rules / here: fp8 x fp8 33 x 8192 of 12288 k 38.1 / 24.1, 64 x 6144 of 8192 k 22.3 / 16.4; int8 64 x 2048 of 12288 k 17.4 / 13.3; over all calls
