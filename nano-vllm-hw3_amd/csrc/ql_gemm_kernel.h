@@ -609,7 +609,8 @@ void qgemm_kernel(const GemmParams p) {
                 // made zero, and its activations are the even step's again (what lies behind them in LDS need not be finite).
                 // A lone step must not take the K = 16 pair: with products of both latencies in front of a join, the
                 // compiler counts the wait of the short one for the results of the long one, which were then read before
-                // they were whole (32 x 32 tile of 1024-k chunks, 33 x 100 x 544: about one call in a thousand wrong).
+                // they were whole (32 x 32 tile of 1024-k chunks, 33 x 100 x 544: about one call in a thousand wrong; tools/mfma_waits.py
+                // finds such reads in the assembly).
                 typedef int i32x8 __attribute__((ext_vector_type(8)));
                 if ((c & 1) == 0) {
                     w_even = w;
