@@ -1,6 +1,6 @@
 """Results of matrix instructions that are read too early, in the assembly of this package's own libraries (CPU only).
 
-    python tools/mfma_waits.py                                   # every kernel of the three libraries: some minutes
+    python tools/mfma_waits.py                                   # every kernel of the three libraries: a minute
     python tools/mfma_waits.py --lib path.so --kernels REGEX
 
 The vector unit may read what a matrix instruction writes a fixed number of wait states behind it, and it is the compiler that counts them.  Where
