@@ -408,7 +408,7 @@ static Plan make_plan(int64_t M, int64_t N, int64_t K, bool group, bool silu = f
         mt = 2; wn = 2; wk = 2; cp = 8;
         // beyond a round of those, 64 x 128 ones of 512-k chunks in one buffer, whose weights run on from chunk to chunk: 0.85 to 0.98 of the time at
         // 17408..32768 columns by 2112..3072 k (19456 x 2560 in fp8, 64 rows 19.1 / 16.1), from 4096 k on 0.87 to 0.99 at 64 rows, 0.97 to 1.06 at 33;
-        // up to 16384 columns 1.02 to 1.32
+        // up to 16384 columns 1.02 to 1.32.  (The one line inside a block of 32 rows: these plans have one slice, so no scratch depends on it.)
         if (N > 16384 && K > 2048 && (K < 4096 || M > 48)) { wn = 4; }
     }
     // a measured plan for this shape, if the table holds one (entries were checked when they were set); for calls that the wide tile is
@@ -712,7 +712,8 @@ size_t ql_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int granularity)
 size_t ql_gemm_workspace_max_bytes(int64_t max_M, int64_t N, int64_t K, int granularity) {
     if (max_M <= 0 || N <= 0 || K <= 0 || K % 32) return 0;
     // every threshold of the tile / split heuristics sits on a multiple of 32 rows and the tiles are multiples
-    // of 32 rows tall, so the plan is the same for all M of one 32-row block: its last M stands for the block
+    // of 32 rows tall, so the plan is the same for all M of one 32-row block: its last M stands for the block (but for gates under SiLU, which
+    // have a line at 48 rows and never more than the one slice that needs no scratch)
     size_t need = 0;
     for (int64_t m = 32;; m += 32) {
         const int64_t mm = m < max_M ? m : max_M;

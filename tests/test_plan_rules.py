@@ -233,3 +233,21 @@ def test_what_a_query_of_staged_quantization_refuses(no_table):
     for form in (Q.QL_PLAN_STAGED, A | S | Q.QL_PLAN_STAGED, A | R | Q.QL_PLAN_STAGED, A | Q.QL_PLAN_PARTIAL | Q.QL_PLAN_STAGED):
         assert lib.ql_gemm_plan_of_call(form, I8, 0, 33, 8192, 12288, out) != 0
     assert lib.ql_gemm_plan_set(A | Q.QL_PLAN_STAGED, 1, 32, 8192, 12288, 1, 2, 4, 4, 1) != 0
+
+
+@pytest.mark.parametrize("form", [S, S | A, S | G, S | NARROW, S | A | NARROW])
+def test_gates_under_silu_have_one_slice_by_the_rules(no_table, form):
+    """Their plans may change inside a block of 32 rows (at 48): the block's last row count need not stand for their scratch."""
+    for N, K in [(384, 256), (2048, 1024), (6144, 1024), (12288, 2048), (19456, 2560), (24576, 4096), (32768, 4096), (65536, 8192), (8192, 12288), (28672, 14336)]:
+        for dtype in (I8, F8):
+            for M in (1, 8, 16, 32, 33, 47, 48, 49, 64, 65, 96, 128, 129, 200, 256, 257, 512, 1024, 1025, 4096):
+                assert Q.plan_query(form, M, N, K, dtype)[4] == 1
+
+
+@pytest.mark.parametrize("form", [0, A, G, A | Q.QL_PLAN_STAGED])
+def test_one_plan_for_every_32_rows(no_table, form):
+    """Scratch is asked for by the last row count of 32, whatever the form (but gates under SiLU, above)."""
+    for N, K in [(1024, 2048), (4096, 1024), (4096, 4096), (2560, 9728), (18496, 2560), (24576, 4096), (8192, 12288), (1344, 7104), (3072, 3072)]:
+        for dtype in (I8, F8):
+            for last in (32, 64, 96, 128, 160, 224, 256, 288, 512):
+                assert len({Q.plan_query(form, M, N, K, dtype) for M in range(last - 31, last + 1)}) == 1
