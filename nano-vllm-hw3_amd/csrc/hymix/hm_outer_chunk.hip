@@ -11,9 +11,9 @@
 //
 // Precision: the stored q, k are bf16 and enter the products exactly; every float32 operand (S, N, R, P, W) enters as the sum of
 // three bf16 numbers, which is the number itself, and of the nine products of two such sums the six above 2^-24 of the result
-// are kept, the leading one in a sum of its own; sums are float32, products of decays double.  Against float64 the results are nearer
-// than the token-by-token walk's: 8 prompts of 900 to 1100 tokens, 16 heads: gated delta 128 x 128 o 2.6e-7 of its norm (walk 2.95e-7),
-// state 4.2e-7 (4.8e-7); state space 128 x 64 o 1.68e-7 (1.68e-7), state 3.19e-7 (3.25e-7).  A token that is not finite spoils
+// are kept, the leading one in a sum of its own (but for K^T W); sums are float32, products of decays double.  Against float64 the results are
+// nearer than the token-by-token walk's: 8 prompts of 900 to 1100 tokens, 8 heads, in norm: gated delta 128 x 128 o 1.30e-7 (walk 1.50e-7), state
+// 1.04e-7 (1.18e-7); state space 128 x 64 o 1.53e-7 (1.91e-7), state 1.41e-7 (1.86e-7).  A token that is not finite spoils
 // its own and later tokens, as in the walk, and none in front of it.
 //
 // The walk is one workgroup of 2 NW waves per (sequence, head, 16 NW value channels).  Wave w < NW keeps 16 columns of the state in the
@@ -24,12 +24,13 @@
 // from the strengths that it is handed through LDS.  One meeting per chunk.
 //
 // Against the walk that takes token after token, bound by the float32 vector unit and its chain of lane sums at two waves per
-// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 22 (prepare) + 72 (walk); one such prompt 9 + 49 us.
+// SIMD: 8 prompts of 900 to 1100 tokens, 16 heads of 128 x 128: 418 us there, here 22 (prepare) + 68 (walk); one such prompt 9 + 46 us.
 // What is left of a chunk's 3800 cycles: the chain S -> K S -> R -> W -> S of one wave, 380 vector instructions of 4.5 cycles (8 for a
 // conversion to bf16) and 85 matrix ones of 16, next to 3300 cycles of its partner, and LDS (58 KB per chunk and 16 columns).
 // With two waves of half the keys each on 32 columns, which both work out the strengths and give each other parts of the results in
-// LDS, the walk took 118 (one prompt: 90); one wave per SIMD with all of a chunk's work 99 (75); the state's terms handed on
-// through LDS so that the partner makes Q S too 85 (63: LDS is then the bound); results in double here as well 78 (57).
+// LDS, the walk took 118 (one prompt: 90).  Against 72 (49), with the state's sums apart: one wave per SIMD with all of a chunk's work 99 (75);
+// the state's terms handed on through LDS so that the partner makes Q S too 85 (63: LDS is then the bound); results in double here as
+// well 78 (57).
 #include "hm_attn_tile.h"
 #include "hm_outer.h"
 
@@ -606,12 +607,14 @@ __global__ __launch_bounds__(128 * NW) void outer_chunk_walk_kernel(const bf16_t
             for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    f32x4 ib = zeros4(), is = zeros4();
-                    is = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[2], is, 0, 0, 0);
-                    ib = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[0], ib, 0, 0, 0);
-                    is = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[1], is, 0, 0, 0);
+                    // (one sum from the smallest terms up: with the leading ones in a sum of their own, as above, the state was up to 2 % further
+                    // from float64, and the walk 2 to 5 % slower)
+                    f32x4 sum = zeros4();
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[2], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[1], sum, 0, 0, 0);
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[ks][half], d.v[0], sum, 0, 0, 0);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) S[ks][half][e] = end * S[ks][half][e] + (ib[e] + is[e]);
+                    for (int e = 0; e < 4; ++e) S[ks][half][e] = end * S[ks][half][e] + sum[e];
                 }
         });
         meet();
@@ -715,8 +718,12 @@ static void launch_chunks(const void* rows_, int64_t stride, int q_off, int k_of
                           int B, int H, int G, int D, int V, int max_q, hipStream_t s) {
     const bf16_t* rows = (const bf16_t*)rows_;
     // Four waves of columns share a chunk's K, Q and prepared part, two have a SIMD each and LDS to themselves: where every CU has at most one
-    // workgroup of two, those (one prompt of 900 tokens, 16 heads of 128 x 128: 49.5 us, four 52.2; 32 heads of 128 x 64 state space 39 and
-    // 48); beyond, a CU has room for one workgroup of either and four take half the rounds.
+    // workgroup of two, those (us of a call, 16 heads, portions of 1000 tokens, two / four: 128 x 128 delta 1 portion 59 / 62, state space 47 / 57).
+    // Beyond: with 128 keys a CU has LDS for one workgroup of either, and four take half the rounds (128 x 64, 12 portions, delta 124 / 88, state
+    // space 103 / 78).  With 64 keys two workgroups of two waves fit and take turns on its SIMDs, each loading its own K, Q and prepared part, where
+    // four waves have those once (64 x 64: 8 portions 59 / 65 and 46 / 58, 12 portions 83 / 73 and 65 / 61, 16 portions 90 / 80 and 70 / 67); from
+    // 513 to 768 workgroups of two, one round and a half of the four's, those are ahead once more (20 portions 121 / 123 and 96 / 106), beyond
+    // that behind (32 portions 171 / 152 and 132 / 129).
     const int nw = V % 64 == 0 && (int64_t)B * H * (V / 32) > 256 ? 4 : 2;
     const dim3 pg((unsigned)((max_q + kChunk - 1) / kChunk), (unsigned)B, (unsigned)H), wg((unsigned)B, (unsigned)H, (unsigned)(V / (16 * nw)));
 #define HM_CHUNKS(DK, NW)                                                                                                              \
