@@ -178,7 +178,7 @@ int hm_state_space(int dtype, const void* rows, int64_t stride, int x_off, int b
 
 /* The two recurrences above over portions of bf16 rows, 32 tokens at a time on the matrix cores; the same arguments, and scratch
  * `work` of hm_outer_chunk_work_bytes(T, B, H) bytes (16-byte aligned).  64 or 128 key channels (states), value channels a multiple
- * of 32; rows, stride and every part's offset on 16 bytes.  gates is not used and may be null. */
+ * of 32; rows, stride and every part's offset on 16 bytes.  gates is not used: null, or 16-byte aligned as above. */
 size_t hm_outer_chunk_work_bytes(int64_t T, int B, int H);
 int hm_gated_delta_chunks(const void* rows, int64_t stride, int q_off, int k_off, int v_off, const void* pre, int64_t pre_stride,
                           int b_off, int a_off, const float* A, const float* dt_bias, float unit_eps, float q_scale, float* gates,

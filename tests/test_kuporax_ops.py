@@ -185,15 +185,17 @@ def test_states_that_hardly_forget_through_portions(device, dtype, sizes):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["delta", "space"])
-@pytest.mark.parametrize("H,G,D,V", [(2, 1, 64, 32), (3, 3, 128, 32), (4, 2, 128, 128), (6, 2, 64, 160)])
-def test_portions_by_chunks_equal_the_walk(monkeypatch, kind, H, G, D, V):
+@pytest.mark.parametrize("H,G,D,V,copies", [(2, 1, 64, 32, 1), (3, 3, 128, 32, 1), (4, 2, 128, 128, 1), (6, 2, 64, 160, 1), (4, 2, 128, 128, 3),
+                                            (4, 4, 64, 64, 5)])
+def test_portions_by_chunks_equal_the_walk(monkeypatch, kind, H, G, D, V, copies):
     """32 tokens at a time and token after token: portions around one and two chunks, new ones and ones that continue a state, rows that
     are a column slice (and one too little aligned for chunks).  Both are float32 sums of exact operands: from the float64 recurrence
     they are within 16 roundings of 2^-24 in norm (D / 64 terms per lane and fold, up to four chunks' states).  A token that is
-    not finite leaves the tokens in front of it and the other portions as they are."""
+    not finite leaves the tokens in front of it and the other portions as they are.  Copies of the portions: workgroups of 64 value channels."""
     g = gen(D + V + H)
-    lens, of = [1, 31, 32, 33, 64, 2, 65, 97], torch.arange(H) // (H // G)
-    starts = [0, 40, 0, 7, 0, 3, 9, 0]
+    lens, of = [1, 31, 32, 33, 64, 2, 65, 97] * copies, torch.arange(H) // (H // G)
+    starts = [0, 40, 0, 7, 0, 3, 9, 0] * copies
+    assert (len(lens) * H * (V // 32) > 256) == (copies > 1)
     n, n_qk = sum(lens), 2 * G * D
     wide = rnd(g, n, n_qk + H * V + 16, dtype=torch.bfloat16)
     pre = rnd(g, n, 2 * H, s=2.0, dtype=torch.bfloat16).cuda()
@@ -249,9 +251,8 @@ def test_portions_by_chunks_equal_the_walk(monkeypatch, kind, H, G, D, V):
 @pytest.mark.parametrize("kind", ["delta", "space"])
 @pytest.mark.parametrize("H,D,V", [(24, 64, 64), (12, 128, 96)])
 def test_long_portions_by_chunks_keep_every_chunks_results(monkeypatch, kind, H, D, V):
-    """Portions of 8 to 47 chunks on more workgroups than the chip runs at once, several times: the two waves of a workgroup exchange
-    parts of a chunk's results, and a part of another chunk in their place is an error of the size of the results in half a chunk's
-    rows.  Every chunk's rows are within 32 roundings of 2^-24 of the walk's in norm (either is within 16 of the exact sums), and
+    """Portions of 8 to 47 chunks on more workgroups than the chip runs at once, several times: a wave hands its partner a chunk's strengths and the
+    state's part of its results, and those of another chunk in their place are an error of the size of the results.  Every chunk's rows are within 32 roundings of 2^-24 of the walk's in norm (either is within 16 of the exact sums), and
     every run gives the same bits."""
     g = gen(H + D)
     lens = [1500, 256, 1023, 777, 1337, 288, 640, 1024] * 3
