@@ -748,7 +748,7 @@ void qgemm_kernel(const GemmParams p) {
     // Qwen3-4B with fp8 weights 39.5 -> 38 us, with groups 46 -> 44.5), up to chunks of 1024 k with groups.  Int8 rows and 8-bit activations
     // need the steps' addresses worked out chunk by chunk (LEAN: kept over the loop they take 15 to 30 registers, and a workgroup per CU with them; that way
     // they gained nothing or lost up to 20 %): 0.84 to 0.93 of the time in the 32 x 64 and 64 x 64 tiles over three chunks and more,
-    // 0.95 to 0.98 in the 32 x 32 ones (936 calls, 1 to 256 rows, weights that no cache holds).  Not in the 32 x 32 tile of 1024-k chunks with
+    // 0.95 to 0.98 in the 32 x 32 ones (936 calls, 1 to 256 rows).  Not in the 32 x 32 tile of 1024-k chunks with
     // fp8 activations, which loses its third workgroup per CU (512 and more of them: 1.08), nor in the 64 x 64 tile with groups, which spills.
     // (STOP: int8 rows where stopping is the faster form all the same, see row_stops in ql_gemm.hip)
     // (an address past the slice's end is the last step's: step() skips what it brings)
