@@ -834,17 +834,18 @@ static int check_rope(const char* fn, const RopeArgs* r, int64_t M, int64_t N) {
 // int8 rows whose weights do not run on from chunk to chunk.  One or two rows on the 32 x 32 tile at more than one workgroup per CU: their activations
 // are there at once and the CU's other workgroup covers the stop (us, stops / runs on: 4096 x 12288 1 row 13.5 / 14.2, 2 rows 13.9 / 14.4, 4 rows
 // 15.0 / 14.6; 1 row of 2560 x 9728 10.4 / 10.7, 6176 x 9216 18.1 / 18.6; at up to one per CU 4096 x 9728 14.0 / 13.0, 6144 x 2560 7.8 / 7.3, at more
-// than four 12288 x 12288 36.1 / 35.5).  And the 32 x 64 tile's slices of one chunk, which have nothing to run on to (6144 x 1024 under SiLU, 1 row 4.9 / 5.0).
-static bool row_stops(const Plan& pl, int64_t M) {
+// than four 12288 x 12288 36.1 / 35.5; slices of one chunk 3968 x 3904 8.5 / 8.1).  And the 32 x 64 tile's slices of one whole chunk, which have
+// nothing to run on to (6144 x 1024 under SiLU, 1 row 4.9 / 5.0; one ragged chunk, 8832 x 896, 6.2 / 5.8: a step's bounds are branches there).
+static bool row_stops(const Plan& pl, int64_t M, int64_t K) {
     if (pl.mt == 1 && pl.wn == 1 && pl.wk == 8 && pl.cp == 4) {
         const int64_t groups = (int64_t)pl.grid.x * pl.grid.y * pl.grid.z;
-        return M <= 2 && groups > 256 && groups <= 1024;
+        return M <= 2 && pl.k_per_split > 1024 && groups > 256 && groups <= 1024;
     }
-    return pl.mt == 1 && pl.wn == 2 && pl.wk == 4 && pl.cp == 8 && pl.k_per_split <= 1024;
+    return pl.mt == 1 && pl.wn == 2 && pl.wk == 4 && pl.cp == 8 && pl.k_per_split <= 1024 && K % 1024 == 0;
 }
 
-static kern_t pick_i8_row(const Plan& pl, int64_t M, bool rope) {
-    return !rope && row_stops(pl, M) ? pick_bf16_i8_row_stop(pl.wn) : pick_bf16_i8_row(pl.mt, pl.wn, pl.wk, pl.cp, rope);
+static kern_t pick_i8_row(const Plan& pl, int64_t M, int64_t K, bool rope) {
+    return !rope && row_stops(pl, M, K) ? pick_bf16_i8_row_stop(pl.wn) : pick_bf16_i8_row(pl.mt, pl.wn, pl.wk, pl.cp, rope);
 }
 
 static int gemm_w8a16(const char* fn, bool silu, int wdtype, int granularity, const void* x, const void* qw,
@@ -907,7 +908,7 @@ static int gemm_w8a16(const char* fn, bool silu, int wdtype, int granularity, co
     } else if (pl.sk_G > 0) {
         if (wdtype == QL_INT8) k = grp ? pick_sk_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_sk_bf16_i8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);
         else k = grp ? pick_sk_bf16_fp8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_sk_bf16_fp8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);
-    } else if (wdtype == QL_INT8) k = grp ? pick_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_i8_row(pl, M, rp);
+    } else if (wdtype == QL_INT8) k = grp ? pick_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_i8_row(pl, M, K, rp);
     else k = grp ? pick_bf16_fp8_group(pl.mt, pl.wn, pl.wk, pl.cp, rp) : pick_bf16_fp8_row(pl.mt, pl.wn, pl.wk, pl.cp, rp);
     return run(k, p, pl, workspace, workspace_bytes, as_stream(stream), fn);
 }
@@ -1019,7 +1020,7 @@ int ql_gemm_w8a16_partial(int wdtype, int granularity, const void* x, const void
     p.partial_rm = partials;
     p.k_per_split = pl.k_per_split;
     kern_t k;
-    if (wdtype == QL_INT8) k = grp ? pick_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp) : pick_i8_row(pl, M, false);
+    if (wdtype == QL_INT8) k = grp ? pick_bf16_i8_group(pl.mt, pl.wn, pl.wk, pl.cp) : pick_i8_row(pl, M, K, false);
     else k = grp ? pick_bf16_fp8_group(pl.mt, pl.wn, pl.wk, pl.cp) : pick_bf16_fp8_row(pl.mt, pl.wn, pl.wk, pl.cp);
     if (!k) { set_error("%s: tile (%d,%d,%d,%d) not built", fn, pl.mt, pl.wn, pl.wk, pl.cp); return QL_EINVAL; }
     hipLaunchKernelGGL(k, pl.grid, dim3(64 * pl.wn * pl.wk), 0, as_stream(stream), p);
